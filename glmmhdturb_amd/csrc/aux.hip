@@ -20,12 +20,19 @@ template <typename T>
 hipError_t launch_ctot(Ptr9<const T> q9dev, size_t n, const Phys<T>& s, unsigned long long* out, hipStream_t st,
                        bool fast)
 {
-    if (fast) hipLaunchKernelGGL((ctot_kernel<T, true>), dim3(grid_for(n, AUX_NT, 4096)), dim3(AUX_NT), 0, st, q9dev, n, s, out);
-    else hipLaunchKernelGGL((ctot_kernel<T, false>), dim3(grid_for(n, AUX_NT, 4096)), dim3(AUX_NT), 0, st, q9dev, n, s, out);
+    if (fast) hipLaunchKernelGGL((ctot_kernel<T, true>), dim3(red_blocks(n)), dim3(AUX_NT), 0, st, q9dev, n, s, out);
+    else hipLaunchKernelGGL((ctot_kernel<T, false>), dim3(red_blocks(n)), dim3(AUX_NT), 0, st, q9dev, n, s, out);
     return hipGetLastError();
 }
 
-size_t diag_nparts(size_t n) { return (n + DIAG_CELLS_PER_BLOCK - 1) / DIAG_CELLS_PER_BLOCK; }
+// Cells of one diagnostics workgroup: 16384 from 256^3 on (which bounds the partials), fewer on smaller
+// grids so that about 1024 workgroups share them: with 16384 a 64^3 grid ran on 16 of the 256 CUs.
+static size_t diag_cells(size_t n)
+{
+    const size_t per = ((n + 1023) / 1024 + AUX_NT - 1) / AUX_NT * AUX_NT;
+    return per < DIAG_CELLS_PER_BLOCK ? per : DIAG_CELLS_PER_BLOCK;
+}
+size_t diag_nparts(size_t n) { const size_t per = diag_cells(n); return (n + per - 1) / per; }
 
 template <typename T>
 hipError_t launch_diag(Ptr9<const T> q9dev, int nx, int ny, int nz, double dx, double smallr, void* parts,
@@ -33,8 +40,8 @@ hipError_t launch_diag(Ptr9<const T> q9dev, int nx, int ny, int nz, double dx, d
 {
     size_t n = (size_t)nx * ny * nz, np = diag_nparts(n);
     hipLaunchKernelGGL((diag_partial_kernel<T>), dim3((unsigned)np), dim3(AUX_NT), 0, st, q9dev, nx, ny, nz, dx, smallr,
-                       (size_t)DIAG_CELLS_PER_BLOCK, (DiagPart*)parts);
-    hipLaunchKernelGGL(diag_final_kernel, dim3(1), dim3(1), 0, st, (const DiagPart*)parts, (int)np, out);
+                       diag_cells(n), (DiagPart*)parts);
+    hipLaunchKernelGGL(diag_final_kernel, dim3(1), dim3(AUX_NT), 0, st, (const DiagPart*)parts, (int)np, out);
     return hipGetLastError();
 }
 

@@ -1,6 +1,6 @@
 // aux_impl.hpp -- reductions and initial-condition kernels for gfx950.
 #pragma once
-#include "physics.hpp"
+#include "gpu_util.hpp"
 
 namespace glm {
 
@@ -14,28 +14,22 @@ GLM_DEV int awrap(int i, int n)
 
 // ---------------------------------------------------------------------------------------------
 // CFL: max over cells of sum_d(|v_d| + c_f(B_d))  (glmmhd_turb.jl:1963-1978), or with FAST the max
-// over cells of max_d c_f(B_d) (the "max fast speed" cleaning speed).  One atomic per wavefront on
-// the bit pattern of a non-negative double (NaN compares largest).
+// over cells of max_d c_f(B_d) (the "max fast speed" cleaning speed), on the bit pattern of a
+// non-negative double (NaN compares largest).
 // ---------------------------------------------------------------------------------------------
 template <typename T, bool FAST>
 __global__ void __launch_bounds__(AUX_NT) ctot_kernel(Ptr9<const T> q9, size_t n, Phys<T> s, unsigned long long* out)
 {
-    double cmax = 0.0;
+    unsigned long long best = 0ull;
     for (size_t c = (size_t)blockIdx.x * AUX_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * AUX_NT) {
         T u[9], p[9];
 #pragma unroll
         for (int v = 0; v < 9; ++v) u[v] = q9[v][c];
         cons2prim(u, p, s);
-        double ct = FAST ? fast_max_speed(p, s) : cfl_speed(p, s);
-        if (!(ct <= cmax)) cmax = ct;
+        const unsigned long long b = (unsigned long long)__double_as_longlong(FAST ? fast_max_speed(p, s) : cfl_speed(p, s));
+        best = b > best ? b : best;
     }
-    unsigned long long bits = (unsigned long long)__double_as_longlong(cmax);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        unsigned long long o = __shfl_xor(bits, off, 64);
-        bits = o > bits ? o : bits;
-    }
-    if ((threadIdx.x & 63) == 0 && bits != 0ull) atomicMax(out, bits);
+    block_max_bits<AUX_NT>(best, out);
 }
 
 __global__ void clear_u64_kernel(unsigned long long* p, int n)
@@ -74,6 +68,36 @@ struct DiagPart {
     KSum sum[NDSUM];
     double divb, rhomin, finite;
 };
+GLM_DEV DiagPart diag_empty()
+{
+    DiagPart d;
+#pragma unroll
+    for (int k = 0; k < NDSUM; ++k) d.sum[k] = KSum{0.0, 0.0};
+    d.divb = 0.0; d.rhomin = INFINITY; d.finite = 1.0;
+    return d;
+}
+GLM_DEV void diag_merge(DiagPart& x, const DiagPart& y)
+{
+#pragma unroll
+    for (int k = 0; k < NDSUM; ++k) x.sum[k] = kmerge(x.sum[k], y.sum[k]);
+    x.divb = fmax(x.divb, y.divb);
+    x.rhomin = fmin(x.rhomin, y.rhomin);
+    x.finite = fmin(x.finite, y.finite);
+}
+// The workgroup's partials combined in a fixed tree; the result is in sh[0].
+GLM_DEV void diag_tree(DiagPart* sh, const DiagPart& d)
+{
+    sh[threadIdx.x] = d;
+    __syncthreads();
+    for (int w = AUX_NT / 2; w >= 1; w >>= 1) {
+        if ((int)threadIdx.x < w) {
+            DiagPart x = sh[threadIdx.x];
+            diag_merge(x, sh[threadIdx.x + w]);
+            sh[threadIdx.x] = x;
+        }
+        __syncthreads();
+    }
+}
 
 template <typename T>
 __global__ void __launch_bounds__(AUX_NT) diag_partial_kernel(Ptr9<const T> q9, int nx, int ny, int nz, double dx,
@@ -83,18 +107,17 @@ __global__ void __launch_bounds__(AUX_NT) diag_partial_kernel(Ptr9<const T> q9, 
     const size_t n = (size_t)nx * ny * nz;
     const size_t c0 = (size_t)blockIdx.x * cells_per_block;
     const size_t c1 = c0 + cells_per_block < n ? c0 + cells_per_block : n;
-    DiagPart d;
-#pragma unroll
-    for (int k = 0; k < NDSUM; ++k) d.sum[k] = KSum{0.0, 0.0};
-    d.divb = 0.0; d.rhomin = INFINITY; d.finite = 1.0;
-    for (size_t c = c0 + threadIdx.x; c < c1; c += AUX_NT) {
-        int i = (int)(c % nx), j = (int)((c / nx) % ny), k = (int)(c / ((size_t)nx * ny));
+    DiagPart d = diag_empty();
+    CellWalk w(c0 + threadIdx.x, AUX_NT, nx, ny);
+    for (size_t c = c0 + threadIdx.x; c < c1; c += AUX_NT, w.next()) {
+        const int i = w.i, j = w.j, k = w.k;
         double r = q9[0][c], a = q9[1][c], b = q9[2][c], e = q9[3][c];
         double m2 = a * a + b * b + e * e;
         double Bx = q9[5][c], By = q9[6][c], Bz = q9[7][c];
         kadd(d.sum[0], r);
-        kadd(d.sum[1], m2 / fmax(r, smallr));
-        kadd(d.sum[2], 0.5 * m2 / r);
+        const double mr = m2 / r;   // halving is exact, and fmax(r, smallr) is r outside floored cells
+        kadd(d.sum[1], r >= smallr ? mr : m2 / fmax(r, smallr));
+        kadd(d.sum[2], 0.5 * mr);
         kadd(d.sum[3], 0.5 * (Bx * Bx + By * By + Bz * Bz));
         kadd(d.sum[4], (a * Bx + b * By + e * Bz) / r);
         kadd(d.sum[5], (double)q9[4][c]);
@@ -114,34 +137,21 @@ __global__ void __launch_bounds__(AUX_NT) diag_partial_kernel(Ptr9<const T> q9, 
         for (int v = 0; v < 9; ++v)
             if (!isfinite((double)q9[v][c])) d.finite = 0.0;
     }
-    sh[threadIdx.x] = d;
-    __syncthreads();
-    for (int w = AUX_NT / 2; w >= 1; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            DiagPart x = sh[threadIdx.x], y = sh[threadIdx.x + w];
-#pragma unroll
-            for (int k = 0; k < NDSUM; ++k) x.sum[k] = kmerge(x.sum[k], y.sum[k]);
-            x.divb = fmax(x.divb, y.divb);
-            x.rhomin = fmin(x.rhomin, y.rhomin);
-            x.finite = fmin(x.finite, y.finite);
-            sh[threadIdx.x] = x;
-        }
-        __syncthreads();
-    }
+    diag_tree(sh, d);
     if (threadIdx.x == 0) parts[blockIdx.x] = sh[0];
 }
 
-__global__ void diag_final_kernel(const DiagPart* parts, int nparts, double* out)
+// The block partials combined by one workgroup: thread t takes partials t, t + 256, ... in order, then
+// the fixed tree of diag_partial_kernel.  (One thread walking all partials in order waited for every
+// load in turn: 483 us for the 1024 partials of 256^3, twice the partial pass.)
+__global__ void __launch_bounds__(AUX_NT) diag_final_kernel(const DiagPart* parts, int nparts, double* out)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    DiagPart d = parts[0];
-    for (int b = 1; b < nparts; ++b) {
-        DiagPart y = parts[b];
-        for (int k = 0; k < NDSUM; ++k) d.sum[k] = kmerge(d.sum[k], y.sum[k]);
-        d.divb = fmax(d.divb, y.divb);
-        d.rhomin = fmin(d.rhomin, y.rhomin);
-        d.finite = fmin(d.finite, y.finite);
-    }
+    __shared__ DiagPart sh[AUX_NT];
+    DiagPart d = diag_empty();
+    for (int b = (int)threadIdx.x; b < nparts; b += AUX_NT) diag_merge(d, parts[b]);
+    diag_tree(sh, d);
+    if (threadIdx.x != 0) return;
+    d = sh[0];
     // out: mass, ke2, divbmax, rhomin, finite, ekin, emag, cross helicity, etot, psi2
     out[0] = d.sum[0].s + d.sum[0].c;
     out[1] = d.sum[1].s + d.sum[1].c;

@@ -3,6 +3,7 @@
 #include "ct_march.hpp"
 #include "ct_tile.hpp"
 #include "ct_launch.hpp"
+#include "aux_launch.hpp"
 
 namespace glm {
 
@@ -47,7 +48,7 @@ hipError_t launch_ct_step(void* const* q, void* const* o, const CTArgsHost& h, v
     if (e != hipSuccess || !h.want_cfl) return e;
     Ptr9<const T> o9;
     for (int v = 0; v < 9; ++v) o9.p[v] = v < 8 ? (const T*)o[v] : nullptr;
-    hipLaunchKernelGGL((ct_ctot_kernel<T>), dim3(2048), b, 0, st, o9, h.nx, h.ny, h.nz, (T)h.gamma, (T)h.smallr,
+    hipLaunchKernelGGL((ct_ctot_kernel<T>), dim3(red_blocks((size_t)h.nx * h.ny * h.nz)), b, 0, st, o9, h.nx, h.ny, h.nz, (T)h.gamma, (T)h.smallr,
                        (T)h.smallp, h.cmax);
     return hipGetLastError();
 }
@@ -66,7 +67,7 @@ hipError_t launch_ct_tiles(void* const* q, void* const* o, const CTArgsHost& h, 
     if (e != hipSuccess || !h.want_cfl) return e;
     Ptr9<const T> o9;
     for (int v = 0; v < 9; ++v) o9.p[v] = v < 8 ? (const T*)o[v] : nullptr;
-    hipLaunchKernelGGL((ct_ctot_kernel<T>), dim3(2048), dim3(CT_NT), 0, st, o9, h.nx, h.ny, h.nz, (T)h.gamma,
+    hipLaunchKernelGGL((ct_ctot_kernel<T>), dim3(red_blocks((size_t)h.nx * h.ny * h.nz)), dim3(CT_NT), 0, st, o9, h.nx, h.ny, h.nz, (T)h.gamma,
                        (T)h.smallr, (T)h.smallp, h.cmax);
     return hipGetLastError();
 }
@@ -124,7 +125,7 @@ hipError_t launch_ct_march(void* const* q, void* const* o, const CTArgsHost& h, 
     if (e != hipSuccess || !h.want_cfl) return e;
     Ptr9<const T> o9;
     for (int v = 0; v < 9; ++v) o9.p[v] = v < 8 ? (const T*)o[v] : nullptr;
-    hipLaunchKernelGGL((ct_ctot_kernel<T>), dim3(2048), dim3(CT_NT), 0, st, o9, h.nx, h.ny, h.nz, (T)h.gamma,
+    hipLaunchKernelGGL((ct_ctot_kernel<T>), dim3(red_blocks((size_t)h.nx * h.ny * h.nz)), dim3(CT_NT), 0, st, o9, h.nx, h.ny, h.nz, (T)h.gamma,
                        (T)h.smallr, (T)h.smallp, h.cmax);
     return hipGetLastError();
 }
@@ -135,7 +136,7 @@ hipError_t launch_ct_ctot(void* const* q, int nx, int ny, int nz, double gamma, 
 {
     Ptr9<const T> q9;
     for (int v = 0; v < 9; ++v) q9.p[v] = v < 8 ? (const T*)q[v] : nullptr;
-    hipLaunchKernelGGL((ct_ctot_kernel<T>), dim3(2048), dim3(CT_NT), 0, st, q9, nx, ny, nz, (T)gamma, (T)smallr,
+    hipLaunchKernelGGL((ct_ctot_kernel<T>), dim3(red_blocks((size_t)nx * ny * nz)), dim3(CT_NT), 0, st, q9, nx, ny, nz, (T)gamma, (T)smallr,
                        (T)smallp, out);
     return hipGetLastError();
 }
@@ -145,7 +146,7 @@ hipError_t launch_ct_divb(void* const* q, int nx, int ny, int nz, double dx, uns
 {
     Ptr9<const T> q9;
     for (int v = 0; v < 9; ++v) q9.p[v] = v < 8 ? (const T*)q[v] : nullptr;
-    hipLaunchKernelGGL((ct_divb_kernel<T>), dim3(2048), dim3(CT_NT), 0, st, q9, nx, ny, nz, dx, out);
+    hipLaunchKernelGGL((ct_divb_kernel<T>), dim3(red_blocks((size_t)nx * ny * nz)), dim3(CT_NT), 0, st, q9, nx, ny, nz, dx, out);
     return hipGetLastError();
 }
 

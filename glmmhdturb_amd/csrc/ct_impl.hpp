@@ -7,7 +7,7 @@
 // (4) the hydro update (:124-136) and the face-B curl update (:156-171) in one kernel, with the
 // optional floor / OU kick / next-step CFL folded in.
 #pragma once
-#include "physics.hpp"
+#include "gpu_util.hpp"
 
 namespace glm {
 
@@ -361,9 +361,11 @@ __global__ void __launch_bounds__(CT_NT) ct_ctot_kernel(Ptr9<const T> q, int nx,
                                                         T smallp, unsigned long long* out)
 {
     size_t n = (size_t)nx * ny * nz;
-    T cmax = T(0);
-    for (size_t c = (size_t)blockIdx.x * CT_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * CT_NT) {
-        int i = (int)(c % nx), j = (int)((c / nx) % ny), k = (int)(c / ((size_t)nx * ny));
+    unsigned long long best = 0ull;
+    const size_t c0 = (size_t)blockIdx.x * CT_NT + threadIdx.x, step = (size_t)gridDim.x * CT_NT;
+    CellWalk w(c0, step, nx, ny);
+    for (size_t c = c0; c < n; c += step, w.next()) {
+        const int i = w.i, j = w.j, k = w.k;
         size_t pl = (size_t)nx * ny;
         T bx = T(0.5) * (q[5][c] + q[5][(size_t)cwrap(i + 1, nx) + (size_t)nx * j + pl * k]);
         T by = T(0.5) * (q[6][c] + q[6][(size_t)i + (size_t)nx * cwrap(j + 1, ny) + pl * k]);
@@ -375,15 +377,10 @@ __global__ void __launch_bounds__(CT_NT) ct_ctot_kernel(Ptr9<const T> q, int nx,
                    smallp);
         T p8[8] = {rho, vx, vy, vz, p, bx, by, bz};
         T ct = (tabs(vx) + ct_cf(p8, bx, gamma)) + (tabs(vy) + ct_cf(p8, by, gamma)) + (tabs(vz) + ct_cf(p8, bz, gamma));
-        if (!(ct <= cmax)) cmax = ct;
+        const unsigned long long b = (unsigned long long)__double_as_longlong((double)ct);
+        best = b > best ? b : best;
     }
-    unsigned long long bits = (unsigned long long)__double_as_longlong((double)cmax);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        unsigned long long o = __shfl_xor(bits, off, 64);
-        bits = o > bits ? o : bits;
-    }
-    if ((threadIdx.x & 63) == 0 && bits != 0ull) atomicMax(out, bits);
+    block_max_bits<CT_NT>(best, out);
 }
 
 // max |div B| from face fields (ct_mhd.jl:191-194)
@@ -392,23 +389,19 @@ __global__ void __launch_bounds__(CT_NT) ct_divb_kernel(Ptr9<const T> q, int nx,
                                                         unsigned long long* out)
 {
     size_t n = (size_t)nx * ny * nz;
-    double m = 0.0;
-    for (size_t c = (size_t)blockIdx.x * CT_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * CT_NT) {
-        int i = (int)(c % nx), j = (int)((c / nx) % ny), k = (int)(c / ((size_t)nx * ny));
+    unsigned long long best = 0ull;
+    const size_t c0 = (size_t)blockIdx.x * CT_NT + threadIdx.x, step = (size_t)gridDim.x * CT_NT;
+    CellWalk w(c0, step, nx, ny);
+    for (size_t c = c0; c < n; c += step, w.next()) {
+        const int i = w.i, j = w.j, k = w.k;
         size_t pl = (size_t)nx * ny;
         double d = (((double)q[5][(size_t)cwrap(i + 1, nx) + (size_t)nx * j + pl * k] - (double)q[5][c]) +
                     ((double)q[6][(size_t)i + (size_t)nx * cwrap(j + 1, ny) + pl * k] - (double)q[6][c]) +
                     ((double)q[7][(size_t)i + (size_t)nx * j + pl * cwrap(k + 1, nz)] - (double)q[7][c])) / dx;
-        d = fabs(d);
-        if (!(d <= m)) m = d;
+        const unsigned long long b = (unsigned long long)__double_as_longlong(fabs(d));
+        best = b > best ? b : best;
     }
-    unsigned long long bits = (unsigned long long)__double_as_longlong(m);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        unsigned long long o = __shfl_xor(bits, off, 64);
-        bits = o > bits ? o : bits;
-    }
-    if ((threadIdx.x & 63) == 0 && bits != 0ull) atomicMax(out, bits);
+    block_max_bits<CT_NT>(best, out);
 }
 
 }  // namespace glm
