@@ -63,7 +63,7 @@ static bool dispatch_faceswise(const AdjArgs& a, dim3 g, hipStream_t st, bool up
 static bool dispatch_back(const AdjArgs& a, int zchunk, hipStream_t st, int pred, int recon, int slope)
 {
     int tx, ty, nzc, zc;
-    march_tiling(a.nx, a.ny, a.nz, zchunk, 256, tx, ty, nzc, zc);   // one workgroup per CU
+    march_tiling<double>(a.nx, a.ny, a.nz, zchunk, Resident{}, tx, ty, nzc, zc);   // one workgroup per CU
     const dim3 g((unsigned)(tx * ty * nzc));
 #define GLM_CASE(P, RC, SL)                                                                          \
     if (pred == P && recon == RC && slope == SL) {                                                   \

@@ -70,6 +70,24 @@ static bool planes_alias(void* const* a, int na, void* const* b, int nb)
 // ------------------------------------------------------------------------------------------
 // context
 // ------------------------------------------------------------------------------------------
+// A kernel's concurrent workgroups, with the scheme key they were asked for (0: none yet).
+struct ResidentOf {
+    int key;
+    Resident r;
+};
+
+static int resident_of(const void* fn, int threads, int key, ResidentOf& out)
+{
+    int dev = 0, cus = 0, occ = 0;
+    HIPCHK(hipGetDevice(&dev));
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, threads, 0));
+    out.r.cus = cus;
+    out.r.occ = occ > 0 ? occ : 1;
+    out.key = key;
+    return GLM_OK;
+}
+
 struct glm_ctx {
     int nx, ny, nz, prec;
     size_t n;
@@ -90,13 +108,8 @@ struct glm_ctx {
     // reverse step: scratch and the forcing-adjoint accumulator
     void* adj_scratch;
     double* d_fdot;
-    // concurrent march workgroups (CUs x resident workgroups per CU) of the last march variant
-    int slots_key;
-    int slots;
-    int ct_slots_key;
-    int ct_slots;
-    int hydro_slots_key;
-    int hydro_slots;
+    // concurrent march workgroups of the last march variant of each kind
+    ResidentOf march_res, ct_res, hydro_res;
 };
 
 static void ctx_free(glm_ctx* c)
@@ -144,8 +157,7 @@ glm_ctx* glm_create(int nx, int ny, int nz, int precision)
         set_err(GLM_ERR_ARG, "glm_create: grid must be >= 1 per axis and precision 8 or 4");
         return nullptr;
     }
-    glm_ctx* c = new glm_ctx();
-    memset(c, 0, sizeof *c);
+    glm_ctx* c = new glm_ctx();   // every field zero
     c->nx = nx; c->ny = ny; c->nz = nz; c->prec = precision;
     c->n = (size_t)nx * ny * nz;
     c->stream = nullptr;
@@ -194,17 +206,12 @@ static int step_impl(glm_ctx* c, void* const* q, void* const* o, const glm_param
     if (planes_alias(q, nv, o, nv)) return set_err(GLM_ERR_ARG, "glm_step: input and output planes must differ");
     a.nx = c->nx; a.ny = c->ny; a.nz = c->nz;
     const int key = floor ? -1 : 1 + (((p->predictor * 4 + p->riemann) * 4 + p->recon) * 4 + p->slope) + 1000 * nsp;
-    if (c->slots_key != key) {
-        int dev = 0, cus = 0, occ = 0;
+    if (c->march_res.key != key) {
         const void* fn = floor ? march_floor_ptr<T>() : march_kernel_ptr<T>(p->predictor, p->riemann, p->recon, p->slope, nsp);
         if (!fn) return set_err(GLM_ERR_ARG, "glm_step: unknown scheme");
-        HIPCHK(hipGetDevice(&dev));
-        HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, NT, 0));
-        c->slots = cus * (occ > 0 ? occ : 1);
-        c->slots_key = key;
+        if (int e = resident_of(fn, NT, key, c->march_res)) return e;
     }
-    march_tiling(c->nx, c->ny, c->nz, p->zchunk, c->slots, a.tiles_x, a.tiles_y, a.nzc, a.zchunk);
+    march_tiling<T>(c->nx, c->ny, c->nz, p->zchunk, c->march_res.r, a.tiles_x, a.tiles_y, a.nzc, a.zchunk);
     a.ph = make_phys<T>(p);
     double dtdx = p->dt / p->dx;
     a.dtdx = (T)dtdx;
@@ -578,19 +585,14 @@ static int ct_step_impl(glm_ctx* ctx, void* const* q, void* const* o, const glm_
     } else if (mode == CT_MARCH) {
         const int ppm = p->recon == GLM_RECON_PPM_SPIKE;
         const int key = 1000 + p->riemann + 10 * nsp + 100 * ppm;
-        if (ctx->ct_slots_key != key) {
-            int dev = 0, cus = 0, occ = 0;
+        if (ctx->ct_res.key != key) {
             const void* fn = ctx->prec == 8 ? ct_march_ptr<double>(p->riemann, nsp, p->recon)
                                             : ct_march_ptr<float>(p->riemann, nsp, p->recon);
             if (!fn) return set_err(GLM_ERR_ARG, "glm_ct_step: unknown Riemann solver");
-            HIPCHK(hipGetDevice(&dev));
-            HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, CT_MARCH_THREADS, 0));
-            ctx->ct_slots = cus * (occ > 0 ? occ : 1);
-            ctx->ct_slots_key = key;
+            if ((e = resident_of(fn, CT_MARCH_THREADS, key, ctx->ct_res))) return e;
         }
-        if (ctx->prec == 8) HIPCHK(launch_ct_march<double>(q, o, h, ctx->ct_slots, ctx->stream));
-        else HIPCHK(launch_ct_march<float>(q, o, h, ctx->ct_slots, ctx->stream));
+        if (ctx->prec == 8) HIPCHK(launch_ct_march<double>(q, o, h, ctx->ct_res.r, ctx->stream));
+        else HIPCHK(launch_ct_march<float>(q, o, h, ctx->ct_res.r, ctx->stream));
     } else {
         if (ctx->prec == 8) HIPCHK(launch_ct_step<double>(q, o, h, ctx->ct_scratch, ctx->stream));
         else HIPCHK(launch_ct_step<float>(q, o, h, ctx->ct_scratch, ctx->stream));
@@ -699,19 +701,14 @@ static int hydro_step_impl(glm_ctx* ctx, void* const* q, void* const* o, const g
     }
     if (h.scheme != 0) h.fallback = 0;   // those builds solve HLL without the fallback (spike_25d.cu:445-483)
     const int key = 2000 + h.fallback + 2 * nsp + 8 * h.cma + 16 * fmt + 128 * h.scheme;
-    if (ctx->hydro_slots_key != key) {
-        int dev = 0, cus = 0, occ = 0;
+    if (ctx->hydro_res.key != key) {
         const void* fn = ctx->prec == 8 ? hydro_march_ptr<double>(h.fallback, nsp, h.cma, fmt, h.scheme)
                                         : hydro_march_ptr<float>(h.fallback, nsp, h.cma, fmt, h.scheme);
         if (!fn) return set_err(GLM_ERR_ARG, "hydro step: no kernel for this format and precision");
-        HIPCHK(hipGetDevice(&dev));
-        HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, HYDRO_THREADS, 0));
-        ctx->hydro_slots = cus * (occ > 0 ? occ : 1);
-        ctx->hydro_slots_key = key;
+        if (int e = resident_of(fn, HYDRO_THREADS, key, ctx->hydro_res)) return e;
     }
-    if (ctx->prec == 8) HIPCHK(launch_hydro_march<double>(q, o, h, ctx->hydro_slots, ctx->stream));
-    else HIPCHK(launch_hydro_march<float>(q, o, h, ctx->hydro_slots, ctx->stream));
+    if (ctx->prec == 8) HIPCHK(launch_hydro_march<double>(q, o, h, ctx->hydro_res.r, ctx->stream));
+    else HIPCHK(launch_hydro_march<float>(q, o, h, ctx->hydro_res.r, ctx->stream));
     return GLM_OK;
 }
 

@@ -99,7 +99,7 @@ const void* ct_march_ptr(int riemann, int nsp, int recon)
 }
 
 template <typename T>
-hipError_t launch_ct_march(void* const* q, void* const* o, const CTArgsHost& h, int slots, hipStream_t st)
+hipError_t launch_ct_march(void* const* q, void* const* o, const CTArgsHost& h, const Resident& res, hipStream_t st)
 {
     if (h.nsp != 0 && h.nsp != 2) return hipErrorInvalidValue;
     CTMArgs<T> a;
@@ -108,7 +108,7 @@ hipError_t launch_ct_march(void* const* q, void* const* o, const CTArgsHost& h, 
         a.o[v] = v < 8 + h.nsp ? (T*)o[v] : nullptr;
     }
     a.nx = h.nx; a.ny = h.ny; a.nz = h.nz;
-    ct_march_tiling(h.nx, h.ny, h.nz, h.zchunk, slots, a.tiles_x, a.tiles_y, a.nzc, a.zchunk);
+    ct_march_tiling<T>(h.nx, h.ny, h.nz, h.zchunk, res, a.tiles_x, a.tiles_y, a.nzc, a.zchunk);
     a.gamma = (T)h.gamma; a.igm1 = (T)(1.0 / (h.gamma - 1.0)); a.smallr = (T)h.smallr; a.smallp = (T)h.smallp;
     double dtdx = h.dt / h.dx;
     a.dtdx = (T)dtdx; a.half_dtdx = (T)(0.5 * dtdx); a.dt = (T)h.dt; a.dx = (T)h.dx;
@@ -163,7 +163,7 @@ const void* ct_kernel_ptr()
     template hipError_t launch_ct_divb<T>(void* const*, int, int, int, double, unsigned long long*, hipStream_t); \
     template const void* ct_kernel_ptr<T>();                                                                    \
     template const void* ct_march_ptr<T>(int, int, int);                                                        \
-    template hipError_t launch_ct_march<T>(void* const*, void* const*, const CTArgsHost&, int, hipStream_t);   \
+    template hipError_t launch_ct_march<T>(void* const*, void* const*, const CTArgsHost&, const Resident&, hipStream_t);   \
     template hipError_t launch_ct_tiles<T>(void* const*, void* const*, const CTArgsHost&, hipStream_t);        \
     template const void* ct_tile_ptr<T>();
 GLM_CT_INST(double)

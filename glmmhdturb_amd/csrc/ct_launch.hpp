@@ -1,6 +1,7 @@
 // ct_launch.hpp -- host launchers of the constrained-transport kernels (ct.hip).
 #pragma once
 #include <hip/hip_runtime.h>
+#include "tiling.hpp"
 #include <stddef.h>
 
 namespace glm {
@@ -28,7 +29,7 @@ template <typename T>
 const void* ct_kernel_ptr();
 // Fused CT step (one z-march kernel) and its kernel for a Riemann solver (occupancy queries).
 template <typename T>
-hipError_t launch_ct_march(void* const* q, void* const* o, const CTArgsHost& h, int slots, hipStream_t st);
+hipError_t launch_ct_march(void* const* q, void* const* o, const CTArgsHost& h, const Resident& res, hipStream_t st);
 template <typename T>
 const void* ct_march_ptr(int riemann, int nsp = 0, int recon = 0);
 // The same step as one kernel over staged 3-D tiles (ct_tile.hpp) and that kernel (resource queries).

@@ -27,6 +27,7 @@
 #include "ct_launch.hpp"
 #include "force.hpp"
 #include "gpu_util.hpp"
+#include "tiling.hpp"
 
 namespace glm {
 
@@ -129,31 +130,12 @@ GLM_DEV void cm_prim(const CTMArgs<T>& a, int x, int y, int z, T p[NV])
     for (int v = 8; v < NV; ++v) p[v] = u[v] * ir;
 }
 
-// Tiles and z-chunks of the CT march on `slots` concurrent workgroups: rounds x (chunk + 2 lead-in
-// planes), the same model as the GLM march's (launch.hpp march_tiling) with its longer lead-in.
-inline void ct_march_tiling(int nx, int ny, int nz, int zchunk_req, int slots, int& tiles_x, int& tiles_y, int& nzc,
-                            int& zchunk)
+// Tiles and z-chunks of the CT march (lead-in: two whole planes of face states and fluxes).
+template <typename T>
+inline void ct_march_tiling(int nx, int ny, int nz, int zchunk_req, const Resident& r, int& tiles_x, int& tiles_y,
+                            int& nzc, int& zchunk)
 {
-    tiles_x = (nx + CM_OX - 1) / CM_OX;
-    tiles_y = (ny + CM_OY - 1) / CM_OY;
-    if (zchunk_req > 0) {
-        zchunk = zchunk_req < nz ? zchunk_req : nz;
-        nzc = (nz + zchunk - 1) / zchunk;
-        return;
-    }
-    const long cols = (long)tiles_x * tiles_y;
-    const long sl = slots > 0 ? slots : 256;
-    const int maxc = nz / 8 > 1 ? nz / 8 : 1;
-    long best = -1;
-    zchunk = nz;
-    for (int c = 1; c <= maxc; ++c) {
-        const int zc = (nz + c - 1) / c;
-        const int n = (nz + zc - 1) / zc;
-        if (n != c) continue;
-        const long cost = ((cols * n + sl - 1) / sl) * (long)(zc + 2);
-        if (best < 0 || cost < best) { best = cost; zchunk = zc; }
-    }
-    nzc = (nz + zchunk - 1) / zchunk;
+    march_tiles(nx, ny, nz, CM_OX, CM_OY, zchunk_req, r, 2.0, sizeof(T) == 8 ? 0.7 : 0.38, tiles_x, tiles_y, nzc, zchunk);
 }
 
 // One step of the CT state with NS passive species (spike_ctm.cu -DNSP: their fluxes ride the

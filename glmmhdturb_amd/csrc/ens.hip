@@ -103,7 +103,7 @@ struct glm_ens {
     std::vector<OUBox> ou;
     hipStream_t stream;
     int any_turb, gmax, nbmax;
-    int cu_count;
+    Resident res;          // concurrent march workgroups
     double clock_khz;
     // device tables
     EnsBox* d_eb;
@@ -143,13 +143,32 @@ void ens_free(glm_ens* e)
     delete e;
 }
 
-// z planes per tile of a box under the configured zchunk (0: automatic, about 32 planes).
-int box_zchunk(int nz, int zreq)
+// z planes per tile of a box for chunks of about z planes: the box's planes shared evenly.
+int box_zchunk(int nz, int z)
 {
-    int z = zreq > 0 ? zreq : 32;
     if (z > nz) z = nz;
     const int nzc = (nz + z - 1) / z;
     return (nz + nzc - 1) / nzc;
+}
+
+// The automatic chunk length: one for all boxes, by the model of the single-grid march over the
+// whole tile list.  (Chunks of 32 planes gave 16 boxes of 32^3..64^3 396 workgroups, of which 140 shared a
+// CU: 512 us a sweep.)
+int ens_zchunk(const glm_ens* e)
+{
+    int nzmax = 1, best = 1;
+    for (const glm_ens_box& x : e->box) nzmax = std::max(nzmax, x.nz);
+    double least = -1.0;
+    for (int z = nzmax; z >= 1; --z) {
+        long W = 0;
+        for (const glm_ens_box& x : e->box) {
+            const int zc = box_zchunk(x.nz, z);
+            W += (long)((x.nx + OX - 1) / OX) * ((x.ny + OY - 1) / OY) * ((x.nz + zc - 1) / zc);
+        }
+        const double t = chunk_cost(W, z + MARCH_LEAD, e->res, march_share(e->prec));
+        if (least < 0.0 || t < least) { least = t; best = z; }
+    }
+    return best;
 }
 
 // The flat tile list of a configuration: position order, tile offsets, per-box tiling.
@@ -170,9 +189,10 @@ Layout make_layout(const glm_ens* e, int zreq, int ord)
     }
     L.tiles_x.resize(n); L.tiles_y.resize(n); L.nzc.resize(n); L.zchunk.resize(n);
     L.tile_off.resize(n + 1);
+    const int z = zreq > 0 ? zreq : ens_zchunk(e);
     for (int b = 0; b < n; ++b) {
         const glm_ens_box& x = e->box[b];
-        march_tiling(x.nx, x.ny, x.nz, box_zchunk(x.nz, zreq), 0, L.tiles_x[b], L.tiles_y[b], L.nzc[b], L.zchunk[b]);
+        march_tiles(x.nx, x.ny, x.nz, OX, OY, box_zchunk(x.nz, z), e->res, 0.0, 0.0, L.tiles_x[b], L.tiles_y[b], L.nzc[b], L.zchunk[b]);
     }
     int off = 0;
     for (int p = 0; p < n; ++p) {
@@ -245,7 +265,7 @@ EnsLaunch<T> make_launch(const glm_ens* e, const void* ma, const int* order, con
 int grid_of(const glm_ens* e, int total, int persistent)
 {
     if (persistent <= 0) return total;
-    const int g = persistent * e->cu_count;
+    const int g = persistent * e->res.cus;
     return g < total ? g : total;
 }
 
@@ -364,7 +384,11 @@ glm_ens* glm_ens_create(int nbox, const glm_ens_box* boxes, const glm_params* sc
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess)
         return fail(GLM_ERR_HIP, "glm_ens_create: device attribute query failed");
-    e->cu_count = cus;
+    e->res.cus = cus;
+    const void* fn = precision == 8 ? ens_kernel_ptr<double>(scheme->predictor, scheme->riemann, scheme->recon, scheme->slope)
+                                    : ens_kernel_ptr<float>(scheme->predictor, scheme->riemann, scheme->recon, scheme->slope);
+    if (!fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&e->res.occ, fn, NT, 0) != hipSuccess || e->res.occ < 1)
+        e->res.occ = 1;
     e->clock_khz = khz > 0 ? (double)khz : 100000.0;
     const size_t logn = (size_t)ENS_LOG * nbox;
     if (hipMalloc(&e->d_eb, nbox * sizeof(EnsBox)) != hipSuccess ||
@@ -560,14 +584,7 @@ int glm_ens_tune(glm_ens* e, int reps, int* best, double* best_ms)
     // writes the other buffer; its CFL max goes to a scratch slot)
     std::vector<EnsBox> eb(e->nbox);
     HIPCHK(hipMemcpy(eb.data(), e->d_eb, eb.size() * sizeof(EnsBox), hipMemcpyDeviceToHost));
-    int occ = 1;
-    {
-        const void* fn = e->prec == 8 ? ens_kernel_ptr<double>(e->scheme.predictor, e->scheme.riemann,
-                                                              e->scheme.recon, e->scheme.slope)
-                                      : ens_kernel_ptr<float>(e->scheme.predictor, e->scheme.riemann,
-                                                              e->scheme.recon, e->scheme.slope);
-        if (!fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, NT, 0) != hipSuccess || occ < 1) occ = 1;
-    }
+    const int occ = e->res.occ;
     void* ma = nullptr;
     int *order = nullptr, *toff = nullptr;
     unsigned long long *slots = nullptr, *t0 = nullptr, *t1 = nullptr;
@@ -585,8 +602,8 @@ int glm_ens_tune(glm_ens* e, int reps, int* best, double* best_ms)
         err = set_err(GLM_ERR_ALLOC, "glm_ens_tune: scratch allocation failed");
     if (!err && (hipEventCreate(&ev0) != hipSuccess || hipEventCreate(&ev1) != hipSuccess))
         err = set_err(GLM_ERR_HIP, "glm_ens_tune: event creation failed");
-    const int zc[] = {16, 24, 32, 48, 64, 128};
-    for (int zi = 0; zi < 6 && !err; ++zi)
+    const int zc[] = {ens_zchunk(e), 16, 24, 32, 48, 64, 128};   // the model's choice first
+    for (int zi = 0; zi < 7 && !err; ++zi)
         for (int pm = 0; pm <= occ && !err; ++pm)
             for (int od = 0; od <= 1 && !err; ++od) {
                 Layout L = make_layout(e, zc[zi], od);

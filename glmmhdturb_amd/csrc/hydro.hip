@@ -63,7 +63,7 @@ static void launch_sv(const HydroArgs<T>& a, dim3 g, int nsp, int cma, hipStream
 }
 
 template <typename T>
-hipError_t launch_hydro_march(void* const* q, void* const* o, const HydroArgsHost& h, int slots, hipStream_t st)
+hipError_t launch_hydro_march(void* const* q, void* const* o, const HydroArgsHost& h, const Resident& res, hipStream_t st)
 {
     if (h.nsp != 0 && h.nsp != 2) return hipErrorInvalidValue;
     if (h.scheme < HY_PLM || h.scheme > HY_DONOR || (h.scheme != HY_PLM && h.fmt != HY_CONS)) return hipErrorInvalidValue;
@@ -83,7 +83,7 @@ hipError_t launch_hydro_march(void* const* q, void* const* o, const HydroArgsHos
         a.oh[v] = narrow ? (unsigned short*)o[v] : nullptr;
     }
     a.nx = h.nx; a.ny = h.ny; a.nz = h.nz;
-    hydro_tiling(h.nx, h.ny, h.nz, h.zchunk, slots, a.tiles_x, a.tiles_y, a.nzc, a.zchunk);
+    hydro_tiling<T>(h.nx, h.ny, h.nz, h.zchunk, res, a.tiles_x, a.tiles_y, a.nzc, a.zchunk);
     a.gamma = (T)h.gamma; a.gm1 = (T)(h.gamma - 1.0); a.igm1 = (T)(1.0 / (h.gamma - 1.0));
     a.dtdx = (T)h.dtdx; a.half_dtdx = (T)(0.5 * h.dtdx);
     a.smallr = (T)h.smallr; a.smallp = (T)h.smallp;
@@ -127,8 +127,8 @@ hipError_t launch_hydro_march(void* const* q, void* const* o, const HydroArgsHos
     return hipGetLastError();
 }
 
-template hipError_t launch_hydro_march<double>(void* const*, void* const*, const HydroArgsHost&, int, hipStream_t);
-template hipError_t launch_hydro_march<float>(void* const*, void* const*, const HydroArgsHost&, int, hipStream_t);
+template hipError_t launch_hydro_march<double>(void* const*, void* const*, const HydroArgsHost&, const Resident&, hipStream_t);
+template hipError_t launch_hydro_march<float>(void* const*, void* const*, const HydroArgsHost&, const Resident&, hipStream_t);
 template const void* hydro_march_ptr<double>(int, int, int, int, int);
 template const void* hydro_march_ptr<float>(int, int, int, int, int);
 

@@ -1,6 +1,7 @@
 // hydro_launch.hpp -- host launcher of the 5-variable hydro march (hydro.hip).
 #pragma once
 #include <hip/hip_runtime.h>
+#include "tiling.hpp"
 
 namespace glm {
 
@@ -20,7 +21,7 @@ struct HydroArgsHost {
 
 constexpr int HYDRO_THREADS = 256;   // lanes of a hydro march workgroup (hydro_march.hpp HM_NT)
 template <typename T>
-hipError_t launch_hydro_march(void* const* q, void* const* o, const HydroArgsHost& h, int slots, hipStream_t st);
+hipError_t launch_hydro_march(void* const* q, void* const* o, const HydroArgsHost& h, const Resident& res, hipStream_t st);
 template <typename T>
 const void* hydro_march_ptr(int fallback, int nsp, int cma, int fmt = 0, int scheme = 0);
 

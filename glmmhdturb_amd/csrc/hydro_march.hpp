@@ -23,6 +23,7 @@
 // cell, as in the reference.
 #pragma once
 #include "gpu_util.hpp"
+#include "tiling.hpp"
 
 namespace glm {
 
@@ -278,31 +279,12 @@ GLM_DEV void hy_dir(const T m2[NV], const T m1[NV], const T c0[NV], const T p1[N
     for (int v = 0; v < NV; ++v) div[v] += Fp[v] - Fm[v];
 }
 
-// z chunking: the chunk length minimising (waves of workgroups) x (planes + priming) for
-// `slots` resident workgroups, or the requested length.
-inline void hydro_tiling(int nx, int ny, int nz, int zchunk_req, int slots, int& tiles_x, int& tiles_y, int& nzc,
+// Tiles and z-chunks of the hydro march (lead-in: the priming z face and the window's load).
+template <typename T>
+inline void hydro_tiling(int nx, int ny, int nz, int zchunk_req, const Resident& r, int& tiles_x, int& tiles_y, int& nzc,
                          int& zchunk)
 {
-    tiles_x = (nx + HM_OX - 1) / HM_OX;
-    tiles_y = (ny + HM_OY - 1) / HM_OY;
-    if (zchunk_req > 0) {
-        zchunk = zchunk_req < nz ? zchunk_req : nz;
-        nzc = (nz + zchunk - 1) / zchunk;
-        return;
-    }
-    const long cols = (long)tiles_x * tiles_y;
-    const long sl = slots > 0 ? slots : 256;
-    const int maxc = nz / 8 > 1 ? nz / 8 : 1;
-    long best = -1;
-    zchunk = nz;
-    for (int c = 1; c <= maxc; ++c) {
-        const int zc = (nz + c - 1) / c;
-        const int n = (nz + zc - 1) / zc;
-        if (n != c) continue;
-        const long cost = ((cols * n + sl - 1) / sl) * (long)(zc + 2);
-        if (best < 0 || cost < best) { best = cost; zchunk = zc; }
-    }
-    nzc = (nz + zchunk - 1) / zchunk;
+    march_tiles(nx, ny, nz, HM_OX, HM_OY, zchunk_req, r, 1.2, sizeof(T) == 8 ? 0.68 : 0.35, tiles_x, tiles_y, nzc, zchunk);
 }
 
 // Resident waves per SIMD the register allocation is held to: as many as the LDS ring allows

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include "march_impl.hpp"
+#include "tiling.hpp"
 
 namespace glm {
 
@@ -75,32 +76,16 @@ inline const void* ens_kernel_ptr(int pred, int riem, int recon, int slope)
     return nullptr;
 }
 
-// Workgroup tiling of the march for an (nx, ny, nz) grid: tiles and z-chunks.  With no requested
-// z-chunk the number of chunks minimises the modelled run time on `slots` concurrent workgroups
-// (CUs x resident workgroups per CU): rounds = ceil(workgroups / slots), each as long as one chunk
-// plus about one plane of lead-in (the first plane's predictor and the chunk's extra z face).
-// A grid whose workgroup count is a multiple of the slots leaves no partly filled last round.
-inline void march_tiling(int nx, int ny, int nz, int zchunk_req, int slots, int& tiles_x, int& tiles_y, int& nzc,
+// Workgroup tiling of the march for an (nx, ny, nz) grid.  A chunk costs about 1.3 planes besides its
+// own: the window's first planes, the lead-in plane's predictor and the face above the last plane.
+// share: the FP64 PPM + HLLD march 0.55, FP32 marches (four resident) 0.29-0.34.
+constexpr double MARCH_LEAD = 1.3;
+inline double march_share(int prec) { return prec == 8 ? 0.55 : 0.32; }
+template <typename T>
+inline void march_tiling(int nx, int ny, int nz, int zchunk_req, const Resident& r, int& tiles_x, int& tiles_y, int& nzc,
                          int& zchunk)
 {
-    tiles_x = (nx + OX - 1) / OX;
-    tiles_y = (ny + OY - 1) / OY;
-    zchunk = zchunk_req > 0 ? zchunk_req : 0;
-    if (zchunk == 0) {
-        const long cols = (long)tiles_x * tiles_y;
-        const long sl = slots > 0 ? slots : 256;
-        const int maxc = nz / 8 > 1 ? nz / 8 : 1;   // chunks of at least 8 planes
-        long best = -1;
-        for (int c = 1; c <= maxc; ++c) {
-            const int zc = (nz + c - 1) / c;
-            const int n = (nz + zc - 1) / zc;      // chunks actually formed
-            if (n != c) continue;
-            const long cost = ((cols * n + sl - 1) / sl) * (long)(zc + 1);
-            if (best < 0 || cost < best) { best = cost; zchunk = zc; }
-        }
-    }
-    if (zchunk > nz) zchunk = nz;
-    nzc = (nz + zchunk - 1) / zchunk;
+    march_tiles(nx, ny, nz, OX, OY, zchunk_req, r, MARCH_LEAD, march_share((int)sizeof(T)), tiles_x, tiles_y, nzc, zchunk);
 }
 
 }  // namespace glm
