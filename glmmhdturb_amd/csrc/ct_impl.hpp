@@ -123,9 +123,9 @@ template <typename T, int D, int NV = 8, int RC = -1, typename A>
 GLM_DEV void ct_cell_states(const T l[NV], const T c[NV], const T r[NV], const A& a, T lo[NV], T hi[NV])
 {
     T hs[NV], mh[NV];
-    const T fac = a.face_slope == 1 ? T(0.25) : T(0.5);
+    const T fac = a.face_slope == 1 ? T(0.5) : T(1);
 #pragma unroll
-    for (int k = 0; k < NV; ++k) hs[k] = fac * moncen(c[k] - l[k], r[k] - c[k]);
+    for (int k = 0; k < NV; ++k) hs[k] = fac * moncen_half(c[k] - l[k], r[k] - c[k]);
     ct_hanc1d<T, D>(c, hs, mh, a);
 #pragma unroll
     for (int k = 8; k < NV; ++k) mh[k] = c[k] - a.half_dtdx * c[1 + D] * (T(2) * hs[k]);

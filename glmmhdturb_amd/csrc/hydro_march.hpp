@@ -121,6 +121,7 @@ GLM_DEV void hy_c2p(const T c[NV], T q[NV], const HydroArgs<T>& a)
 template <typename T>
 GLM_DEV T hy_moncen(T l, T m, T r)
 {
+    if (sizeof(T) == 4) return T(2) * moncen_half(m - l, r - m);
     const T dl = m - l, dr = r - m, dc = T(0.5) * (r - l);
     const T s = tmin(tabs(dc), tmin(T(2) * tabs(dl), T(2) * tabs(dr)));
     return dl * dr <= T(0) ? T(0) : (dl > T(0) ? s : -s);

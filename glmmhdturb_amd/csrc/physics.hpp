@@ -307,6 +307,8 @@ GLM_HD T minmod(T a, T b)
 {
     return (a * b <= T(0)) ? T(0) : (tabs(a) < tabs(b) ? a : b);
 }
+GLM_HD float tmed3(float a, float b, float c);
+GLM_HD float minmod(float a, float b) { return tmed3(a, b, 0.0f); }
 // Half the MonCen slope without selects: with s the sign of dl + dr, a = s dl and b = s dr,
 // 0.5 moncen(dl, dr) = s max(0, min(a, b, |dl + dr| / 4)).  When dl and dr share a sign, a and b are
 // |dl| and |dr| and the min is 0.5 min(2|dl|, 2|dr|, |dc|) exactly (powers of two); otherwise one of
@@ -350,19 +352,23 @@ GLM_HD void ppm_edges(T qm, T q0, T qp, T& lo, T& hi)
 // With s the sign of a + b (that is, of the slope) a' = s max(0, min(s a, 2 s b)) and b' = s max(0, min(s b, 2 s a)):
 // the same limited parabola up to rounding, with no selects (the limiter is continuous at each
 // switch, so a switch decided differently by rounding moves the result by rounding only).
-GLM_HD double flip_sign(double x, double ref)
-{
-    const unsigned long long m = __builtin_bit_cast(unsigned long long, ref) & 0x8000000000000000ull;
-    return __builtin_bit_cast(double, __builtin_bit_cast(unsigned long long, x) ^ m);
-}
-GLM_HD float flip_sign(float x, float ref)
-{
-    const unsigned m = __builtin_bit_cast(unsigned, ref) & 0x80000000u;
-    return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) ^ m);
-}
-// The sign is applied by multiplying with s = +-1 rather than by flipping the sign bit: a product is
-// a canonical float, so the min/max that follow need no NaN-quieting of their operands (a bit
+// In FP64 the sign is applied by multiplying with s = +-1 rather than by flipping the sign bit: a product
+// is a canonical float, so the min/max that follow need no NaN-quieting of their operands (a bit
 // operation's result would get one).  Multiplying by +-1 is exact, so the values are the same.
+//
+// In FP32 the limiters are medians with 0, one v_med3_f32 each: med3(a, b, 0) is the smaller of a and b
+// in magnitude where they share a sign and 0 where they do not (minmod), so half the MonCen slope is
+// med3(med3(dl, dr, 0), (dl + dr)/4, 0) (6 instructions with the differences instead of 11) and a
+// limited PPM offset is med3(a, 2b, 0).  The FP32 marches issue VALU instructions nearly all the
+// time, so their time follows the count: see the figures at GLM_WAVES_F32_NS0.
+GLM_HD float tmed3(float a, float b, float c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_fmed3f(a, b, c);
+#else
+    return __builtin_fmaxf(__builtin_fminf(a, b), __builtin_fminf(__builtin_fmaxf(a, b), c));
+#endif
+}
 GLM_HD double moncen_half(double dl, double dr)
 {
     const double sum = dl + dr;
@@ -372,10 +378,23 @@ GLM_HD double moncen_half(double dl, double dr)
 }
 GLM_HD float moncen_half(float dl, float dr)
 {
-    const float sum = dl + dr;
-    const float sg = __builtin_copysignf(1.0f, sum);
-    const float a = sg * dl, b = sg * dr;
-    return sg * __builtin_fmaxf(__builtin_fminf(__builtin_fminf(a, b), 0.25f * __builtin_fabsf(sum)), 0.0f);
+    return tmed3(tmed3(dl, dr, 0.0f), 0.25f * (dl + dr), 0.0f);
+}
+// The limited offsets of a parabola with unlimited offsets a and b of slope sign(d): minmod(a, 2b) and
+// minmod(b, 2a).  s = sign(d): where a and b share a sign it is theirs (a + b = 2d up to rounding,
+// which keeps signs), and where they do not both offsets are 0 whatever s is.
+template <typename T>
+GLM_HD void limit_offsets(T d, T a, T b, T& dl, T& dr)
+{
+    const T sg = tcopysign(T(1), d);
+    const T sa = sg * a, sb = sg * b;
+    dl = sg * tmax(tmin(sa, sb + sb), T(0));
+    dr = sg * tmax(tmin(sb, sa + sa), T(0));
+}
+GLM_HD void limit_offsets(float, float a, float b, float& dl, float& dr)
+{
+    dl = tmed3(a, b + b, 0.0f);
+    dr = tmed3(b, a + a, 0.0f);
 }
 template <typename T>
 GLM_HD void ppm_offsets(T qm, T q0, T qp, T& dl, T& dr)
@@ -383,13 +402,7 @@ GLM_HD void ppm_offsets(T qm, T q0, T qp, T& dl, T& dr)
     T slope = T(0.25) * (qp - qm);
     T curve = (qm - T(2) * q0 + qp) * T(1.0 / 12.0);
     T a = slope - curve, b = slope + curve;
-    // s = sign(slope): where a and b share a sign it is theirs (a + b = 2 slope up to rounding, which
-    // keeps signs), and where they do not both offsets are 0 whatever s is.  s is applied as a
-    // factor +-1 (exact), whose products need no NaN-quieting before the min/max.
-    const T sg = tcopysign(T(1), slope);
-    T sa = sg * a, sb = sg * b;
-    dl = sg * tmax(tmin(sa, sb + sb), T(0));
-    dr = sg * tmax(tmin(sb, sa + sa), T(0));
+    limit_offsets(slope, a, b, dl, dr);
 }
 
 // spike_mhd.cu:164-172 ppm1 as edge offsets dl = q0 - lo, dr = hi - q0, in min/max form.  The
@@ -406,10 +419,7 @@ GLM_HD void ppm_offsets_spike(T qm, T q0, T qp, T& dl, T& dr)
 {
     const T d = T(0.25) * (qp - qm), cu = (qm - T(2) * q0 + qp) * (T(1) / T(6));
     const T a = d + cu, b = d - cu;
-    const T sg = tcopysign(T(1), d);
-    const T sa = sg * a, sb = sg * b;
-    dl = sg * tmax(tmin(sa, sb + sb), T(0));
-    dr = sg * tmax(tmin(sb, sa + sa), T(0));
+    limit_offsets(d, a, b, dl, dr);
 }
 // spike_mhd.cu:164-172 ppm1 (both edges).
 template <typename T>

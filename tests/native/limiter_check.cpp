@@ -27,4 +27,14 @@ void lc_ppm_spike(const double* qm, const double* q0, const double* qp, double* 
     for (long i = 0; i < n; ++i) glm::ppm_edges_spike(qm[i], q0[i], qp[i], lo[i], hi[i]);
 }
 
+// the FP32 forms: MonCen's half slope, minmod, and the limited offsets of unlimited ones a and b
+void lc_limiters_f32(const float* a, const float* b, float* half, float* mm, float* dl, float* dr, long n)
+{
+    for (long i = 0; i < n; ++i) {
+        half[i] = glm::moncen_half(a[i], b[i]);
+        mm[i] = glm::minmod(a[i], b[i]);
+        glm::limit_offsets(a[i] + b[i], a[i], b[i], dl[i], dr[i]);
+    }
+}
+
 }
