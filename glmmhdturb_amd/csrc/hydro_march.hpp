@@ -12,25 +12,36 @@
 // :251, :298), their flux the HLL/LLF flux of rho*s or, with CMA (-DCMA), the HLL mass flux times
 // the upwind face value of s (:321, :367).
 //
-// Kernel shape.  A workgroup owns a 32 x 8 column tile and a chunk of z planes; lane (tx, ty)
-// owns one column.  Each plane of the tile plus a 2-cell halo (36 x 12 cells) is read from HBM
-// once, converted to primitives once, and kept in a ring of 4 LDS planes: plane k+3 is fetched
-// before plane k is updated and stored after it (one barrier per plane).  The x and y stencils read plane k; the z
-// stencil is the lane's own column of planes k-1..k+2, kept in registers as it passes through
-// the ring.  The z face k+1/2 solved for plane k is the face k+1/2 of plane k+1, so it is
-// carried, not solved again; the first z face of a chunk is solved by the same code in a priming
-// iteration, so every chunking gives the same bits.  x and y faces are solved once per adjacent
-// cell, as in the reference.
+// Kernel shape.  A workgroup of 256 lanes owns a 30 x 16 column tile and a chunk of z planes.  Half a
+// wavefront is one row of 32 cells (the 30 owned and one more on each side), and each lane carries the
+// columns of two neighbouring rows.  What bounds it is the issue of VALU instructions, so each face
+// state and face is computed as few times as its direction allows without a workgroup barrier:
+//   x: every lane builds the states of its own cell once and solves its lower face; the upper face of the
+//      lower neighbour and the flux of the upper one come from the next lane (DPP wave shift, no LDS
+//      round trip);
+//   y: four cells' states and three faces for a lane's two rows, from the LDS plane;
+//   z: one cell's states and one face per plane and row; the upper state is carried to the next plane.
+// Per owned cell that is 4 slopes and half steps and 3.5 solves (times 32/30), where a lane per column
+// with both its faces in each direction took 8 and 5: 480^3 FP32 2.52 -> 1.90 ms.
+//   LDS holds the primitives of planes k and k+1 over the tile grown by two cells (34 x 20): a lane's own
+// cells reach plane k+2 in registers, the halo's plane k+1 is fetched during plane k, so one barrier
+// per plane suffices.  The loop starts two planes early so that the chunk's first z states and face
+// come from the loop's own code, and the flux functions are not contracted by the compiler (their
+// fused operations are written out): a face has the same bits in every row, lane and chunking.
 #pragma once
 #include "gpu_util.hpp"
 #include "tiling.hpp"
 
 namespace glm {
 
-constexpr int HM_OX = 32, HM_OY = 8, HM_G = 2;
-constexpr int HM_LX = HM_OX + 2 * HM_G, HM_LY = HM_OY + 2 * HM_G;
-constexpr int HM_NPL = HM_LX * HM_LY;   // 432 cells of a haloed plane
-constexpr int HM_NT = HM_OX * HM_OY;    // 256 lanes, one per owned column
+constexpr int HM_OX = 30, HM_OY = 16;
+constexpr int HM_W = HM_OX + 2;                      // lanes of a row
+constexpr int HM_LX = HM_OX + 4, HM_LY = HM_OY + 4;  // LDS plane: the tile grown by two cells
+constexpr int HM_NPL = HM_LX * HM_LY;
+constexpr int HM_NT = HM_W * HM_OY / 2;              // 256 lanes, two rows each
+constexpr int HM_NHALO = 4 * HM_W + 2 * HM_OY;       // plane cells no lane owns: two rows below and above, the outer columns
+constexpr int HM_SEAM_X = 32, HM_SEAM_Y = 8;         // the reference's 32 x 8 tiles, whose seams HY_DONOR treats
+static_assert(HM_W == 32 && HM_NT == 256 && HM_NHALO <= HM_NT, "two rows of 32 lanes per wavefront");
 
 constexpr int HM_NVMAX = 7;   // 5 hydro variables + 2 passive scalars (-DSCALARS)
 
@@ -116,98 +127,22 @@ GLM_DEV void hy_c2p(const T c[NV], T q[NV], const HydroArgs<T>& a)
     for (int v = 5; v < NV; ++v) q[v] = LG ? c[v] : c[v] * ir;
 }
 
-// spike_25d.cu:207-213 moncen (full slope).  The selects stay: a select-free form (the sign of dc
-// applied as a factor) measured 2-3% slower in this kernel (480^3 FP32).
-template <typename T>
-GLM_DEV T hy_moncen(T l, T m, T r)
-{
-    if (sizeof(T) == 4) return T(2) * moncen_half(m - l, r - m);
-    const T dl = m - l, dr = r - m, dc = T(0.5) * (r - l);
-    const T s = tmin(tabs(dc), tmin(T(2) * tabs(dl), T(2) * tabs(dr)));
-    return dl * dr <= T(0) ? T(0) : (dl > T(0) ? s : -s);
-}
+// a*b + c as one operation.  The flux functions below are compiled without contraction and write their
+// fused operations out, so that every copy of them (two rows, three faces, three directions) rounds alike.
+GLM_DEV double tfma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+GLM_DEV float tfma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
-// spike_25d.cu:231-244 primFlux and :245-255 toCons (with LG the scalars are log2 X, decoded for the
-// flux and the conserved rho X, :248-250)
-template <typename T, int D, int NV, bool LG = false>
-GLM_DEV void hy_flux_cons(const T q[NV], T f[NV], T u[NV], const HydroArgs<T>& a)
+// spike_25d.cu:245-255 toCons (with LG the scalars are log2 X, decoded for the conserved rho X, :248-250)
+template <typename T, int NV, bool LG = false>
+GLM_DEV void hy_cons(const T q[NV], T u[NV], const HydroArgs<T>& a)
 {
-    const T un = q[1 + D];
-    const T E = q[4] * a.igm1 + T(0.5) * q[0] * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
-    const T mu = q[0] * un;
-    f[0] = mu;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) f[1 + c] = q[0] * q[1 + c] * un + (c == D ? q[4] : T(0));
-    f[4] = (E + q[4]) * un;
+#pragma clang fp contract(off)
     u[0] = q[0];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) u[1 + c] = q[0] * q[1 + c];
-    u[4] = E;
+    for (int c = 1; c < 4; ++c) u[c] = q[0] * q[c];
+    u[4] = tfma(q[4], a.igm1, T(0.5) * q[0] * tfma(q[1], q[1], tfma(q[2], q[2], q[3] * q[3])));
 #pragma unroll
-    for (int v = 5; v < NV; ++v) {
-        const T x = LG ? hy_exp2(q[v]) : q[v];
-        f[v] = mu * x;
-        u[v] = q[0] * x;
-    }
-}
-
-// spike_25d.cu:287-301 hanc1d: normal-only Hancock half step along D
-template <typename T, int D, int NV>
-GLM_DEV void hy_hanc1d(const T m[NV], const T s[NV], T mh[NV], const HydroArgs<T>& a)
-{
-    const T un = m[1 + D], sn = s[1 + D];
-    const T ir = trcp(m[0]);
-    const T h = a.half_dtdx;
-    mh[0] = m[0] - h * (un * s[0] + m[0] * sn);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) mh[1 + c] = m[1 + c] - h * (un * s[1 + c] + (c == D ? s[4] * ir : T(0)));
-    mh[4] = m[4] - h * (un * s[4] + a.gamma * m[4] * sn);
-    const T hu = h * un;
-#pragma unroll
-    for (int v = 5; v < NV; ++v) mh[v] = m[v] - hu * s[v];   // passive advection (:298)
-}
-
-// spike_25d.cu:222-230 edge: mh + sign*s/2, clamped at SMALLR/SMALLP
-template <typename T, int NV>
-GLM_DEV void hy_edge(const T mh[NV], const T s[NV], T sign, T e[NV], const HydroArgs<T>& a)
-{
-    const T hs = sign * T(0.5);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) e[v] = mh[v] + hs * s[v];
-    e[0] = tmax(e[0], a.smallr);
-    e[4] = tmax(e[4], a.smallp);
-}
-
-// HLL (spike_25d.cu:302-330); with FB, LLF where a face state is below the fallback floors
-// (riemann_fb, :335-376).  Both combine the same FL, FR, UL, UR.  With CMA the scalar fluxes of
-// the HLL fan are the mass flux times the upwind face value (:321, :367).
-template <typename T, int D, bool FB, int NV, bool CMA, bool LG = false>
-GLM_DEV void hy_riemann(const T L[NV], const T R[NV], T F[NV], const HydroArgs<T>& a)
-{
-    const T unL = L[1 + D], unR = R[1 + D];
-    const T aL = tsqrt_pos(a.gamma * L[4] * trcp(L[0])), aR = tsqrt_pos(a.gamma * R[4] * trcp(R[0]));
-    T FL[NV], FR[NV], UL[NV], UR[NV];
-    hy_flux_cons<T, D, NV, LG>(L, FL, UL, a);
-    hy_flux_cons<T, D, NV, LG>(R, FR, UR, a);
-    const T sL = tmin(unL - aL, unR - aR), sR = tmax(unL + aL, unR + aR);
-    const T inv = trcp(sR - sL), slsr = sL * sR;
-    const bool llf = FB && (L[0] < a.fb_dmin || L[4] < a.fb_pmin || R[0] < a.fb_dmin || R[4] < a.fb_pmin);
-    const T sm = tmax(tabs(unL) + aL, tabs(unR) + aR);
-    const T hll0 = (sR * FL[0] - sL * FR[0] + slsr * (UR[0] - UL[0])) * inv;
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        T hll = v == 0 ? hll0 : (sR * FL[v] - sL * FR[v] + slsr * (UR[v] - UL[v])) * inv;
-        if (CMA && v >= 5) hll = hll0 >= T(0) ? hll0 * (LG ? hy_exp2(L[v]) : L[v]) : hll0 * (LG ? hy_exp2(R[v]) : R[v]);
-        const T h = sL >= T(0) ? FL[v] : (sR <= T(0) ? FR[v] : hll);
-        F[v] = llf ? T(0.5) * (FL[v] + FR[v]) - T(0.5) * sm * (UR[v] - UL[v]) : h;
-    }
-}
-
-template <typename T, int NV>
-GLM_DEV void hy_slopes(const T l[NV], const T m[NV], const T r[NV], T s[NV])
-{
-#pragma unroll
-    for (int v = 0; v < NV; ++v) s[v] = hy_moncen(l[v], m[v], r[v]);
+    for (int v = 5; v < NV; ++v) u[v] = q[0] * (LG ? hy_exp2(q[v]) : q[v]);
 }
 
 // Scheme variants of the march (spike_25d.cu build flags): HY_PLM the light march (-DHANCOCK1D:
@@ -219,103 +154,139 @@ GLM_DEV void hy_slopes(const T l[NV], const T m[NV], const T r[NV], T s[NV])
 // without the fallback.
 enum { HY_PLM = 0, HY_PPM1D = 1, HY_DONOR = 2 };
 
-// The upper (SIGN = +1) or lower (-1) face state of cell c with neighbours l, r, slope sl and half
-// step mh: the light march's edge mh +- s/2 clamped at SMALLR/SMALLP, or the PPM1D parabola's edge
-// plus mh - c, unclamped (spike_25d.cu:476-479).
-template <typename T, int NV, int SV, int SIGN>
-GLM_DEV void hy_state(const T l[NV], const T c[NV], const T r[NV], const T sl[NV], const T mh[NV], T e[NV],
-                      const HydroArgs<T>& a)
+// The two face states of cell c along D from its neighbours l and r: half the MonCen slope (:207-221), the
+// normal-only Hancock half step mh (:287-301), then mh -+ half slope clamped at SMALLR/SMALLP (:222-230)
+// or the PPM1D parabola's edges plus mh - c, unclamped (:476-479).
+template <typename T, int D, int NV, int SV>
+GLM_DEV void hy_states(const T l[NV], const T c[NV], const T r[NV], T lo[NV], T hi[NV], const HydroArgs<T>& a)
 {
+#pragma clang fp contract(off)
+    T hs[NV], mh[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) hs[v] = moncen_half(c[v] - l[v], r[v] - c[v]);
+    // the half step is dt/dx times the half slope
+    const T un = c[1 + D], sn = hs[1 + D], k = -a.dtdx;
+    const T kn = k * un;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) mh[v] = tfma(kn, hs[v], c[v]);   // advection, the whole of a scalar's half step (:298)
+    mh[0] = tfma(k * c[0], sn, mh[0]);
+    mh[1 + D] = tfma(k * trcp(c[0]), hs[4], mh[1 + D]);
+    mh[4] = tfma(k * a.gamma * c[4], sn, mh[4]);
     if (SV == HY_PPM1D) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             T dl, dr;   // the edge is c - dl or c + dr; plus mh - c
             ppm_offsets_spike(l[v], c[v], r[v], dl, dr);
-            e[v] = SIGN > 0 ? mh[v] + dr : mh[v] - dl;
+            lo[v] = mh[v] - dl;
+            hi[v] = mh[v] + dr;
         }
     } else {
-        hy_edge<T, NV>(mh, sl, T(SIGN), e, a);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) { lo[v] = mh[v] - hs[v]; hi[v] = mh[v] + hs[v]; }
+        lo[0] = tmax(lo[0], a.smallr); hi[0] = tmax(hi[0], a.smallr);
+        lo[4] = tmax(lo[4], a.smallp); hi[4] = tmax(hi[4], a.smallp);
     }
 }
 
-// Flux through the face between cells c1 and c2 of the stencil c0 c1 | c2 c3 along D.
-template <typename T, int D, bool FB, int NV, bool CMA, bool LG = false, int SV = HY_PLM>
-GLM_DEV void hy_face(const T c0[NV], const T c1[NV], const T c2[NV], const T c3[NV], T F[NV], const HydroArgs<T>& a)
+// HLL (spike_25d.cu:302-330); with FB, LLF where a face state is below the fallback floors
+// (riemann_fb, :335-376).  With CMA the scalar fluxes of the HLL fan are the mass flux times the upwind
+// face value (:321, :367).
+//
+// F = [sR FL - sL FR + sL sR (UR - UL)] / (sR - sL) = wL (FL - sL UL) + wR (FR - sR UR) with
+// wL = sR / (sR - sL) and wR = -sL / (sR - sL).  FL - sL UL needs no momenta and no flux of its own (its mass
+// part rho (u - sL) times each velocity is its momentum part); speeds clamped at 0 make it the upwind flux
+// on supersonic faces, and speeds -+max(|u| + a) make it LLF: two selects instead of one per component.
+template <typename T, int D, bool FB, int NV, bool CMA, bool LG = false>
+GLM_DEV void hy_riemann(const T L[NV], const T R[NV], T F[NV], const HydroArgs<T>& a)
 {
-    T s[NV], mh[NV], L[NV], R[NV];
-    hy_slopes<T, NV>(c0, c1, c2, s);
-    hy_hanc1d<T, D, NV>(c1, s, mh, a);
-    hy_state<T, NV, SV, 1>(c0, c1, c2, s, mh, L, a);
-    hy_slopes<T, NV>(c1, c2, c3, s);
-    hy_hanc1d<T, D, NV>(c2, s, mh, a);
-    hy_state<T, NV, SV, -1>(c1, c2, c3, s, mh, R, a);
-    hy_riemann<T, D, FB && SV == HY_PLM, NV, CMA, LG>(L, R, F, a);
-}
-
-// div += F(+1/2) - F(-1/2) along D for the cell c0 of the stencil m2 m1 c0 p1 p2: the centre
-// cell's slope and half step are shared by its two faces (spike_25d.cu:462-466 forms them once
-// per face).  lob / hib: the lower / upper face is a tile seam (HY_DONOR: donor-cell HLL of the
-// two cell states, :445-448).
-template <typename T, int D, bool FB, int NV, bool CMA, bool LG = false, int SV = HY_PLM>
-GLM_DEV void hy_dir(const T m2[NV], const T m1[NV], const T c0[NV], const T p1[NV], const T p2[NV], T div[NV],
-                    const HydroArgs<T>& a, bool lob = false, bool hib = false)
-{
-    constexpr bool fb = FB && SV == HY_PLM;
-    T s[NV], mh[NV], L[NV], R[NV], Fm[NV], Fp[NV];
-    hy_slopes<T, NV>(m2, m1, c0, s);
-    hy_hanc1d<T, D, NV>(m1, s, mh, a);
-    hy_state<T, NV, SV, 1>(m2, m1, c0, s, mh, L, a);
-    hy_slopes<T, NV>(m1, c0, p1, s);
-    hy_hanc1d<T, D, NV>(c0, s, mh, a);
-    hy_state<T, NV, SV, -1>(m1, c0, p1, s, mh, R, a);
-    if (SV == HY_DONOR && lob) hy_riemann<T, D, false, NV, CMA, LG>(m1, c0, Fm, a);
-    else hy_riemann<T, D, fb, NV, CMA, LG>(L, R, Fm, a);
-    hy_state<T, NV, SV, 1>(m1, c0, p1, s, mh, L, a);
-    hy_slopes<T, NV>(c0, p1, p2, s);
-    hy_hanc1d<T, D, NV>(p1, s, mh, a);
-    hy_state<T, NV, SV, -1>(c0, p1, p2, s, mh, R, a);
-    if (SV == HY_DONOR && hib) hy_riemann<T, D, false, NV, CMA, LG>(c0, p1, Fp, a);
-    else hy_riemann<T, D, fb, NV, CMA, LG>(L, R, Fp, a);
+#pragma clang fp contract(off)
+    const T uL = L[1 + D], uR = R[1 + D];
+    const T aL = tsqrt_pos(a.gamma * L[4] * trcp(L[0])), aR = tsqrt_pos(a.gamma * R[4] * trcp(R[0]));
+    T sL = tmin(tmin(uL - aL, uR - aR), T(0)), sR = tmax(tmax(uL + aL, uR + aR), T(0));
+    bool llf = false;
+    if (FB) {
+        llf = L[0] < a.fb_dmin || L[4] < a.fb_pmin || R[0] < a.fb_dmin || R[4] < a.fb_pmin;
+        const T sm = tmax(tabs(uL) + aL, tabs(uR) + aR);
+        sL = llf ? -sm : sL;
+        sR = llf ? sm : sR;
+    }
+    const T inv = trcp(sR - sL), wL = sR * inv, wR = -sL * inv;
+    const T dL = uL - sL, dR = uR - sR;
+    const T mL = wL * (L[0] * dL), mR = wR * (R[0] * dR);
+    F[0] = mL + mR;
 #pragma unroll
-    for (int v = 0; v < NV; ++v) div[v] += Fp[v] - Fm[v];
+    for (int c = 1; c < 4; ++c) F[c] = tfma(mL, L[c], mR * R[c]);
+    F[1 + D] = F[1 + D] + tfma(wL, L[4], wR * R[4]);
+    const T EL = tfma(L[4], a.igm1, T(0.5) * L[0] * tfma(L[1], L[1], tfma(L[2], L[2], L[3] * L[3])));
+    const T ER = tfma(R[4], a.igm1, T(0.5) * R[0] * tfma(R[1], R[1], tfma(R[2], R[2], R[3] * R[3])));
+    F[4] = tfma(wL, tfma(EL, dL, L[4] * uL), wR * tfma(ER, dR, R[4] * uR));
+#pragma unroll
+    for (int v = 5; v < NV; ++v) {
+        if (CMA) {
+            const T x = F[0] >= T(0) ? L[v] : R[v];
+            F[v] = F[0] * (LG ? hy_exp2(x) : x);
+            if (FB && llf) F[v] = tfma(mL, LG ? hy_exp2(L[v]) : L[v], mR * (LG ? hy_exp2(R[v]) : R[v]));
+        } else {
+            F[v] = tfma(mL, L[v], mR * R[v]);
+        }
+    }
 }
 
-// Tiles and z-chunks of the hydro march (lead-in: the priming z face and the window's load).
+// The value of the previous / next lane of the wavefront.
+GLM_DEV float lane_prev(float x)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x138, 0xf, 0xf, false));
+}
+GLM_DEV float lane_next(float x)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x130, 0xf, 0xf, false));
+}
+GLM_DEV double lane_prev(double x)
+{
+    int2 w = __builtin_bit_cast(int2, x);
+    w.x = __builtin_amdgcn_update_dpp(0, w.x, 0x138, 0xf, 0xf, false);
+    w.y = __builtin_amdgcn_update_dpp(0, w.y, 0x138, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, w);
+}
+GLM_DEV double lane_next(double x)
+{
+    int2 w = __builtin_bit_cast(int2, x);
+    w.x = __builtin_amdgcn_update_dpp(0, w.x, 0x130, 0xf, 0xf, false);
+    w.y = __builtin_amdgcn_update_dpp(0, w.y, 0x130, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, w);
+}
+
+// Tiles and z-chunks of the hydro march (lead-in: the two priming iterations and the window's load; a
+// plane takes 2.65 us alone and 6.0 with three resident in FP32, 3.9 and 8 with two in FP64).
 template <typename T>
 inline void hydro_tiling(int nx, int ny, int nz, int zchunk_req, const Resident& r, int& tiles_x, int& tiles_y, int& nzc,
                          int& zchunk)
 {
-    march_tiles(nx, ny, nz, HM_OX, HM_OY, zchunk_req, r, 1.2, sizeof(T) == 8 ? 0.68 : 0.35, tiles_x, tiles_y, nzc, zchunk);
+    march_tiles(nx, ny, nz, HM_OX, HM_OY, zchunk_req, r, 0.7, sizeof(T) == 8 ? 0.9 : 0.6, tiles_x, tiles_y, nzc, zchunk);
 }
 
-// Resident waves per SIMD the register allocation is held to: as many as the LDS ring allows
-// (FP64: 2 workgroups per CU of 69 KB, 1 of 97 KB with scalars; FP32: 4 of 35 KB), except FP32 with
-// scalars, where 3 workgroups of 48 KB would hold it to 168 registers and spill: 2 workgroups and
-// no spills run 1.4x faster (480^3, measured).
-// The PPM1D and DONOR builds in FP32: 3 waves per SIMD without scalars (4 would hold them to 128
-// registers and spill), 1 with scalars (PPM1D with scalars at 1: 20.8 Gcell/s, at 2: 19.9; 480^3).
-#ifndef GLM_HYDRO_SV_WAVES0
-#define GLM_HYDRO_SV_WAVES0 3
+// Resident wavefronts per SIMD that the register allocation is held to.  FP32: 3 (168 registers, no
+// spills; at 4, 128 registers with 20 B of spills, 480^3 took 2.01 ms instead of 1.90, the fallback build
+// 2.63 instead of 1.97), with scalars 2 (2.58 ms; 3 with 36 B of spills 2.89).  FP64: 2 (3.58 ms; the
+// fallback build with 60 B of spills 4.21, at one wavefront 4.11), with scalars or donor seams, which
+// would spill 136-550 B at 256 registers, 1 (scalars 5.11 ms, at two 9.86; donor 3.72, at two 6.05).
+#ifndef GLM_HY_WAVES
+#define GLM_HY_WAVES(T, NSP, SV) (sizeof(T) == 8 ? ((NSP) || (SV) == HY_DONOR ? 1 : 2) : ((NSP) ? 2 : 3))
 #endif
-#ifndef GLM_HYDRO_SV_WAVES2
-#define GLM_HYDRO_SV_WAVES2 1
-#endif
-#define GLM_HYDRO_WAVES_PER_EU(T, NSP, SV) \
-    (sizeof(T) == 8 ? ((NSP) ? 1 : 2) : (SV) == HY_PLM ? ((NSP) ? 2 : 4) : ((NSP) ? GLM_HYDRO_SV_WAVES2 : GLM_HYDRO_SV_WAVES0))
 
 template <typename T, bool FB, int NSP, bool CMA, int FMT = HY_CONS, int SV = HY_PLM>
-__global__ void __launch_bounds__(HM_NT) __attribute__((amdgpu_waves_per_eu(GLM_HYDRO_WAVES_PER_EU(T, NSP, SV))))
+__global__ void __launch_bounds__(HM_NT) __attribute__((amdgpu_waves_per_eu(GLM_HY_WAVES(T, NSP, SV))))
 hydro_march_kernel(HydroArgs<T> a)
 {
     constexpr int NV = 5 + NSP;
     constexpr bool LG = FMT == HY_U16SP;      // species held as log2 X
     constexpr bool PRIM = FMT == HY_F16P || FMT == HY_U16P;   // primitive storage: no conversion on load
+    constexpr bool fb = FB && SV == HY_PLM;
     static_assert(FMT == HY_CONS || (sizeof(T) == 4 && (FMT != HY_U16SP || (NSP == 2 && CMA)) &&
                                      (FMT == HY_U16SP || NSP == 0)), "compact formats: FP32; U16SP with 2 CMA species");
-    // ring of 4 haloed primitive planes: plane j lives in buffer (j - k0 + 2) & 3
-    __shared__ T P[4][NV][HM_NPL];
+    __shared__ T P[2][NV][HM_NPL];   // primitives of plane j in P[j & 1]
     const int tid = threadIdx.x;
-    const int tx = tid % HM_OX, ty = tid / HM_OX;
+    const int lx = tid % HM_W, ly = tid / HM_W * 2;   // the lane's column in the row of 32, its lower row
     const int ntile = a.tiles_x * a.tiles_y;
     const int w = xcd_block((int)blockIdx.x, (int)gridDim.x);   // neighbouring tiles share an XCD's L2
     const int tile = w % ntile, zc = w / ntile;
@@ -323,167 +294,191 @@ hydro_march_kernel(HydroArgs<T> a)
     const int k0 = zc * a.zchunk;
     const int k1 = k0 + a.zchunk < a.nz ? k0 + a.zchunk : a.nz;
     const size_t plane = (size_t)a.nx * a.ny;
-    // the lane's column; lanes past the grid edge compute a wrapped column and store nothing
-    const int gx = x0 + tx, gy = y0 + ty;
-    const bool own = gx < a.nx && gy < a.ny;
-    const size_t col = (size_t)wrapi(gx, a.nx) + (size_t)a.nx * wrapi(gy, a.ny);
-    const int li = (ty + HM_G) * HM_LX + tx + HM_G;
+    // the lane's columns; those outside the tile or the grid are wrapped and store nothing
+    const int gx = wrapi(x0 - 1 + lx, a.nx), gy0 = wrapi(y0 + ly, a.ny), gy1 = wrapi(y0 + ly + 1, a.ny);
+    const size_t col[2] = {(size_t)gx + (size_t)a.nx * gy0, (size_t)gx + (size_t)a.nx * gy1};
+    const bool ownx = lx >= 1 && lx <= HM_OX && x0 - 1 + lx < a.nx;
+    const bool own[2] = {ownx && y0 + ly < a.ny, ownx && y0 + ly + 1 < a.ny};
+    const int li = (ly + 2) * HM_LX + lx + 1;   // the lower row's cell of the LDS plane
+    // the halo cell this lane brings in: rows -2, -1, 16, 17 of the lanes' columns, then columns -2 and 31
+    const bool halo = tid < HM_NHALO;
+    int hpx = 1 + lx, hpy = ly / 2 < 2 ? ly / 2 : HM_OY + ly / 2;
+    if (tid >= 4 * HM_W) {
+        hpx = (tid & 1) ? HM_LX - 1 : 0;
+        hpy = 2 + (tid - 4 * HM_W) / 2;
+    }
+    const int hi_ = halo ? hpy * HM_LX + hpx : 0;
+    const size_t hcol = halo ? (size_t)wrapi(x0 - 2 + hpx, a.nx) + (size_t)a.nx * wrapi(y0 - 2 + hpy, a.ny) : 0;
 
-    // every primitive value of the kernel comes from hy_c2p, which is not contracted, so a cell
-    // has the same bits in every stencil and every chunking.  A plane is fetched from HBM into
-    // registers (`pre`, two cells per lane) at the top of an iteration and converted into its
-    // LDS buffer at the bottom, so the fetch latency is hidden behind the plane's compute.
-    T pre[2][NV];
-    auto fetch = [&](int k) {
-        const size_t zoff = (size_t)wrapi(k, a.nz) * plane;
+    // a cell as it lies in HBM, decoded (cell g of the state)
+    auto fetch = [&](size_t g, T c[NV]) {
+        if (FMT == HY_CONS) {
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const int c = tid + r * HM_NT;
-            if (c < HM_NPL) {
-                const int lx = c % HM_LX, ly = c / HM_LX;
-                const size_t g = zoff + wrapi(x0 - HM_G + lx, a.nx) + (size_t)a.nx * wrapi(y0 - HM_G + ly, a.ny);
-                if (FMT == HY_CONS) {
+            for (int v = 0; v < NV; ++v) c[v] = gload(a.q[v] + g);
+        } else if (FMT == HY_F16P) {
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) pre[r][v] = gload(a.q[v] + g);
-                } else if (FMT == HY_F16P) {
+            for (int v = 0; v < 5; ++v) c[v] = (T)hy_f16_to_f32(gload(a.qh[v] + g));
+        } else if (FMT == HY_U16P) {   // spike_25d.cu:397-402
+            c[0] = (T)exp2f(hy_dec_log2s(gload(a.qh[0] + g)));
 #pragma unroll
-                    for (int v = 0; v < 5; ++v) pre[r][v] = (T)hy_f16_to_f32(gload(a.qh[v] + g));
-                } else if (FMT == HY_U16P) {   // spike_25d.cu:397-402
-                    pre[r][0] = (T)exp2f(hy_dec_log2s(gload(a.qh[0] + g)));
+            for (int v = 1; v < 4; ++v) c[v] = (T)hy_dec_vel(gload(a.qh[v] + g));
+            c[4] = (T)exp2f(hy_dec_log2s(gload(a.qh[4] + g)));
+        } else {                       // HY_U16SP, :409-411
 #pragma unroll
-                    for (int v = 1; v < 4; ++v) pre[r][v] = (T)hy_dec_vel(gload(a.qh[v] + g));
-                    pre[r][4] = (T)exp2f(hy_dec_log2s(gload(a.qh[4] + g)));
-                } else {                       // HY_U16SP, :409-411
+            for (int v = 0; v < 5; ++v) c[v] = gload(a.q[v] + g);
 #pragma unroll
-                    for (int v = 0; v < 5; ++v) pre[r][v] = gload(a.q[v] + g);
-#pragma unroll
-                    for (int v = 5; v < NV; ++v) pre[r][v] = (T)hy_dec_log2(gload(a.qh[v] + g));
-                }
-            }
+            for (int v = 5; v < NV; ++v) c[v] = (T)hy_dec_log2(gload(a.qh[v] + g));
         }
     };
-    auto commit = [&](int k) {
-        const int b = (k - k0 + 2) & 3;
+    // its primitives: every primitive value of the kernel comes from here
+    auto prim = [&](const T c[NV], T q[NV]) {
+        if (PRIM) {   // make_prim (spike_25d.cu:204-206)
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const int c = tid + r * HM_NT;
-            if (c < HM_NPL) {
-                T qq[NV];
-                if (PRIM) {   // make_prim (spike_25d.cu:204-206)
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) qq[v] = pre[r][v];
-                    qq[0] = tmax(qq[0], a.smallr);
-                    qq[4] = tmax(qq[4], a.smallp);
-                } else {
-                    hy_c2p<T, NV, LG>(pre[r], qq, a);
-                }
-#pragma unroll
-                for (int v = 0; v < NV; ++v) P[b][v][c] = qq[v];
-            }
+            for (int v = 0; v < NV; ++v) q[v] = c[v];
+            q[0] = tmax(q[0], a.smallr);
+            q[4] = tmax(q[4], a.smallp);
+        } else {
+            hy_c2p<T, NV, LG>(c, q, a);
         }
     };
-    auto load_plane = [&](int k) {
-        fetch(k);
-        commit(k);
-    };
-    auto own_cell = [&](int k, T qq[NV]) {
-        const int b = (k - k0 + 2) & 3;
+    auto zoff = [&](int k) { return (size_t)wrapi(k, a.nz) * plane; };
+    auto lds = [&](int k, int at, T q[NV]) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) qq[v] = P[b][v][li];
+        for (int v = 0; v < NV; ++v) q[v] = P[k & 1][v][at];
+    };
+    // U1 = toCons(prim(U0)) - dtdx div of cell g
+    auto store = [&](size_t g, const T p0[NV], const T div[NV]) {
+        T U[NV];
+        hy_cons<T, NV, LG>(p0, U, a);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) U[v] = tfma(-a.dtdx, div[v], U[v]);
+        if (FMT == HY_CONS) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) a.o[v][g] = U[v];
+        } else if (PRIM) {   // c2p -> store primitive (spike_25d.cu:499-511)
+            const T ir = T(1) / tmax(U[0], a.smallr);
+            const T vx = U[1] * ir, vy = U[2] * ir, vz = U[3] * ir;
+            const T ke = T(0.5) * U[0] * (vx * vx + vy * vy + vz * vz);
+            const T pp = tmax(a.gm1 * (U[4] - ke), a.smallp);
+            if (FMT == HY_F16P) {
+                a.oh[0][g] = hy_f32_to_f16((float)U[0]);
+                a.oh[1][g] = hy_f32_to_f16((float)vx);
+                a.oh[2][g] = hy_f32_to_f16((float)vy);
+                a.oh[3][g] = hy_f32_to_f16((float)vz);
+                a.oh[4][g] = hy_f32_to_f16((float)pp);
+            } else {
+                a.oh[0][g] = hy_enc_log2s(log2f((float)tmax(U[0], a.smallr)));
+                a.oh[1][g] = hy_enc_vel((float)vx);
+                a.oh[2][g] = hy_enc_vel((float)vy);
+                a.oh[3][g] = hy_enc_vel((float)vz);
+                a.oh[4][g] = hy_enc_log2s(log2f((float)pp));
+            }
+        } else {             // HY_U16SP: X_new = (rho X)_new / rho_new -> log2 -> uint16 (:514-517)
+#pragma unroll
+            for (int v = 0; v < 5; ++v) a.o[v][g] = U[v];
+            const T rinv = T(1) / tmax(U[0], a.smallr);
+#pragma unroll
+            for (int v = 5; v < NV; ++v) a.oh[v][g] = hy_enc_log2(log2f(fmaxf((float)(U[v] * rinv), 7.7e-34f)));
+        }
     };
 
-    T W[4][NV];   // the lane's column at planes k-1 .. k+2 (iteration k)
-    T Fz[NV];     // z flux through face k-1/2
-    load_plane(k0 - 2);
-    load_plane(k0 - 1);
-    load_plane(k0);
-    load_plane(k0 + 1);
-    __syncthreads();
-    own_cell(k0 - 2, W[1]);
-    own_cell(k0 - 1, W[2]);
-    own_cell(k0, W[3]);
-    __syncthreads();   // plane k0-2's buffer is reloaded in the first iteration
+    T pp[2][NV];      // the lane's cells of plane k+1
+    T zprev[2][NV];   // upper z states of its cells of plane k
+    T Fz[2][NV];      // z fluxes through face k-1/2
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        T c[NV], q[NV];
+        fetch(zoff(k0 - 2) + col[r], c);
+        prim(c, q);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) { P[k0 & 1][v][li + r * HM_LX] = q[v]; zprev[r][v] = T(1); Fz[r][v] = T(0); }
+        fetch(zoff(k0 - 1) + col[r], c);
+        prim(c, pp[r]);
+    }
 
-    // iteration k0-1 only computes the z face k0-1/2 (with the same code as every later face)
+    // iterations k0-2 and k0-1 only form the z states and the face below plane k0
 #pragma clang loop unroll(disable)
-    for (int k = k0 - 1; k < k1; ++k) {
-        const bool more = k + 3 <= k1 + 1;   // planes up to k1+1 are read
-        if (more) fetch(k + 3);
+    for (int k = k0 - 2; k < k1; ++k) {
+        T pre[2][NV], hpre[NV];   // plane k+2 of the lane's cells, plane k+1 of its halo cell
+        const bool more = k + 1 >= k0 && k + 1 < k1;
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            W[0][v] = W[1][v];
-            W[1][v] = W[2][v];
-            W[2][v] = W[3][v];
-        }
-        own_cell(k + 2, W[3]);
-        T div[NV];
+        for (int r = 0; r < 2; ++r) fetch(zoff(k + 2) + col[r], pre[r]);
+        if (more && halo) fetch(zoff(k + 1) + hcol, hpre);
+        // plane k+1 into the buffer of plane k-1, last read before the previous barrier
 #pragma unroll
-        for (int v = 0; v < NV; ++v) div[v] = T(0);
-        const bool upd = k >= k0;
-        if (upd) {
-            const int b = (k - k0 + 2) & 3;
-            T m2[NV], m1[NV], c0[NV], p1[NV], p2[NV];
+        for (int r = 0; r < 2; ++r)
 #pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                m2[v] = P[b][v][li - 2]; m1[v] = P[b][v][li - 1]; c0[v] = P[b][v][li];
-                p1[v] = P[b][v][li + 1]; p2[v] = P[b][v][li + 2];
-            }
-            // tile seams of HY_DONOR: faces at x = i - 1/2 with i mod 32 = 0, y = j - 1/2 with j mod 8 = 0
-            // (the periodic face after the last cell included)
-            const bool lox = SV == HY_DONOR && gx % HM_OX == 0, hix = SV == HY_DONOR && ((gx + 1) % a.nx) % HM_OX == 0;
-            const bool loy = SV == HY_DONOR && gy % HM_OY == 0, hiy = SV == HY_DONOR && ((gy + 1) % a.ny) % HM_OY == 0;
-            hy_dir<T, 0, FB, NV, CMA, LG, SV>(m2, m1, c0, p1, p2, div, a, lox, hix);
+            for (int v = 0; v < NV; ++v) P[(k + 1) & 1][v][li + r * HM_LX] = pp[r][v];
+
+        T div[2][NV];
+        if (k >= k0) {
+            // ---- x: the lane's own states, its lower face; the neighbours by wave shift ----------------
+            const bool seam = SV == HY_DONOR && gx % HM_SEAM_X == 0;
 #pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                m2[v] = P[b][v][li - 2 * HM_LX]; m1[v] = P[b][v][li - HM_LX];
-                p1[v] = P[b][v][li + HM_LX]; p2[v] = P[b][v][li + 2 * HM_LX];
-            }
-            hy_dir<T, 1, FB, NV, CMA, LG, SV>(m2, m1, c0, p1, p2, div, a, loy, hiy);
-        }
-        T Fp[NV];
-        hy_face<T, 2, FB, NV, CMA, LG, SV>(W[0], W[1], W[2], W[3], Fp, a);   // face k+1/2
-        if (upd) {
+            for (int r = 0; r < 2; ++r) {
+                T l[NV], c[NV], n[NV], lo[NV], hi[NV], F[NV];
+                lds(k, li + r * HM_LX - 1, l);
+                lds(k, li + r * HM_LX, c);
+                lds(k, li + r * HM_LX + 1, n);
+                hy_states<T, 0, NV, SV>(l, c, n, lo, hi, a);
 #pragma unroll
-            for (int v = 0; v < NV; ++v) div[v] += Fp[v] - Fz[v];
-            T U[NV], f[NV];
-            hy_flux_cons<T, 0, NV, LG>(W[1], f, U, a);   // toCons(prim(U0)); the flux is unused
-            if (own) {
-                const size_t g = (size_t)k * plane + col;
+                for (int v = 0; v < NV; ++v) hi[v] = lane_prev(hi[v]);
+                if (seam) {
 #pragma unroll
-                for (int v = 0; v < NV; ++v) U[v] = U[v] - a.dtdx * div[v];
-                if (FMT == HY_CONS) {
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) a.o[v][g] = U[v];
-                } else if (PRIM) {   // c2p -> store primitive (spike_25d.cu:499-511)
-                    const T ir = T(1) / tmax(U[0], a.smallr);
-                    const T vx = U[1] * ir, vy = U[2] * ir, vz = U[3] * ir;
-                    const T ke = T(0.5) * U[0] * (vx * vx + vy * vy + vz * vz);
-                    const T pp = tmax(a.gm1 * (U[4] - ke), a.smallp);
-                    if (FMT == HY_F16P) {
-                        a.oh[0][g] = hy_f32_to_f16((float)U[0]);
-                        a.oh[1][g] = hy_f32_to_f16((float)vx);
-                        a.oh[2][g] = hy_f32_to_f16((float)vy);
-                        a.oh[3][g] = hy_f32_to_f16((float)vz);
-                        a.oh[4][g] = hy_f32_to_f16((float)pp);
-                    } else {
-                        a.oh[0][g] = hy_enc_log2s(log2f((float)tmax(U[0], a.smallr)));
-                        a.oh[1][g] = hy_enc_vel((float)vx);
-                        a.oh[2][g] = hy_enc_vel((float)vy);
-                        a.oh[3][g] = hy_enc_vel((float)vz);
-                        a.oh[4][g] = hy_enc_log2s(log2f((float)pp));
-                    }
-                } else {             // HY_U16SP: X_new = (rho X)_new / rho_new -> log2 -> uint16 (:514-517)
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) a.o[v][g] = U[v];
-                    const T rinv = T(1) / tmax(U[0], a.smallr);
-#pragma unroll
-                    for (int v = 5; v < NV; ++v) a.oh[v][g] = hy_enc_log2(log2f(fmaxf((float)(U[v] * rinv), 7.7e-34f)));
+                    for (int v = 0; v < NV; ++v) { hi[v] = l[v]; lo[v] = c[v]; }
                 }
+                hy_riemann<T, 0, fb, NV, CMA, LG>(hi, lo, F, a);
+#pragma unroll
+                for (int v = 0; v < NV; ++v) div[r][v] = lane_next(F[v]) - F[v];
+            }
+            // ---- y: rows -1 .. 2 around the lane's rows 0 and 1, three faces -----------------------------
+            const bool seam0 = SV == HY_DONOR && gy0 % HM_SEAM_Y == 0, seam1 = SV == HY_DONOR && gy1 % HM_SEAM_Y == 0;
+            const bool seam2 = SV == HY_DONOR && ((gy1 + 1) % a.ny) % HM_SEAM_Y == 0;
+            T l[NV], c[NV], n[NV], up[NV], lo[NV], hi[NV], F0[NV], F1[NV];
+            lds(k, li - 2 * HM_LX, l);
+            lds(k, li - HM_LX, c);
+            lds(k, li, n);
+            hy_states<T, 1, NV, SV>(l, c, n, lo, up, a);
+#pragma unroll
+            for (int f = 0; f < 3; ++f) {   // face below row f: (c | n) with c's upper state in `up`
+                T nn[NV];
+                lds(k, li + (f + 1) * HM_LX, nn);
+                hy_states<T, 1, NV, SV>(c, n, nn, lo, hi, a);
+                if (f == 0 ? seam0 : f == 1 ? seam1 : seam2) {
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) { up[v] = c[v]; lo[v] = n[v]; }
+                }
+                hy_riemann<T, 1, fb, NV, CMA, LG>(up, lo, F1, a);
+                if (f > 0) {
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) div[f - 1][v] += F1[v] - F0[v];
+                }
+#pragma unroll
+                for (int v = 0; v < NV; ++v) { F0[v] = F1[v]; c[v] = n[v]; n[v] = nn[v]; up[v] = hi[v]; }
             }
         }
+        // ---- z: states of plane k+1, the face k+1/2, the update of plane k ---------------------------------
 #pragma unroll
-        for (int v = 0; v < NV; ++v) Fz[v] = Fp[v];
-        if (more) commit(k + 3);   // into plane k-1's buffer, last read before the previous barrier
+        for (int r = 0; r < 2; ++r) {
+            T p0[NV], pn[NV], lo[NV], hi[NV], F[NV];
+            lds(k, li + r * HM_LX, p0);
+            prim(pre[r], pn);
+            hy_states<T, 2, NV, SV>(p0, pp[r], pn, lo, hi, a);
+            hy_riemann<T, 2, fb, NV, CMA, LG>(zprev[r], lo, F, a);
+            if (k >= k0 && own[r]) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) div[r][v] += F[v] - Fz[r][v];
+                store((size_t)k * plane + col[r], p0, div[r]);
+            }
+#pragma unroll
+            for (int v = 0; v < NV; ++v) { zprev[r][v] = hi[v]; Fz[r][v] = F[v]; pp[r][v] = pn[v]; }
+        }
+        if (more && halo) {
+            T q[NV];
+            prim(hpre, q);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) P[(k + 1) & 1][v][hi_] = q[v];
+        }
         __syncthreads();
     }
 }

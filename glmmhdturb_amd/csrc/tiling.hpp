@@ -16,8 +16,9 @@ struct Resident {
 // Modelled time, in planes of a workgroup that has its CU for itself, of W workgroups of `len` planes:
 // the CU with the most workgroups takes n = ceil(W / cus) of them, occ at a time, and m resident
 // workgroups slow each other down by 1 + share (m - 1).  share 0 would be perfect overlap, 1 none; the
-// measured marches lie at 0.5-0.7 in FP64 (two resident: 7.7 us a plane alone, 11.8 together) and
-// 0.29-0.38 in FP32 (three or four resident).  Against the sweep of all chunk lengths on grids from
+// measured GLM and CT marches lie at 0.5-0.7 in FP64 (two resident: 7.7 us a plane alone, 11.8 together)
+// and 0.29-0.38 in FP32 (three or four resident), the hydro march, which keeps the VALU busier alone, at
+// 0.9 and 0.6.  Against the sweep of all chunk lengths on grids from
 // 32^3 to 256^3 the choice is within 5% of the best.  (Counting whole rounds over all slots as if
 // resident workgroups did not slow each other, with chunks of at least 8 planes, took 72 us instead
 // of 25 for 32^3 FP64 and 60 instead of 40 for 64^3 FP32.)
