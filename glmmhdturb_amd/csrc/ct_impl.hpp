@@ -50,26 +50,6 @@ GLM_DEV size_t cidx(const CTArgs<T>& a, int i, int j, int k)
     return (size_t)i + (size_t)a.nx * ((size_t)j + (size_t)a.ny * (size_t)k);
 }
 
-// ct_mhd.jl:39-55 dflux in direction D (8 components, F[Bn] = 0)
-template <typename T, int D>
-GLM_DEV void ct_dflux(const T q[8], T f[8], T igm1)
-{
-    const T rho = q[0], vx = q[1], vy = q[2], vz = q[3], p = q[4], bx = q[5], by = q[6], bz = q[7];
-    T b2 = bx * bx + by * by + bz * bz, ptot = p + T(0.5) * b2;
-    T E = p * igm1 + T(0.5) * rho * (vx * vx + vy * vy + vz * vz) + T(0.5) * b2;
-    T vb = vx * bx + vy * by + vz * bz;
-    const T un = D == 0 ? vx : (D == 1 ? vy : vz);
-    const T bn = D == 0 ? bx : (D == 1 ? by : bz);
-    f[0] = rho * un;
-    f[1] = rho * un * vx - bn * bx + (D == 0 ? ptot : T(0));
-    f[2] = rho * un * vy - bn * by + (D == 1 ? ptot : T(0));
-    f[3] = rho * un * vz - bn * bz + (D == 2 ? ptot : T(0));
-    f[4] = (E + ptot) * un - bn * vb;
-    f[5] = D == 0 ? T(0) : un * bx - vx * bn;
-    f[6] = D == 1 ? T(0) : un * by - vy * bn;
-    f[7] = D == 2 ? T(0) : un * bz - vz * bn;
-}
-
 template <typename T>
 GLM_DEV void ct_toC(const T q[8], T u[8], T igm1)
 {
@@ -92,16 +72,14 @@ GLM_DEV T ct_cf(const T q[8], T bn, T gamma)
 template <typename T, int D, typename A>
 GLM_DEV void ct_hanc1d(const T q[8], const T hs[8], T mh[8], const A& a)
 {
-    T t[8], FL[8], FR[8], U[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) t[k] = q[k] - hs[k];
-    ct_dflux<T, D>(t, FL, a.igm1);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) t[k] = q[k] + hs[k];
-    ct_dflux<T, D>(t, FR, a.igm1);
+    const T q9[9] = {q[0], q[1], q[2], q[3], q[4], q[5], q[6], q[7], T(0)};
+    const T h9[9] = {hs[0], hs[1], hs[2], hs[3], hs[4], hs[5], hs[6], hs[7], T(0)};
+    T o[9], U[8], v2, b2, vb;
+    squares(q9, v2, b2, vb);
+    flux_odd<T, D>(q9, h9, v2, b2, vb, o, a.igm1);
     ct_toC(q, U, a.igm1);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) U[k] = U[k] - a.half_dtdx * (FR[k] - FL[k]);
+    for (int k = 0; k < 8; ++k) U[k] = U[k] - T(2) * a.half_dtdx * o[k];
     T rho = tmax(U[0], a.smallr), ir = trcp(rho);
     T vx = U[1] * ir, vy = U[2] * ir, vz = U[3] * ir;
     T p = ct_pressure(U[4], rho, vx, vy, vz, U[5], U[6], U[7], a.gamma, a.smallp);
@@ -155,38 +133,20 @@ GLM_DEV void ct_riemann8(const T Lq[8], const T Rq[8], T bn, const A& a, T f[8])
 #pragma unroll
     for (int k = 0; k < 8; ++k) { L[k] = Lq[k]; R[k] = Rq[k]; }
     L[5 + D] = bn; R[5 + D] = bn;
-    if (RIEM == RIEM_HLLD) {
-        // rotate D to x, Miyoshi-Kusano with the face-normal B and F[Bn] = 0, rotate back
-        constexpr int A_ = D % 3, B_ = (D + 1) % 3, C_ = (D + 2) % 3;
-        T Lr[9] = {L[0], L[1 + A_], L[1 + B_], L[1 + C_], L[4], L[5 + A_], L[5 + B_], L[5 + C_], T(0)};
-        T Rr[9] = {R[0], R[1 + A_], R[1 + B_], R[1 + C_], R[4], R[5 + A_], R[5 + B_], R[5 + C_], T(0)};
-        Phys<T> s;
-        s.gamma = a.gamma; s.igm1 = a.igm1; s.smallr = a.smallr; s.pfl = a.smallp;
-        s.ch = T(1); s.ch2 = T(1); s.half_ich = T(0.5); s.llf_dmin = T(0); s.llf_pmin = T(0);
-        T fx[9];
-        hlld_x(Lr, Rr, fx, s);
-        f[0] = fx[0]; f[4] = fx[4];
-        f[1 + A_] = fx[1]; f[1 + B_] = fx[2]; f[1 + C_] = fx[3];
-        f[5 + A_] = T(0); f[5 + B_] = fx[6]; f[5 + C_] = fx[7];
-        return;
-    }
-    T FL[8], FR[8], UL[8], UR[8];
-    ct_dflux<T, D>(L, FL, a.igm1);
-    ct_dflux<T, D>(R, FR, a.igm1);
-    ct_toC(L, UL, a.igm1);
-    ct_toC(R, UR, a.igm1);
-    const T uL = L[1 + D], uR = R[1 + D];
-    const T cL = ct_cf(L, L[5 + D], a.gamma), cR = ct_cf(R, R[5 + D], a.gamma);
-    if (RIEM == RIEM_LLF) {
-        T smax = tmax(tabs(uL) + cL, tabs(uR) + cR);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) f[k] = T(0.5) * (FL[k] + FR[k]) - T(0.5) * smax * (UR[k] - UL[k]);
-    } else {
-        T SL = tmin(tmin(uL - cL, uR - cR), T(0)), SR = tmax(tmax(uL + cL, uR + cR), T(0));
-        T ih = trcp(SR - SL);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) f[k] = (SR * FL[k] - SL * FR[k] + SL * SR * (UR[k] - UL[k])) * ih;
-    }
+    // rotate D to x, solve with the face-normal B and F[Bn] = 0, rotate back
+    constexpr int A_ = D % 3, B_ = (D + 1) % 3, C_ = (D + 2) % 3;
+    T Lr[9] = {L[0], L[1 + A_], L[1 + B_], L[1 + C_], L[4], L[5 + A_], L[5 + B_], L[5 + C_], T(0)};
+    T Rr[9] = {R[0], R[1 + A_], R[1 + B_], R[1 + C_], R[4], R[5 + A_], R[5 + B_], R[5 + C_], T(0)};
+    Phys<T> s;
+    s.gamma = a.gamma; s.igm1 = a.igm1; s.smallr = a.smallr; s.pfl = a.smallp;
+    s.ch = T(0); s.ch2 = T(0); s.half_ich = T(0); s.llf_dmin = T(0); s.llf_pmin = T(0);   // no cleaning, no switch
+    T fx[9];
+    if (RIEM == RIEM_HLLD) hlld_x(Lr, Rr, fx, s);
+    else if (RIEM == RIEM_LLF) llf_x<T, false>(Lr, Rr, fx, s);
+    else hll_x(Lr, Rr, fx, s);
+    f[0] = fx[0]; f[4] = fx[4];
+    f[1 + A_] = fx[1]; f[1 + B_] = fx[2]; f[1 + C_] = fx[3];
+    f[5 + A_] = T(0); f[5 + B_] = fx[6]; f[5 + C_] = fx[7];
 }
 
 // ct_riemann8 plus the species fluxes of an NV-value state: F_s = F_rho X_s of the upwind face

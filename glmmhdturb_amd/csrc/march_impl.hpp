@@ -181,16 +181,12 @@ GLM_DEV void guard(T f[NV], const T m0[NV], int g, const Phys<T>& s)
 template <typename T, int D, int NV>
 GLM_DEV void hanc1d(const T c0[NV], const T hs[NV], T mh[NV], T half_dtdx, const Phys<T>& s)
 {
-    T t[9], fa[9], fb[9], u[9];
-#pragma unroll
-    for (int v = 0; v < 9; ++v) t[v] = c0[v] - hs[v];
-    flux_dir<T, D>(t, fa, s);
-#pragma unroll
-    for (int v = 0; v < 9; ++v) t[v] = c0[v] + hs[v];
-    flux_dir<T, D>(t, fb, s);
+    T o[9], u[9], v2, b2, vb;
+    squares(c0, v2, b2, vb);
+    flux_odd<T, D>(c0, hs, v2, b2, vb, o, s.igm1);
     prim2cons(c0, u, s);
 #pragma unroll
-    for (int v = 0; v < 9; ++v) u[v] -= half_dtdx * (fb[v] - fa[v]);
+    for (int v = 0; v < 9; ++v) u[v] -= T(2) * half_dtdx * o[v];
     cons2prim(u, mh, s);
     // species: the advective half step X - dt/dx u_D hs (spike_mhd.cu:155-159, hs the half slope)
 #pragma unroll
@@ -404,50 +400,30 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile)
         if (PRED == PRED_FULL && !MF) {
             // glmmhd_turb.jl:165-172 hancock, :391-395 revert: U0 - dt/(2dx) sum_d [F_d(m0+s_d) - F_d(m0-s_d)];
             // species: the advective half step X - dt/dx (u hs_x + v hs_y + w hs_z)
-            T acc[9], t[9], f[9], hs[NV], sadv[NS > 0 ? NS : 1];
+            T acc[9], t[9], f[9], hs[NV], sadv[NS > 0 ? NS : 1], v2, b2, vb;
+            squares(p0, v2, b2, vb);
 #pragma unroll
             for (int v = 0; v < NV; ++v) hs[v] = half_slope<T, SLOPE>(P[v][lo_own - 1], p0[v], P[v][lo_own + 1]);
 #pragma unroll
             for (int v = 9; v < NV; ++v) sadv[v - 9] = p0[1] * hs[v];
-#pragma unroll
-            for (int v = 0; v < 9; ++v) t[v] = p0[v] + hs[v];
-            flux_dir<T, 0>(t, acc, s);
-#pragma unroll
-            for (int v = 0; v < 9; ++v) t[v] = p0[v] - hs[v];
-            flux_dir<T, 0>(t, f, s);
-#pragma unroll
-            for (int v = 0; v < 9; ++v) acc[v] -= f[v];
+            flux_odd<T, 0>(p0, hs, v2, b2, vb, acc, s.igm1);
 #pragma unroll
             for (int v = 0; v < NV; ++v) hs[v] = half_slope<T, SLOPE>(P[v][lo_own - PX], p0[v], P[v][lo_own + PX]);
 #pragma unroll
             for (int v = 9; v < NV; ++v) sadv[v - 9] = sadv[v - 9] + p0[2] * hs[v];
-#pragma unroll
-            for (int v = 0; v < 9; ++v) t[v] = p0[v] + hs[v];
-            flux_dir<T, 1>(t, f, s);
+            flux_odd<T, 1>(p0, hs, v2, b2, vb, f, s.igm1);
 #pragma unroll
             for (int v = 0; v < 9; ++v) acc[v] += f[v];
-#pragma unroll
-            for (int v = 0; v < 9; ++v) t[v] = p0[v] - hs[v];
-            flux_dir<T, 1>(t, f, s);
-#pragma unroll
-            for (int v = 0; v < 9; ++v) acc[v] -= f[v];
 #pragma unroll
             for (int v = 0; v < NV; ++v) hs[v] = half_slope<T, SLOPE>(pm[v], p0[v], pp[v]);
 #pragma unroll
             for (int v = 9; v < NV; ++v) sadv[v - 9] = sadv[v - 9] + p0[3] * hs[v];
-#pragma unroll
-            for (int v = 0; v < 9; ++v) t[v] = p0[v] + hs[v];
-            flux_dir<T, 2>(t, f, s);
+            flux_odd<T, 2>(p0, hs, v2, b2, vb, f, s.igm1);
 #pragma unroll
             for (int v = 0; v < 9; ++v) acc[v] += f[v];
-#pragma unroll
-            for (int v = 0; v < 9; ++v) t[v] = p0[v] - hs[v];
-            flux_dir<T, 2>(t, f, s);
-#pragma unroll
-            for (int v = 0; v < 9; ++v) acc[v] -= f[v];
             prim2cons(p0, t, s);
 #pragma unroll
-            for (int v = 0; v < 9; ++v) t[v] = t[v] - a.half_dtdx * acc[v];
+            for (int v = 0; v < 9; ++v) t[v] = t[v] - a.dtdx * acc[v];   // acc: half the differences
             cons2prim(t, mh, s);
 #pragma unroll
             for (int v = 9; v < NV; ++v) mh[v] = p0[v] - a.dtdx * sadv[v - 9];
