@@ -94,6 +94,25 @@ __global__ void __launch_bounds__(ENS_MAX_BOXES) ens_ctl_kernel(EnsBox* eb, Marc
     t1[(size_t)slot * nbox + b] = 0ull;
 }
 
+// The CFL max of every box's first buffer (blockIdx.y: the box) into its control block.
+template <typename T>
+__global__ void __launch_bounds__(256) ens_ctot_kernel(EnsBox* eb, const MarchArgs<T>* ma)
+{
+    EnsBox& e = eb[blockIdx.y];
+    const MarchArgs<T>& m = ma[blockIdx.y];
+    const size_t n = (size_t)m.nx * m.ny * m.nz;
+    unsigned long long best = 0ull;
+    for (size_t c = (size_t)blockIdx.x * 256 + threadIdx.x; c < n; c += (size_t)gridDim.x * 256) {
+        T u[9], p[9];
+#pragma unroll
+        for (int v = 0; v < 9; ++v) u[v] = gload((const T*)e.u[0][v] + c);
+        cons2prim(u, p, m.ph);
+        const unsigned long long b = (unsigned long long)__double_as_longlong(cfl_speed(p, m.ph));
+        best = b > best ? b : best;
+    }
+    block_max_bits<256>(best, &e.cmax);
+}
+
 }  // namespace glm
 
 struct glm_ens {
@@ -109,8 +128,7 @@ struct glm_ens {
     EnsBox* d_eb;
     void* d_ma;            // MarchArgs<T>[nbox]
     OUBox* d_ou;
-    int* d_order;
-    int* d_tile_off;
+    EnsTile* d_tiles;         // flat tile list: box and its local tile (replaced when the layout changes)
     unsigned int* d_queue;
     long long* d_sweep;
     double* d_log;
@@ -120,6 +138,7 @@ struct glm_ens {
     int total, grid;
     // graph
     int use_graph;
+    long long enqueued;    // sweeps enqueued since the last reset: each flips every box's buffers
     hipGraph_t graph;
     hipGraphExec_t exec;
 };
@@ -134,7 +153,7 @@ void ens_free(glm_ens* e)
     if (e->exec) (void)hipGraphExecDestroy(e->exec);
     if (e->graph) (void)hipGraphDestroy(e->graph);
     if (e->stream) (void)hipStreamSynchronize(e->stream);
-    void* ptrs[] = {e->d_eb, e->d_ma, e->d_ou, e->d_order, e->d_tile_off, e->d_queue, e->d_sweep, e->d_log,
+    void* ptrs[] = {e->d_eb, e->d_ma, e->d_ou, e->d_tiles, e->d_queue, e->d_sweep, e->d_log,
                     e->d_t0, e->d_t1};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -173,7 +192,8 @@ int ens_zchunk(const glm_ens* e)
 
 // The flat tile list of a configuration: position order, tile offsets, per-box tiling.
 struct Layout {
-    std::vector<int> order, tile_off, tiles_x, tiles_y, nzc, zchunk;
+    std::vector<int> order, tiles_x, tiles_y, nzc, zchunk;
+    std::vector<EnsTile> tiles;   // box and local tile of every flat tile
     int total = 0;
 };
 
@@ -188,20 +208,14 @@ Layout make_layout(const glm_ens* e, int zreq, int ord)
         std::stable_sort(L.order.begin(), L.order.end(), [&](int a, int b) { return cells(a) > cells(b); });
     }
     L.tiles_x.resize(n); L.tiles_y.resize(n); L.nzc.resize(n); L.zchunk.resize(n);
-    L.tile_off.resize(n + 1);
     const int z = zreq > 0 ? zreq : ens_zchunk(e);
     for (int b = 0; b < n; ++b) {
         const glm_ens_box& x = e->box[b];
         march_tiles(x.nx, x.ny, x.nz, OX, OY, box_zchunk(x.nz, z), e->res, 0.0, 0.0, L.tiles_x[b], L.tiles_y[b], L.nzc[b], L.zchunk[b]);
     }
-    int off = 0;
-    for (int p = 0; p < n; ++p) {
-        L.tile_off[p] = off;
-        const int b = L.order[p];
-        off += L.tiles_x[b] * L.tiles_y[b] * L.nzc[b];
-    }
-    L.tile_off[n] = off;
-    L.total = off;
+    for (int b : L.order)
+        for (int t = 0; t < L.tiles_x[b] * L.tiles_y[b] * L.nzc[b]; ++t) L.tiles.push_back(EnsTile{b, t});
+    L.total = (int)L.tiles.size();
     return L;
 }
 
@@ -244,14 +258,12 @@ std::vector<MarchArgs<T>> make_args(const glm_ens* e, const Layout& L, unsigned 
 }
 
 template <typename T>
-EnsLaunch<T> make_launch(const glm_ens* e, const void* ma, const int* order, const int* tile_off, int total,
-                         int persistent, unsigned long long* t0, unsigned long long* t1)
+EnsLaunch<T> make_launch(const glm_ens* e, const void* ma, const EnsTile* tiles, int total, int persistent,
+                         unsigned long long* t0, unsigned long long* t1)
 {
     EnsLaunch<T> l;
     l.boxes = (const MarchArgs<T>*)ma;
-    l.order = order;
-    l.tile_off = tile_off;
-    l.npos = e->nbox;
+    l.tiles = tiles;
     l.total = total;
     l.persistent = persistent > 0 ? 1 : 0;
     l.nbox = e->nbox;
@@ -269,11 +281,28 @@ int grid_of(const glm_ens* e, int total, int persistent)
     return g < total ? g : total;
 }
 
+// The tile list of a layout in device memory (the caller's to free).
+int upload_tiles(const Layout& L, EnsTile** out)
+{
+    if (hipMalloc(out, L.tiles.size() * sizeof(EnsTile)) != hipSuccess)
+        return set_err(GLM_ERR_ALLOC, "glm_ens: tile list allocation failed");
+    if (hipMemcpy(*out, L.tiles.data(), L.tiles.size() * sizeof(EnsTile), hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipFree(*out);
+        *out = nullptr;
+        return set_err(GLM_ERR_HIP, "glm_ens: tile list upload failed");
+    }
+    return GLM_OK;
+}
+
 int apply_config(glm_ens* e, int zreq, int persistent, int ord)
 {
     Layout L = make_layout(e, zreq, ord);
     if (L.total <= 0) return set_err(GLM_ERR_ARG, "glm_ens: empty tile list");
     HIPCHK(hipStreamSynchronize(e->stream));
+    EnsTile* tiles = nullptr;
+    if (int err = upload_tiles(L, &tiles)) return err;
+    if (e->d_tiles) (void)hipFree(e->d_tiles);
+    e->d_tiles = tiles;
     // the step control rewrites the per-step fields every sweep; the rest comes from here
     if (e->prec == 8) {
         auto v = make_args<double>(e, L, nullptr);
@@ -284,8 +313,6 @@ int apply_config(glm_ens* e, int zreq, int persistent, int ord)
         for (int b = 0; b < e->nbox; ++b) v[b].cmax = &e->d_eb[b].cmax;
         HIPCHK(hipMemcpy(e->d_ma, v.data(), v.size() * sizeof v[0], hipMemcpyHostToDevice));
     }
-    HIPCHK(hipMemcpy(e->d_order, L.order.data(), e->nbox * sizeof(int), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(e->d_tile_off, L.tile_off.data(), (e->nbox + 1) * sizeof(int), hipMemcpyHostToDevice));
     e->zchunk = zreq; e->persistent = persistent; e->order = ord;
     e->total = L.total;
     e->grid = grid_of(e, L.total, persistent);
@@ -308,11 +335,11 @@ int enqueue_sweep(glm_ens* e)
     HIPCHK(hipGetLastError());
     if (e->any_turb) HIPCHK(launch_ou_advance(e->prec, e->d_ou, e->nbox, e->gmax, e->nbmax, -1, e->stream));
     if (e->prec == 8)
-        HIPCHK(launch_ens<double>(make_launch<double>(e, e->d_ma, e->d_order, e->d_tile_off, e->total, e->persistent,
+        HIPCHK(launch_ens<double>(make_launch<double>(e, e->d_ma, e->d_tiles, e->total, e->persistent,
                                                       e->d_t0, e->d_t1),
                                   p.predictor, p.riemann, p.recon, p.slope, e->grid, e->stream));
     else
-        HIPCHK(launch_ens<float>(make_launch<float>(e, e->d_ma, e->d_order, e->d_tile_off, e->total, e->persistent,
+        HIPCHK(launch_ens<float>(make_launch<float>(e, e->d_ma, e->d_tiles, e->total, e->persistent,
                                                     e->d_t0, e->d_t1),
                                  p.predictor, p.riemann, p.recon, p.slope, e->grid, e->stream));
     return GLM_OK;
@@ -394,8 +421,6 @@ glm_ens* glm_ens_create(int nbox, const glm_ens_box* boxes, const glm_params* sc
     if (hipMalloc(&e->d_eb, nbox * sizeof(EnsBox)) != hipSuccess ||
         hipMalloc(&e->d_ma, nbox * ma_bytes(precision)) != hipSuccess ||
         hipMalloc(&e->d_ou, nbox * sizeof(OUBox)) != hipSuccess ||
-        hipMalloc(&e->d_order, nbox * sizeof(int)) != hipSuccess ||
-        hipMalloc(&e->d_tile_off, (nbox + 1) * sizeof(int)) != hipSuccess ||
         hipMalloc(&e->d_queue, NXCD * sizeof(unsigned int)) != hipSuccess ||
         hipMalloc(&e->d_sweep, sizeof(long long)) != hipSuccess ||
         hipMalloc(&e->d_log, logn * 8 * sizeof(double)) != hipSuccess ||
@@ -451,27 +476,19 @@ int glm_ens_reset(glm_ens* e)
         }
     }
     HIPCHK(hipMemcpy(e->d_eb, eb.data(), eb.size() * sizeof(EnsBox), hipMemcpyHostToDevice));
-    for (int b = 0; b < e->nbox; ++b)
-        if (e->box[b].do_turb) HIPCHK(ou_box_reset(e->ou[b], e->prec, e->stream));
     HIPCHK(hipMemcpyAsync(e->d_ou, e->ou.data(), e->nbox * sizeof(OUBox), hipMemcpyHostToDevice, e->stream));
     const long long minus1 = -1;
     HIPCHK(hipMemcpyAsync(e->d_sweep, &minus1, sizeof minus1, hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipMemsetAsync(e->d_log, 0, (size_t)ENS_LOG * e->nbox * 8 * sizeof(double), e->stream));
-    for (int b = 0; b < e->nbox; ++b) {
-        const glm_ens_box& x = e->box[b];
-        const size_t n = (size_t)x.nx * x.ny * x.nz;
-        glm_params p = e->scheme;
-        p.ch = 1.0;
-        if (e->prec == 8) {
-            Ptr9<const double> q;
-            for (int v = 0; v < 9; ++v) q.p[v] = (const double*)x.u0[v];
-            HIPCHK(launch_ctot<double>(q, n, make_phys<double>(&p), &e->d_eb[b].cmax, e->stream));
-        } else {
-            Ptr9<const float> q;
-            for (int v = 0; v < 9; ++v) q.p[v] = (const float*)x.u0[v];
-            HIPCHK(launch_ctot<float>(q, n, make_phys<float>(&p), &e->d_eb[b].cmax, e->stream));
-        }
-    }
+    // one launch each for all boxes: 16 boxes took 48 fills and 16 maxima one after another, 0.6 ms
+    if (e->any_turb) HIPCHK(launch_ou_reset(e->prec, e->d_ou, e->nbox, e->gmax, e->stream));
+    size_t nmax = 1;
+    for (const glm_ens_box& x : e->box) nmax = std::max(nmax, (size_t)x.nx * x.ny * x.nz);
+    const dim3 grid(red_blocks(nmax), (unsigned)e->nbox);
+    if (e->prec == 8) hipLaunchKernelGGL((ens_ctot_kernel<double>), grid, dim3(256), 0, e->stream, e->d_eb, (const MarchArgs<double>*)e->d_ma);
+    else hipLaunchKernelGGL((ens_ctot_kernel<float>), grid, dim3(256), 0, e->stream, e->d_eb, (const MarchArgs<float>*)e->d_ma);
+    HIPCHK(hipGetLastError());
+    e->enqueued = 0;
     HIPCHK(hipStreamSynchronize(e->stream));
     return GLM_OK;
 }
@@ -485,6 +502,7 @@ int glm_ens_step(glm_ens* e, int nsweeps)
             int err = enqueue_sweep(e);
             if (err) return err;
         }
+        e->enqueued += 1;
     }
     return GLM_OK;
 }
@@ -524,10 +542,8 @@ long long glm_ens_sweeps(glm_ens* e)
 int glm_ens_current(glm_ens* e, int box, void** planes)
 {
     if (!e || !planes || box < 0 || box >= e->nbox) return set_err(GLM_ERR_ARG, "glm_ens_current: bad argument");
-    int par = 0;
-    HIPCHK(hipMemcpyAsync(&par, (char*)(e->d_eb + box) + offsetof(EnsBox, parity), sizeof par,
-                          hipMemcpyDeviceToHost, e->stream));
     HIPCHK(hipStreamSynchronize(e->stream));
+    const int par = (int)(e->enqueued & 1);   // the step control starts at u0 and flips every box in each sweep
     for (int v = 0; v < 9; ++v) planes[v] = par ? e->box[box].u1[v] : e->box[box].u0[v];
     return GLM_OK;
 }
@@ -586,7 +602,7 @@ int glm_ens_tune(glm_ens* e, int reps, int* best, double* best_ms)
     HIPCHK(hipMemcpy(eb.data(), e->d_eb, eb.size() * sizeof(EnsBox), hipMemcpyDeviceToHost));
     const int occ = e->res.occ;
     void* ma = nullptr;
-    int *order = nullptr, *toff = nullptr;
+    EnsTile* tiles = nullptr;
     unsigned long long *slots = nullptr, *t0 = nullptr, *t1 = nullptr;
     const size_t logn = (size_t)ENS_LOG * e->nbox;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -594,8 +610,6 @@ int glm_ens_tune(glm_ens* e, int reps, int* best, double* best_ms)
     double bms = 1e300;
     int bz = e->zchunk, bp = e->persistent, bo = e->order;
     if (hipMalloc(&ma, e->nbox * ma_bytes(e->prec)) != hipSuccess ||
-        hipMalloc(&order, e->nbox * sizeof(int)) != hipSuccess ||
-        hipMalloc(&toff, (e->nbox + 1) * sizeof(int)) != hipSuccess ||
         hipMalloc(&slots, e->nbox * sizeof(unsigned long long)) != hipSuccess ||
         hipMalloc(&t0, logn * sizeof(unsigned long long)) != hipSuccess ||
         hipMalloc(&t1, logn * sizeof(unsigned long long)) != hipSuccess)
@@ -628,11 +642,9 @@ int glm_ens_tune(glm_ens* e, int reps, int* best, double* best_ms)
                 };
                 err = e->prec == 8 ? fill(double()) : fill(float());
                 if (err) break;
-                if (hipMemcpy(order, L.order.data(), e->nbox * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
-                    hipMemcpy(toff, L.tile_off.data(), (e->nbox + 1) * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
-                    err = set_err(GLM_ERR_HIP, "glm_ens_tune: table upload failed");
-                    break;
-                }
+                if (tiles) (void)hipFree(tiles);
+                tiles = nullptr;
+                if ((err = upload_tiles(L, &tiles))) break;
                 const int grid = grid_of(e, L.total, pm);
                 std::vector<float> ms;
                 for (int r = 0; r <= reps && !err; ++r) {   // one untimed warm-up launch
@@ -643,9 +655,9 @@ int glm_ens_tune(glm_ens* e, int reps, int* best, double* best_ms)
                         break;
                     }
                     hipError_t le = e->prec == 8
-                        ? launch_ens<double>(make_launch<double>(e, ma, order, toff, L.total, pm, t0, t1), e->scheme.predictor,
+                        ? launch_ens<double>(make_launch<double>(e, ma, tiles, L.total, pm, t0, t1), e->scheme.predictor,
                                              e->scheme.riemann, e->scheme.recon, e->scheme.slope, grid, e->stream)
-                        : launch_ens<float>(make_launch<float>(e, ma, order, toff, L.total, pm, t0, t1), e->scheme.predictor,
+                        : launch_ens<float>(make_launch<float>(e, ma, tiles, L.total, pm, t0, t1), e->scheme.predictor,
                                             e->scheme.riemann, e->scheme.recon, e->scheme.slope, grid, e->stream);
                     if (le != hipSuccess || hipEventRecord(ev1, e->stream) != hipSuccess ||
                         hipEventSynchronize(ev1) != hipSuccess) {
@@ -663,7 +675,7 @@ int glm_ens_tune(glm_ens* e, int reps, int* best, double* best_ms)
             }
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
-    void* ptrs[] = {ma, order, toff, slots, t0, t1};
+    void* ptrs[] = {ma, tiles, slots, t0, t1};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (err) return err;

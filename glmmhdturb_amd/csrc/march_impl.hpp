@@ -605,18 +605,22 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GLM_WAV
 
 // ---------------------------------------------------------------------------------------------
 // Ensemble: many boxes of uneven size in one launch per sweep.  The boxes' tiles form one flat
-// list (box positions in a chosen order, each box's tiles contiguous in its own x, y, z-chunk
-// order); tile_off[pos] is the first flat tile of position pos.  Each box's MarchArgs live in
+// list (boxes in a chosen order, each box's tiles contiguous in its own x, y, z-chunk order), one
+// entry a tile with its box and local tile, so that a workgroup finds its work in one load (a
+// search over the boxes' offsets was 4-5 dependent ones).  Each box's MarchArgs live in
 // device memory and are refreshed every sweep by the step-control kernel (ens.hip).
 // ---------------------------------------------------------------------------------------------
 constexpr int ENS_LOG = 256;   // sweeps kept in the per-box log and timing records
 
+struct EnsTile {
+    int box, lt;
+};
+
 template <typename T>
 struct EnsLaunch {
     const MarchArgs<T>* boxes;   // per box
-    const int* order;            // flat position -> box
-    const int* tile_off;         // [npos + 1]
-    int npos, total;             // positions and flat tiles
+    const EnsTile* tiles;        // [total]
+    int total;                   // flat tiles
     int persistent;              // 0: workgroup w marches flat tile xcd_block(w); 1: workgroups take
                                  // tiles from per-XCD queues and steal from the others when theirs is empty
     int nbox;
@@ -635,47 +639,35 @@ GLM_DEV int xcd_start(int x, int total)
 }
 GLM_DEV int xcd_count(int x, int total) { return total / NXCD + (x < total % NXCD ? 1 : 0); }
 
-// Thread 0 claims the workgroup's next tile (flat: its own, once; persistent: a ticket from the
-// XCD queues, stealing when its own is empty), finds the box by binary search over the tile
-// offsets and stages the box's cold arguments; the job is published in s_job after a barrier.
-template <typename T, bool PERSIST>
-GLM_DEV void ens_claim(const EnsLaunch<T>& e, int it, int& xq, unsigned long long* s_tb, MarchLDS<T>& L, int* s_job)
+// A persistent workgroup's next tile (thread 0): a ticket from the XCD queues, stealing from the others when
+// its own is empty.  Publishes box (-1: no more work) and local tile in s_job.
+template <typename T>
+GLM_DEV void ens_claim(const EnsLaunch<T>& e, int& xq, int* s_job)
 {
     int tile = -1;
-    if (!PERSIST) {
-        if (it == 0) tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
-    } else {
-        for (int k = 0; k < NXCD && tile < 0; ++k) {
-            const int x = (xq + k) % NXCD;
-            const unsigned tk = atomicAdd(&e.queue[x], 1u);
-            if (tk < (unsigned)xcd_count(x, e.total)) {
-                tile = xcd_start(x, e.total) + (int)tk;
-                xq = x;
-            }
+    for (int k = 0; k < NXCD && tile < 0; ++k) {
+        const int x = (xq + k) % NXCD;
+        const unsigned tk = atomicAdd(&e.queue[x], 1u);
+        if (tk < (unsigned)xcd_count(x, e.total)) {
+            tile = xcd_start(x, e.total) + (int)tk;
+            xq = x;
         }
     }
-    int box = -1, lt = 0;
-    if (tile >= 0) {
-        int lo = 0, hi = e.npos;   // tile_off[lo] <= tile < tile_off[lo + 1]
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (e.tile_off[mid] <= tile) lo = mid; else hi = mid;
-        }
-        box = e.order[lo];
-        lt = tile - e.tile_off[lo];
-        stage_cold(e.boxes[box], L.ca);
-        *s_tb = (unsigned long long)wall_clock64();
-    }
-    s_job[0] = box;
-    s_job[1] = lt;
+    s_job[0] = tile >= 0 ? e.tiles[tile].box : -1;
+    s_job[1] = tile >= 0 ? e.tiles[tile].lt : 0;
 }
 
 // The march of one claimed tile, its CFL merge into the box's slot and the box's timing record
 // (the start time waits in LDS, out of the registers the march needs).
 template <typename T, int PRED, int RIEM, int RECON, int SLOPE>
-GLM_DEV void ens_tile(const EnsLaunch<T>& e, MarchLDS<T>& L, int box, int lt, int slot, const unsigned long long* s_tb)
+GLM_DEV void ens_tile(const EnsLaunch<T>& e, MarchLDS<T>& L, int box, int lt, int slot, unsigned long long* s_tb)
 {
     const auto& a = constant_ref(e.boxes + box);
+    if (threadIdx.x == 0) {
+        stage_cold(e.boxes[box], L.ca);
+        *s_tb = (unsigned long long)wall_clock64();
+    }
+    __syncthreads();
     const double cmax = march_tile<T, PRED, RIEM, RECON, SLOPE>(a, L, lt);
     cfl_merge(L, cmax, a.cmax);
     if (threadIdx.x == 0) {
@@ -692,22 +684,17 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GLM_WAV
 {
     __shared__ MarchLDS<T> L;
     __shared__ int s_job[2];   // box (-1: no more work) and its local tile
-    __shared__ unsigned long long s_tb;   // wall clock at the claim
-    const int tid = threadIdx.x;
+    __shared__ unsigned long long s_tb;   // wall clock at the start of the tile
     const long long sw = *e.sweep;   // -1 before the first sweep (tuning launches)
     const int slot = (int)((sw < 0 ? 0 : sw) % ENS_LOG);
-    int xq = (int)blockIdx.x % NXCD;
     if (!PERSIST) {
-        if (tid == 0) ens_claim<T, false>(e, 0, xq, &s_tb, L, s_job);
-        __syncthreads();
-        const int box = __builtin_amdgcn_readfirstlane(s_job[0]);
-        const int lt = __builtin_amdgcn_readfirstlane(s_job[1]);
-        if (box < 0) return;
-        ens_tile<T, PRED, RIEM, RECON, SLOPE>(e, L, box, lt, slot, &s_tb);
+        const auto& t = constant_ref(e.tiles + xcd_block((int)blockIdx.x, (int)gridDim.x));
+        ens_tile<T, PRED, RIEM, RECON, SLOPE>(e, L, t.box, t.lt, slot, &s_tb);
         return;
     }
-    for (int it = 0;; ++it) {
-        if (tid == 0) ens_claim<T, true>(e, it, xq, &s_tb, L, s_job);
+    int xq = (int)blockIdx.x % NXCD;
+    for (;;) {
+        if (threadIdx.x == 0) ens_claim(e, xq, s_job);
         __syncthreads();
         const int box = __builtin_amdgcn_readfirstlane(s_job[0]);
         const int lt = __builtin_amdgcn_readfirstlane(s_job[1]);

@@ -66,15 +66,6 @@ void ou_box_free(OUBox& b)
     memset(&b, 0, sizeof b);
 }
 
-hipError_t ou_box_reset(const OUBox& b, int prec, hipStream_t st)
-{
-    const size_t nb = b.nb, gg = (size_t)b.g * b.g;
-    hipError_t e = hipMemsetAsync(b.fre, 0, 3 * nb * nb * nb * 8, st);
-    if (e == hipSuccess) e = hipMemsetAsync(b.fim, 0, 3 * nb * nb * nb * 8, st);
-    if (e == hipSuccess) e = hipMemsetAsync(b.afield, 0, 3 * gg * b.g * prec, st);
-    return e;
-}
-
 static unsigned blocks_for(size_t work, int nbox)
 {
     size_t cap = (size_t)(2048 / (nbox > 0 ? nbox : 1));
@@ -91,10 +82,25 @@ hipError_t launch_ou_advance(int prec, const OUBox* d_boxes, int nbox, int gmax,
     dim3 bl(256);
     hipLaunchKernelGGL(ou_band_step_kernel, dim3(blocks_for(nb * nb * nb, nbox), nbox), bl, 0, st, d_boxes, step_all);
     hipLaunchKernelGGL(ou_pass_x_kernel, dim3(blocks_for(3 * nb * nb * g, nbox), nbox), bl, 0, st, d_boxes, step_all);
+    // one plane of the y and z passes in LDS where its nb x g complex values fit (kmax 3 on a 64^3 forcing
+    // grid: 7 KB); the separate passes for wide bands on large grids
+    const size_t lds = 2 * nb * g * sizeof(double);
+    if (lds <= 64 * 1024) {
+        dim3 gp((unsigned)(3 * g), nbox);
+        if (prec == 8) hipLaunchKernelGGL((ou_pass_yz_kernel<double>), gp, bl, lds, st, d_boxes, step_all);
+        else hipLaunchKernelGGL((ou_pass_yz_kernel<float>), gp, bl, lds, st, d_boxes, step_all);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(ou_pass_y_kernel, dim3(blocks_for(3 * nb * g * g, nbox), nbox), bl, 0, st, d_boxes, step_all);
     dim3 gz(blocks_for(3 * g * g * g, nbox), nbox);
     if (prec == 8) hipLaunchKernelGGL((ou_pass_z_kernel<double>), gz, bl, 0, st, d_boxes, step_all);
     else hipLaunchKernelGGL((ou_pass_z_kernel<float>), gz, bl, 0, st, d_boxes, step_all);
+    return hipGetLastError();
+}
+
+hipError_t launch_ou_reset(int prec, const OUBox* d_boxes, int nbox, int gmax, hipStream_t st)
+{
+    hipLaunchKernelGGL(ou_reset_kernel, dim3(blocks_for(3 * (size_t)gmax * gmax * gmax, nbox), nbox), dim3(256), 0, st, d_boxes, prec);
     return hipGetLastError();
 }
 

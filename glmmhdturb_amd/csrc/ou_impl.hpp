@@ -172,4 +172,69 @@ __global__ void ou_pass_z_kernel(const OUBox* boxes, long long step_all)
     }
 }
 
+// The y and z passes as one: a workgroup takes one (component, j) plane, sums w2[ed][i] for it into LDS and
+// the g x g outputs (k, i) from there, so w2 does not go through memory.  The twiddle index (mode * j) mod g
+// of successive modes is carried by addition (with a division per term the y and z passes of 16 boxes on 32^3..64^3
+// forcing grids took 125 us, now 75).  The sums run over the modes in the passes' order.
+template <typename T>
+__global__ void __launch_bounds__(256) ou_pass_yz_kernel(const OUBox* boxes, long long step_all)
+{
+    extern __shared__ double ou_w2[];   // [nb][g] real parts, then imaginary parts
+    const OUBox& b = boxes[blockIdx.y];
+    unsigned long long step;
+    if (!ou_active(b, step_all, step)) return;
+    const int g = b.g, nb = b.nb, K = b.K;
+    const size_t gg = (size_t)g * g, g3 = gg * g;
+    double *w2r = ou_w2, *w2i = ou_w2 + (size_t)nb * g;
+    T* af = (T*)b.afield;
+    for (int cj = blockIdx.x; cj < 3 * g; cj += gridDim.x) {
+        const int c = cj / g, j = cj % g;
+        const int jump_j = (int)(((size_t)band_mode(K + 1 < nb ? K + 1 : 0, nb, K, g) * j) % g);
+        for (int e = threadIdx.x; e < nb * g; e += blockDim.x) {
+            const int ed = e / g, i = e % g;
+            const size_t base = ((size_t)c * nb + ed) * nb * g + i;
+            double sr = 0.0, si = 0.0;
+            int tw = 0;   // (band_mode(eb) * j) mod g
+            for (int eb = 0; eb < nb; ++eb) {
+                if (eb == K + 1) tw = jump_j;
+                const double xr = b.w1r[base + (size_t)eb * g], xi = b.w1i[base + (size_t)eb * g];
+                sr += xr * b.cs[tw] - xi * b.sn[tw];
+                si += xr * b.sn[tw] + xi * b.cs[tw];
+                tw += j;
+                if (tw >= g) tw -= g;
+            }
+            w2r[e] = sr;
+            w2i[e] = si;
+        }
+        __syncthreads();
+        for (int e = threadIdx.x; e < g * g; e += blockDim.x) {
+            const int k = e / g, i = e % g;
+            double sr = 0.0;
+            int tw = 0;   // (band_mode(ed) * k) mod g
+            for (int ed = 0; ed < nb; ++ed) {
+                if (ed == K + 1) tw = (int)(((size_t)band_mode(ed, nb, K, g) * k) % g);
+                sr += w2r[ed * g + i] * b.cs[tw] - w2i[ed * g + i] * b.sn[tw];
+                tw += k;
+                if (tw >= g) tw -= g;
+            }
+            af[c * g3 + k * gg + (size_t)j * g + i] = (T)(sr * b.scale);
+        }
+        __syncthreads();
+    }
+}
+
+// Zero the OU state and the forcing field of every box (blockIdx.y): a restart from F = 0.
+__global__ void __launch_bounds__(256) ou_reset_kernel(const OUBox* boxes, int prec)
+{
+    const OUBox& b = boxes[blockIdx.y];
+    if (!b.fre) return;   // an unforced box
+    const size_t nf = 3 * (size_t)b.nb * b.nb * b.nb, na = 3 * (size_t)b.g * b.g * b.g;
+    const size_t t0 = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+    for (size_t t = t0; t < nf; t += step) { b.fre[t] = 0.0; b.fim[t] = 0.0; }
+    for (size_t t = t0; t < na; t += step) {
+        if (prec == 8) ((double*)b.afield)[t] = 0.0;
+        else ((float*)b.afield)[t] = 0.0f;
+    }
+}
+
 }  // namespace glm

@@ -28,8 +28,8 @@ int ou_band_width(int g, double kmax);
 hipError_t ou_box_alloc(OUBox& b, int g, double kmin, double kmax, double T, int ndt, double comp, double amp,
                         unsigned long long seed, int prec, hipStream_t st);
 void ou_box_free(OUBox& b);
-// Zero the OU state and the forcing field (a restart from F = 0).
-hipError_t ou_box_reset(const OUBox& b, int prec, hipStream_t st);
+// Zero the OU state and the forcing field of nbox boxes (descriptors in device memory), a restart from F = 0.
+hipError_t launch_ou_reset(int prec, const OUBox* d_boxes, int nbox, int gmax, hipStream_t st);
 
 // One OU advance of nbox boxes (descriptors in device memory): step_all >= 0 advances every box
 // with that Philox step counter; step_all < 0 advances the boxes whose `due` flag is set, each
