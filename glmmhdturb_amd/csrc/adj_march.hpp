@@ -6,7 +6,7 @@
 // re-reading 63 + 9 contribution planes.  Inputs are the planes the front passes wrote: W = c2p(u0),
 // the predicted states MH, the face-state adjoints LFS and LPRE; the output is lam0.
 //
-// Layout: the forward march's tile (march_impl.hpp): 248 lanes, a 16 x 12 owned tile and its
+// Layout: the forward march's tile (march_impl.hpp): 252 lanes, a 16 x 12 owned tile and its
 // one-cell ring, each lane one column, marching z; W of plane q over the tile grown by two cells in
 // LDS.  Per plane q every lane takes the face-state adjoints of its cell in x, y, z and the
 // predictor adjoint; the contributions to its in-plane neighbours go through LDS (one slot per
@@ -47,9 +47,9 @@ adj_back_kernel(AdjArgs a, int tiles_x, int tiles_y, int zchunk)
     const bool owned = tid < NO && gxu < nx && gyu < ny;
     const size_t col = (size_t)gx + (size_t)nx * gy;
     const int lo = (ty + 1) * PX + (tx + 1);
-    const bool helper = tid < NHELP;
+    const bool helper = tid >= NO && tid - NO < NHELP;
     int hx = 0, hy = 0;
-    helper_cell(helper ? tid : 0, hx, hy);
+    helper_cell(helper ? tid - NO : 0, hx, hy);
     const size_t hcol = (size_t)wrapi(tile_x * OX - 2 + hx, nx) + (size_t)nx * wrapi(tile_y * OY - 2 + hy, ny);
     const int lo_ring = hy * PX + hx;
     const double* W = plane(a, ADJ_W, n);

@@ -17,7 +17,7 @@ struct CTArgsHost {
 };
 
 size_t ct_scratch_bytes(size_t n, int prec);
-constexpr int CT_MARCH_THREADS = 252;   // lanes of a CT march workgroup (ct_march.hpp CM_NT)
+constexpr int CT_MARCH_THREADS = 256;   // lanes of a CT march workgroup (ct_march.hpp CM_NT)
 template <typename T>
 hipError_t launch_ct_step(void* const* q, void* const* o, const CTArgsHost& h, void* scratch, hipStream_t st);
 template <typename T>

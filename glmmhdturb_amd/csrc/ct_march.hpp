@@ -7,7 +7,7 @@
 // and OU kick.  The point functions are the same ones (ct_cell_states, ct_riemann).
 //
 // Layout on the GPU (the GLM march's, adapted to CT):
-//   * A workgroup of 252 lanes owns a 16 x 12 column tile and a z-chunk.  Lanes 0..191 own the
+//   * A workgroup of 256 lanes owns a 16 x 12 column tile and a z-chunk.  Lanes 0..191 own the
 //     tile row by row; lanes 192..251 are the one-cell ring around it, corners included (the
 //     EMF at an edge of the tile needs fluxes of the ring's corner cells).  Every lane builds the
 //     x, y and z face states of its cell; the LDS plane holds the primitives of plane q over the
@@ -34,13 +34,14 @@ namespace glm {
 constexpr int CM_OX = 16, CM_OY = 12;
 constexpr int CM_NO = CM_OX * CM_OY;                           // owned lanes
 constexpr int CM_NH = 2 * (CM_OX + 2) + 2 * CM_OY;             // one-cell ring with corners
-constexpr int CM_NT = CM_NO + CM_NH;                           // 252
+constexpr int CM_NL = CM_NO + CM_NH;                           // 252 lanes with a cell of their own
+constexpr int CM_NT = 256;                                     // and 4 that only help (they repeat the last lane)
 constexpr int CM_PX = CM_OX + 4, CM_PY = CM_OY + 4;            // LDS plane (two-cell ring)
 constexpr int CM_NPL = CM_PX * CM_PY;
 constexpr int CM_LX = CM_OX + 2;                               // row of the lanes' grown tile
 static_assert(CM_LX * (CM_OY + 2) == CM_OX * CM_OY + 2 * (CM_OX + 2) + 2 * CM_OY, "one lane per grown-tile cell");
 constexpr int CM_NHELP = 2 * (CM_OX + 2) + 2 * (CM_OY + 2);    // two-cell ring without its corners
-static_assert(CM_NT <= 256 && CM_NT >= CM_NHELP && CM_NO % 64 == 0, "CT tile shape");
+static_assert(CM_NL <= CM_NT && CM_NT - CM_NO >= CM_NHELP && CM_NO % 64 == 0, "CT tile shape");
 static_assert(CM_NT == CT_MARCH_THREADS, "launch width of the CT march");
 
 #ifndef GLM_CT_WAVES_F64
@@ -102,10 +103,10 @@ GLM_DEV void cm_helper_cell(int h, int& px, int& py)
 template <typename T, int NV = 8>
 struct CTMarchLDS {
     T P[NV][CM_NPL];       // primitives (and species fractions) of plane q (two-cell ring)
-    T XB[NV][CM_NT];       // +x face states, then x fluxes (0..4 and species 8.., By in 6) and the z flux's Bx (5), By (7)
-    T YB[NV][CM_NT];       // +y face states, then y fluxes (0..4 and species 8.., Bx in 5)
+    T XB[NV][CM_NL];       // +x face states, then x fluxes (0..4 and species 8.., By in 6) and the z flux's Bx (5), By (7)
+    T YB[NV][CM_NL];       // +y face states, then y fluxes (0..4 and species 8.., Bx in 5)
     T E[2][3][CM_NPL];     // edge EMFs ex, ey, ez of the last two planes (plane k in slot k & 1)
-    T FCB[6][CM_NT];       // forcing interpolation cache (ForceCache)
+    T FCB[6][CM_NO];       // forcing interpolation cache (ForceCache) of the owned columns
 };
 
 // Primitives with cell-centred B of cell (x, y, z) (ct_mhd.jl:26-34, :85-96), then the species
@@ -152,12 +153,12 @@ ct_march_kernel(CTMArgs<T> a_)
     constexpr int NV = 8 + NS, NH = 5 + NS;   // values per cell; hydro-updated values (species at 5..)
     __shared__ CTMarchLDS<T, NV> L;
     T (&P)[NV][CM_NPL] = L.P;
-    T (&XB)[NV][CM_NT] = L.XB;
-    T (&YB)[NV][CM_NT] = L.YB;
+    T (&XB)[NV][CM_NL] = L.XB;
+    T (&YB)[NV][CM_NL] = L.YB;
     const int tid = threadIdx.x;
     int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
     int tx, ty;
-    cm_lane_cell(tid, tx, ty);
+    cm_lane_cell(tid < CM_NL ? tid : CM_NL - 1, tx, ty);
     const int tile_x = tile % a.tiles_x; tile /= a.tiles_x;
     const int tile_y = tile % a.tiles_y; tile /= a.tiles_y;
     const int zs = tile * a.zchunk;
@@ -177,9 +178,10 @@ ct_march_kernel(CTMArgs<T> a_)
     const size_t col = (size_t)gx + (size_t)nx * gy;
     const int lo = (ty + 1) * CM_PX + (tx + 1);
     const int li = ty * CM_LX + tx;
-    const bool helper = tid < CM_NHELP;
+    const bool helper = tid >= CM_NO;   // the halo wavefront, which has no update, brings in the two-cell ring (the first
+                                        // one did: 2.46 instead of 2.70 ms at 256^3 FP64)
     int hx = 0, hy = 0;
-    cm_helper_cell(helper ? tid : 0, hx, hy);
+    cm_helper_cell(helper ? tid - CM_NO : 0, hx, hy);
     const int hgx = cwrap(tile_x * CM_OX - 2 + hx, nx), hgy = cwrap(tile_y * CM_OY - 2 + hy, ny);
     const int lo_ring = hy * CM_PX + hx;
 
@@ -209,9 +211,9 @@ ct_march_kernel(CTMArgs<T> a_)
     for (int v = 0; v < NV; ++v) zprev[v] = T(0);
 #pragma unroll
     for (int v = 0; v < NH; ++v) { fzp[v] = T(0); pend[v] = T(0); }
-    ForceCache<T, CM_NT> fc;
+    ForceCache<T, CM_NO> fc;
     fc.k0 = -0x7fffffff;
-    fc.b = &L.FCB[0][tid];
+    fc.b = &L.FCB[0][tid < CM_NO ? tid : 0];
 
     for (int q = zs - 1; q <= ze; ++q) {
         const int zq = cwrap(q, nz);

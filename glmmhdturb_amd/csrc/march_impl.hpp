@@ -39,8 +39,9 @@ namespace glm {
 
 // Owned tile OX x OY (16 doubles = one 128-byte line per row).  Lanes 0..NO-1 own the tile row by
 // row (4 rows per wavefront, so each row is stored by one instruction as a whole line); lanes
-// NO..NT-1 are the tile's one-cell halo without its corners and form the last wavefront, which
-// therefore skips the z solve and the update as a whole.
+// NO..NT-1 are the tile's one-cell halo and form the last wavefront, which therefore skips the z solve and
+// the update as a whole; it also brings in the two-cell ring that no lane owns (done by the first wavefront,
+// whose SIMD then had the most to do, the FP64 step at 256^3 took 2.35 ms instead of 2.31).
 #ifndef GLM_OX
 #define GLM_OX 16
 #endif
@@ -49,13 +50,13 @@ namespace glm {
 #endif
 constexpr int OX = GLM_OX, OY = GLM_OY;
 constexpr int NO = OX * OY;                 // owned lanes
-constexpr int NH = 2 * OX + 2 * OY;         // halo lanes (one-cell ring without corners)
+constexpr int NH = 2 * OX + 2 * OY + 4;     // halo lanes (one-cell ring, corners last)
 constexpr int NT = NO + NH;                 // threads per workgroup
 constexpr int PX = OX + 4, PY = OY + 4;     // LDS primitive plane (two-cell ring)
 constexpr int NPL = PX * PY;
-constexpr int NHELP = 4 + NH;               // plane cells no lane owns: the 4 one-cell corners and the
-                                            // two-cell ring without corners (in-plane neighbours of halo lanes)
-static_assert(NT <= 256 && NT >= NHELP && NO % 64 == 0, "tile shape");
+constexpr int NHELP = 2 * OX + 2 * OY;      // plane cells no lane owns: the two-cell ring without corners
+                                            // (in-plane neighbours of halo lanes), one for each of the first halo lanes
+static_assert(NT <= 256 && NH >= NHELP && NO % 64 == 0, "tile shape");
 
 // Minimum resident wavefronts per SIMD requested from the register allocator.
 #ifndef GLM_WAVES_F64
@@ -119,14 +120,13 @@ GLM_DEV void lane_cell(int t, int& tx, int& ty)
     if (h < OX) { tx = 1 + h; ty = 0; }
     else if (h < 2 * OX) { tx = 1 + h - OX; ty = OY + 1; }
     else if (h < 2 * OX + OY) { tx = 0; ty = 1 + h - 2 * OX; }
-    else { tx = OX + 1; ty = 1 + h - 2 * OX - OY; }
+    else if (h < 2 * OX + 2 * OY) { tx = OX + 1; ty = 1 + h - 2 * OX - OY; }
+    else { tx = (h & 1) ? OX + 1 : 0; ty = (h & 2) ? OY + 1 : 0; }   // h - 2 OX - 2 OY = 0..3
 }
 
-// LDS plane position (px, py) of helper cell h (0 <= h < NHELP).
-GLM_DEV void helper_cell(int h, int& px, int& py)
+// LDS plane position (px, py) of helper cell r (0 <= r < NHELP).
+GLM_DEV void helper_cell(int r, int& px, int& py)
 {
-    if (h < 4) { px = (h & 1) ? PX - 2 : 1; py = (h & 2) ? PY - 2 : 1; return; }
-    const int r = h - 4;
     if (r < OX) { px = 2 + r; py = 0; }
     else if (r < 2 * OX) { px = 2 + r - OX; py = PY - 1; }
     else if (r < 2 * OX + OY) { px = 0; py = 2 + r - 2 * OX; }
@@ -254,7 +254,7 @@ GLM_DEV void faces_dir(const T l[NV], const T m0[NV], const T r[NV], const T mhf
 // (glmmhd_turb.jl:1963-1971).  acc = (Fx_lo - Fx_hi) + (Fy_lo - Fy_hi) + (Fz_lo - Fz_hi).
 template <int NV, typename T>
 GLM_DEV double update_cell(T r[NV], const T acc[NV], const ColdArgs<T>& a, const Phys<T>& s, bool want_cfl,
-                           ForceCache<T, NT>& fc, int gx, int gy, int gz)
+                           ForceCache<T, NO>& fc, int gx, int gy, int gz)
 {
     T xold[NV > 9 ? NV - 9 : 1];   // species fractions at the start of the step (for the floor)
     if (NV > 9) {
@@ -300,7 +300,7 @@ struct MarchLDS {
     T P[NV][NPL];    // primitives of the current plane over the tile grown by two cells
     T XB[NV][NPL];   // +x face states, then x fluxes, at the LDS plane position of the cell
     T YB[NV][NPL];
-    T FCB[6][NT];   // forcing interpolation cache (ForceCache)
+    T FCB[6][NO];   // forcing interpolation cache (ForceCache) of the owned columns
     ColdArgs<T> ca;
 };
 
@@ -345,9 +345,9 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile)
     const bool need_y = tx >= 1 && tx <= OX && ty >= 1;      // this lane solves the y face at ty - 1/2
     const size_t col = (size_t)gx + (size_t)nx * gy;
     const int lo_own = (ty + 1) * PX + (tx + 1);
-    const bool helper = tid < NHELP;
+    const bool helper = tid >= NO && tid - NO < NHELP;
     int hx = 0, hy = 0;
-    helper_cell(helper ? tid : 0, hx, hy);
+    helper_cell(helper ? tid - NO : 0, hx, hy);
     const size_t hcol = (size_t)wrapi(tile_x * OX - 2 + hx, nx) + (size_t)nx * wrapi(tile_y * OY - 2 + hy, ny);
     const int lo_ring = hy * PX + hx;
 
@@ -376,9 +376,9 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile)
 #pragma unroll
     for (int v = 0; v < NV; ++v) { zprev[v] = T(0); pend[v] = T(0); }
     double cmax = 0.0;
-    ForceCache<T, NT> fc;
+    ForceCache<T, NO> fc;
     fc.k0 = -0x7fffffff;
-    fc.b = &L.FCB[0][tid];
+    fc.b = &L.FCB[0][tid < NO ? tid : 0];
 
     for (int q = zs - 1; q <= ze; ++q) {
         const bool last = q == ze;
