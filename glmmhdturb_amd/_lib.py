@@ -134,5 +134,5 @@ def check(code: int) -> None:
 
 def plane_array(ptrs):
     """Host array of device plane addresses (the float** / void* const* of the ABI)."""
-    arr = (C.c_void_p * len(ptrs))(*[C.c_void_p(int(p)) for p in ptrs])
-    return C.cast(arr, C.POINTER(C.c_void_p)), arr
+    arr = (C.c_void_p * len(ptrs))(*ptrs)
+    return arr, arr

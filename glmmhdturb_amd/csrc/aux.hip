@@ -16,6 +16,12 @@ hipError_t launch_clear_u64(unsigned long long* p, int n, hipStream_t st)
     return hipGetLastError();
 }
 
+hipError_t launch_publish_u64(unsigned long long* slot, unsigned long long* host, bool clear, hipStream_t st)
+{
+    hipLaunchKernelGGL(publish_u64_kernel, dim3(1), dim3(1), 0, st, slot, host, clear ? 1 : 0);
+    return hipGetLastError();
+}
+
 template <typename T>
 hipError_t launch_ctot(Ptr9<const T> q9dev, size_t n, const Phys<T>& s, unsigned long long* out, hipStream_t st,
                        bool fast)

@@ -32,6 +32,14 @@ __global__ void __launch_bounds__(AUX_NT) ctot_kernel(Ptr9<const T> q9, size_t n
     block_max_bits<AUX_NT>(best, out);
 }
 
+// One 8-byte result into host memory that the device can write, clearing its slot for the next reduction when
+// asked to: a call that waits for its result then needs no copy and no clear launch of its own.
+__global__ void publish_u64_kernel(unsigned long long* slot, unsigned long long* host, int clear)
+{
+    __hip_atomic_store(host, *slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (clear) *slot = 0ull;
+}
+
 __global__ void clear_u64_kernel(unsigned long long* p, int n)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;

@@ -17,6 +17,8 @@ inline unsigned red_blocks(size_t n)
 }
 
 hipError_t launch_clear_u64(unsigned long long* p, int n, hipStream_t st);
+// *host = *slot (host: device-mapped host memory), then *slot = 0 when clear.
+hipError_t launch_publish_u64(unsigned long long* slot, unsigned long long* host, bool clear, hipStream_t st);
 template <typename T>
 hipError_t launch_ctot(Ptr9<const T> q9dev, size_t n, const Phys<T>& s, unsigned long long* out, hipStream_t st,
                        bool fast = false);

@@ -74,6 +74,7 @@ static bool planes_alias(void* const* a, int na, void* const* b, int nb)
 struct ResidentOf {
     int key;
     Resident r;
+    int zauto;   // the modelled chunk length of the context's grid (0: not asked for yet)
 };
 
 static int resident_of(const void* fn, int threads, int key, ResidentOf& out)
@@ -84,6 +85,7 @@ static int resident_of(const void* fn, int threads, int key, ResidentOf& out)
     HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, threads, 0));
     out.r.cus = cus;
     out.r.occ = occ > 0 ? occ : 1;
+    out.zauto = 0;
     out.key = key;
     return GLM_OK;
 }
@@ -93,10 +95,11 @@ struct glm_ctx {
     size_t n;
     hipStream_t stream;
     unsigned long long* d_cmax;  // [0],[1] march CFL ping-pong, [2] CT step CFL, [3] standalone reductions
+    bool red_dirty;              // slot 3 may hold a value: a reduction was started and not read back
+    unsigned long long* h_out;   // pinned and device-mapped: results of the calls that wait for them
     int cfl_parity;              // slot the next march step accumulates into
     int cfl_slot;                // slot holding the CFL max of the last step with want_cfl (-1: none)
     void* d_parts;
-    double* d_diag;
     // OU forcing: one band-limited box (host copy of the descriptor, and the device copy)
     int g;
     long long nstep;
@@ -115,11 +118,36 @@ struct glm_ctx {
 static void ctx_free(glm_ctx* c)
 {
     if (!c) return;
-    void* ptrs[] = {c->d_cmax, c->d_parts, c->d_diag, c->d_ou, c->ct_scratch, c->adj_scratch, c->d_fdot};
+    void* ptrs[] = {c->d_cmax, c->d_parts, c->d_ou, c->ct_scratch, c->adj_scratch, c->d_fdot};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    if (c->h_out) (void)hipHostFree(c->h_out);
     ou_box_free(c->ou);
     delete c;
+}
+
+// Wait for the context's stream and return the 8 bytes of a device slot; clear: zero the slot behind them.
+// (An 8-byte hipMemcpyAsync to the caller's memory took about 6 us more than the one-lane kernel.)
+static int read_slot(glm_ctx* c, unsigned long long* slot, bool clear, double* out)
+{
+    HIPCHK(launch_publish_u64(slot, c->h_out, clear, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    memcpy(out, c->h_out, sizeof *out);
+    return GLM_OK;
+}
+
+// The standalone reductions accumulate into slot 3, which every complete one leaves at zero.
+static int begin_reduction(glm_ctx* c)
+{
+    if (c->red_dirty) HIPCHK(launch_clear_u64(c->d_cmax + 3, 1, c->stream));
+    c->red_dirty = true;
+    return GLM_OK;
+}
+static int end_reduction(glm_ctx* c, double* out)
+{
+    if (int e = read_slot(c, c->d_cmax + 3, true, out)) return e;
+    c->red_dirty = false;
+    return GLM_OK;
 }
 
 extern "C" {
@@ -166,8 +194,8 @@ glm_ctx* glm_create(int nx, int ny, int nz, int precision)
     c->cfl_slot = -1;
     if (hipMalloc(&c->d_cmax, 4 * sizeof(unsigned long long)) != hipSuccess ||
         hipMalloc(&c->d_parts, np * diag_part_bytes()) != hipSuccess ||
-        hipMalloc(&c->d_diag, GLM_NDIAG * sizeof(double)) != hipSuccess) {
-        set_err(GLM_ERR_ALLOC, "glm_create: device allocation failed");
+        hipHostMalloc((void**)&c->h_out, GLM_NDIAG * sizeof(double), hipHostMallocMapped) != hipSuccess) {
+        set_err(GLM_ERR_ALLOC, "glm_create: allocation failed");
         ctx_free(c);
         return nullptr;
     }
@@ -211,7 +239,9 @@ static int step_impl(glm_ctx* c, void* const* q, void* const* o, const glm_param
         if (!fn) return set_err(GLM_ERR_ARG, "glm_step: unknown scheme");
         if (int e = resident_of(fn, NT, key, c->march_res)) return e;
     }
-    march_tiling<T>(c->nx, c->ny, c->nz, p->zchunk, c->march_res.r, a.tiles_x, a.tiles_y, a.nzc, a.zchunk);
+    march_tiling<T>(c->nx, c->ny, c->nz, p->zchunk > 0 ? p->zchunk : c->march_res.zauto, c->march_res.r, a.tiles_x, a.tiles_y,
+                    a.nzc, a.zchunk);
+    if (p->zchunk <= 0) c->march_res.zauto = a.zchunk;
     a.ph = make_phys<T>(p);
     double dtdx = p->dt / p->dx;
     a.dtdx = (T)dtdx;
@@ -277,11 +307,7 @@ int glm_cfl_max(glm_ctx* ctx, double* cmax)
 {
     if (!ctx || !cmax) return set_err(GLM_ERR_ARG, "glm_cfl_max: null argument");
     if (ctx->cfl_slot < 0) return set_err(GLM_ERR_STATE, "glm_cfl_max: no step with want_cfl has run");
-    unsigned long long bits = 0;
-    HIPCHK(hipMemcpyAsync(&bits, ctx->d_cmax + ctx->cfl_slot, sizeof bits, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    memcpy(cmax, &bits, sizeof bits);
-    return GLM_OK;
+    return read_slot(ctx, ctx->d_cmax + ctx->cfl_slot, false, cmax);
 }
 
 }  // extern "C"
@@ -317,15 +343,11 @@ static int ctot_impl(glm_ctx* ctx, void* const* q, const glm_params* p, double* 
     int e = check_planes(q, 9, msg);
     if (!e) e = check_params(p);
     if (e) return e;
-    HIPCHK(launch_clear_u64(ctx->d_cmax + 3, 1, ctx->stream));
+    if ((e = begin_reduction(ctx))) return e;
     if (ctx->prec == 8)
         HIPCHK(launch_ctot<double>(cptr9<double>(q), ctx->n, make_phys<double>(p), ctx->d_cmax + 3, ctx->stream, fast));
     else HIPCHK(launch_ctot<float>(cptr9<float>(q), ctx->n, make_phys<float>(p), ctx->d_cmax + 3, ctx->stream, fast));
-    unsigned long long bits = 0;
-    HIPCHK(hipMemcpyAsync(&bits, ctx->d_cmax + 3, sizeof bits, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    memcpy(cmax, &bits, sizeof bits);
-    return GLM_OK;
+    return end_reduction(ctx, cmax);
 }
 
 extern "C" {
@@ -347,11 +369,11 @@ int glm_diagnostics(glm_ctx* ctx, void* const* q, const glm_params* p, double* o
     if (!e) e = check_params(p);
     if (e) return e;
     if (ctx->prec == 8)
-        HIPCHK(launch_diag<double>(cptr9<double>(q), ctx->nx, ctx->ny, ctx->nz, p->dx, p->smallr, ctx->d_parts, ctx->d_diag, ctx->stream));
+        HIPCHK(launch_diag<double>(cptr9<double>(q), ctx->nx, ctx->ny, ctx->nz, p->dx, p->smallr, ctx->d_parts, (double*)ctx->h_out, ctx->stream));
     else
-        HIPCHK(launch_diag<float>(cptr9<float>(q), ctx->nx, ctx->ny, ctx->nz, p->dx, p->smallr, ctx->d_parts, ctx->d_diag, ctx->stream));
-    HIPCHK(hipMemcpyAsync(out, ctx->d_diag, GLM_NDIAG * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHK(launch_diag<float>(cptr9<float>(q), ctx->nx, ctx->ny, ctx->nz, p->dx, p->smallr, ctx->d_parts, (double*)ctx->h_out, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    memcpy(out, ctx->h_out, GLM_NDIAG * sizeof(double));
     return GLM_OK;
 }
 
@@ -498,7 +520,7 @@ static int step_adjoint_impl(glm_ctx* ctx, void* const* u0, void* const* lam1, v
             ctx->d_fdot = nullptr;
             return set_err(GLM_ERR_ALLOC, "glm_step_adjoint: allocation failed");
         }
-        HIPCHK(hipMemsetAsync(ctx->d_fdot, 0, sizeof(double), ctx->stream));
+        HIPCHK(launch_clear_u64((unsigned long long*)ctx->d_fdot, 1, ctx->stream));
     }
     AdjArgs a;
     memset(&a, 0, sizeof a);
@@ -542,10 +564,7 @@ int glm_adjoint_force_dot(glm_ctx* ctx, int reset, double* out)
     if (!ctx || !out) return set_err(GLM_ERR_ARG, "glm_adjoint_force_dot: null argument");
     *out = 0.0;
     if (!ctx->d_fdot) return GLM_OK;
-    HIPCHK(hipMemcpyAsync(out, ctx->d_fdot, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (reset) HIPCHK(hipMemsetAsync(ctx->d_fdot, 0, sizeof(double), ctx->stream));
-    return GLM_OK;
+    return read_slot(ctx, (unsigned long long*)ctx->d_fdot, reset != 0, out);
 }
 
 // CT step paths: the multi-pass kernel sequence, the fused z-march, the staged 3-D tiles.
@@ -578,7 +597,7 @@ static int ct_step_impl(glm_ctx* ctx, void* const* q, void* const* o, const glm_
     h.face_slope = ct_face_slope; h.riemann = p->riemann; h.recon = p->recon;
     h.update_floor = p->update_floor; h.do_turb = p->do_turb; h.tgs = ctx->g; h.afield = ctx->afield;
     h.want_cfl = p->want_cfl; h.cmax = ctx->d_cmax + 2; h.zchunk = p->zchunk; h.nsp = nsp;
-    if (p->want_cfl) HIPCHK(launch_clear_u64(ctx->d_cmax + 2, 1, ctx->stream));
+    if (p->want_cfl && mode != CT_MARCH) HIPCHK(launch_clear_u64(ctx->d_cmax + 2, 1, ctx->stream));   // the march clears it itself
     if (mode == CT_TILES) {
         if (ctx->prec == 8) HIPCHK(launch_ct_tiles<double>(q, o, h, ctx->stream));
         else HIPCHK(launch_ct_tiles<float>(q, o, h, ctx->stream));
@@ -590,6 +609,12 @@ static int ct_step_impl(glm_ctx* ctx, void* const* q, void* const* o, const glm_
                                             : ct_march_ptr<float>(p->riemann, nsp, p->recon);
             if (!fn) return set_err(GLM_ERR_ARG, "glm_ct_step: unknown Riemann solver");
             if ((e = resident_of(fn, CT_MARCH_THREADS, key, ctx->ct_res))) return e;
+        }
+        if (h.zchunk <= 0) {
+            if (!ctx->ct_res.zauto)
+                ctx->ct_res.zauto = ctx->prec == 8 ? ct_march_chunk<double>(h.nx, h.ny, h.nz, ctx->ct_res.r)
+                                                   : ct_march_chunk<float>(h.nx, h.ny, h.nz, ctx->ct_res.r);
+            h.zchunk = ctx->ct_res.zauto;
         }
         if (ctx->prec == 8) HIPCHK(launch_ct_march<double>(q, o, h, ctx->ct_res.r, ctx->stream));
         else HIPCHK(launch_ct_march<float>(q, o, h, ctx->ct_res.r, ctx->stream));
@@ -628,30 +653,23 @@ int glm_ct_ctot_max(glm_ctx* ctx, void* const* q, const glm_params* p, double* c
     if (!e) e = check_params(p);
     if (e) return e;
     double smallp = p->pfl > 0.0 ? p->pfl : p->smallr * p->smallc * p->smallc / p->gamma;
-    HIPCHK(launch_clear_u64(ctx->d_cmax + 3, 1, ctx->stream));
+    if ((e = begin_reduction(ctx))) return e;
     if (ctx->prec == 8)
         HIPCHK(launch_ct_ctot<double>(q, ctx->nx, ctx->ny, ctx->nz, p->gamma, p->smallr, smallp, ctx->d_cmax + 3, ctx->stream));
     else
         HIPCHK(launch_ct_ctot<float>(q, ctx->nx, ctx->ny, ctx->nz, p->gamma, p->smallr, smallp, ctx->d_cmax + 3, ctx->stream));
-    unsigned long long bits = 0;
-    HIPCHK(hipMemcpyAsync(&bits, ctx->d_cmax + 3, sizeof bits, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    memcpy(cmax, &bits, sizeof bits);
-    return GLM_OK;
+    return end_reduction(ctx, cmax);
 }
 
 int glm_ct_divb_max(glm_ctx* ctx, void* const* q, double dx, double* out)
 {
     if (!ctx || !out || !(dx > 0.0)) return set_err(GLM_ERR_ARG, "glm_ct_divb_max: bad argument");
-    if (int e = check_planes(q, 8, "glm_ct_divb_max: null plane pointer")) return e;
-    HIPCHK(launch_clear_u64(ctx->d_cmax + 3, 1, ctx->stream));
+    int e = check_planes(q, 8, "glm_ct_divb_max: null plane pointer");
+    if (e) return e;
+    if ((e = begin_reduction(ctx))) return e;
     if (ctx->prec == 8) HIPCHK(launch_ct_divb<double>(q, ctx->nx, ctx->ny, ctx->nz, dx, ctx->d_cmax + 3, ctx->stream));
     else HIPCHK(launch_ct_divb<float>(q, ctx->nx, ctx->ny, ctx->nz, dx, ctx->d_cmax + 3, ctx->stream));
-    unsigned long long bits = 0;
-    HIPCHK(hipMemcpyAsync(&bits, ctx->d_cmax + 3, sizeof bits, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    memcpy(out, &bits, sizeof bits);
-    return GLM_OK;
+    return end_reduction(ctx, out);
 }
 
 // The hydro march (spike_25d.cu:383-516 as build_march.sh builds it), with nsp = 0 or 2 passive
@@ -706,6 +724,12 @@ static int hydro_step_impl(glm_ctx* ctx, void* const* q, void* const* o, const g
                                         : hydro_march_ptr<float>(h.fallback, nsp, h.cma, fmt, h.scheme);
         if (!fn) return set_err(GLM_ERR_ARG, "hydro step: no kernel for this format and precision");
         if (int e = resident_of(fn, HYDRO_THREADS, key, ctx->hydro_res)) return e;
+    }
+    if (h.zchunk <= 0) {
+        if (!ctx->hydro_res.zauto)
+            ctx->hydro_res.zauto = ctx->prec == 8 ? hydro_march_chunk<double>(h.nx, h.ny, h.nz, ctx->hydro_res.r)
+                                                  : hydro_march_chunk<float>(h.nx, h.ny, h.nz, ctx->hydro_res.r);
+        h.zchunk = ctx->hydro_res.zauto;
     }
     if (ctx->prec == 8) HIPCHK(launch_hydro_march<double>(q, o, h, ctx->hydro_res.r, ctx->stream));
     else HIPCHK(launch_hydro_march<float>(q, o, h, ctx->hydro_res.r, ctx->stream));

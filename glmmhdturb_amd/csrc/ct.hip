@@ -99,6 +99,14 @@ const void* ct_march_ptr(int riemann, int nsp, int recon)
 }
 
 template <typename T>
+int ct_march_chunk(int nx, int ny, int nz, const Resident& res)
+{
+    int tx, ty, nzc, zc;
+    ct_march_tiling<T>(nx, ny, nz, 0, res, tx, ty, nzc, zc);
+    return zc;
+}
+
+template <typename T>
 hipError_t launch_ct_march(void* const* q, void* const* o, const CTArgsHost& h, const Resident& res, hipStream_t st)
 {
     if (h.nsp != 0 && h.nsp != 2) return hipErrorInvalidValue;
@@ -117,6 +125,7 @@ hipError_t launch_ct_march(void* const* q, void* const* o, const CTArgsHost& h, 
     a.face_slope = h.face_slope; a.recon = h.recon; a.update_floor = h.update_floor;
     a.do_turb = h.do_turb; a.tgs = h.tgs;
     a.afield = (const T*)h.afield;
+    a.cmax = h.want_cfl ? h.cmax : nullptr;
     const void* fn = ct_march_ptr<T>(h.riemann, h.nsp, h.recon);
     if (!fn) return hipErrorInvalidValue;
     void* args[] = {&a};
@@ -162,6 +171,7 @@ const void* ct_kernel_ptr()
                                           unsigned long long*, hipStream_t);                                    \
     template hipError_t launch_ct_divb<T>(void* const*, int, int, int, double, unsigned long long*, hipStream_t); \
     template const void* ct_kernel_ptr<T>();                                                                    \
+    template int ct_march_chunk<T>(int, int, int, const Resident&);                                             \
     template const void* ct_march_ptr<T>(int, int, int);                                                        \
     template hipError_t launch_ct_march<T>(void* const*, void* const*, const CTArgsHost&, const Resident&, hipStream_t);   \
     template hipError_t launch_ct_tiles<T>(void* const*, void* const*, const CTArgsHost&, hipStream_t);        \

@@ -31,6 +31,8 @@ const void* ct_kernel_ptr();
 template <typename T>
 hipError_t launch_ct_march(void* const* q, void* const* o, const CTArgsHost& h, const Resident& res, hipStream_t st);
 template <typename T>
+int ct_march_chunk(int nx, int ny, int nz, const Resident& res);   // the modelled z planes per tile
+template <typename T>
 const void* ct_march_ptr(int riemann, int nsp = 0, int recon = 0);
 // The same step as one kernel over staged 3-D tiles (ct_tile.hpp) and that kernel (resource queries).
 template <typename T>

@@ -76,6 +76,7 @@ struct CTMArgs {
     T gamma, igm1, smallr, smallp, dtdx, half_dtdx, dt, dx, lx, ly, lz, smallc, turb_min_rho, ramp;
     int face_slope, recon, update_floor, do_turb, tgs;
     const T* afield;
+    unsigned long long* cmax;   // cleared here for the CFL reduction that follows, or null
 };
 
 // Lane t's cell (tx, ty) in the tile grown by one cell (tx in 0..OX+1, ty in 0..OY+1).
@@ -156,6 +157,7 @@ ct_march_kernel(CTMArgs<T> a_)
     T (&XB)[NV][CM_NL] = L.XB;
     T (&YB)[NV][CM_NL] = L.YB;
     const int tid = threadIdx.x;
+    if (a.cmax && blockIdx.x == 0 && tid == 0) *a.cmax = 0ull;
     int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
     int tx, ty;
     cm_lane_cell(tid < CM_NL ? tid : CM_NL - 1, tx, ty);
@@ -178,8 +180,8 @@ ct_march_kernel(CTMArgs<T> a_)
     const size_t col = (size_t)gx + (size_t)nx * gy;
     const int lo = (ty + 1) * CM_PX + (tx + 1);
     const int li = ty * CM_LX + tx;
-    const bool helper = tid >= CM_NO;   // the halo wavefront, which has no update, brings in the two-cell ring (the first
-                                        // one did: 2.46 instead of 2.70 ms at 256^3 FP64)
+    const bool helper = tid >= CM_NO;   // the halo wavefront, which has no update, brings in the two-cell ring (when
+                                        // the first owned one did: 2.70 ms at 256^3 FP64, now 2.46)
     int hx = 0, hy = 0;
     cm_helper_cell(helper ? tid - CM_NO : 0, hx, hy);
     const int hgx = cwrap(tile_x * CM_OX - 2 + hx, nx), hgy = cwrap(tile_y * CM_OY - 2 + hy, ny);

@@ -63,6 +63,14 @@ static void launch_sv(const HydroArgs<T>& a, dim3 g, int nsp, int cma, hipStream
 }
 
 template <typename T>
+int hydro_march_chunk(int nx, int ny, int nz, const Resident& res)
+{
+    int tx, ty, nzc, zc;
+    hydro_tiling<T>(nx, ny, nz, 0, res, tx, ty, nzc, zc);
+    return zc;
+}
+
+template <typename T>
 hipError_t launch_hydro_march(void* const* q, void* const* o, const HydroArgsHost& h, const Resident& res, hipStream_t st)
 {
     if (h.nsp != 0 && h.nsp != 2) return hipErrorInvalidValue;
@@ -129,6 +137,8 @@ hipError_t launch_hydro_march(void* const* q, void* const* o, const HydroArgsHos
 
 template hipError_t launch_hydro_march<double>(void* const*, void* const*, const HydroArgsHost&, const Resident&, hipStream_t);
 template hipError_t launch_hydro_march<float>(void* const*, void* const*, const HydroArgsHost&, const Resident&, hipStream_t);
+template int hydro_march_chunk<double>(int, int, int, const Resident&);
+template int hydro_march_chunk<float>(int, int, int, const Resident&);
 template const void* hydro_march_ptr<double>(int, int, int, int, int);
 template const void* hydro_march_ptr<float>(int, int, int, int, int);
 

@@ -23,6 +23,8 @@ constexpr int HYDRO_THREADS = 256;   // lanes of a hydro march workgroup (hydro_
 template <typename T>
 hipError_t launch_hydro_march(void* const* q, void* const* o, const HydroArgsHost& h, const Resident& res, hipStream_t st);
 template <typename T>
+int hydro_march_chunk(int nx, int ny, int nz, const Resident& res);   // the modelled z planes per workgroup
+template <typename T>
 const void* hydro_march_ptr(int fallback, int nsp, int cma, int fmt = 0, int scheme = 0);
 
 }  // namespace glm

@@ -212,7 +212,9 @@ class Solver:
     def _planes(self, u, nv=NV):
         if u.dtype != self.dtype or not u.is_contiguous() or tuple(u.shape) != (nv, self.nz, self.ny, self.nx):
             raise ValueError(f"state must be a contiguous {self.dtype} tensor of shape {(nv, self.nz, self.ny, self.nx)}")
-        return plane_array([u[v].data_ptr() for v in range(nv)])
+        # the planes of a contiguous state lie one after another (a view per plane costs a microsecond each)
+        base, step = u.data_ptr(), self.nx * self.ny * self.nz * u.element_size()
+        return plane_array(range(base, base + nv * step, step))
 
     # ---- initial conditions -------------------------------------------------------------
     def ic(self, u, kind: str, args):
