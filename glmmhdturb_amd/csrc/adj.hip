@@ -63,7 +63,7 @@ static bool dispatch_faceswise(const AdjArgs& a, dim3 g, hipStream_t st, bool up
 static bool dispatch_back(const AdjArgs& a, int zchunk, hipStream_t st, int pred, int recon, int slope)
 {
     int tx, ty, nzc, zc;
-    march_tiling<double>(a.nx, a.ny, a.nz, zchunk, Resident{}, tx, ty, nzc, zc);   // one workgroup per CU
+    march_tiling<double>(a.nx, a.ny, a.nz, zchunk, Resident{256, adj_waves(pred)}, tx, ty, nzc, zc);
     const dim3 g((unsigned)(tx * ty * nzc));
 #define GLM_CASE(P, RC, SL)                                                                          \
     if (pred == P && recon == RC && slope == SL) {                                                   \
@@ -91,7 +91,8 @@ hipError_t launch_step_adjoint(AdjArgs a, void* scratch, int pred, int riem, int
     if (!dispatch_faceswise(a, g, st, true, riem)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(adj_fdot_kernel, dim3(1), dim3(ADJ_NT), 0, st, (const double*)a.part, (int)g.x, fdot);
     dispatch_faceswise(a, g, st, false, riem);
-    if (fused) {
+    // the march's 32-bit offsets reach over one z plane of the scratch (2.29 million cells)
+    if (fused && (size_t)ADJ_NPLANES * sizeof(double) * a.nx * a.ny <= UINT32_MAX) {
         dispatch_back(a, zchunk, st, pred, recon, slope);
     } else {
         dispatch_cellwise(a, g, st, false, pred, recon, slope);

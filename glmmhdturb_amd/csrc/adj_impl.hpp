@@ -30,38 +30,58 @@ GLM_DEV int adj_wrap(int i, int n)
 }
 
 struct Cell {
-    size_t c;
+    size_t c, o;   // index in the caller's planes and in the scratch
     int i, j, k;
 };
-GLM_DEV Cell cell_of(size_t c, int nx, int ny)
+// Scratch index: the ADJ_NPLANES values of a cell row lie together, row by row.  As planes of n cells the
+// 60 to 120 streams of a pass were as many pages, and every access of a wavefront a translation of its
+// own: the Riemann adjoint took 618 us at 128^3 (505 now), the reverse step as a whole 6% more.
+GLM_DEV size_t adj_index(const AdjArgs& a, int i, int j, int k)
+{
+    return (size_t)i + (size_t)a.nx * ADJ_NPLANES * ((size_t)j + (size_t)a.ny * k);
+}
+GLM_DEV Cell cell_of(const AdjArgs& a, size_t c)
 {
     Cell r;
     r.c = c;
-    r.i = (int)(c % nx);
-    r.j = (int)((c / nx) % ny);
-    r.k = (int)(c / ((size_t)nx * ny));
+    r.i = (int)(c % a.nx);
+    r.j = (int)((c / a.nx) % a.ny);
+    r.k = (int)(c / ((size_t)a.nx * a.ny));
+    r.o = adj_index(a, r.i, r.j, r.k);
     return r;
 }
-// neighbour index in direction d (0..2), offset o (-1 or +1)
-GLM_DEV size_t nbr(const Cell& x, int d, int o, int nx, int ny, int nz)
+// scratch index of the neighbour in direction d (0..2), offset o (-1 or +1)
+GLM_DEV size_t nbr(const AdjArgs& a, const Cell& x, int d, int o)
 {
     int i = x.i, j = x.j, k = x.k;
-    if (d == 0) i = adj_wrap(i + o, nx);
-    else if (d == 1) j = adj_wrap(j + o, ny);
-    else k = adj_wrap(k + o, nz);
-    return (size_t)i + (size_t)nx * ((size_t)j + (size_t)ny * k);
+    if (d == 0) i = adj_wrap(i + o, a.nx);
+    else if (d == 1) j = adj_wrap(j + o, a.ny);
+    else k = adj_wrap(k + o, a.nz);
+    return adj_index(a, i, j, k);
 }
 
-GLM_DEV double* plane(const AdjArgs& a, int p, size_t n) { return a.scr + (size_t)p * n; }
-GLM_DEV void ld9(const double* base, size_t n, size_t c, double x[9])
+// plane p of the scratch; the nine planes of a group are a.nx apart
+GLM_DEV double* plane(const AdjArgs& a, int p) { return a.scr + (size_t)p * a.nx; }
+GLM_DEV void ld9(const AdjArgs& a, int p, size_t o, double x[9])
 {
+    const double* b = plane(a, p) + o;
 #pragma unroll
-    for (int v = 0; v < 9; ++v) x[v] = base[(size_t)v * n + c];
+    for (int v = 0; v < 9; ++v) x[v] = b[(size_t)v * a.nx];
 }
-GLM_DEV void st9(double* base, size_t n, size_t c, const double x[9])
+GLM_DEV void st9(const AdjArgs& a, int p, size_t o, const double x[9])
 {
+    double* b = plane(a, p) + o;
 #pragma unroll
-    for (int v = 0; v < 9; ++v) base[(size_t)v * n + c] = x[v];
+    for (int v = 0; v < 9; ++v) b[(size_t)v * a.nx] = x[v];
+}
+
+// The predicted state as the face states use it: MH holds the predictor's result before the revert,
+// which is what its adjoint needs.
+GLM_DEV void mh_revert(const AdjArgs& a, const double p0[9], double mh[9])
+{
+    const bool rev = hancock_reverts(mh, a.mh_revert, a.ph);
+#pragma unroll
+    for (int v = 0; v < 9; ++v) mh[v] = rev ? p0[v] : mh[v];
 }
 // face-state slot: direction d, side 0 (low face) or 1 (high face)
 GLM_DEV int fs_slot(int d, int side) { return (d * 2 + side) * 9; }
@@ -75,7 +95,7 @@ __global__ void __launch_bounds__(ADJ_NT) adj_prim_kernel(AdjArgs a)
 #pragma unroll
         for (int v = 0; v < 9; ++v) u[v] = a.u0[v][c];
         cons2prim(u, w, a.ph);
-        st9(plane(a, ADJ_W, n), n, c, w);
+        st9(a, ADJ_W, cell_of(a, c).o, w);
     }
 }
 
@@ -85,13 +105,13 @@ GLM_DEV bool ppm_up(const double p0[9], const double (*nb)[9])
     return !(spj(nb[0][4], p0[4], nb[1][4]) || spj(nb[2][4], p0[4], nb[3][4]) || spj(nb[4][4], p0[4], nb[5][4]));
 }
 
-GLM_DEV void load_stencil(const AdjArgs& a, const Cell& x, size_t n, double p0[9], double nb[6][9])
+GLM_DEV void load_p(const AdjArgs& a, size_t o, double* out9) { ld9(a, ADJ_W, o, out9); }
+GLM_DEV void load_stencil(const AdjArgs& a, const Cell& x, double p0[9], double nb[6][9])
 {
-    const double* W = plane(a, ADJ_W, n);
-    ld9(W, n, x.c, p0);
+    load_p(a, x.o, p0);
     for (int d = 0; d < 3; ++d) {
-        ld9(W, n, nbr(x, d, -1, a.nx, a.ny, a.nz), nb[2 * d]);
-        ld9(W, n, nbr(x, d, +1, a.nx, a.ny, a.nz), nb[2 * d + 1]);
+        load_p(a, nbr(a, x, d, -1), nb[2 * d]);
+        load_p(a, nbr(a, x, d, +1), nb[2 * d + 1]);
     }
 }
 
@@ -102,23 +122,24 @@ __global__ void __launch_bounds__(ADJ_NT) adj_faces_kernel(AdjArgs a)
     const size_t n = (size_t)a.nx * a.ny * a.nz;
     const FaceOpts o{a.mh_revert, a.face_guard};
     for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        const Cell x = cell_of(c, a.nx, a.ny);
+        const Cell x = cell_of(a, c);
         double p0[9], nb[6][9], mh[9], lo[9], hi[9];
-        load_stencil(a, x, n, p0, nb);
+        load_stencil(a, x, p0, nb);
         const bool up = RECON == RECON_PPM ? ppm_up(p0, nb) : true;
         if (PRED == PRED_FULL) {
-            hancock_fwd<double, SLOPE>(p0, nb, mh, a.half_dtdx, a.mh_revert, a.ph);
-            st9(plane(a, ADJ_MH, n), n, c, mh);
+            hancock_fwd<double, SLOPE>(p0, nb, mh, a.half_dtdx, 0, a.ph);
+            st9(a, ADJ_MH, x.o, mh);
+            mh_revert(a, p0, mh);
         }
         faces_fwd<double, PRED, RECON, SLOPE, 0>(nb[0], p0, nb[1], mh, up, a.half_dtdx, o, a.ph, lo, hi);
-        st9(plane(a, ADJ_FS + fs_slot(0, 0), n), n, c, lo);
-        st9(plane(a, ADJ_FS + fs_slot(0, 1), n), n, c, hi);
+        st9(a, ADJ_FS + fs_slot(0, 0), x.o, lo);
+        st9(a, ADJ_FS + fs_slot(0, 1), x.o, hi);
         faces_fwd<double, PRED, RECON, SLOPE, 1>(nb[2], p0, nb[3], mh, up, a.half_dtdx, o, a.ph, lo, hi);
-        st9(plane(a, ADJ_FS + fs_slot(1, 0), n), n, c, lo);
-        st9(plane(a, ADJ_FS + fs_slot(1, 1), n), n, c, hi);
+        st9(a, ADJ_FS + fs_slot(1, 0), x.o, lo);
+        st9(a, ADJ_FS + fs_slot(1, 1), x.o, hi);
         faces_fwd<double, PRED, RECON, SLOPE, 2>(nb[4], p0, nb[5], mh, up, a.half_dtdx, o, a.ph, lo, hi);
-        st9(plane(a, ADJ_FS + fs_slot(2, 0), n), n, c, lo);
-        st9(plane(a, ADJ_FS + fs_slot(2, 1), n), n, c, hi);
+        st9(a, ADJ_FS + fs_slot(2, 0), x.o, lo);
+        st9(a, ADJ_FS + fs_slot(2, 1), x.o, hi);
     }
 }
 
@@ -148,11 +169,11 @@ GLM_DEV void adj_force(const AdjArgs& a, int i, int j, int k, double a3[3])
 }
 
 template <int RIEM, int D>
-GLM_DEV void face_flux(const AdjArgs& a, size_t n, size_t cl, size_t cr, double f[9])
+GLM_DEV void face_flux(const AdjArgs& a, size_t cl, size_t cr, double f[9])
 {
     double L[9], R[9];
-    ld9(plane(a, ADJ_FS + fs_slot(D, 1), n), n, cl, L);
-    ld9(plane(a, ADJ_FS + fs_slot(D, 0), n), n, cr, R);
+    ld9(a, ADJ_FS + fs_slot(D, 1), cl, L);
+    ld9(a, ADJ_FS + fs_slot(D, 0), cr, R);
     riemann<double, RIEM, D>(L, R, f, a.ph);
 }
 
@@ -163,14 +184,14 @@ __global__ void __launch_bounds__(ADJ_NT) adj_flux_kernel(AdjArgs a)
 {
     const size_t n = (size_t)a.nx * a.ny * a.nz;
     for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        const Cell x = cell_of(c, a.nx, a.ny);
+        const Cell x = cell_of(a, c);
         double f[9];
-        face_flux<RIEM, 0>(a, n, nbr(x, 0, -1, a.nx, a.ny, a.nz), c, f);
-        st9(plane(a, ADJ_FLX, n), n, c, f);
-        face_flux<RIEM, 1>(a, n, nbr(x, 1, -1, a.nx, a.ny, a.nz), c, f);
-        st9(plane(a, ADJ_FLX + 9, n), n, c, f);
-        face_flux<RIEM, 2>(a, n, nbr(x, 2, -1, a.nx, a.ny, a.nz), c, f);
-        st9(plane(a, ADJ_FLX + 18, n), n, c, f);
+        face_flux<RIEM, 0>(a, nbr(a, x, 0, -1), x.o, f);
+        st9(a, ADJ_FLX, x.o, f);
+        face_flux<RIEM, 1>(a, nbr(a, x, 1, -1), x.o, f);
+        st9(a, ADJ_FLX + 9, x.o, f);
+        face_flux<RIEM, 2>(a, nbr(a, x, 2, -1), x.o, f);
+        st9(a, ADJ_FLX + 18, x.o, f);
     }
 }
 
@@ -182,18 +203,18 @@ __global__ void __launch_bounds__(ADJ_NT) adj_upre_kernel(AdjArgs a)
     const UpdOpts o{a.update_floor, a.do_turb};
     double fdot = 0.0;
     for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        const Cell x = cell_of(c, a.nx, a.ny);
+        const Cell x = cell_of(a, c);
         double acc[9], fl[9], fh[9];
-        ld9(plane(a, ADJ_FLX, n), n, c, fl);
-        ld9(plane(a, ADJ_FLX, n), n, nbr(x, 0, +1, a.nx, a.ny, a.nz), fh);
+        ld9(a, ADJ_FLX, x.o, fl);
+        ld9(a, ADJ_FLX, nbr(a, x, 0, +1), fh);
 #pragma unroll
         for (int v = 0; v < 9; ++v) acc[v] = fl[v] - fh[v];
-        ld9(plane(a, ADJ_FLX + 9, n), n, c, fl);
-        ld9(plane(a, ADJ_FLX + 9, n), n, nbr(x, 1, +1, a.nx, a.ny, a.nz), fh);
+        ld9(a, ADJ_FLX + 9, x.o, fl);
+        ld9(a, ADJ_FLX + 9, nbr(a, x, 1, +1), fh);
 #pragma unroll
         for (int v = 0; v < 9; ++v) acc[v] += fl[v] - fh[v];
-        ld9(plane(a, ADJ_FLX + 18, n), n, c, fl);
-        ld9(plane(a, ADJ_FLX + 18, n), n, nbr(x, 2, +1, a.nx, a.ny, a.nz), fh);
+        ld9(a, ADJ_FLX + 18, x.o, fl);
+        ld9(a, ADJ_FLX + 18, nbr(a, x, 2, +1), fh);
         double r[9], lam[9], rb[9];
 #pragma unroll
         for (int v = 0; v < 9; ++v) {
@@ -205,7 +226,7 @@ __global__ void __launch_bounds__(ADJ_NT) adj_upre_kernel(AdjArgs a)
         double a3[3] = {0.0, 0.0, 0.0}, a3b[3] = {0.0, 0.0, 0.0};
         if (a.do_turb) adj_force(a, x.i, x.j, x.k, a3);
         epilogue_adj<double>(r, a3, a.glm_fac, a.smallc, a.turb_min_rho, a.dt, o, a.ph, lam, rb, a3b);
-        st9(plane(a, ADJ_LPRE, n), n, c, rb);
+        st9(a, ADJ_LPRE, x.o, rb);
         fdot += a3b[0] * a3[0] + a3b[1] * a3[1] + a3b[2] * a3[2];
     }
     red[threadIdx.x] = fdot;
@@ -219,14 +240,14 @@ __global__ void __launch_bounds__(ADJ_NT) adj_upre_kernel(AdjArgs a)
 
 // ---- pass 4 ----------------------------------------------------------------------------------
 template <int RIEM, int D>
-GLM_DEV void face_adj(const AdjArgs& a, size_t n, const Cell& x)
+GLM_DEV void face_adj(const AdjArgs& a, const Cell& x)
 {
-    const size_t cl = nbr(x, D, -1, a.nx, a.ny, a.nz), cr = x.c;
+    const size_t cl = nbr(a, x, D, -1), cr = x.o;
     double L[9], R[9], lr[9], ll[9], ob[9];
-    ld9(plane(a, ADJ_FS + fs_slot(D, 1), n), n, cl, L);
-    ld9(plane(a, ADJ_FS + fs_slot(D, 0), n), n, cr, R);
-    ld9(plane(a, ADJ_LPRE, n), n, cr, lr);
-    ld9(plane(a, ADJ_LPRE, n), n, cl, ll);
+    ld9(a, ADJ_FS + fs_slot(D, 1), cl, L);
+    ld9(a, ADJ_FS + fs_slot(D, 0), cr, R);
+    ld9(a, ADJ_LPRE, cr, lr);
+    ld9(a, ADJ_LPRE, cl, ll);
     double Lb[9], Rb[9];
 #pragma unroll
     for (int v = 0; v < 9; ++v) {
@@ -235,18 +256,18 @@ GLM_DEV void face_adj(const AdjArgs& a, size_t n, const Cell& x)
         Rb[v] = 0.0;
     }
     riemann_adj<double, RIEM, D>(L, R, ob, Lb, Rb, a.ph);
-    st9(plane(a, ADJ_LFS + fs_slot(D, 1), n), n, cl, Lb);
-    st9(plane(a, ADJ_LFS + fs_slot(D, 0), n), n, cr, Rb);
+    st9(a, ADJ_LFS + fs_slot(D, 1), cl, Lb);
+    st9(a, ADJ_LFS + fs_slot(D, 0), cr, Rb);
 }
 template <int RIEM>
 __global__ void __launch_bounds__(ADJ_NT) adj_riemann_kernel(AdjArgs a)
 {
     const size_t n = (size_t)a.nx * a.ny * a.nz;
     for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        const Cell x = cell_of(c, a.nx, a.ny);
-        face_adj<RIEM, 0>(a, n, x);
-        face_adj<RIEM, 1>(a, n, x);
-        face_adj<RIEM, 2>(a, n, x);
+        const Cell x = cell_of(a, c);
+        face_adj<RIEM, 0>(a, x);
+        face_adj<RIEM, 1>(a, x);
+        face_adj<RIEM, 2>(a, x);
     }
 }
 
@@ -256,103 +277,88 @@ __global__ void __launch_bounds__(ADJ_NT) adj_riemann_kernel(AdjArgs a)
 // 1 + 2D and 2 + 2D, plus the cell's own slot 0 and the predictor adjoint MHB (the D = 0 launch
 // stores, the others add).  5h (full predictor): the predictor adjoint -> slots 0..6 (added).
 // One direction per launch keeps each thread's live set small.
-GLM_DEV void load_p(const AdjArgs& a, size_t n, size_t c, double* out9) { ld9(plane(a, ADJ_W, n), n, c, out9); }
-
 template <int PRED, int RECON, int SLOPE, int D>
 __global__ void __launch_bounds__(ADJ_NT) adj_cell_dir_kernel(AdjArgs a)
 {
     const size_t n = (size_t)a.nx * a.ny * a.nz;
     const FaceOpts o{a.mh_revert, a.face_guard};
-    double* C = plane(a, ADJ_CON, n);
-    double* MHB = plane(a, ADJ_MHB, n);
     for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        const Cell x = cell_of(c, a.nx, a.ny);
+        const Cell x = cell_of(a, c);
         double p0[9], l[9], r[9], mh[9], lob[9], hib[9], lb[9], m0b[9], rb[9], mhb[9];
-        load_p(a, n, c, p0);
-        load_p(a, n, nbr(x, D, -1, a.nx, a.ny, a.nz), l);
-        load_p(a, n, nbr(x, D, +1, a.nx, a.ny, a.nz), r);
+        load_p(a, x.o, p0);
+        load_p(a, nbr(a, x, D, -1), l);
+        load_p(a, nbr(a, x, D, +1), r);
         bool up = true;
         if (RECON == RECON_PPM) {
-            const double* P = plane(a, ADJ_W, n) + 4 * n;
+            const double* P = plane(a, ADJ_W + 4);
             double pr[6];
             for (int d = 0; d < 3; ++d) {
-                pr[2 * d] = P[nbr(x, d, -1, a.nx, a.ny, a.nz)];
-                pr[2 * d + 1] = P[nbr(x, d, +1, a.nx, a.ny, a.nz)];
+                pr[2 * d] = P[nbr(a, x, d, -1)];
+                pr[2 * d + 1] = P[nbr(a, x, d, +1)];
             }
             up = !(spj(pr[0], p0[4], pr[1]) || spj(pr[2], p0[4], pr[3]) || spj(pr[4], p0[4], pr[5]));
         }
-        if (PRED == PRED_FULL) ld9(plane(a, ADJ_MH, n), n, c, mh);
-        else for (int v = 0; v < 9; ++v) mh[v] = 0.0;
-        ld9(plane(a, ADJ_LFS + fs_slot(D, 0), n), n, c, lob);
-        ld9(plane(a, ADJ_LFS + fs_slot(D, 1), n), n, c, hib);
+        if (PRED == PRED_FULL) {
+            ld9(a, ADJ_MH, x.o, mh);
+            mh_revert(a, p0, mh);
+        } else for (int v = 0; v < 9; ++v) mh[v] = 0.0;
+        ld9(a, ADJ_LFS + fs_slot(D, 0), x.o, lob);
+        ld9(a, ADJ_LFS + fs_slot(D, 1), x.o, hib);
         for (int v = 0; v < 9; ++v) { lb[v] = 0.0; m0b[v] = 0.0; rb[v] = 0.0; mhb[v] = 0.0; }
         faces_adj<double, PRED, RECON, SLOPE, D>(l, p0, r, mh, up, a.half_dtdx, o, a.ph, lob, hib, lb, m0b, rb, mhb);
-        st9(C + (size_t)(1 + 2 * D) * 9 * n, n, c, lb);
-        st9(C + (size_t)(2 + 2 * D) * 9 * n, n, c, rb);
+        st9(a, ADJ_CON + (1 + 2 * D) * 9, x.o, lb);
+        st9(a, ADJ_CON + (2 + 2 * D) * 9, x.o, rb);
         if (D > 0) {
             double t[9];
-            ld9(C, n, c, t);
+            ld9(a, ADJ_CON, x.o, t);
             for (int v = 0; v < 9; ++v) m0b[v] += t[v];
             if (PRED == PRED_FULL) {
-                ld9(MHB, n, c, t);
+                ld9(a, ADJ_MHB, x.o, t);
                 for (int v = 0; v < 9; ++v) mhb[v] += t[v];
             }
         }
-        st9(C, n, c, m0b);
-        if (PRED == PRED_FULL) st9(MHB, n, c, mhb);
+        st9(a, ADJ_CON, x.o, m0b);
+        if (PRED == PRED_FULL) st9(a, ADJ_MHB, x.o, mhb);
     }
 }
 
 template <int SLOPE, int D>
-GLM_DEV void hancock_dir_add(const AdjArgs& a, size_t n, const Cell& x, const double p0[9], const double accb[9],
+GLM_DEV void hancock_dir_add(const AdjArgs& a, const Cell& x, const double p0[9], const double accb[9],
                              double p0b[9])
 {
     double l[9], r[9], lb[9], rb[9], t[9];
-    const size_t cl = nbr(x, D, -1, a.nx, a.ny, a.nz), cr = nbr(x, D, +1, a.nx, a.ny, a.nz);
-    load_p(a, n, cl, l);
-    load_p(a, n, cr, r);
+    const size_t cl = nbr(a, x, D, -1), cr = nbr(a, x, D, +1);
+    load_p(a, cl, l);
+    load_p(a, cr, r);
     for (int v = 0; v < 9; ++v) { lb[v] = 0.0; rb[v] = 0.0; }
     hancock_adj_dir<double, SLOPE, D>(p0, l, r, accb, p0b, lb, rb, a.ph);
-    double* C = plane(a, ADJ_CON, n);
-    ld9(C + (size_t)(1 + 2 * D) * 9 * n, n, x.c, t);
+    ld9(a, ADJ_CON + (1 + 2 * D) * 9, x.o, t);
     for (int v = 0; v < 9; ++v) t[v] += lb[v];
-    st9(C + (size_t)(1 + 2 * D) * 9 * n, n, x.c, t);
-    ld9(C + (size_t)(2 + 2 * D) * 9 * n, n, x.c, t);
+    st9(a, ADJ_CON + (1 + 2 * D) * 9, x.o, t);
+    ld9(a, ADJ_CON + (2 + 2 * D) * 9, x.o, t);
     for (int v = 0; v < 9; ++v) t[v] += rb[v];
-    st9(C + (size_t)(2 + 2 * D) * 9 * n, n, x.c, t);
+    st9(a, ADJ_CON + (2 + 2 * D) * 9, x.o, t);
 }
-template <int SLOPE, int D>
-GLM_DEV void hancock_acc_load(const AdjArgs& a, size_t n, const Cell& x, const double p0[9], double acc[9])
-{
-    double l[9], r[9];
-    load_p(a, n, nbr(x, D, -1, a.nx, a.ny, a.nz), l);
-    load_p(a, n, nbr(x, D, +1, a.nx, a.ny, a.nz), r);
-    hancock_acc_dir<double, SLOPE, D>(p0, l, r, acc, a.ph);
-}
-
 template <int SLOPE>
 __global__ void __launch_bounds__(ADJ_NT) adj_hancock_kernel(AdjArgs a)
 {
     const size_t n = (size_t)a.nx * a.ny * a.nz;
-    double* C = plane(a, ADJ_CON, n);
     for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        const Cell x = cell_of(c, a.nx, a.ny);
-        double p0[9], acc[9], mhb[9], p0b[9], accb[9];
-        load_p(a, n, c, p0);
-        ld9(plane(a, ADJ_MHB, n), n, c, mhb);
-        for (int v = 0; v < 9; ++v) { acc[v] = 0.0; p0b[v] = 0.0; }
-        hancock_acc_load<SLOPE, 0>(a, n, x, p0, acc);
-        hancock_acc_load<SLOPE, 1>(a, n, x, p0, acc);
-        hancock_acc_load<SLOPE, 2>(a, n, x, p0, acc);
-        if (hancock_core_from_acc(p0, acc, mhb, p0b, accb, a.half_dtdx, a.mh_revert, a.ph)) {
-            hancock_dir_add<SLOPE, 0>(a, n, x, p0, accb, p0b);
-            hancock_dir_add<SLOPE, 1>(a, n, x, p0, accb, p0b);
-            hancock_dir_add<SLOPE, 2>(a, n, x, p0, accb, p0b);
+        const Cell x = cell_of(a, c);
+        double p0[9], mh[9], mhb[9], p0b[9], accb[9];
+        load_p(a, x.o, p0);
+        ld9(a, ADJ_MHB, x.o, mhb);
+        ld9(a, ADJ_MH, x.o, mh);
+        for (int v = 0; v < 9; ++v) p0b[v] = 0.0;
+        if (hancock_adj_core(p0, mh, mhb, p0b, accb, a.half_dtdx, a.mh_revert, a.ph)) {
+            hancock_dir_add<SLOPE, 0>(a, x, p0, accb, p0b);
+            hancock_dir_add<SLOPE, 1>(a, x, p0, accb, p0b);
+            hancock_dir_add<SLOPE, 2>(a, x, p0, accb, p0b);
         }
         double t[9];
-        ld9(C, n, c, t);
+        ld9(a, ADJ_CON, x.o, t);
         for (int v = 0; v < 9; ++v) t[v] += p0b[v];
-        st9(C, n, c, t);
+        st9(a, ADJ_CON, x.o, t);
     }
 }
 
@@ -360,22 +366,20 @@ __global__ void __launch_bounds__(ADJ_NT) adj_hancock_kernel(AdjArgs a)
 __global__ void __launch_bounds__(ADJ_NT) adj_gather_kernel(AdjArgs a)
 {
     const size_t n = (size_t)a.nx * a.ny * a.nz;
-    const double* C = plane(a, ADJ_CON, n);
     for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        const Cell x = cell_of(c, a.nx, a.ny);
-        double wb[9], t[9], u[9], lb[9];
-        ld9(C, n, c, wb);
+        const Cell x = cell_of(a, c);
+        double wb[9], t[9], w[9], lb[9];
+        ld9(a, ADJ_CON, x.o, wb);
         for (int d = 0; d < 3; ++d) {
             // the -d neighbour's +d contribution and the +d neighbour's -d contribution aim at c
-            ld9(C + (size_t)(2 + 2 * d) * 9 * n, n, nbr(x, d, -1, a.nx, a.ny, a.nz), t);
+            ld9(a, ADJ_CON + (2 + 2 * d) * 9, nbr(a, x, d, -1), t);
             for (int v = 0; v < 9; ++v) wb[v] += t[v];
-            ld9(C + (size_t)(1 + 2 * d) * 9 * n, n, nbr(x, d, +1, a.nx, a.ny, a.nz), t);
+            ld9(a, ADJ_CON + (1 + 2 * d) * 9, nbr(a, x, d, +1), t);
             for (int v = 0; v < 9; ++v) wb[v] += t[v];
         }
-#pragma unroll
-        for (int v = 0; v < 9; ++v) u[v] = a.u0[v][c];
-        ld9(plane(a, ADJ_LPRE, n), n, c, lb);
-        cons2prim_adj(u, wb, lb, a.ph);
+        load_p(a, x.o, w);
+        ld9(a, ADJ_LPRE, x.o, lb);
+        cons2prim_adj_q(w, wb, lb, a.ph);
 #pragma unroll
         for (int v = 0; v < 9; ++v) a.lam0[v][c] = lb[v];
     }

@@ -7,7 +7,7 @@ namespace glm {
 
 constexpr int ADJ_NT = 256;
 
-// Scratch planes of the reverse step (n doubles each).
+// Scratch planes of the reverse step (n doubles each, interleaved row by row: adj_impl.hpp adj_index).
 constexpr int ADJ_W = 0, ADJ_MH = 9, ADJ_FS = 18, ADJ_LPRE = 72, ADJ_LFS = 81, ADJ_CON = 135, ADJ_MHB = 198,
               ADJ_FLX = 207, ADJ_NPLANES = 234;   // ADJ_FLX: the flux through each cell's three lower faces
 
@@ -30,9 +30,9 @@ struct AdjArgs {
 size_t adj_scratch_bytes(size_t n);
 // Launch the reverse step and add the step's sum of (kick acceleration adjoint . acceleration)
 // to *fdot (device).  With fused, the face-state and predictor adjoints and the gather run as one
-// z-march kernel (adj_march.hpp, z planes per tile: zchunk, 0 = the occupancy model); otherwise as
-// the separate passes 5 and 6.  a.scr and a.part must come from a scratch of adj_scratch_bytes(n).
-// Returns hipErrorInvalidValue for an unsupported scheme.
+// z-march kernel (adj_march.hpp, z planes per tile: zchunk, 0 = the occupancy model) where a z plane
+// of the scratch is below 4 GiB; otherwise as the separate passes 5 and 6.  a.scr and a.part must come
+// from a scratch of adj_scratch_bytes(n).  Returns hipErrorInvalidValue for an unsupported scheme.
 hipError_t launch_step_adjoint(AdjArgs a, void* scratch, int pred, int riem, int recon, int slope, double* fdot,
                                bool fused, int zchunk, hipStream_t st);
 

@@ -49,6 +49,23 @@ GLM_HD void cons2prim_adj(const T c[9], const T qb[9], T cb[9], const Phys<T>& s
     for (int j = 5; j <= 8; ++j) cb[j] += qb[j];
 }
 
+// The same from q = cons2prim(c): the floors act where q sits on them, and c enters only through the
+// density and the velocities q holds.
+template <typename T>
+GLM_HD void cons2prim_adj_q(const T q[9], const T qb[9], T cb[9], const Phys<T>& s)
+{
+    const T ir = trcp(q[0]);
+    const T g = q[4] > s.pfl ? (s.gamma - T(1)) * qb[4] : T(0);
+    const T vb = q[1] * qb[1] + q[2] * qb[2] + q[3] * qb[3];
+    const T v2 = q[1] * q[1] + q[2] * q[2] + q[3] * q[3];
+    const T rho_b = qb[0] - ir * vb + g * T(0.5) * v2;
+    cb[0] += q[0] > s.smallr ? rho_b : T(0);
+    for (int i = 1; i <= 3; ++i) cb[i] += qb[i] * ir - g * q[i];
+    cb[4] += g;
+    for (int j = 5; j <= 7; ++j) cb[j] += qb[j] - g * q[j];
+    cb[8] += qb[8];
+}
+
 // ---- prim2cons (glmmhd_turb.jl:79-86) ------------------------------------------------------
 template <typename T>
 GLM_HD void prim2cons_adj(const T q[9], const T cb[9], T qb[9], const Phys<T>& s)
@@ -62,28 +79,37 @@ GLM_HD void prim2cons_adj(const T q[9], const T cb[9], T qb[9], const Phys<T>& s
 }
 
 // ---- flux_dir (glmmhd_turb.jl:98-115 in direction D) --------------------------------------
+// (the set form writes qb[0..7]; the flux does not depend on psi)
 template <typename T, int D>
-GLM_HD void flux_dir_adj(const T q[9], const T fb[9], T qb[9], const Phys<T>& s)
+GLM_HD void flux_dir_adj_set(const T q[9], const T fb[9], T qb[8], const Phys<T>& s)
 {
     constexpr int A = D % 3, B = (D + 1) % 3, C = (D + 2) % 3;
     const T rho = q[0], un = q[1 + A], u1 = q[1 + B], u2 = q[1 + C], p = q[4];
     const T bn = q[5 + A], b1 = q[5 + B], b2_ = q[5 + C];
-    const T b2 = bn * bn + b1 * b1 + b2_ * b2_;
-    const T ptot = p + T(0.5) * b2;
+    const T bt = b1 * b1 + b2_ * b2_;
     const T u2s = un * un + u1 * u1 + u2 * u2;
-    const T E = p * s.igm1 + T(0.5) * rho * u2s + T(0.5) * b2;
-    const T vdotb = un * bn + u1 * b1 + u2 * b2_;
+    const T g1 = s.igm1 + T(1);                                        // E + ptot - bn^2 = g1 p + rho u^2 / 2 + bt
     const T g0 = fb[0], gA = fb[1 + A], gB = fb[1 + B], gC = fb[1 + C], g4 = fb[4];
     const T hB = fb[5 + B], hC = fb[5 + C];
-    qb[0] += g0 * un + gA * un * un + gB * un * u1 + gC * un * u2 + g4 * un * T(0.5) * u2s;
-    qb[1 + A] += g0 * rho + gA * T(2) * rho * un + gB * rho * u1 + gC * rho * u2 +
-                 g4 * ((E + ptot) + rho * un * un - bn * bn) + hB * b1 + hC * b2_;
-    qb[1 + B] += gB * rho * un + g4 * (rho * un * u1 - bn * b1) - hB * bn;
-    qb[1 + C] += gC * rho * un + g4 * (rho * un * u2 - bn * b2_) - hC * bn;
-    qb[4] += gA + g4 * un * (s.igm1 + T(1));
-    qb[5 + A] += -gA * bn - gB * b1 - gC * b2_ + g4 * (un * bn - vdotb) - hB * u1 - hC * u2;
-    qb[5 + B] += gA * b1 - gB * bn + g4 * (T(2) * un * b1 - bn * u1) + hB * un;
-    qb[5 + C] += gA * b2_ - gC * bn + g4 * (T(2) * un * b2_ - bn * u2) + hC * un;
+    const T m = rho * un, t = g4 * un;
+    const T x = g0 + gA * un + gB * u1 + gC * u2;
+    const T kB = gB + g4 * u1, kC = gC + g4 * u2;
+    const T jB = hB + g4 * b1, jC = hC + g4 * b2_;
+    qb[0] = un * (x + T(0.5) * g4 * u2s);
+    qb[1 + A] = rho * (x + gA * un) + g4 * (g1 * p + T(0.5) * rho * u2s + bt) + m * t + hB * b1 + hC * b2_;
+    qb[1 + B] = m * kB - bn * jB;
+    qb[1 + C] = m * kC - bn * jC;
+    qb[4] = gA + t * g1;
+    qb[5 + A] = -(gA * bn + b1 * kB + b2_ * kC + hB * u1 + hC * u2);
+    qb[5 + B] = b1 * (gA + T(2) * t) - bn * kB + hB * un;
+    qb[5 + C] = b2_ * (gA + T(2) * t) - bn * kC + hC * un;
+}
+template <typename T, int D>
+GLM_HD void flux_dir_adj(const T q[9], const T fb[9], T qb[9], const Phys<T>& s)
+{
+    T x[8];
+    flux_dir_adj_set<T, D>(q, fb, x, s);
+    for (int v = 0; v < 8; ++v) qb[v] += x[v];
 }
 
 // ---- fast_speed (glmmhd_turb.jl:89-95) ------------------------------------------------------
@@ -116,46 +142,55 @@ GLM_HD void fast_speed_adj(T rho, T p, T b2, T bn, T cfb, T& rho_b, T& p_b, T& b
 }
 
 // ---- limiters and reconstructions -----------------------------------------------------------
-// moncen (glmmhd_turb.jl:145-150): adjoint w.r.t. (dl, dr)
+// Written with weights picked by selects: one weight pair per variable instead of a tree of divergent
+// branches (in the reverse march nine variables x three directions took every arm of every one).
+// moncen (glmmhd_turb.jl:145-150): adjoint w.r.t. (dl, dr).  Where the slope is not zero dl, dr and
+// dc share a sign, so m = 2 dl, 2 dr or dc.
 template <typename T>
 GLM_HD void moncen_adj(T dl, T dr, T mb, T& dl_b, T& dr_b)
 {
-    if (dl * dr <= T(0)) return;
-    const T dc = T(0.5) * (dl + dr);
-    const T a = T(2) * tmin(tabs(dl), tabs(dr)), b = tabs(dc);
-    const T g = mb * sgn1(dc);   // d copysign(m, dc)/dm
-    if (a < b) {
-        if (tabs(dl) <= tabs(dr)) dl_b += T(2) * sgn1(dl) * g;
-        else dr_b += T(2) * sgn1(dr) * g;
-    } else {
-        const T dc_b = g * sgn1(dc);
-        dl_b += T(0.5) * dc_b;
-        dr_b += T(0.5) * dc_b;
-    }
+    const T al = tabs(dl), ar = tabs(dr);
+    const bool two = T(2) * tmin(al, ar) < tabs(T(0.5) * (dl + dr));
+    const bool left = al <= ar;
+    const T g = dl * dr <= T(0) ? T(0) : mb;
+    dl_b = (two ? (left ? T(2) : T(0)) : T(0.5)) * g;
+    dr_b = (two ? (left ? T(0) : T(2)) : T(0.5)) * g;
 }
 template <typename T>
 GLM_HD void minmod_adj(T a, T b, T mb, T& a_b, T& b_b)
 {
-    if (a * b <= T(0)) return;
-    if (tabs(a) < tabs(b)) a_b += mb;
-    else b_b += mb;
+    const bool left = tabs(a) < tabs(b);
+    const T g = a * b <= T(0) ? T(0) : mb;
+    a_b = left ? g : T(0);
+    b_b = left ? T(0) : g;
 }
-// half slope h(l, m, r) (glmmhd_turb.jl:153-155, :302-303)
+// half slope h(l, m, r) (glmmhd_turb.jl:153-155, :302-303): sets the neighbours' adjoints
 template <typename T, int SLOPE>
-GLM_HD void half_slope_adj(T l, T m, T r, T hb, T& l_b, T& m_b, T& r_b)
+GLM_HD void half_slope_adj_set(T l, T m, T r, T hb, T& l_b, T& m_b, T& r_b)
 {
     const T dl = m - l, dr = r - m;
-    T dl_b = T(0), dr_b = T(0);
+    T dl_b, dr_b;
     if (SLOPE == SLOPE_MINMOD) minmod_adj(dl, dr, T(0.5) * hb, dl_b, dr_b);
     else moncen_adj(dl, dr, T(0.5) * hb, dl_b, dr_b);
     m_b += dl_b - dr_b;
-    l_b -= dl_b;
-    r_b += dr_b;
+    l_b = -dl_b;
+    r_b = dr_b;
+}
+template <typename T, int SLOPE>
+GLM_HD void half_slope_adj(T l, T m, T r, T hb, T& l_b, T& m_b, T& r_b)
+{
+    T a, b;
+    half_slope_adj_set<T, SLOPE>(l, m, r, hb, a, m_b, b);
+    l_b += a;
+    r_b += b;
 }
 
-// ppm_edges (glmmhd_turb.jl:917-923)
+// ppm_edges (glmmhd_turb.jl:917-923) relative to the cell value: adjoint of (ql - q0, qr - q0), the
+// offsets the face states are built from.  The reset edges are ql = 3 q0 - 2 qr and qr = 3 q0 - 2 ql,
+// so with a and b the adjoints that reach the unlimited edges, the offsets' pull on q0 is that of the
+// parabola's curvature alone.  Sets the neighbours' adjoints.
 template <typename T>
-GLM_HD void ppm_edges_adj(T qm, T q0, T qp, T lo_b, T hi_b, T& qm_b, T& q0_b, T& qp_b)
+GLM_HD void ppm_offsets_adj(T qm, T q0, T qp, T lo_b, T hi_b, T& qm_b, T& q0_b, T& qp_b)
 {
     const T slope = T(0.25) * (qp - qm);
     const T curve = (qm - T(2) * q0 + qp) * T(1.0 / 12.0);
@@ -166,21 +201,24 @@ GLM_HD void ppm_edges_adj(T qm, T q0, T qp, T lo_b, T hi_b, T& qm_b, T& q0_b, T&
     const bool flat = (qr - q0) * (q0 - ql) <= T(0);
     const bool hi_os = diff > lim;
     const bool lo_os = diff < -lim;
-    T ql_b = T(0), qr_b = T(0);
-    if (flat) {
-        q0_b += lo_b + hi_b;
-        return;
-    }
-    if (hi_os) { q0_b += T(3) * lo_b; qr_b -= T(2) * lo_b; }
-    else ql_b += lo_b;
-    if (hi_os) qr_b += hi_b;
-    else if (lo_os) { q0_b += T(3) * hi_b; ql_b -= T(2) * hi_b; }
-    else qr_b += hi_b;
-    q0_b += ql_b + qr_b;
-    const T slope_b = qr_b - ql_b, curve_b = (ql_b + qr_b) * T(1.0 / 12.0);
-    qp_b += T(0.25) * slope_b + curve_b;
-    qm_b += -T(0.25) * slope_b + curve_b;
-    q0_b += -T(2) * curve_b;
+    T a = hi_os ? T(0) : (lo_os ? lo_b - T(2) * hi_b : lo_b);
+    T b = hi_os ? hi_b - T(2) * lo_b : (lo_os ? T(0) : hi_b);
+    a = flat ? T(0) : a;
+    b = flat ? T(0) : b;
+    const T slope_b = T(0.25) * (b - a), curve_b = (a + b) * T(1.0 / 12.0);
+    qp_b = curve_b + slope_b;
+    qm_b = curve_b - slope_b;
+    q0_b -= T(2) * curve_b;
+}
+// ppm_edges itself.
+template <typename T>
+GLM_HD void ppm_edges_adj(T qm, T q0, T qp, T lo_b, T hi_b, T& qm_b, T& q0_b, T& qp_b)
+{
+    T a, b;
+    q0_b += lo_b + hi_b;
+    ppm_offsets_adj(qm, q0, qp, lo_b, hi_b, a, q0_b, b);
+    qm_b += a;
+    qp_b += b;
 }
 
 // ---- Riemann solvers (x frame; L, R floored and GLM-cleaned) ---------------------------------
@@ -652,6 +690,12 @@ GLM_HD void hanc1d_adj(const T c0[9], const T hs[9], const T mhb[9], T c0b[9], T
     for (int v = 0; v < 9; ++v) { c0b[v] += tpb[v] + tmb[v]; hsb[v] += tpb[v] - tmb[v]; }
 }
 
+// Is the predictor's result mh (before the revert) one that reverts to the cell's own state?
+template <typename T>
+GLM_HD bool hancock_reverts(const T mh[9], int mh_revert, const Phys<T>& s)
+{
+    return mh_revert && (mh[0] <= s.smallr || mh[4] <= s.pfl);
+}
 // Full-transverse Hancock predictor of one cell (glmmhd_turb.jl:165-172, revert :391-395) from
 // its six neighbours nb[2d] (low) and nb[2d+1] (high) in direction d.  Returns true if reverted.
 template <typename T, int SLOPE>
@@ -672,7 +716,7 @@ GLM_HD bool hancock_fwd(const T p0[9], const T (*nb)[9], T mh[9], T half_dtdx, i
     prim2cons(p0, t, s);
     for (int v = 0; v < 9; ++v) t[v] = t[v] - half_dtdx * acc[v];
     cons2prim(t, mh, s);
-    if (mh_revert && (mh[0] <= s.smallr || mh[4] <= s.pfl)) {
+    if (hancock_reverts(mh, mh_revert, s)) {
         for (int v = 0; v < 9; ++v) mh[v] = p0[v];
         return true;
     }
@@ -680,78 +724,55 @@ GLM_HD bool hancock_fwd(const T p0[9], const T (*nb)[9], T mh[9], T half_dtdx, i
 }
 // The predictor's adjoint in two parts, so that a kernel can take the directions one at a time:
 // the core (conversions and the revert) gives the adjoint of the flux sum, accb; each direction
-// then adds its flux and slope adjoints.  Returns false if the predictor reverted (mh = p0).
-template <typename T, int SLOPE, int D>
-GLM_HD void hancock_acc_dir(const T p0[9], const T l[9], const T r[9], T acc[9], const Phys<T>& s)
-{
-    T t[9], f[9];
-    for (int sgn = 0; sgn < 2; ++sgn) {
-        for (int v = 0; v < 9; ++v) {
-            const T h = half_slope<T, SLOPE>(l[v], p0[v], r[v]);
-            t[v] = sgn == 0 ? p0[v] + h : p0[v] - h;
-        }
-        flux_dir<T, D>(t, f, s);
-        for (int v = 0; v < 9; ++v) acc[v] = sgn == 0 ? acc[v] + f[v] : acc[v] - f[v];
-    }
-}
-// Core from the flux sum acc of the three directions.
+// then adds its flux and slope adjoints.  mh is the predictor's result before the revert; returns
+// false (accb is not set) where it reverts.
 template <typename T>
-GLM_HD bool hancock_core_from_acc(const T p0[9], const T acc[9], const T mhb[9], T p0b[9], T accb[9], T half_dtdx,
-                                  int mh_revert, const Phys<T>& s)
+GLM_HD bool hancock_adj_core(const T p0[9], const T mh[9], const T mhb[9], T p0b[9], T accb[9], T half_dtdx,
+                             int mh_revert, const Phys<T>& s)
 {
-    T u[9], mh[9];
-    prim2cons(p0, u, s);
-    for (int v = 0; v < 9; ++v) u[v] = u[v] - half_dtdx * acc[v];
-    cons2prim(u, mh, s);
-    if (mh_revert && (mh[0] <= s.smallr || mh[4] <= s.pfl)) {
+    if (hancock_reverts(mh, mh_revert, s)) {
         for (int v = 0; v < 9; ++v) p0b[v] += mhb[v];
         return false;
     }
     T ub[9] = {T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
-    cons2prim_adj(u, mhb, ub, s);
+    cons2prim_adj_q(mh, mhb, ub, s);
     prim2cons_adj(p0, ub, p0b, s);
     for (int v = 0; v < 9; ++v) accb[v] = -half_dtdx * ub[v];
     return true;
 }
-template <typename T, int SLOPE>
-GLM_HD bool hancock_adj_core(const T p0[9], const T (*nb)[9], const T mhb[9], T p0b[9], T accb[9], T half_dtdx,
-                             int mh_revert, const Phys<T>& s)
+// Flux part of one direction: from the flux-sum adjoint accb to the adjoints of the cell (added to
+// p0b) and of its half slopes hs (hsb is set); psi has no flux here.
+template <typename T, int D>
+GLM_HD void hancock_adj_flux(const T p0[9], const T hs[9], const T accb[9], T p0b[9], T hsb[8], const Phys<T>& s)
 {
-    T acc[9];
-    for (int v = 0; v < 9; ++v) acc[v] = T(0);
-    hancock_acc_dir<T, SLOPE, 0>(p0, nb[0], nb[1], acc, s);
-    hancock_acc_dir<T, SLOPE, 1>(p0, nb[2], nb[3], acc, s);
-    hancock_acc_dir<T, SLOPE, 2>(p0, nb[4], nb[5], acc, s);
-    return hancock_core_from_acc(p0, acc, mhb, p0b, accb, half_dtdx, mh_revert, s);
+    T t[9], tb[8];
+    for (int v = 0; v < 9; ++v) t[v] = p0[v] + hs[v];
+    flux_dir_adj_set<T, D>(t, accb, hsb, s);
+    for (int v = 0; v < 9; ++v) t[v] = p0[v] - hs[v];
+    flux_dir_adj_set<T, D>(t, accb, tb, s);
+    for (int v = 0; v < 8; ++v) {
+        p0b[v] += hsb[v] - tb[v];
+        hsb[v] += tb[v];
+    }
 }
 template <typename T, int SLOPE, int D>
 GLM_HD void hancock_adj_dir(const T p0[9], const T l[9], const T r[9], const T accb[9], T p0b[9], T lb[9], T rb[9],
                             const Phys<T>& s)
 {
-    T hs[9], hsb[9];
-    for (int v = 0; v < 9; ++v) { hs[v] = half_slope<T, SLOPE>(l[v], p0[v], r[v]); hsb[v] = T(0); }
-    for (int sgn = 0; sgn < 2; ++sgn) {
-        T t[9], fb_[9], tb[9];
-        for (int v = 0; v < 9; ++v) {
-            t[v] = sgn == 0 ? p0[v] + hs[v] : p0[v] - hs[v];
-            fb_[v] = sgn == 0 ? accb[v] : -accb[v];
-            tb[v] = T(0);
-        }
-        flux_dir_adj<T, D>(t, fb_, tb, s);
-        for (int v = 0; v < 9; ++v) {
-            p0b[v] += tb[v];
-            hsb[v] += sgn == 0 ? tb[v] : -tb[v];
-        }
-    }
-    for (int v = 0; v < 9; ++v) half_slope_adj<T, SLOPE>(l[v], p0[v], r[v], hsb[v], lb[v], p0b[v], rb[v]);
+    T hs[9], hsb[8];
+    for (int v = 0; v < 8; ++v) hs[v] = half_slope<T, SLOPE>(l[v], p0[v], r[v]);
+    hs[8] = T(0);
+    hancock_adj_flux<T, D>(p0, hs, accb, p0b, hsb, s);
+    for (int v = 0; v < 8; ++v) half_slope_adj<T, SLOPE>(l[v], p0[v], r[v], hsb[v], lb[v], p0b[v], rb[v]);
 }
 
 template <typename T, int SLOPE>
 GLM_HD void hancock_adj(const T p0[9], const T (*nb)[9], const T mhb[9], T p0b[9], T (*nbb)[9], T half_dtdx,
                         int mh_revert, const Phys<T>& s)
 {
-    T accb[9];
-    if (!hancock_adj_core<T, SLOPE>(p0, nb, mhb, p0b, accb, half_dtdx, mh_revert, s)) return;
+    T mh[9], accb[9];
+    hancock_fwd<T, SLOPE>(p0, nb, mh, half_dtdx, 0, s);
+    if (!hancock_adj_core(p0, mh, mhb, p0b, accb, half_dtdx, mh_revert, s)) return;
     hancock_adj_dir<T, SLOPE, 0>(p0, nb[0], nb[1], accb, p0b, nbb[0], nbb[1], s);
     hancock_adj_dir<T, SLOPE, 1>(p0, nb[2], nb[3], accb, p0b, nbb[2], nbb[3], s);
     hancock_adj_dir<T, SLOPE, 2>(p0, nb[4], nb[5], accb, p0b, nbb[4], nbb[5], s);
@@ -856,8 +877,10 @@ GLM_HD void faces_adj(const T l[9], const T m0[9], const T r[9], const T mhf[9],
     if (RECON == RECON_PPM) {
         if (up) {
             for (int v = 0; v < 9; ++v) {
-                m0b[v] -= lob[v] + hib[v];
-                ppm_edges_adj(l[v], m0[v], r[v], lob[v], hib[v], lb[v], m0b[v], rb[v]);
+                T a, b;
+                ppm_offsets_adj(l[v], m0[v], r[v], lob[v], hib[v], a, m0b[v], b);
+                lb[v] += a;
+                rb[v] += b;
             }
         } else {
             for (int v = 0; v < 9; ++v) {

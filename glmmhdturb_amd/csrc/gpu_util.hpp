@@ -77,6 +77,28 @@ GLM_DEV T gload(const T* p)
     return *p;   // host pass of the kernel templates: never executed
 #endif
 }
+// The same at a byte offset from a base that is one for the wavefront: where the offset is a 32-bit
+// value of its own the instruction adds the two.
+template <typename T>
+GLM_DEV T gload_at(const T* base, unsigned off)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const __attribute__((address_space(1))) char* b = (const __attribute__((address_space(1))) char*)base;
+    return *(const __attribute__((address_space(1))) T*)(b + off);
+#else
+    return *(const T*)((const char*)base + off);
+#endif
+}
+template <typename T>
+GLM_DEV void gstore_at(T* base, unsigned off, T x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    __attribute__((address_space(1))) char* b = (__attribute__((address_space(1))) char*)base;
+    *(__attribute__((address_space(1))) T*)(b + off) = x;
+#else
+    *(T*)((char*)base + off) = x;
+#endif
+}
 
 template <typename T>
 GLM_DEV void gstore_nt(T v, T* p)
