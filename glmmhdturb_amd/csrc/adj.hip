@@ -3,6 +3,8 @@
 #include "adj_march.hpp"
 #include "launch.hpp"
 
+#include <cstring>
+
 namespace glm {
 
 constexpr unsigned ADJ_GRID_MAX = 2048;
@@ -13,69 +15,73 @@ static unsigned adj_grid(size_t n)
     return (unsigned)(g < ADJ_GRID_MAX ? (g > 0 ? g : 1) : ADJ_GRID_MAX);
 }
 
-size_t adj_scratch_bytes(size_t n) { return (size_t)ADJ_NPLANES * n * sizeof(double) + ADJ_GRID_MAX * sizeof(double); }
+size_t adj_scratch_bytes(size_t n) { return (size_t)(ADJ_NPLANES + 1) * n * sizeof(double); }
+
+// Passes 1-3 as one march; nparts: the workgroups, each with a partial sum in a.part.
+static hipError_t dispatch_front(const AdjArgs& a, int zchunk, hipStream_t st, int pred, int riem, int recon, int slope,
+                                 int& nparts)
+{
+    MarchArgs<double> m;
+    memset(&m, 0, sizeof m);
+    for (int v = 0; v < 9; ++v) m.q[v] = a.u0[v];
+    m.nx = a.nx; m.ny = a.ny; m.nz = a.nz;
+    march_tiling<double>(a.nx, a.ny, a.nz, zchunk, Resident{256, 2}, m.tiles_x, m.tiles_y, m.nzc, m.zchunk);
+    m.ph = a.ph;
+    m.dtdx = a.dtdx; m.half_dtdx = a.half_dtdx; m.glm_fac = a.glm_fac;
+    m.smallc = a.smallc; m.turb_min_rho = a.turb_min_rho; m.ramp = a.ramp; m.dt = a.dt;
+    m.dx = a.dx; m.lx = a.lx; m.ly = a.ly; m.lz = a.lz;
+    m.recon = recon; m.slope = slope;
+    m.mh_revert = a.mh_revert; m.face_guard = a.face_guard; m.update_floor = a.update_floor;
+    m.do_turb = a.do_turb; m.tgs = a.tgs; m.afield = a.afield;
+    nparts = m.tiles_x * m.tiles_y * m.nzc;
+#define GLM_CASE(P, R) if (pred == P && riem == R) return launch_adj_front_pr<P, R>(m, a, recon, slope, st);
+    GLM_CASE(PRED_FULL, RIEM_LLF) GLM_CASE(PRED_FULL, RIEM_LLFB) GLM_CASE(PRED_FULL, RIEM_HLL) GLM_CASE(PRED_FULL, RIEM_HLLD)
+    GLM_CASE(PRED_ONED, RIEM_LLF) GLM_CASE(PRED_ONED, RIEM_LLFB) GLM_CASE(PRED_ONED, RIEM_HLL) GLM_CASE(PRED_ONED, RIEM_HLLD)
+#undef GLM_CASE
+    return hipErrorInvalidValue;
+}
 
 template <int PRED, int RECON, int SLOPE>
-static void launch_cellwise(const AdjArgs& a, dim3 g, hipStream_t st, bool faces)
+static void launch_cellwise(const AdjArgs& a, dim3 g, hipStream_t st)
 {
-    if (faces) {
-        hipLaunchKernelGGL((adj_faces_kernel<PRED, RECON, SLOPE>), g, dim3(ADJ_NT), 0, st, a);
-        return;
-    }
     hipLaunchKernelGGL((adj_cell_dir_kernel<PRED, RECON, SLOPE, 0>), g, dim3(ADJ_NT), 0, st, a);
     hipLaunchKernelGGL((adj_cell_dir_kernel<PRED, RECON, SLOPE, 1>), g, dim3(ADJ_NT), 0, st, a);
     hipLaunchKernelGGL((adj_cell_dir_kernel<PRED, RECON, SLOPE, 2>), g, dim3(ADJ_NT), 0, st, a);
     if (PRED == PRED_FULL) hipLaunchKernelGGL((adj_hancock_kernel<SLOPE>), g, dim3(ADJ_NT), 0, st, a);
 }
 
-static bool dispatch_cellwise(const AdjArgs& a, dim3 g, hipStream_t st, bool faces, int pred, int recon, int slope)
+static void dispatch_cellwise(const AdjArgs& a, dim3 g, hipStream_t st, int pred, int recon, int slope)
 {
 #define GLM_CASE(P, RC, SL)                                          \
-    if (pred == P && recon == RC && slope == SL) {                   \
-        launch_cellwise<P, RC, SL>(a, g, st, faces);                 \
-        return true;                                                 \
-    }
+    if (pred == P && recon == RC && slope == SL) launch_cellwise<P, RC, SL>(a, g, st);
     GLM_CASE(PRED_FULL, RECON_PLM, SLOPE_MONCEN) GLM_CASE(PRED_FULL, RECON_PLM, SLOPE_MINMOD)
     GLM_CASE(PRED_FULL, RECON_PPM, SLOPE_MONCEN) GLM_CASE(PRED_FULL, RECON_PPM, SLOPE_MINMOD)
     GLM_CASE(PRED_ONED, RECON_PLM, SLOPE_MONCEN) GLM_CASE(PRED_ONED, RECON_PLM, SLOPE_MINMOD)
     GLM_CASE(PRED_ONED, RECON_PPM, SLOPE_MONCEN) GLM_CASE(PRED_ONED, RECON_PPM, SLOPE_MINMOD)
 #undef GLM_CASE
-    return false;
 }
 
-static bool dispatch_faceswise(const AdjArgs& a, dim3 g, hipStream_t st, bool upre, int riem)
+static void dispatch_riemann(const AdjArgs& a, dim3 g, hipStream_t st, int riem)
 {
-#define GLM_CASE(R)                                                                                       \
-    if (riem == R) {                                                                                      \
-        if (upre) {                                                                                       \
-            hipLaunchKernelGGL((adj_flux_kernel<R>), g, dim3(ADJ_NT), 0, st, a);                          \
-            hipLaunchKernelGGL(adj_upre_kernel, g, dim3(ADJ_NT), 0, st, a);                               \
-        } else {                                                                                          \
-            hipLaunchKernelGGL((adj_riemann_kernel<R>), g, dim3(ADJ_NT), 0, st, a);                       \
-        }                                                                                                 \
-        return true;                                                                                      \
-    }
+#define GLM_CASE(R) \
+    if (riem == R) hipLaunchKernelGGL((adj_riemann_kernel<R>), g, dim3(ADJ_NT), 0, st, a);
     GLM_CASE(RIEM_LLF) GLM_CASE(RIEM_LLFB) GLM_CASE(RIEM_HLL) GLM_CASE(RIEM_HLLD)
 #undef GLM_CASE
-    return false;
 }
 
-static bool dispatch_back(const AdjArgs& a, int zchunk, hipStream_t st, int pred, int recon, int slope)
+static void dispatch_back(const AdjArgs& a, int zchunk, hipStream_t st, int pred, int recon, int slope)
 {
     int tx, ty, nzc, zc;
     march_tiling<double>(a.nx, a.ny, a.nz, zchunk, Resident{256, adj_waves(pred)}, tx, ty, nzc, zc);
     const dim3 g((unsigned)(tx * ty * nzc));
 #define GLM_CASE(P, RC, SL)                                                                          \
-    if (pred == P && recon == RC && slope == SL) {                                                   \
-        hipLaunchKernelGGL((adj_back_kernel<P, RC, SL>), g, dim3(NT), 0, st, a, tx, ty, zc);         \
-        return true;                                                                                 \
-    }
+    if (pred == P && recon == RC && slope == SL)                                                     \
+        hipLaunchKernelGGL((adj_back_kernel<P, RC, SL>), g, dim3(NT), 0, st, a, tx, ty, zc);
     GLM_CASE(PRED_FULL, RECON_PLM, SLOPE_MONCEN) GLM_CASE(PRED_FULL, RECON_PLM, SLOPE_MINMOD)
     GLM_CASE(PRED_FULL, RECON_PPM, SLOPE_MONCEN) GLM_CASE(PRED_FULL, RECON_PPM, SLOPE_MINMOD)
     GLM_CASE(PRED_ONED, RECON_PLM, SLOPE_MONCEN) GLM_CASE(PRED_ONED, RECON_PLM, SLOPE_MINMOD)
     GLM_CASE(PRED_ONED, RECON_PPM, SLOPE_MONCEN) GLM_CASE(PRED_ONED, RECON_PPM, SLOPE_MINMOD)
 #undef GLM_CASE
-    return false;
 }
 
 hipError_t launch_step_adjoint(AdjArgs a, void* scratch, int pred, int riem, int recon, int slope, double* fdot,
@@ -86,16 +92,16 @@ hipError_t launch_step_adjoint(AdjArgs a, void* scratch, int pred, int riem, int
     a.scr = (double*)scratch;
     a.part = a.scr + (size_t)ADJ_NPLANES * n;
     const dim3 g(adj_grid(n));
-    hipLaunchKernelGGL(adj_prim_kernel, g, dim3(ADJ_NT), 0, st, a);
-    if (!dispatch_cellwise(a, g, st, true, pred, recon, slope)) return hipErrorInvalidValue;
-    if (!dispatch_faceswise(a, g, st, true, riem)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(adj_fdot_kernel, dim3(1), dim3(ADJ_NT), 0, st, (const double*)a.part, (int)g.x, fdot);
-    dispatch_faceswise(a, g, st, false, riem);
-    // the march's 32-bit offsets reach over one z plane of the scratch (2.29 million cells)
+    int nparts = 0;
+    const hipError_t e = dispatch_front(a, zchunk, st, pred, riem, recon, slope, nparts);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(adj_fdot_kernel, dim3(1), dim3(ADJ_NT), 0, st, (const double*)a.part, nparts, fdot);
+    dispatch_riemann(a, g, st, riem);
+    // the march's 32-bit offsets reach over one z plane of the scratch (2.59 million cells)
     if (fused && (size_t)ADJ_NPLANES * sizeof(double) * a.nx * a.ny <= UINT32_MAX) {
         dispatch_back(a, zchunk, st, pred, recon, slope);
     } else {
-        dispatch_cellwise(a, g, st, false, pred, recon, slope);
+        dispatch_cellwise(a, g, st, pred, recon, slope);
         hipLaunchKernelGGL(adj_gather_kernel, g, dim3(ADJ_NT), 0, st, a);
     }
     return hipGetLastError();

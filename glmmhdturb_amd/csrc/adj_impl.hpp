@@ -2,13 +2,10 @@
 //
 // Given the state u0 a step started from and the adjoint lam1 of the state it produced, the
 // kernels below compute lam0 = (dU1/dU0)^T lam1 for that step with its scalars (dt, ch, psi
-// decay, ramp, forcing field) held fixed.  The step is re-derived in passes, one thread per cell
-// (every pass is a stencil over the periodic grid):
-//   1 prim    W = c2p(u0)
-//   2 faces   predictor (full Hancock) and the six face states of every cell
-//   3 upre    the flux through every face, each solved once (FLX), then the step's flux
-//             divergence -> the pre-epilogue state and the epilogue adjoint (kick, psi decay,
-//             floor): LPRE = adjoint of the pre-epilogue state
+// decay, ramp, forcing field) held fixed.  The step is re-derived in passes over the periodic grid:
+//   1-3 front (adj_front.hpp, a z-march): W = c2p(u0), the predicted state, the six face states of
+//             every cell; the step's flux divergence -> the pre-epilogue state and the epilogue
+//             adjoint (kick, psi decay, floor): LPRE = adjoint of the pre-epilogue state
 //   4 riemann per lower face: lambda_F = dtdx (LPRE(c) - LPRE(c - e_d)), Riemann adjoint ->
 //             adjoints of the two face states meeting there (each slot has one writer)
 //   5 cell    face-state adjoints (one launch per direction) and the predictor adjoint of every
@@ -83,160 +80,7 @@ GLM_DEV void mh_revert(const AdjArgs& a, const double p0[9], double mh[9])
 #pragma unroll
     for (int v = 0; v < 9; ++v) mh[v] = rev ? p0[v] : mh[v];
 }
-// face-state slot: direction d, side 0 (low face) or 1 (high face)
-GLM_DEV int fs_slot(int d, int side) { return (d * 2 + side) * 9; }
-
-// ---- pass 1 ----------------------------------------------------------------------------------
-__global__ void __launch_bounds__(ADJ_NT) adj_prim_kernel(AdjArgs a)
-{
-    const size_t n = (size_t)a.nx * a.ny * a.nz;
-    for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        double u[9], w[9];
-#pragma unroll
-        for (int v = 0; v < 9; ++v) u[v] = a.u0[v][c];
-        cons2prim(u, w, a.ph);
-        st9(a, ADJ_W, cell_of(a, c).o, w);
-    }
-}
-
-// PPM strong-pressure-jump flag of a cell from its pressure stencil (glmmhd_turb.jl:959)
-GLM_DEV bool ppm_up(const double p0[9], const double (*nb)[9])
-{
-    return !(spj(nb[0][4], p0[4], nb[1][4]) || spj(nb[2][4], p0[4], nb[3][4]) || spj(nb[4][4], p0[4], nb[5][4]));
-}
-
 GLM_DEV void load_p(const AdjArgs& a, size_t o, double* out9) { ld9(a, ADJ_W, o, out9); }
-GLM_DEV void load_stencil(const AdjArgs& a, const Cell& x, double p0[9], double nb[6][9])
-{
-    load_p(a, x.o, p0);
-    for (int d = 0; d < 3; ++d) {
-        load_p(a, nbr(a, x, d, -1), nb[2 * d]);
-        load_p(a, nbr(a, x, d, +1), nb[2 * d + 1]);
-    }
-}
-
-// ---- pass 2 ----------------------------------------------------------------------------------
-template <int PRED, int RECON, int SLOPE>
-__global__ void __launch_bounds__(ADJ_NT) adj_faces_kernel(AdjArgs a)
-{
-    const size_t n = (size_t)a.nx * a.ny * a.nz;
-    const FaceOpts o{a.mh_revert, a.face_guard};
-    for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        const Cell x = cell_of(a, c);
-        double p0[9], nb[6][9], mh[9], lo[9], hi[9];
-        load_stencil(a, x, p0, nb);
-        const bool up = RECON == RECON_PPM ? ppm_up(p0, nb) : true;
-        if (PRED == PRED_FULL) {
-            hancock_fwd<double, SLOPE>(p0, nb, mh, a.half_dtdx, 0, a.ph);
-            st9(a, ADJ_MH, x.o, mh);
-            mh_revert(a, p0, mh);
-        }
-        faces_fwd<double, PRED, RECON, SLOPE, 0>(nb[0], p0, nb[1], mh, up, a.half_dtdx, o, a.ph, lo, hi);
-        st9(a, ADJ_FS + fs_slot(0, 0), x.o, lo);
-        st9(a, ADJ_FS + fs_slot(0, 1), x.o, hi);
-        faces_fwd<double, PRED, RECON, SLOPE, 1>(nb[2], p0, nb[3], mh, up, a.half_dtdx, o, a.ph, lo, hi);
-        st9(a, ADJ_FS + fs_slot(1, 0), x.o, lo);
-        st9(a, ADJ_FS + fs_slot(1, 1), x.o, hi);
-        faces_fwd<double, PRED, RECON, SLOPE, 2>(nb[4], p0, nb[5], mh, up, a.half_dtdx, o, a.ph, lo, hi);
-        st9(a, ADJ_FS + fs_slot(2, 0), x.o, lo);
-        st9(a, ADJ_FS + fs_slot(2, 1), x.o, hi);
-    }
-}
-
-// Forcing acceleration at the centre of cell (i,j,k) (glmmhd_turb.jl:483-505), ramp applied.
-GLM_DEV void adj_force(const AdjArgs& a, int i, int j, int k, double a3[3])
-{
-    const int g = a.tgs;
-    const double gg = (double)g;
-    const double cx = (((double)i + 0.5) * a.dx) / a.lx * gg;
-    const double cy = (((double)j + 0.5) * a.dx) / a.ly * gg;
-    const double cz = (((double)k + 0.5) * a.dx) / a.lz * gg;
-    const double fx = floor(cx), fy = floor(cy), fz = floor(cz);
-    const int i0 = (int)fx, j0 = (int)fy, k0 = (int)fz;
-    const double wx = cx - fx, wy = cy - fy, wz = cz - fz;
-    const int i0w = adj_wrap(i0, g), i1w = adj_wrap(i0 + 1, g), j0w = adj_wrap(j0, g), j1w = adj_wrap(j0 + 1, g);
-    const int k0w = adj_wrap(k0, g), k1w = adj_wrap(k0 + 1, g);
-    const size_t g3 = (size_t)g * g * g;
-    for (int cc = 0; cc < 3; ++cc) {
-        const double* af = a.afield + cc * g3;
-        auto at = [&](int ii, int jj, int kk) { return af[(size_t)ii + (size_t)g * ((size_t)jj + (size_t)g * kk)]; };
-        const double b0 = (at(i0w, j0w, k0w) * (1.0 - wx) + at(i1w, j0w, k0w) * wx) * (1.0 - wy) +
-                          (at(i0w, j1w, k0w) * (1.0 - wx) + at(i1w, j1w, k0w) * wx) * wy;
-        const double b1 = (at(i0w, j0w, k1w) * (1.0 - wx) + at(i1w, j0w, k1w) * wx) * (1.0 - wy) +
-                          (at(i0w, j1w, k1w) * (1.0 - wx) + at(i1w, j1w, k1w) * wx) * wy;
-        a3[cc] = a.ramp * (b0 * (1.0 - wz) + b1 * wz);
-    }
-}
-
-template <int RIEM, int D>
-GLM_DEV void face_flux(const AdjArgs& a, size_t cl, size_t cr, double f[9])
-{
-    double L[9], R[9];
-    ld9(a, ADJ_FS + fs_slot(D, 1), cl, L);
-    ld9(a, ADJ_FS + fs_slot(D, 0), cr, R);
-    riemann<double, RIEM, D>(L, R, f, a.ph);
-}
-
-// ---- pass 3 ----------------------------------------------------------------------------------
-// 3a: the flux through each cell's three lower faces, each face solved once -> FLX (27 planes)
-template <int RIEM>
-__global__ void __launch_bounds__(ADJ_NT) adj_flux_kernel(AdjArgs a)
-{
-    const size_t n = (size_t)a.nx * a.ny * a.nz;
-    for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        const Cell x = cell_of(a, c);
-        double f[9];
-        face_flux<RIEM, 0>(a, nbr(a, x, 0, -1), x.o, f);
-        st9(a, ADJ_FLX, x.o, f);
-        face_flux<RIEM, 1>(a, nbr(a, x, 1, -1), x.o, f);
-        st9(a, ADJ_FLX + 9, x.o, f);
-        face_flux<RIEM, 2>(a, nbr(a, x, 2, -1), x.o, f);
-        st9(a, ADJ_FLX + 18, x.o, f);
-    }
-}
-
-// 3b: flux divergence from FLX, then the epilogue adjoint
-__global__ void __launch_bounds__(ADJ_NT) adj_upre_kernel(AdjArgs a)
-{
-    __shared__ double red[ADJ_NT];
-    const size_t n = (size_t)a.nx * a.ny * a.nz;
-    const UpdOpts o{a.update_floor, a.do_turb};
-    double fdot = 0.0;
-    for (size_t c = (size_t)blockIdx.x * ADJ_NT + threadIdx.x; c < n; c += (size_t)gridDim.x * ADJ_NT) {
-        const Cell x = cell_of(a, c);
-        double acc[9], fl[9], fh[9];
-        ld9(a, ADJ_FLX, x.o, fl);
-        ld9(a, ADJ_FLX, nbr(a, x, 0, +1), fh);
-#pragma unroll
-        for (int v = 0; v < 9; ++v) acc[v] = fl[v] - fh[v];
-        ld9(a, ADJ_FLX + 9, x.o, fl);
-        ld9(a, ADJ_FLX + 9, nbr(a, x, 1, +1), fh);
-#pragma unroll
-        for (int v = 0; v < 9; ++v) acc[v] += fl[v] - fh[v];
-        ld9(a, ADJ_FLX + 18, x.o, fl);
-        ld9(a, ADJ_FLX + 18, nbr(a, x, 2, +1), fh);
-        double r[9], lam[9], rb[9];
-#pragma unroll
-        for (int v = 0; v < 9; ++v) {
-            acc[v] += fl[v] - fh[v];
-            r[v] = a.u0[v][c] + a.dtdx * acc[v];
-            lam[v] = a.lam1[v][c];
-            rb[v] = 0.0;
-        }
-        double a3[3] = {0.0, 0.0, 0.0}, a3b[3] = {0.0, 0.0, 0.0};
-        if (a.do_turb) adj_force(a, x.i, x.j, x.k, a3);
-        epilogue_adj<double>(r, a3, a.glm_fac, a.smallc, a.turb_min_rho, a.dt, o, a.ph, lam, rb, a3b);
-        st9(a, ADJ_LPRE, x.o, rb);
-        fdot += a3b[0] * a3[0] + a3b[1] * a3[1] + a3b[2] * a3[2];
-    }
-    red[threadIdx.x] = fdot;
-    __syncthreads();
-    for (int s = ADJ_NT / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) a.part[blockIdx.x] = red[0];
-}
 
 // ---- pass 4 ----------------------------------------------------------------------------------
 template <int RIEM, int D>
@@ -385,7 +229,7 @@ __global__ void __launch_bounds__(ADJ_NT) adj_gather_kernel(AdjArgs a)
     }
 }
 
-// Sum of the per-block partials of pass 3, added to *acc.  One block: thread t sums partials
+// Sum of the front half's per-workgroup partials, added to *acc.  One block: thread t sums partials
 // t, t + 256, ... in order, then a fixed tree; deterministic for a given grid.
 __global__ void __launch_bounds__(ADJ_NT) adj_fdot_kernel(const double* part, int nparts, double* acc)
 {

@@ -9,7 +9,10 @@ constexpr int ADJ_NT = 256;
 
 // Scratch planes of the reverse step (n doubles each, interleaved row by row: adj_impl.hpp adj_index).
 constexpr int ADJ_W = 0, ADJ_MH = 9, ADJ_FS = 18, ADJ_LPRE = 72, ADJ_LFS = 81, ADJ_CON = 135, ADJ_MHB = 198,
-              ADJ_FLX = 207, ADJ_NPLANES = 234;   // ADJ_FLX: the flux through each cell's three lower faces
+              ADJ_NPLANES = 207;
+
+// face-state slot: direction d, side 0 (low face) or 1 (high face)
+__host__ __device__ constexpr int fs_slot(int d, int side) { return (d * 2 + side) * 9; }
 
 struct AdjArgs {
     const double* u0[9];
@@ -21,13 +24,18 @@ struct AdjArgs {
     int mh_revert, face_guard, update_floor, do_turb;
     const double* afield;   // 3 planes of tgs^3 (the step's forcing field), or null
     double* scr;            // ADJ_NPLANES planes of n
-    double* part;           // per-block partial sums of a_bar . a (pass 3)
+    double* part;           // per-workgroup partial sums of a_bar . a (front half)
 };
 
 
 // Device scratch of one reverse step over n cells, in bytes (ADJ_NPLANES planes plus the
-// per-block partial sums).
+// front half's partial sums: its workgroups are at most as many as the cells).
 size_t adj_scratch_bytes(size_t n);
+template <typename T>
+struct MarchArgs;
+// One (predictor, Riemann) family of front kernels (adj_front.hpp), built from adj_front_inst.hip.
+template <int PRED, int RIEM>
+hipError_t launch_adj_front_pr(const MarchArgs<double>& m, const AdjArgs& a, int recon, int slope, hipStream_t st);
 // Launch the reverse step and add the step's sum of (kick acceleration adjoint . acceleration)
 // to *fdot (device).  With fused, the face-state and predictor adjoints and the gather run as one
 // z-march kernel (adj_march.hpp, z planes per tile: zchunk, 0 = the occupancy model) where a z plane

@@ -314,14 +314,21 @@ GLM_DEV void stage_cold(const MarchArgs<T>& a, ColdArgs<T>& ca)
     ca.update_floor = a.update_floor; ca.do_turb = a.do_turb; ca.tgs = a.tgs;
 }
 
+// The plain step: march_tile updates each cell and stores it.  With REVERSE the stages' values go to the
+// object instead (adj_front.hpp) and nothing is updated.
+struct StepStages {
+    static constexpr bool REVERSE = false;
+};
+
 // The march of one tile: the workgroup's lanes march the columns of tile (tile_x, tile_y) through
 // z-chunk zc, tile = tile_x + tiles_x * (tile_y + tiles_y * zc), and write the updated planes.
 // L.ca must hold `a`'s cold arguments, published by a barrier.  Returns the lane's max CFL speed
 // over the cells it updated.  MF (the memory floor, spike_mhd.cu -DMEMFLOOR): the same loads,
 // primitive conversion, LDS staging, update-base read and stores, with no predictor, faces, fluxes
 // or epilogue: each cell is stored as read.
-template <typename T, int PRED, int RIEM, int RECON, int SLOPE, int NS = 0, bool MF = false, typename A = MarchArgs<T>>
-GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile)
+template <typename T, int PRED, int RIEM, int RECON, int SLOPE, int NS = 0, bool MF = false, typename A = MarchArgs<T>,
+          class H>
+GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile, H& h)
 {
     constexpr int NV = 9 + NS;   // the GLM-MHD planes and NS passive species
     T (&P)[NV][NPL] = L.P;
@@ -390,6 +397,9 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile)
 #pragma unroll
         for (int v = 0; v < NV; ++v) p0[v] = P[v][lo_own];
 
+        if constexpr (H::REVERSE) {
+            if (owned && inplane) h.prim(gx, gy, q, p0);
+        }
         // ---- reconstruction of this column's cell in plane q --------------------------------
         bool up = true;   // PPM strong-pressure-jump fallback flag (glmmhd_turb.jl:959)
         if (RECON == RECON_PPM && !MF) {
@@ -427,6 +437,9 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile)
             cons2prim(t, mh, s);
 #pragma unroll
             for (int v = 9; v < NV; ++v) mh[v] = p0[v] - a.dtdx * sadv[v - 9];
+            if constexpr (H::REVERSE) {
+                if (owned && inplane) h.predicted(gx, gy, q, mh);
+            }
             if (a.mh_revert && __builtin_expect(mh[0] <= s.smallr || mh[4] <= s.pfl, 0)) {
 #pragma unroll
                 for (int v = 0; v < NV; ++v) mh[v] = p0[v];
@@ -440,6 +453,9 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile)
         if (owned && !MF) {
             T zlo[NV], zhi[NV];
             faces_dir<T, PRED, RECON, SLOPE, 2, NV>(pm, p0, pp, mh, up, a, zlo, zhi);
+            if constexpr (H::REVERSE) {
+                if (inplane) h.faces(2, gx, gy, q, zlo, zhi);
+            }
             if (q >= zs) {
                 riemann<T, RIEM, 2>(zprev, zlo, fz, s);
                 species_flux<NV>(zprev, zlo, fz);
@@ -457,16 +473,23 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile)
 #pragma unroll
             for (int v = 0; v < NV; ++v) u0[v] = gload(ca.q[v] + col + plane * wrapi(q - 1, nz));
             const int zq = wrapi(q - 1, nz);
-            if (!MF) {
+            if constexpr (H::REVERSE) {
+                T acc[NV];
+#pragma unroll
+                for (int v = 0; v < NV; ++v) acc[v] = pend[v] - fz[v];
+                h.update(u0, acc, ca, fc, s, gx, gy, zq);
+            } else if (!MF) {
                 T acc[NV];
 #pragma unroll
                 for (int v = 0; v < NV; ++v) acc[v] = pend[v] - fz[v];
                 double ct = update_cell<NV>(u0, acc, ca, s, a.want_cfl != 0, fc, gx, gy, zq);
                 if (!(ct <= cmax)) cmax = ct;
             }
-            const size_t off = col + plane * zq;
+            if constexpr (!H::REVERSE) {
+                const size_t off = col + plane * zq;
 #pragma unroll
-            for (int v = 0; v < NV; ++v) gstore_nt(u0[v], ca.o[v] + off);
+                for (int v = 0; v < NV; ++v) gstore_nt(u0[v], ca.o[v] + off);
+            }
         }
         if (last) break;
 
@@ -486,11 +509,17 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile)
 #pragma unroll
                 for (int v = 0; v < NV; ++v) { l[v] = P[v][lo_own - 1]; r[v] = P[v][lo_own + 1]; }
                 faces_dir<T, PRED, RECON, SLOPE, 0, NV>(l, p0, r, mh, up, a, xlo, hi);
+                if constexpr (H::REVERSE) {
+                    if (owned) h.faces(0, gx, gy, q, xlo, hi);
+                }
 #pragma unroll
                 for (int v = 0; v < NV; ++v) XB[v][lo_own] = hi[v];
 #pragma unroll
                 for (int v = 0; v < NV; ++v) { l[v] = P[v][lo_own - PX]; r[v] = P[v][lo_own + PX]; }
                 faces_dir<T, PRED, RECON, SLOPE, 1, NV>(l, p0, r, mh, up, a, ylo, hi);
+                if constexpr (H::REVERSE) {
+                    if (owned) h.faces(1, gx, gy, q, ylo, hi);
+                }
 #pragma unroll
                 for (int v = 0; v < NV; ++v) YB[v][lo_own] = hi[v];
             }
@@ -583,7 +612,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GLM_WAV
     const auto& ak = kernarg_ref<MarchArgs<T>>();
     if (threadIdx.x == 0) stage_cold(a, L.ca);
     __syncthreads();
-    const double cmax = march_tile<T, PRED, RIEM, RECON, SLOPE, NS>(ak, L, xcd_block((int)blockIdx.x, (int)gridDim.x));
+    StepStages h;
+    const double cmax = march_tile<T, PRED, RIEM, RECON, SLOPE, NS>(ak, L, xcd_block((int)blockIdx.x, (int)gridDim.x), h);
     if (ak.want_cfl) {
         cfl_merge(L, cmax, ak.cmax);
         if (blockIdx.x == 0 && threadIdx.x == 0) *ak.cmax_next = 0ull;
@@ -600,7 +630,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GLM_WAV
     const auto& ak = kernarg_ref<MarchArgs<T>>();
     if (threadIdx.x == 0) stage_cold(a, L.ca);
     __syncthreads();
-    (void)march_tile<T, PRED_FULL, RIEM_HLLD, RECON_PPM, SLOPE_MONCEN, 0, true>(ak, L, xcd_block((int)blockIdx.x, (int)gridDim.x));
+    StepStages h;
+    (void)march_tile<T, PRED_FULL, RIEM_HLLD, RECON_PPM, SLOPE_MONCEN, 0, true>(ak, L, xcd_block((int)blockIdx.x, (int)gridDim.x), h);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -668,7 +699,8 @@ GLM_DEV void ens_tile(const EnsLaunch<T>& e, MarchLDS<T>& L, int box, int lt, in
         *s_tb = (unsigned long long)wall_clock64();
     }
     __syncthreads();
-    const double cmax = march_tile<T, PRED, RIEM, RECON, SLOPE>(a, L, lt);
+    StepStages h;
+    const double cmax = march_tile<T, PRED, RIEM, RECON, SLOPE>(a, L, lt, h);
     cfl_merge(L, cmax, a.cmax);
     if (threadIdx.x == 0) {
         const size_t k = (size_t)slot * e.nbox + box;

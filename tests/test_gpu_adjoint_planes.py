@@ -8,11 +8,11 @@ pytestmark = pytest.mark.gpu
 from glmmhdturb_amd import Params, Solver, step_args  # noqa: E402
 
 
-@pytest.mark.parametrize("ny", [1433, 1434])
+@pytest.mark.parametrize("ny", [1620, 1621])
 def test_reverse_step_at_the_offset_limit(ny):
-    """1600 x 1433 cells x 234 scratch planes x 8 bytes is the last multiple below 4 GiB."""
+    """1600 x 1620 cells x 207 scratch planes x 8 bytes is the last multiple below 4 GiB."""
     nx, nz = 1600, 2
-    assert (nx * 234 * 8 * ny <= 2**32 - 1) == (ny == 1433)
+    assert (nx * 207 * 8 * ny <= 2**32 - 1) == (ny == 1620)
     p = Params(N=nx, nx=nx, ny=ny, nz=nz, gamma=5.0 / 3.0, courant=0.4)
     s = Solver(p, "f64")
     g = torch.Generator(device="cuda").manual_seed(ny)
