@@ -61,8 +61,12 @@ static void dispatch_cellwise(const AdjArgs& a, dim3 g, hipStream_t st, int pred
 #undef GLM_CASE
 }
 
+// HLLD: one workgroup a CU is resident and each walks its share of the cells (adj_riemann_kernel).
+constexpr unsigned ADJ_HLLD_GRID = 256;
+
 static void dispatch_riemann(const AdjArgs& a, dim3 g, hipStream_t st, int riem)
 {
+    if (riem == RIEM_HLLD && g.x > ADJ_HLLD_GRID) g.x = ADJ_HLLD_GRID;
 #define GLM_CASE(R) \
     if (riem == R) hipLaunchKernelGGL((adj_riemann_kernel<R>), g, dim3(ADJ_NT), 0, st, a);
     GLM_CASE(RIEM_LLF) GLM_CASE(RIEM_LLFB) GLM_CASE(RIEM_HLL) GLM_CASE(RIEM_HLLD)

@@ -20,7 +20,7 @@ GLM_HD T sgn1(T x) { return x >= T(0) ? T(1) : T(-1); }
 
 // d sqrt(x) with sqrt(x) = y
 template <typename T>
-GLM_HD T dsqrt(T y) { return y > T(0) ? T(0.5) / y : T(0); }
+GLM_HD T dsqrt(T y) { return y > T(0) ? T(0.5) * trcp(y) : T(0); }
 
 // ---- cons2prim (glmmhd_turb.jl:68-77) ------------------------------------------------------
 template <typename T>
@@ -564,8 +564,8 @@ GLM_HD void hlld_x_adj(const T L[9], const T R[9], const T fb[9], T Lb[9], T Rb[
     sqdRs_b += -SRs_b * absbn * rR * rR;
     bn_b += absbn_b * sgn1(bn);
     // sqrt, floors
-    dLs_b += sqdLs_b * dsqrt(sqdLs);
-    dRs_b += sqdRs_b * dsqrt(sqdRs);
+    dLs_b += sqdLs_b * T(0.5) * rL;
+    dRs_b += sqdRs_b * T(0.5) * rR;
     if (XL > T(1e-12)) { dL_b += dLs_b * aL * iL; aL_b += dLs_b * dL * iL; iL_b += dLs_b * dL * aL; }
     if (XR > T(1e-12)) { dR_b += dRs_b * aR * iR; aR_b += dRs_b * dR * iR; iR_b += dRs_b * dR * aR; }
     SL_b += -iL * iL * iL_b; SM_b += iL * iL * iL_b;
@@ -602,10 +602,12 @@ GLM_HD void hlld_x_adj(const T L[9], const T R[9], const T fb[9], T Lb[9], T Rb[
         if (uL >= uR) uL_b += SR_b; else uR_b += SR_b;
         cfm_b += SR_b;
     }
-    T cfL_b = T(0), cfR_b = T(0);
-    if (cfL >= cfR) cfL_b += cfm_b; else cfR_b += cfm_b;
-    fast_speed_adj(dL, pL, b2L, bn, cfL_b, dL_b, pL_b, b2L_b, bn_b, s);
-    fast_speed_adj(dR, pR, b2R, bn, cfR_b, dR_b, pR_b, b2R_b, bn_b, s);
+    // the adjoint of the larger speed belongs to one side: one evaluation on that side's values
+    const bool cl = cfL >= cfR;
+    T dm_b = T(0), pm_b = T(0), b2m_b = T(0);
+    fast_speed_adj(cl ? dL : dR, cl ? pL : pR, cl ? b2L : b2R, bn, cfm_b, dm_b, pm_b, b2m_b, bn_b, s);
+    dL_b += cl ? dm_b : T(0); pL_b += cl ? pm_b : T(0); b2L_b += cl ? b2m_b : T(0);
+    dR_b += cl ? T(0) : dm_b; pR_b += cl ? T(0) : pm_b; b2R_b += cl ? T(0) : b2m_b;
     pL_b += ptL_b; b2L_b += T(0.5) * ptL_b;
     pR_b += ptR_b; b2R_b += T(0.5) * ptR_b;
     bn_b += T(2) * bn * (b2L_b + b2R_b);
