@@ -18,13 +18,14 @@
 // (VALU busy 24%, 224 B spilled, 1.64 ms at 128^3).  Two workgroups need 256 registers and 80 KiB of
 // LDS each: so the variables of a stage are finished one by one, what a later stage can read again
 // from LDS is not kept, Wb of the plane below rests in LDS, and a stage's planes are requested where
-// the stage before has let go of its registers.  0.78 ms (VALU busy 40%); requests two stages ahead or
-// spread over a stage, and 3 or 9 variables at a time, measured 2 to 4% slower.
+// the stage before has let go of its registers: 0.78 ms.  The last wavefront holds the ring, whose
+// loads take a line per lane: it skips the z contributions, which nobody reads (0.73), and LDS rows have
+// odd pitches for its columns (0.70, VALU busy 43%).  Requests two stages ahead or spread over a stage,
+// the c2p adjoint behind the next plane's barrier, and 3 or 9 variables at a time measured 2 to 4% slower.
 #pragma once
 #include "adj_impl.hpp"
 #include "gpu_util.hpp"
 #include "march_impl.hpp"
-
 
 namespace glm {
 
@@ -33,12 +34,12 @@ namespace glm {
 // + MonCen at 128^3: 2.05 against 3.03 ms; with the full predictor 2.30 against 2.09).
 constexpr int adj_waves(int pred) { return pred == PRED_FULL ? 2 : 1; }
 constexpr int ADJ_GRP = 2;     // variables in work at a time
-constexpr int ADJ_EX = 18;     // exchange row: the tile's columns with their ring
-constexpr int ADJ_EXN = ADJ_EX * (NT / ADJ_EX);
-static_assert(ADJ_EXN == NT, "every lane has a slot");
+// LDS rows: odd pitches, so that the ring's columns (one lane a row) fall on different banks.
+constexpr int APX = OX + 5, ANPL = APX * PY;            // W: the tile with its two-cell ring
+constexpr int ADJ_EX = OX + 3, ADJ_EXN = ADJ_EX * (OY + 2);   // exchange: the tile with its one-cell ring
 
 struct AdjBackLDS {
-    double P[9][NPL];                     // W of plane q (two-cell ring)
+    double P[9][ANPL];                     // W of plane q (two-cell ring)
     double LO[9][ADJ_EXN], HI[9][ADJ_EXN];   // a lane's contributions to its lower and its upper neighbour
     double PT[9][ADJ_EXN];                // Wb of plane q-1 without plane q's share (each lane its own slot)
 };
@@ -68,10 +69,10 @@ GLM_DEV void reread()
 // neighbours, out(v, lb, rb) takes the contributions to them; the cell's own go to s0 and mhb.
 // With the full predictor the variables are independent once the guards are known, so each one is read,
 // finished and handed out by itself: nine of anything would not fit the registers next to the march's
-// state.  m0, m4: the predicted density and pressure (the guards look at those two only).
+// state.  give: the lane's contributions are wanted (the halo's in z are not).  m0, m4: the predicted density and pressure (the guards look at those two only).
 template <int PRED, int RECON, int SLOPE, int D, class LR, class OUT>
 GLM_DEV void back_faces(const AdjArgs& a, bool up, double m0, double m4, double lob[9], double hib[9], LR lr, OUT out,
-                        double s0[9], double mhb[9])
+                        bool give, double s0[9], double mhb[9])
 {
     const FaceOpts o{a.mh_revert, a.face_guard};
     if (PRED == PRED_ONED) {
@@ -113,7 +114,10 @@ GLM_DEV void back_faces(const AdjArgs& a, bool up, double m0, double m4, double 
             hib[4] = fh[1] > a.ph.pfl ? hib[4] : 0.0;
         }
     }
-    if (RECON == RECON_PPM && up) {
+    if (!give) {
+#pragma unroll
+        for (int v = 0; v < 9; ++v) mhb[v] += lob[v] + hib[v];
+    } else if (RECON == RECON_PPM && up) {
 #pragma unroll
         for (int v = 0; v < 9; ++v) {
             double l, p0, r, lb, rb;
@@ -174,7 +178,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(adj_wav
 adj_back_kernel(AdjArgs a, int tiles_x, int tiles_y, int zchunk)
 {
     __shared__ AdjBackLDS L;
-    double (&P)[9][NPL] = L.P;
+    double (&P)[9][ANPL] = L.P;
     const int tid = threadIdx.x;
     int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
     int tx, ty;
@@ -192,13 +196,13 @@ adj_back_kernel(AdjArgs a, int tiles_x, int tiles_y, int zchunk)
     // this kernel only where the former stay below 4 GiB)
     const unsigned row = 8u * ADJ_NPLANES * (unsigned)nx;
     const unsigned col = 8u * (unsigned)gx + row * (unsigned)gy, ccol = 8u * (unsigned)(gx + nx * gy);
-    const int lo = (ty + 1) * PX + (tx + 1), e = ty * ADJ_EX + tx;
+    const int lo = (ty + 1) * APX + (tx + 1), e = ty * ADJ_EX + tx;
     const bool helper = tid >= NO && tid - NO < NHELP;
     int hx = 0, hy = 0;
     helper_cell(helper ? tid - NO : 0, hx, hy);
     const unsigned hcol =
         8u * (unsigned)wrapi(tile_x * OX - 2 + hx, nx) + row * (unsigned)wrapi(tile_y * OY - 2 + hy, ny);
-    const int lo_ring = hy * PX + hx;
+    const int lo_ring = hy * APX + hx;
     // nine planes of the scratch from plane p on, of z plane q at the lane's offset.  The offset is made
     // opaque per use: hoisted out of the loop as 64 bits it costs an addition and two registers a load,
     // next to the load it is the load's own offset operand.
@@ -254,7 +258,7 @@ adj_back_kernel(AdjArgs a, int tiles_x, int tiles_y, int zchunk)
 #pragma unroll
         for (int v = 0; v < 9; ++v) { s0[v] = up1[v]; up1[v] = 0.0; mhb[v] = 0.0; }
         auto lrx = [&](int v, double& l, double& m, double& r) { l = P[v][lo - 1]; m = P[v][lo]; r = P[v][lo + 1]; };
-        auto lry = [&](int v, double& l, double& m, double& r) { l = P[v][lo - PX]; m = P[v][lo]; r = P[v][lo + PX]; };
+        auto lry = [&](int v, double& l, double& m, double& r) { l = P[v][lo - APX]; m = P[v][lo]; r = P[v][lo + APX]; };
         auto lrz = [&](int v, double& l, double& m, double& r) { l = pm[v]; m = P[v][lo]; r = pp[v]; };
         auto side = [&](int v, double lb, double rb) { L.LO[v][e] = lb; L.HI[v][e] = rb; };
         auto column = [&](int v, double lb, double rb) { L.PT[v][e] += lb; up1[v] += rb; };
@@ -271,15 +275,15 @@ adj_back_kernel(AdjArgs a, int tiles_x, int tiles_y, int zchunk)
             if (PRED == PRED_FULL && a.mh_revert && (m0 <= a.ph.smallr || m4 <= a.ph.pfl)) { m0 = P[0][lo]; m4 = p0; }
             bool up = true;   // PPM strong-pressure-jump flag (glmmhd_turb.jl:959), stencil order of ppm_up
             if (RECON == RECON_PPM)
-                up = !(spj(P[4][lo - 1], p0, P[4][lo + 1]) || spj(P[4][lo - PX], p0, P[4][lo + PX]) || spj(pm[4], p0, pr));
-            back_faces<PRED, RECON, SLOPE, 0>(a, up, m0, m4, lob, hib, lrx, side, s0, mhb);
+                up = !(spj(P[4][lo - 1], p0, P[4][lo + 1]) || spj(P[4][lo - APX], p0, P[4][lo + APX]) || spj(pm[4], p0, pr));
+            back_faces<PRED, RECON, SLOPE, 0>(a, up, m0, m4, lob, hib, lrx, side, true, s0, mhb);
             ldL(1, q);
             adj_collect<1, 9>(L, e, owned, s0);
-            back_faces<PRED, RECON, SLOPE, 1>(a, up, m0, m4, lob, hib, lry, side, s0, mhb);
+            back_faces<PRED, RECON, SLOPE, 1>(a, up, m0, m4, lob, hib, lry, side, true, s0, mhb);
             ldL(2, q);
             adj_collect<ADJ_EX, 9>(L, e, owned, s0);
             if (PRED != PRED_FULL) ldX(xp);
-            back_faces<PRED, RECON, SLOPE, 2>(a, up, m0, m4, lob, hib, lrz, column, s0, mhb);
+            back_faces<PRED, RECON, SLOPE, 2>(a, up, m0, m4, lob, hib, lrz, column, owned, s0, mhb);
         }
 
         // predictor adjoint
@@ -300,7 +304,8 @@ adj_back_kernel(AdjArgs a, int tiles_x, int tiles_y, int zchunk)
             adj_collect<1, 8>(L, e, owned, s0);
             back_hancock<SLOPE, 1>(a, ok, accb, lry, side, none, s0);
             adj_collect<ADJ_EX, 8>(L, e, owned, s0);
-            back_hancock<SLOPE, 2>(a, ok, accb, lrz, column, [&] { ldX(xp); }, s0);
+            if (owned) back_hancock<SLOPE, 2>(a, ok, accb, lrz, column, [&] { ldX(xp); }, s0);
+            else ldX(xp);
         }
         const bool last = q == ze;
         if (!last) {
