@@ -110,6 +110,33 @@ GLM_DEV void gstore_nt(T v, T* p)
 #endif
 }
 
+template <typename T>
+GLM_DEV void gstore_nt_at(T v, T* base, unsigned off)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    __attribute__((address_space(1))) char* b = (__attribute__((address_space(1))) char*)base;
+    __builtin_nontemporal_store(v, (__attribute__((address_space(1))) T*)(b + off));
+#else
+    *(T*)((char*)base + off) = v;
+#endif
+}
+// Uses behind this point take the value as a new one: what is derived from it is not carried from
+// before (an offset widened ahead of a loop, a pointer table read ahead of it).
+template <typename P>
+GLM_DEV void renew_s(P& p)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(p));
+#endif
+}
+template <typename V>
+GLM_DEV void renew_v(V& x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(x));
+#endif
+}
+
 // An argument block as a reference into the constant address space: a kernel reads each field with
 // a scalar load where it needs it, instead of holding a copy of the whole block in registers (which
 // cost the ensemble kernel 64 B per lane of spills).

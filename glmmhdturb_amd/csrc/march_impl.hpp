@@ -7,9 +7,9 @@
 // and LLF/HLL/HLLD Riemann fluxes with Dedner GLM cleaning (glmmhd_turb.jl:175-354).
 //
 // How it is laid out on the GPU:
-//   * A workgroup of TX x TY = 18 x 14 threads owns a 16 x 12 column tile and a z-chunk (16
-//     doubles = one 128-byte line per row, so row stores are whole lines).  Each thread owns one
-//     (x,y) column of the tile grown by one halo cell and marches z.  Its column's primitives for
+//   * A workgroup of 252 threads owns a 16 x 12 column tile and a z-chunk (16 doubles = one
+//     128-byte line per row, so row stores are whole lines).  Each thread owns one (x,y) column of
+//     the tile grown by one halo cell (18 x 14) and marches z.  Its column's primitives for
 //     planes q-1 and q+1 live in registers; plane q is read back from LDS where it is needed.
 //   * LDS holds the primitives of the current plane q over the tile grown by two cells
 //     (20 x 16): the in-plane neighbours for slopes, PPM edges and the transverse predictor.
@@ -29,7 +29,7 @@
 //     lane: the next planes are prefetched only after the plane's Riemann solves, and plane q and
 //     the predicted state are parked in LDS across the phases that do not use them.
 //   * The epilogue also folds the next step's CFL signal speed (glmmhd_turb.jl:1963-1971) into a
-//     per-thread max, reduced per wavefront and merged with one atomic per wavefront.
+//     per-thread max, reduced over the workgroup and merged with one atomic.
 #pragma once
 #include "force.hpp"
 #include "gpu_util.hpp"
@@ -101,12 +101,10 @@ struct MarchArgs {
     unsigned long long* cmax_next;  // the slot the next step accumulates into (zeroed here)
 };
 
-// Arguments used only at the loads, stores and the update epilogue.  They are staged in LDS at
-// kernel entry so they do not hold scalar registers across the march loop.
+// Arguments used only in the update epilogue.  They are staged in LDS at kernel entry so they do
+// not hold scalar registers across the march loop.
 template <typename T>
 struct ColdArgs {
-    const T* q[NVMAX];
-    T* o[NVMAX];
     const T* afield;
     T dtdx, glm_fac, smallc, turb_min_rho, ramp, dt, dx, lx, ly, lz;
     int update_floor, do_turb, tgs, pad_;
@@ -133,11 +131,30 @@ GLM_DEV void helper_cell(int r, int& px, int& py)
     else { px = PX - 1; py = 2 + r - 2 * OX - OY; }
 }
 
-template <int NV, typename T>
-GLM_DEV void loadv(const ColdArgs<T>& a, size_t off, T c[NV])
+// A lane's column of the grid: the byte offset within a z plane where that fits 32 bits (the plane's base
+// is then one for the wavefront and the access adds the offset itself), else the wide one.
+struct Column {
+    unsigned off;
+    size_t wide;   // in cells
+};
+
+// The NV values of a column's cell `zoff` cells into each plane.  The plane pointers are read from the
+// arguments here: carried across the march they cost 36 scalar registers, from LDS an addition each
+// (64-bit additions and LDS reads were 2% of a plane's instructions: the FP64 PPM + HLLD march at 256^3
+// 2.29 -> 2.26 ms, the FP32 normal-only PLM + HLL one at 480^3 4.77 -> 4.71).
+template <int NV, typename T, typename A>
+GLM_DEV void loadv(const A& a, size_t zoff, Column k, bool narrow, T c[NV])
 {
+    const auto* p = &a;
+    renew_s(p);
+    if (__builtin_expect(narrow, 1)) {
+        renew_v(k.off);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) c[v] = gload(a.q[v] + off);
+        for (int v = 0; v < NV; ++v) c[v] = gload_at((const T*)p->q[v] + zoff, k.off);
+    } else {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) c[v] = gload((const T*)p->q[v] + zoff + k.wide);
+    }
 }
 
 // cons2prim plus the species fractions X = (rho X) / max(rho, smallr) (spike_mhd.cu:243-244).
@@ -307,7 +324,6 @@ struct MarchLDS {
 template <typename T>
 GLM_DEV void stage_cold(const MarchArgs<T>& a, ColdArgs<T>& ca)
 {
-    for (int v = 0; v < NVMAX; ++v) { ca.q[v] = a.q[v]; ca.o[v] = a.o[v]; }
     ca.afield = a.afield;
     ca.dtdx = a.dtdx; ca.glm_fac = a.glm_fac; ca.smallc = a.smallc; ca.turb_min_rho = a.turb_min_rho;
     ca.ramp = a.ramp; ca.dt = a.dt; ca.dx = a.dx; ca.lx = a.lx; ca.ly = a.ly; ca.lz = a.lz;
@@ -350,27 +366,28 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile, H& h)
     const bool owned = tid < NO && gxu < nx && gyu < ny;
     const bool need_x = ty >= 1 && ty <= OY && tx >= 1;      // this lane solves the x face at tx - 1/2
     const bool need_y = tx >= 1 && tx <= OX && ty >= 1;      // this lane solves the y face at ty - 1/2
-    const size_t col = (size_t)gx + (size_t)nx * gy;
+    const bool narrow = plane * sizeof(T) <= 0xffffffffu;
+    const Column col{(unsigned)sizeof(T) * ((unsigned)gx + (unsigned)nx * (unsigned)gy), (size_t)gx + (size_t)nx * gy};
     const int lo_own = (ty + 1) * PX + (tx + 1);
     const bool helper = tid >= NO && tid - NO < NHELP;
     int hx = 0, hy = 0;
     helper_cell(helper ? tid - NO : 0, hx, hy);
-    const size_t hcol = (size_t)wrapi(tile_x * OX - 2 + hx, nx) + (size_t)nx * wrapi(tile_y * OY - 2 + hy, ny);
+    const int hgx = wrapi(tile_x * OX - 2 + hx, nx), hgy = wrapi(tile_y * OY - 2 + hy, ny);
+    const Column hcol{(unsigned)sizeof(T) * ((unsigned)hgx + (unsigned)nx * (unsigned)hgy), (size_t)hgx + (size_t)nx * hgy};
     const int lo_ring = hy * PX + hx;
-
 
     // column window: primitives of planes q-1, q, q+1
     T pm[NV], pp[NV];
     {
         T c[NV], p0[NV];
-        loadv<NV>(ca, col + plane * wrapi(zs - 2, nz), c); c2p<NV>(c, pm, s);
-        loadv<NV>(ca, col + plane * wrapi(zs - 1, nz), c); c2p<NV>(c, p0, s);
-        loadv<NV>(ca, col + plane * wrapi(zs, nz), c); c2p<NV>(c, pp, s);
+        loadv<NV>(a, plane * wrapi(zs - 2, nz), col, narrow, c); c2p<NV>(c, pm, s);
+        loadv<NV>(a, plane * wrapi(zs - 1, nz), col, narrow, c); c2p<NV>(c, p0, s);
+        loadv<NV>(a, plane * wrapi(zs, nz), col, narrow, c); c2p<NV>(c, pp, s);
 #pragma unroll
         for (int v = 0; v < NV; ++v) P[v][lo_own] = p0[v];
         if (helper) {
             T h[NV];
-            loadv<NV>(ca, hcol + plane * wrapi(zs - 1, nz), c); c2p<NV>(c, h, s);
+            loadv<NV>(a, plane * wrapi(zs - 1, nz), hcol, narrow, c); c2p<NV>(c, h, s);
 #pragma unroll
             for (int v = 0; v < NV; ++v) P[v][lo_ring] = h[v];
         }
@@ -470,9 +487,8 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile, H& h)
             for (int v = 0; v < NV; ++v) XB[v][lo_own] = mh[v];
         }
         if (do_upd) {
-#pragma unroll
-            for (int v = 0; v < NV; ++v) u0[v] = gload(ca.q[v] + col + plane * wrapi(q - 1, nz));
             const int zq = wrapi(q - 1, nz);
+            loadv<NV>(a, plane * zq, col, narrow, u0);
             if constexpr (H::REVERSE) {
                 T acc[NV];
 #pragma unroll
@@ -486,9 +502,17 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile, H& h)
                 if (!(ct <= cmax)) cmax = ct;
             }
             if constexpr (!H::REVERSE) {
-                const size_t off = col + plane * zq;
+                const auto* p = &a;
+                renew_s(p);
+                if (__builtin_expect(narrow, 1)) {
+                    unsigned off = col.off;
+                    renew_v(off);
 #pragma unroll
-                for (int v = 0; v < NV; ++v) gstore_nt(u0[v], ca.o[v] + off);
+                    for (int v = 0; v < NV; ++v) gstore_nt_at(u0[v], (T*)p->o[v] + plane * zq, off);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) gstore_nt(u0[v], (T*)p->o[v] + plane * zq + col.wide);
+                }
             }
         }
         if (last) break;
@@ -559,8 +583,8 @@ GLM_DEV double march_tile(const A& a, MarchLDS<T, 9 + NS>& L, int tile, H& h)
 
         if (!MF) __builtin_amdgcn_s_setprio(1);   // (set already when this plane's faces were solved)
         T cn[NV], hr[NV];
-        loadv<NV>(ca, col + plane * wrapi(q + 2, nz), cn);
-        if (helper) loadv<NV>(ca, hcol + plane * wrapi(q + 1, nz), hr);
+        loadv<NV>(a, plane * wrapi(q + 2, nz), col, narrow, cn);
+        if (helper) loadv<NV>(a, plane * wrapi(q + 1, nz), hcol, narrow, hr);
         // ---- advance the column window and publish plane q+1 to LDS ------------------------------
         // The last reads of plane q's LDS cells precede the face-state barrier when this plane's
         // faces were solved; otherwise (the lead-in plane) they are the predictor's.

@@ -180,18 +180,23 @@ GLM_HD T tsqrt_nn(T a) { return tsqrt(a); }
 // Gas pressure (gamma-1)(E - |m|^2/(2 rho) - |B|^2/2), floored (glmmhd_turb.jl:75).  With FP32 state
 // the subtraction is carried out in FP64: in low-beta or high-Mach cells E is dominated by the
 // magnetic or kinetic part and the FP32 difference would lose the thermal part.
+// The fused operations are written out and no others are made: the pressure has the same bits at every
+// place a march takes it (its window's first planes and its loop), which chunk lengths must not show.
 GLM_HD double gas_pressure(const double c[9], double ir, double gm1, double pfl)
 {
-    double ekin = 0.5 * (c[1] * c[1] + c[2] * c[2] + c[3] * c[3]) * ir;
-    double emag = 0.5 * (c[5] * c[5] + c[6] * c[6] + c[7] * c[7]);
-    return __builtin_fmax(gm1 * (c[4] - ekin - emag), pfl);
+#pragma clang fp contract(off)
+    const double m2 = __builtin_fma(c[3], c[3], __builtin_fma(c[2], c[2], c[1] * c[1]));
+    const double b2 = __builtin_fma(c[7], c[7], __builtin_fma(c[6], c[6], c[5] * c[5]));
+    return __builtin_fmax(gm1 * __builtin_fma(-0.5, b2, __builtin_fma(-0.5 * m2, ir, c[4])), pfl);
 }
 GLM_HD float gas_pressure(const float c[9], float ir, float gm1, float pfl)
 {
-    double m1 = c[1], m2 = c[2], m3 = c[3], b1 = c[5], b2 = c[6], b3 = c[7];
-    double ekin = 0.5 * (m1 * m1 + m2 * m2 + m3 * m3) * (double)ir;
-    double emag = 0.5 * (b1 * b1 + b2 * b2 + b3 * b3);
-    return __builtin_fmaxf((float)((double)gm1 * ((double)c[4] - ekin - emag)), pfl);
+#pragma clang fp contract(off)
+    const double m1 = c[1], m2 = c[2], m3 = c[3], b1 = c[5], b2 = c[6], b3 = c[7];
+    const double mm = __builtin_fma(m3, m3, __builtin_fma(m2, m2, m1 * m1));
+    const double bb = __builtin_fma(b3, b3, __builtin_fma(b2, b2, b1 * b1));
+    const double e = __builtin_fma(-0.5, bb, __builtin_fma(-0.5 * mm, (double)ir, (double)c[4]));
+    return __builtin_fmaxf((float)((double)gm1 * e), pfl);
 }
 
 // glmmhd_turb.jl:68-77 cons2prim
