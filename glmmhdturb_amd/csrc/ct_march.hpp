@@ -110,23 +110,50 @@ struct CTMarchLDS {
     T FCB[6][CM_NO];       // forcing interpolation cache (ForceCache) of the owned columns
 };
 
-// Primitives with cell-centred B of cell (x, y, z) (ct_mhd.jl:26-34, :85-96), then the species
-// fractions X_s = rho X_s / max(rho, smallr) (spike_ctm.cu:260-263).
-template <typename T, int NV = 8>
-GLM_DEV void cm_prim(const CTMArgs<T>& a, int x, int y, int z, T p[NV])
+// A column (x, y) of the grid and the byte offsets, within a z plane, of its cells and of their upper x
+// and y neighbours, for planes below 4 GiB: the plane's base is one for the wavefront and an access adds
+// its offset itself.  (64-bit lane addresses, a multiplication or two and an addition each, were 4% of a
+// plane's instructions: the HLLD + PLM step at 256^3 FP64 2.43 -> 2.27 ms.)
+struct CmColumn {
+    int x, y;
+    unsigned c, x1, y1;
+};
+template <typename T>
+GLM_DEV CmColumn cm_column(int x, int y, int nx, int ny)
 {
-    const size_t pl = (size_t)a.nx * a.ny;
-    const size_t c = (size_t)x + (size_t)a.nx * y + pl * z;
-    T u[NV];
+    const unsigned row = (unsigned)nx * (unsigned)y;
+    return {x, y, (unsigned)sizeof(T) * ((unsigned)x + row), (unsigned)sizeof(T) * ((unsigned)cwrap(x + 1, nx) + row),
+            (unsigned)sizeof(T) * ((unsigned)x + (unsigned)nx * (unsigned)cwrap(y + 1, ny))};
+}
+
+// Primitives with cell-centred B of a column's cell in plane z (ct_mhd.jl:26-34, :85-96), then the
+// species fractions X_s = rho X_s / max(rho, smallr) (spike_ctm.cu:260-263).
+template <typename T, int NV = 8, typename A>
+GLM_DEV void cm_prim(const A& a, CmColumn k, int z, bool narrow, T p[NV])
+{
+    const size_t pl = (size_t)a.nx * a.ny, z0 = pl * z, z1 = pl * cwrap(z + 1, a.nz);
+    T u[NV], bx1, by1, bz1;
+    const auto* ap = &a;
+    renew_s(ap);
+    if (__builtin_expect(narrow, 1)) {
+        renew_v(k.c); renew_v(k.x1); renew_v(k.y1);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) u[v] = gload(a.q[v] + c);
-    const T bx1 = gload(a.q[5] + ((size_t)cwrap(x + 1, a.nx) + (size_t)a.nx * y + pl * z));
-    const T by1 = gload(a.q[6] + ((size_t)x + (size_t)a.nx * cwrap(y + 1, a.ny) + pl * z));
-    const T bz1 = gload(a.q[7] + ((size_t)x + (size_t)a.nx * y + pl * cwrap(z + 1, a.nz)));
+        for (int v = 0; v < NV; ++v) u[v] = gload_at((const T*)ap->q[v] + z0, k.c);
+        bx1 = gload_at((const T*)ap->q[5] + z0, k.x1);
+        by1 = gload_at((const T*)ap->q[6] + z0, k.y1);
+        bz1 = gload_at((const T*)ap->q[7] + z1, k.c);
+    } else {
+        const size_t row = (size_t)a.nx * k.y, c = (size_t)k.x + row;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) u[v] = gload(a.q[v] + (c + z0));
+        bx1 = gload(a.q[5] + ((size_t)cwrap(k.x + 1, a.nx) + row + z0));
+        by1 = gload(a.q[6] + ((size_t)k.x + (size_t)a.nx * cwrap(k.y + 1, a.ny) + z0));
+        bz1 = gload(a.q[7] + (c + z1));
+    }
     const T bx = T(0.5) * (u[5] + bx1), by = T(0.5) * (u[6] + by1), bz = T(0.5) * (u[7] + bz1);
     T rho = tmax(u[0], a.smallr), ir = trcp(rho);
     T vx = u[1] * ir, vy = u[2] * ir, vz = u[3] * ir;
-    T pr = ct_pressure(u[4], rho, vx, vy, vz, bx, by, bz, a.gamma, a.smallp);
+    T pr = ct_pressure(u[4], rho, vx, vy, vz, bx, by, bz, (T)a.gamma, (T)a.smallp);
     p[0] = rho; p[1] = vx; p[2] = vy; p[3] = vz; p[4] = pr; p[5] = bx; p[6] = by; p[7] = bz;
 #pragma unroll
     for (int v = 8; v < NV; ++v) p[v] = u[v] * ir;
@@ -177,28 +204,30 @@ ct_march_kernel(CTMArgs<T> a_)
     const bool emf_z = tx >= 1 && ty >= 1;            // ez at the lane's lower x-y edge
     const bool emf_x = tx >= 1 && tx <= CM_OX && ty >= 1;
     const bool emf_y = tx >= 1 && ty >= 1 && ty <= CM_OY;
-    const size_t col = (size_t)gx + (size_t)nx * gy;
+    const bool narrow = plane * sizeof(T) <= 0xffffffffu;
+    const CmColumn col = cm_column<T>(gx, gy, nx, ny);
     const int lo = (ty + 1) * CM_PX + (tx + 1);
     const int li = ty * CM_LX + tx;
     const bool helper = tid >= CM_NO;   // the halo wavefront, which has no update, brings in the two-cell ring (when
                                         // the first owned one did: 2.70 ms at 256^3 FP64, now 2.46)
     int hx = 0, hy = 0;
     cm_helper_cell(helper ? tid - CM_NO : 0, hx, hy);
-    const int hgx = cwrap(tile_x * CM_OX - 2 + hx, nx), hgy = cwrap(tile_y * CM_OY - 2 + hy, ny);
+    const CmColumn hcol =
+        cm_column<T>(cwrap(tile_x * CM_OX - 2 + hx, nx), cwrap(tile_y * CM_OY - 2 + hy, ny), nx, ny);
     const int lo_ring = hy * CM_PX + hx;
 
     // column window: primitives of planes q-1 and q+1 (plane q is read back from LDS)
     T pm[NV], pp[NV];
     {
         T p0[NV];
-        cm_prim<T, NV>(a, gx, gy, cwrap(zs - 2, nz), pm);
-        cm_prim<T, NV>(a, gx, gy, cwrap(zs - 1, nz), p0);
-        cm_prim<T, NV>(a, gx, gy, cwrap(zs, nz), pp);
+        cm_prim<T, NV>(a, col, cwrap(zs - 2, nz), narrow, pm);
+        cm_prim<T, NV>(a, col, cwrap(zs - 1, nz), narrow, p0);
+        cm_prim<T, NV>(a, col, cwrap(zs, nz), narrow, pp);
 #pragma unroll
         for (int v = 0; v < NV; ++v) P[v][lo] = p0[v];
         if (helper) {
             T h[NV];
-            cm_prim<T, NV>(a, hgx, hgy, cwrap(zs - 1, nz), h);
+            cm_prim<T, NV>(a, hcol, cwrap(zs - 1, nz), narrow, h);
 #pragma unroll
             for (int v = 0; v < NV; ++v) P[v][lo_ring] = h[v];
         }
@@ -220,10 +249,21 @@ ct_march_kernel(CTMArgs<T> a_)
     for (int q = zs - 1; q <= ze; ++q) {
         const int zq = cwrap(q, nz);
         const bool lead = q == zs - 1;
-        const size_t off = col + plane * zq;
 
         // face-normal fields of this cell's lower faces, loaded ahead of their Riemann solves
-        const T bnx = gload(a.q[5] + off), bny = gload(a.q[6] + off), bnz = gload(a.q[7] + off);
+        T bnx, bny, bnz;
+        if (__builtin_expect(narrow, 1)) {
+            const auto* ap = &a;
+            unsigned off = col.c;
+            renew_s(ap);
+            renew_v(off);
+            bnx = gload_at((const T*)ap->q[5] + plane * zq, off);
+            bny = gload_at((const T*)ap->q[6] + plane * zq, off);
+            bnz = gload_at((const T*)ap->q[7] + plane * zq, off);
+        } else {
+            const size_t off = (size_t)gx + (size_t)nx * gy + plane * zq;
+            bnx = gload(a.q[5] + off); bny = gload(a.q[6] + off); bnz = gload(a.q[7] + off);
+        }
 
         // ---- x and y face states of this lane's cell in plane q -----------------------------------
         T xlo[NV], ylo[NV];
@@ -308,16 +348,29 @@ ct_march_kernel(CTMArgs<T> a_)
             // ---- update of plane q-1 (ct_mhd.jl:124-136, :156-171) --------------------------------
             if (owned && q >= zs + 1) {
                 const int zu = cwrap(q - 1, nz);
-                const size_t ou = col + plane * zu;
-                T r[NH], b0[NH];   // hydro values, then species (plane 8 + s at index 5 + s)
+                const size_t zo = plane * zu, ow = (size_t)gx + (size_t)nx * gy + zo;
+                T r[NH], b0[NH], bo[3];   // hydro values, then species (plane 8 + s at index 5 + s); face fields
+                const auto* ap = &a;
+                renew_s(ap);
+                if (__builtin_expect(narrow, 1)) {
+                    unsigned off = col.c;
+                    renew_v(off);
 #pragma unroll
-                for (int t = 0; t < NH; ++t) b0[t] = gload(a.q[t < 5 ? t : t + 3] + ou);
+                    for (int t = 0; t < NH; ++t) b0[t] = gload_at((const T*)ap->q[t < 5 ? t : t + 3] + zo, off);
+#pragma unroll
+                    for (int t = 0; t < 3; ++t) bo[t] = gload_at((const T*)ap->q[5 + t] + zo, off);
+                } else {
+#pragma unroll
+                    for (int t = 0; t < NH; ++t) b0[t] = gload(a.q[t < 5 ? t : t + 3] + ow);
+#pragma unroll
+                    for (int t = 0; t < 3; ++t) bo[t] = gload(a.q[5 + t] + ow);
+                }
 #pragma unroll
                 for (int t = 0; t < NH; ++t) r[t] = b0[t] + a.dtdx * (pend[t] + (fzp[t] - fz[t < 5 ? t : t + 3]));
                 const T ex0 = Ep[0][lo], ey0 = Ep[1][lo], ez0 = Ep[2][lo];
-                const T bxn = gload(a.q[5] + ou) - a.dtdx * ((Ep[2][lo + CM_PX] - ez0) - (ey - ey0));
-                const T byn = gload(a.q[6] + ou) - a.dtdx * ((ex - ex0) - (Ep[2][lo + 1] - ez0));
-                const T bzn = gload(a.q[7] + ou) - a.dtdx * ((Ep[1][lo + 1] - ey0) - (Ep[0][lo + CM_PX] - ex0));
+                const T bxn = bo[0] - a.dtdx * ((Ep[2][lo + CM_PX] - ez0) - (ey - ey0));
+                const T byn = bo[1] - a.dtdx * ((ex - ex0) - (Ep[2][lo + 1] - ez0));
+                const T bzn = bo[2] - a.dtdx * ((Ep[1][lo + 1] - ey0) - (Ep[0][lo + CM_PX] - ex0));
                 if (a.update_floor && r[0] < a.smallr) {
                     T emag = T(0.5) * (pm[5] * pm[5] + pm[6] * pm[6] + pm[7] * pm[7]);
                     r[0] = a.smallr; r[1] = T(0); r[2] = T(0); r[3] = T(0); r[4] = a.smallp * a.igm1 + emag;
@@ -338,13 +391,21 @@ ct_march_kernel(CTMArgs<T> a_)
                     e = tmax(e + T(0.5) * m4 * m4 * irm, fl);
                     r[1] = m2; r[2] = m3; r[3] = m4; r[4] = e;
                 }
+                const T bn[3] = {bxn, byn, bzn};
+                renew_s(ap);
+                if (__builtin_expect(narrow, 1)) {
+                    unsigned off = col.c;
+                    renew_v(off);
 #pragma unroll
-                for (int t = 0; t < 5; ++t) gstore_nt(r[t], a.o[t] + ou);
+                    for (int t = 0; t < NH; ++t) gstore_nt_at(r[t], (T*)ap->o[t < 5 ? t : t + 3] + zo, off);
 #pragma unroll
-                for (int t = 5; t < NH; ++t) gstore_nt(r[t], a.o[t + 3] + ou);
-                gstore_nt(bxn, a.o[5] + ou);
-                gstore_nt(byn, a.o[6] + ou);
-                gstore_nt(bzn, a.o[7] + ou);
+                    for (int t = 0; t < 3; ++t) gstore_nt_at(bn[t], (T*)ap->o[5 + t] + zo, off);
+                } else {
+#pragma unroll
+                    for (int t = 0; t < NH; ++t) gstore_nt(r[t], (T*)a.o[t < 5 ? t : t + 3] + ow);
+#pragma unroll
+                    for (int t = 0; t < 3; ++t) gstore_nt(bn[t], (T*)a.o[5 + t] + ow);
+                }
             }
             // in-plane flux differences of plane q for its update in the next pass
             if (owned) {
@@ -366,8 +427,8 @@ ct_march_kernel(CTMArgs<T> a_)
         // workgroups reach the plane's last barrier sooner (FP32 PPM +2%, FP64 HLLD + PLM +1.7%).
         __builtin_amdgcn_s_setprio(1);
         T pn[NV], hn[NV];
-        cm_prim<T, NV>(a, gx, gy, cwrap(q + 2, nz), pn);
-        if (helper) cm_prim<T, NV>(a, hgx, hgy, cwrap(q + 1, nz), hn);
+        cm_prim<T, NV>(a, col, cwrap(q + 2, nz), narrow, pn);
+        if (helper) cm_prim<T, NV>(a, hcol, cwrap(q + 1, nz), narrow, hn);
         __syncthreads();   // every read of plane q's LDS cells and of the flux exchange is done
 #pragma unroll
         for (int v = 0; v < NV; ++v) { pm[v] = P[v][lo]; P[v][lo] = pp[v]; pp[v] = pn[v]; }
