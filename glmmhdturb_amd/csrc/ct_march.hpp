@@ -113,7 +113,13 @@ struct CTMarchLDS {
 // A column (x, y) of the grid and the byte offsets, within a z plane, of its cells and of their upper x
 // and y neighbours, for planes below 4 GiB: the plane's base is one for the wavefront and an access adds
 // its offset itself.  (64-bit lane addresses, a multiplication or two and an addition each, were 4% of a
-// plane's instructions: the HLLD + PLM step at 256^3 FP64 2.43 -> 2.27 ms.)
+// plane's instructions: the HLLD + PLM step at 256^3 FP64 2.43 -> 2.27 ms.)  Where the offsets are used
+// (192^3, us with 64-bit addresses and with offsets): FP64 PLM HLLD 885 -> 837 (HLL 632 -> 637); FP32 PLM
+// HLLD 424 -> 412, PPM HLL 374 -> 356, PPM HLLD 485 -> 457.  Not in the FP64 builds at one wavefront a SIMD,
+// which have the registers and wait longer for the pointers (PPM HLL 924 -> 985, HLLD 1097 -> 1125; species
+// HLL 1018 -> 1078, HLLD 1148 -> 1218), nor for FP32 PLM HLL (324 -> 327) and species (HLLD 521 -> 526).
+template <typename T, int RIEM, int NS, int RC>
+constexpr bool CM_OFFSETS = NS == 0 && (sizeof(T) == 8 ? RC == RECON_PLM : RIEM == RIEM_HLLD || RC != RECON_PLM);
 struct CmColumn {
     int x, y;
     unsigned c, x1, y1;
@@ -126,37 +132,55 @@ GLM_DEV CmColumn cm_column(int x, int y, int nx, int ny)
             (unsigned)sizeof(T) * ((unsigned)x + (unsigned)nx * (unsigned)cwrap(y + 1, ny))};
 }
 
-// Primitives with cell-centred B of a column's cell in plane z (ct_mhd.jl:26-34, :85-96), then the
-// species fractions X_s = rho X_s / max(rho, smallr) (spike_ctm.cu:260-263).
-template <typename T, int NV = 8, typename A>
-GLM_DEV void cm_prim(const A& a, CmColumn k, int z, bool narrow, T p[NV])
+// Primitives with cell-centred B of a cell (ct_mhd.jl:26-34, :85-96) from its values and the face
+// fields of its upper neighbours, then the species fractions X_s = rho X_s / max(rho, smallr)
+// (spike_ctm.cu:260-263).
+template <typename T, int NV>
+GLM_DEV void cm_prim_of(const CTMArgs<T>& a, const T u[NV], T bx1, T by1, T bz1, T p[NV])
 {
-    const size_t pl = (size_t)a.nx * a.ny, z0 = pl * z, z1 = pl * cwrap(z + 1, a.nz);
-    T u[NV], bx1, by1, bz1;
-    const auto* ap = &a;
-    renew_s(ap);
-    if (__builtin_expect(narrow, 1)) {
-        renew_v(k.c); renew_v(k.x1); renew_v(k.y1);
-#pragma unroll
-        for (int v = 0; v < NV; ++v) u[v] = gload_at((const T*)ap->q[v] + z0, k.c);
-        bx1 = gload_at((const T*)ap->q[5] + z0, k.x1);
-        by1 = gload_at((const T*)ap->q[6] + z0, k.y1);
-        bz1 = gload_at((const T*)ap->q[7] + z1, k.c);
-    } else {
-        const size_t row = (size_t)a.nx * k.y, c = (size_t)k.x + row;
-#pragma unroll
-        for (int v = 0; v < NV; ++v) u[v] = gload(a.q[v] + (c + z0));
-        bx1 = gload(a.q[5] + ((size_t)cwrap(k.x + 1, a.nx) + row + z0));
-        by1 = gload(a.q[6] + ((size_t)k.x + (size_t)a.nx * cwrap(k.y + 1, a.ny) + z0));
-        bz1 = gload(a.q[7] + (c + z1));
-    }
     const T bx = T(0.5) * (u[5] + bx1), by = T(0.5) * (u[6] + by1), bz = T(0.5) * (u[7] + bz1);
     T rho = tmax(u[0], a.smallr), ir = trcp(rho);
     T vx = u[1] * ir, vy = u[2] * ir, vz = u[3] * ir;
-    T pr = ct_pressure(u[4], rho, vx, vy, vz, bx, by, bz, (T)a.gamma, (T)a.smallp);
+    T pr = ct_pressure(u[4], rho, vx, vy, vz, bx, by, bz, a.gamma, a.smallp);
     p[0] = rho; p[1] = vx; p[2] = vy; p[3] = vz; p[4] = pr; p[5] = bx; p[6] = by; p[7] = bz;
 #pragma unroll
     for (int v = 8; v < NV; ++v) p[v] = u[v] * ir;
+}
+// of cell (x, y, z)
+template <typename T, int NV = 8>
+GLM_DEV void cm_prim(const CTMArgs<T>& a, int x, int y, int z, T p[NV])
+{
+    const size_t pl = (size_t)a.nx * a.ny;
+    const size_t c = (size_t)x + (size_t)a.nx * y + pl * z;
+    T u[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) u[v] = gload(a.q[v] + c);
+    const T bx1 = gload(a.q[5] + ((size_t)cwrap(x + 1, a.nx) + (size_t)a.nx * y + pl * z));
+    const T by1 = gload(a.q[6] + ((size_t)x + (size_t)a.nx * cwrap(y + 1, a.ny) + pl * z));
+    const T bz1 = gload(a.q[7] + ((size_t)x + (size_t)a.nx * y + pl * cwrap(z + 1, a.nz)));
+    cm_prim_of<T, NV>(a, u, bx1, by1, bz1, p);
+}
+// of a column's cell in plane z, by offsets where `narrow`
+template <typename T, int NV, bool OFF, typename A>
+GLM_DEV void cm_prim_at(const A& a, CmColumn k, int z, bool narrow, T p[NV])
+{
+    if constexpr (OFF) {
+        if (__builtin_expect(narrow, 1)) {
+            const auto* ap = &a;
+            renew_s(ap);
+            const size_t pl = (size_t)a.nx * a.ny, z0 = pl * z, z1 = pl * cwrap(z + 1, a.nz);
+            renew_v(k.c); renew_v(k.x1); renew_v(k.y1);
+            T u[NV];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) u[v] = gload_at((const T*)ap->q[v] + z0, k.c);
+            const T bx1 = gload_at((const T*)ap->q[5] + z0, k.x1);
+            const T by1 = gload_at((const T*)ap->q[6] + z0, k.y1);
+            const T bz1 = gload_at((const T*)ap->q[7] + z1, k.c);
+            cm_prim_of<T, NV>(a, u, bx1, by1, bz1, p);
+            return;
+        }
+    }
+    cm_prim<T, NV>(a, k.x, k.y, z, p);
 }
 
 // Tiles and z-chunks of the CT march (lead-in: two whole planes of face states and fluxes).
@@ -204,7 +228,9 @@ ct_march_kernel(CTMArgs<T> a_)
     const bool emf_z = tx >= 1 && ty >= 1;            // ez at the lane's lower x-y edge
     const bool emf_x = tx >= 1 && tx <= CM_OX && ty >= 1;
     const bool emf_y = tx >= 1 && ty >= 1 && ty <= CM_OY;
-    const bool narrow = plane * sizeof(T) <= 0xffffffffu;
+    constexpr bool OFF = CM_OFFSETS<T, RIEM, NS, RC>;
+    const bool narrow = OFF && plane * sizeof(T) <= 0xffffffffu;
+    const size_t wcol = (size_t)gx + (size_t)nx * gy;
     const CmColumn col = cm_column<T>(gx, gy, nx, ny);
     const int lo = (ty + 1) * CM_PX + (tx + 1);
     const int li = ty * CM_LX + tx;
@@ -220,14 +246,14 @@ ct_march_kernel(CTMArgs<T> a_)
     T pm[NV], pp[NV];
     {
         T p0[NV];
-        cm_prim<T, NV>(a, col, cwrap(zs - 2, nz), narrow, pm);
-        cm_prim<T, NV>(a, col, cwrap(zs - 1, nz), narrow, p0);
-        cm_prim<T, NV>(a, col, cwrap(zs, nz), narrow, pp);
+        cm_prim_at<T, NV, OFF>(a, col, cwrap(zs - 2, nz), narrow, pm);
+        cm_prim_at<T, NV, OFF>(a, col, cwrap(zs - 1, nz), narrow, p0);
+        cm_prim_at<T, NV, OFF>(a, col, cwrap(zs, nz), narrow, pp);
 #pragma unroll
         for (int v = 0; v < NV; ++v) P[v][lo] = p0[v];
         if (helper) {
             T h[NV];
-            cm_prim<T, NV>(a, hcol, cwrap(zs - 1, nz), narrow, h);
+            cm_prim_at<T, NV, OFF>(a, hcol, cwrap(zs - 1, nz), narrow, h);
 #pragma unroll
             for (int v = 0; v < NV; ++v) P[v][lo_ring] = h[v];
         }
@@ -261,7 +287,7 @@ ct_march_kernel(CTMArgs<T> a_)
             bny = gload_at((const T*)ap->q[6] + plane * zq, off);
             bnz = gload_at((const T*)ap->q[7] + plane * zq, off);
         } else {
-            const size_t off = (size_t)gx + (size_t)nx * gy + plane * zq;
+            const size_t off = wcol + plane * zq;
             bnx = gload(a.q[5] + off); bny = gload(a.q[6] + off); bnz = gload(a.q[7] + off);
         }
 
@@ -348,7 +374,7 @@ ct_march_kernel(CTMArgs<T> a_)
             // ---- update of plane q-1 (ct_mhd.jl:124-136, :156-171) --------------------------------
             if (owned && q >= zs + 1) {
                 const int zu = cwrap(q - 1, nz);
-                const size_t zo = plane * zu, ow = (size_t)gx + (size_t)nx * gy + zo;
+                const size_t zo = plane * zu, ow = wcol + zo;
                 T r[NH], b0[NH], bo[3];   // hydro values, then species (plane 8 + s at index 5 + s); face fields
                 const auto* ap = &a;
                 renew_s(ap);
@@ -363,14 +389,15 @@ ct_march_kernel(CTMArgs<T> a_)
 #pragma unroll
                     for (int t = 0; t < NH; ++t) b0[t] = gload(a.q[t < 5 ? t : t + 3] + ow);
 #pragma unroll
-                    for (int t = 0; t < 3; ++t) bo[t] = gload(a.q[5 + t] + ow);
+                    for (int t = 0; t < 3 && OFF; ++t) bo[t] = gload(a.q[5 + t] + ow);
                 }
 #pragma unroll
                 for (int t = 0; t < NH; ++t) r[t] = b0[t] + a.dtdx * (pend[t] + (fzp[t] - fz[t < 5 ? t : t + 3]));
                 const T ex0 = Ep[0][lo], ey0 = Ep[1][lo], ez0 = Ep[2][lo];
-                const T bxn = bo[0] - a.dtdx * ((Ep[2][lo + CM_PX] - ez0) - (ey - ey0));
-                const T byn = bo[1] - a.dtdx * ((ex - ex0) - (Ep[2][lo + 1] - ez0));
-                const T bzn = bo[2] - a.dtdx * ((Ep[1][lo + 1] - ey0) - (Ep[0][lo + CM_PX] - ex0));
+                auto face_b = [&](int t) { return OFF ? bo[t] : gload(a.q[5 + t] + ow); };
+                const T bxn = face_b(0) - a.dtdx * ((Ep[2][lo + CM_PX] - ez0) - (ey - ey0));
+                const T byn = face_b(1) - a.dtdx * ((ex - ex0) - (Ep[2][lo + 1] - ez0));
+                const T bzn = face_b(2) - a.dtdx * ((Ep[1][lo + 1] - ey0) - (Ep[0][lo + CM_PX] - ex0));
                 if (a.update_floor && r[0] < a.smallr) {
                     T emag = T(0.5) * (pm[5] * pm[5] + pm[6] * pm[6] + pm[7] * pm[7]);
                     r[0] = a.smallr; r[1] = T(0); r[2] = T(0); r[3] = T(0); r[4] = a.smallp * a.igm1 + emag;
@@ -427,8 +454,8 @@ ct_march_kernel(CTMArgs<T> a_)
         // workgroups reach the plane's last barrier sooner (FP32 PPM +2%, FP64 HLLD + PLM +1.7%).
         __builtin_amdgcn_s_setprio(1);
         T pn[NV], hn[NV];
-        cm_prim<T, NV>(a, col, cwrap(q + 2, nz), narrow, pn);
-        if (helper) cm_prim<T, NV>(a, hcol, cwrap(q + 1, nz), narrow, hn);
+        cm_prim_at<T, NV, OFF>(a, col, cwrap(q + 2, nz), narrow, pn);
+        if (helper) cm_prim_at<T, NV, OFF>(a, hcol, cwrap(q + 1, nz), narrow, hn);
         __syncthreads();   // every read of plane q's LDS cells and of the flux exchange is done
 #pragma unroll
         for (int v = 0; v < NV; ++v) { pm[v] = P[v][lo]; P[v][lo] = pp[v]; pp[v] = pn[v]; }

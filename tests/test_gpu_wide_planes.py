@@ -1,7 +1,6 @@
-"""The GLM and CT marches on z planes at the reach of its 32-bit offsets (csrc/march_impl.hpp Column,
-csrc/ct_march.hpp CmColumn): the largest
-FP32 plane below 4 GiB and the first at 4 GiB, each a periodic repetition of a small grid, so that every
-cell must come out with the bits of the small grid's step."""
+"""The GLM and CT marches on z planes at the reach of their 32-bit offsets (csrc/march_impl.hpp Column,
+csrc/ct_march.hpp CmColumn): the largest FP32 plane below 4 GiB and the first at 4 GiB, each a periodic
+repetition of a small grid, so that every cell must come out with the bits of the small grid's step."""
 import pytest
 
 torch = pytest.importorskip("torch")
