@@ -113,9 +113,9 @@ struct CTMarchLDS {
 // A column (x, y) of the grid and the byte offsets, within a z plane, of its cells and of their upper x
 // and y neighbours, for planes below 4 GiB: the plane's base is one for the wavefront and an access adds
 // its offset itself.  (64-bit lane addresses, a multiplication or two and an addition each, were 4% of a
-// plane's instructions: the HLLD + PLM step at 256^3 FP64 2.43 -> 2.27 ms.)  Where the offsets are used
-// (192^3, us with 64-bit addresses and with offsets): FP64 PLM HLLD 885 -> 837 (HLL 632 -> 637); FP32 PLM
-// HLLD 424 -> 412, PPM HLL 374 -> 356, PPM HLLD 485 -> 457.  Not in the FP64 builds at one wavefront a SIMD,
+// plane's instructions: the HLLD + PLM step at 256^3 FP64 2.43 -> 2.24 ms.)  Where the offsets are used
+// (192^3, us with 64-bit addresses and with offsets): FP64 PLM HLLD 886 -> 829 (HLL 632 -> 633); FP32 PLM
+// HLLD 416 -> 415, PPM HLL 374 -> 347, PPM HLLD 486 -> 448.  Not in the FP64 builds at one wavefront a SIMD,
 // which have the registers and wait longer for the pointers (PPM HLL 924 -> 985, HLLD 1097 -> 1125; species
 // HLL 1018 -> 1078, HLLD 1148 -> 1218), nor for FP32 PLM HLL (324 -> 327) and species (HLLD 521 -> 526).
 template <typename T, int RIEM, int NS, int RC>
@@ -179,6 +179,8 @@ GLM_DEV void cm_prim_at(const A& a, CmColumn k, int z, bool narrow, T p[NV])
             cm_prim_of<T, NV>(a, u, bx1, by1, bz1, p);
             return;
         }
+        renew_v(k.x);   // nothing of the wide addresses is kept across the march
+        renew_v(k.y);
     }
     cm_prim<T, NV>(a, k.x, k.y, z, p);
 }
@@ -230,7 +232,11 @@ ct_march_kernel(CTMArgs<T> a_)
     const bool emf_y = tx >= 1 && ty >= 1 && ty <= CM_OY;
     constexpr bool OFF = CM_OFFSETS<T, RIEM, NS, RC>;
     const bool narrow = OFF && plane * sizeof(T) <= 0xffffffffu;
-    const size_t wcol = (size_t)gx + (size_t)nx * gy;
+    auto wide = [&] {   // the column's index within a z plane
+        int x = gx, y = gy;
+        if (OFF) { renew_v(x); renew_v(y); }
+        return (size_t)x + (size_t)nx * y;
+    };
     const CmColumn col = cm_column<T>(gx, gy, nx, ny);
     const int lo = (ty + 1) * CM_PX + (tx + 1);
     const int li = ty * CM_LX + tx;
@@ -287,7 +293,7 @@ ct_march_kernel(CTMArgs<T> a_)
             bny = gload_at((const T*)ap->q[6] + plane * zq, off);
             bnz = gload_at((const T*)ap->q[7] + plane * zq, off);
         } else {
-            const size_t off = wcol + plane * zq;
+            const size_t off = wide() + plane * zq;
             bnx = gload(a.q[5] + off); bny = gload(a.q[6] + off); bnz = gload(a.q[7] + off);
         }
 
@@ -374,7 +380,8 @@ ct_march_kernel(CTMArgs<T> a_)
             // ---- update of plane q-1 (ct_mhd.jl:124-136, :156-171) --------------------------------
             if (owned && q >= zs + 1) {
                 const int zu = cwrap(q - 1, nz);
-                const size_t zo = plane * zu, ow = wcol + zo;
+                const size_t zo = plane * zu;
+                size_t ow = OFF ? 0 : wide() + zo;
                 T r[NH], b0[NH], bo[3];   // hydro values, then species (plane 8 + s at index 5 + s); face fields
                 const auto* ap = &a;
                 renew_s(ap);
@@ -386,6 +393,7 @@ ct_march_kernel(CTMArgs<T> a_)
 #pragma unroll
                     for (int t = 0; t < 3; ++t) bo[t] = gload_at((const T*)ap->q[5 + t] + zo, off);
                 } else {
+                    if (OFF) ow = wide() + zo;
 #pragma unroll
                     for (int t = 0; t < NH; ++t) b0[t] = gload(a.q[t < 5 ? t : t + 3] + ow);
 #pragma unroll
@@ -428,6 +436,7 @@ ct_march_kernel(CTMArgs<T> a_)
 #pragma unroll
                     for (int t = 0; t < 3; ++t) gstore_nt_at(bn[t], (T*)ap->o[5 + t] + zo, off);
                 } else {
+                    if (OFF) ow = wide() + zo;
 #pragma unroll
                     for (int t = 0; t < NH; ++t) gstore_nt(r[t], (T*)a.o[t < 5 ? t : t + 3] + ow);
 #pragma unroll
