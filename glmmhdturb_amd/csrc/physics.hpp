@@ -527,30 +527,31 @@ GLM_HD bool spj(T a, T b, T c)
 // (Bx = bn*); fbn/fpsi are the GLM fluxes placed in slots 5 and 8.
 // ----------------------------------------------------------------------------------------
 
-// wL (FL - SL UL) + wR (FR - SR UR): the HLL flux with wL = SR / (SR - SL) and wR = -SL / (SR - SL), the LLF
-// one with SL = -smax, SR = smax and both weights 1/2.  FL - SL UL needs neither the momenta nor the plain
-// flux: with kL = wL (u - SL) its mass part is rho kL, whose products with the velocities are the
-// momentum parts, and the common Bn multiplies the weighted sums once: 60 operations where
-// (SR FL - SL FR + SL SR (UR - UL)) / (SR - SL) took 95.
+// wL FL + wR FR + k (UL - UR): the HLL flux with wL = SR / (SR - SL), wR = -SL / (SR - SL) and k = -SL wL, the
+// LLF one with both weights 1/2 and k = smax/2.  The plain fluxes' products with the velocities share wL u and
+// the common Bn multiplies the weighted sums once: about 75 operations where
+// (SR FL - SL FR + SL SR (UR - UL)) / (SR - SL) took 95.  The jumps U_L - U_R are formed before they are
+// multiplied: folded into the sides, as wL (FL - SL UL) + wR (FR - SR UR) (60 operations), the terms -+k U are
+// rounded before they cancel, and at Mach 0.01 with 2% jumps the mass flux loses a factor of 70 of its accuracy.
 template <typename T>
-GLM_HD void two_wave_x(const T L[9], const T R[9], T SL, T SR, T wL, T wR, T f[9], T igm1)
+GLM_HD void two_wave_x(const T L[9], const T R[9], T wL, T wR, T k, T f[9], T igm1)
 {
     const T bn = L[5], bn2 = bn * bn;
     const T b2L = bn2 + L[6] * L[6] + L[7] * L[7], b2R = bn2 + R[6] * R[6] + R[7] * R[7];
     const T ptL = L[4] + T(0.5) * b2L, ptR = R[4] + T(0.5) * b2R;
-    const T kL = wL * (L[1] - SL), kR = wR * (R[1] - SR);
-    const T mL = L[0] * kL, mR = R[0] * kR;
-    f[0] = mL + mR;
-    f[1] = mL * L[1] + mR * R[1] + (wL * ptL + wR * ptR) - bn2;
-    f[2] = mL * L[2] + mR * R[2] - bn * (wL * L[6] + wR * R[6]);
-    f[3] = mL * L[3] + mR * R[3] - bn * (wL * L[7] + wR * R[7]);
+    const T aL = wL * L[1], aR = wR * R[1];
+    const T mL = L[0] * aL, mR = R[0] * aR;
+    f[0] = mL + mR + k * (L[0] - R[0]);
+    f[1] = wL * ptL + wR * ptR + (mL * L[1] + mR * R[1] + k * (L[0] * L[1] - R[0] * R[1]) - bn2);
+    f[2] = mL * L[2] + mR * R[2] - bn * (wL * L[6] + wR * R[6]) + k * (L[0] * L[2] - R[0] * R[2]);
+    f[3] = mL * L[3] + mR * R[3] - bn * (wL * L[7] + wR * R[7]) + k * (L[0] * L[3] - R[0] * R[3]);
     const T EL = L[4] * igm1 + T(0.5) * (L[0] * (L[1] * L[1] + L[2] * L[2] + L[3] * L[3]) + b2L);
     const T ER = R[4] * igm1 + T(0.5) * (R[0] * (R[1] * R[1] + R[2] * R[2] + R[3] * R[3]) + b2R);
     const T vbL = L[1] * bn + L[2] * L[6] + L[3] * L[7], vbR = R[1] * bn + R[2] * R[6] + R[3] * R[7];
-    f[4] = EL * kL + ER * kR + (wL * (ptL * L[1] - bn * vbL) + wR * (ptR * R[1] - bn * vbR));
+    f[4] = aL * (EL + ptL) + aR * (ER + ptR) - bn * (wL * vbL + wR * vbR) + k * (EL - ER);
     f[5] = T(0);
-    f[6] = L[6] * kL + R[6] * kR - bn * (wL * L[2] + wR * R[2]);
-    f[7] = L[7] * kL + R[7] * kR - bn * (wL * L[3] + wR * R[3]);
+    f[6] = aL * L[6] + aR * R[6] - bn * (wL * L[2] + wR * R[2]) + k * (L[6] - R[6]);
+    f[7] = aL * L[7] + aR * R[7] - bn * (wL * L[3] + wR * R[3]) + k * (L[7] - R[7]);
     f[8] = T(0);
 }
 
@@ -569,7 +570,7 @@ GLM_HD void llf_x(const T L[9], const T R[9], T f[9], const Phys<T>& s)
         cR = fast_speed(R[0], R[4], b2R, R[5], s);
     }
     T smax = tmax(tmax(tabs(L[1]) + cL, tabs(R[1]) + cR), s.ch);
-    two_wave_x(L, R, -smax, smax, T(0.5), T(0.5), f, s.igm1);
+    two_wave_x(L, R, T(0.5), T(0.5), T(0.5) * smax, f, s.igm1);
 }
 
 // glmmhd_turb.jl:335-343 hll_x
@@ -582,7 +583,8 @@ GLM_HD void hll_x(const T L[9], const T R[9], T f[9], const Phys<T>& s)
     T SL = tmin(tmin(L[1] - cfL, R[1] - cfR), T(0));
     T SR = tmax(tmax(L[1] + cfL, R[1] + cfR), T(0));
     T ihd = trcp(SR - SL);
-    two_wave_x(L, R, SL, SR, SR * ihd, -SL * ihd, f, s.igm1);
+    const T wL = SR * ihd;
+    two_wave_x(L, R, wL, -SL * ihd, -SL * wL, f, s.igm1);
 }
 
 // glmmhd_turb.jl:193-272 hlld_x (Miyoshi & Kusano 2005).  Only the side that the sampling

@@ -1,0 +1,27 @@
+// flux_check.cpp -- the kernels' two-wave fluxes (HLL, LLF) as host functions, for their rounding error and their
+// one-sided limits.  Built by tests/native/Makefile (a host-only pass of hipcc); used by the CPU tests.
+#include "../../glmmhdturb_amd/csrc/physics.hpp"
+
+using namespace glm;
+
+namespace {
+
+// n faces: x-frame states of nine values each (rho, vx, vy, vz, p, Bx, By, Bz, psi), no floors, no cleaning
+template <typename T>
+void mhd(int llf, const T* L, const T* R, T* f, long n, double gamma)
+{
+    Phys<T> s;
+    s.gamma = (T)gamma; s.igm1 = (T)(1.0 / (gamma - 1.0)); s.smallr = T(0); s.pfl = T(0);
+    s.ch = T(0); s.ch2 = T(0); s.half_ich = T(0); s.llf_dmin = T(0); s.llf_pmin = T(0);
+    for (long i = 0; i < n; ++i) {
+        if (llf) llf_x<T, false>(L + 9 * i, R + 9 * i, f + 9 * i, s);
+        else hll_x(L + 9 * i, R + 9 * i, f + 9 * i, s);
+    }
+}
+
+}  // namespace
+
+extern "C" {
+void fc_mhd_f32(int llf, const float* L, const float* R, float* f, long n, double g) { mhd(llf, L, R, f, n, g); }
+void fc_mhd_f64(int llf, const double* L, const double* R, double* f, long n, double g) { mhd(llf, L, R, f, n, g); }
+}

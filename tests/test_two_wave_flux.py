@@ -1,0 +1,73 @@
+"""The two-wave fluxes (csrc/physics.hpp two_wave_x: HLL and LLF) against 80-bit arithmetic on states down to Mach
+0.01, where U_L - U_R has to be formed before it is multiplied by the wave speeds."""
+import ctypes as C
+import os
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "glmmhdturb_amd", "_build", "libfluxcheck.so")
+G = 1.4
+X = np.longdouble
+
+
+def solve(name, kind, L, R):
+    if not os.path.exists(LIB):
+        pytest.skip("host flux build is missing (tests/native)")
+    f = np.empty_like(L)
+    ptr = [a.ctypes.data_as(C.c_void_p) for a in (L, R, f)]
+    getattr(C.CDLL(LIB), name)(C.c_int(kind), *ptr, C.c_long(len(L)), C.c_double(G))
+    return f
+
+
+def pair(nv, mach, jump, dtype, n=4000):
+    """Two states a face: the same one and up to `jump` of relative change in every value."""
+    r = np.random.default_rng(5)
+    b = np.zeros((n, nv))
+    b[:, 0], b[:, 4] = r.uniform(0.5, 2, n), r.uniform(0.5, 2, n)
+    a = np.sqrt(G * b[:, 4] / b[:, 0])
+    b[:, 1:4] = mach * a[:, None] * r.uniform(-1, 1, (n, 3))
+    if nv == 9:
+        b[:, 5:8] = r.uniform(-1, 1, (n, 3))
+    L, R = (b * (1 + jump * r.uniform(-1, 1, b.shape)) for _ in range(2))
+    if nv == 9:
+        R[:, 5] = L[:, 5]   # the face's normal field is one value
+    return L.astype(dtype), R.astype(dtype)
+
+
+def two_wave(L, R, llf, fast):
+    """Weights and k of wL FL + wR FR + k (UL - UR) in 80 bits."""
+    cl, cr = fast(L), fast(R)
+    if llf:
+        s = np.maximum(abs(L[1]) + cl, abs(R[1]) + cr)
+        sl, sr = -s, s
+    else:
+        sl = np.minimum(np.minimum(L[1] - cl, R[1] - cr), 0)
+        sr = np.maximum(np.maximum(L[1] + cl, R[1] + cr), 0)
+    return sr / (sr - sl), -sl / (sr - sl), -sl * sr / (sr - sl)
+
+
+@pytest.mark.parametrize("llf", [0, 1], ids=["hll", "llf"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("mach,jump", [(0.01, 0.02), (0.1, 0.02), (1.0, 0.02), (1.0, 0.5)])
+def test_mhd_flux_error_follows_the_jump(mach, jump, dtype, llf):
+    """Mass and transverse field, whose jump is exact: every term is a product of up to four rounded factors (the
+    speeds to 4 ulp), so 8 ulp of the sum of their magnitudes.  Terms of +-k U would leave 0.5 ulp of k U each."""
+    L, R = pair(9, mach, jump, dtype)
+    f = solve("fc_mhd_f32" if dtype == np.float32 else "fc_mhd_f64", llf, L, R).T
+    l, r = L.astype(X).T, R.astype(X).T
+
+    def fast(q):
+        b2 = q[5] ** 2 + q[6] ** 2 + q[7] ** 2
+        h = 0.5 * (G * q[4] + b2) / q[0]
+        return np.sqrt(h + np.sqrt(np.maximum(h * h - X(G) * q[4] * q[5] ** 2 / q[0] ** 2, 0)))
+
+    wl, wr, k = two_wave(l, r, llf, fast)
+    terms = {0: (l[0] * l[1], r[0] * r[1], k * (l[0] - r[0])),
+             6: (l[6] * l[1] - l[5] * l[2], r[6] * r[1] - r[5] * r[2], k * (l[6] - r[6]))}
+    size = {0: abs(l[0] * l[1]) + abs(r[0] * r[1]),
+            6: abs(l[6] * l[1]) + abs(l[5] * l[2]) + abs(r[6] * r[1]) + abs(r[5] * r[2])}
+    for c, (fl, fr, d) in terms.items():
+        err = abs(f[c] - (wl * fl + wr * fr + d))
+        assert np.all(err <= 8 * np.finfo(dtype).eps * (size[c] + abs(d))), (c, float((err / (size[c] + abs(d))).max()))
