@@ -533,6 +533,8 @@ GLM_HD bool spj(T a, T b, T c)
 // (SR FL - SL FR + SL SR (UR - UL)) / (SR - SL) took 95.  The jumps U_L - U_R are formed before they are
 // multiplied: folded into the sides, as wL (FL - SL UL) + wR (FR - SR UR) (60 operations), the terms -+k U are
 // rounded before they cancel, and at Mach 0.01 with 2% jumps the mass flux loses a factor of 70 of its accuracy.
+// The energy comes first, the components that let go of the most values of the states next: as the switch of the
+// FP32 HLLD + PPM builds, in component order, it made them spill 68 B a lane instead of 56 (6% of their time).
 template <typename T>
 GLM_HD void two_wave_x(const T L[9], const T R[9], T wL, T wR, T k, T f[9], T igm1)
 {
@@ -541,17 +543,17 @@ GLM_HD void two_wave_x(const T L[9], const T R[9], T wL, T wR, T k, T f[9], T ig
     const T ptL = L[4] + T(0.5) * b2L, ptR = R[4] + T(0.5) * b2R;
     const T aL = wL * L[1], aR = wR * R[1];
     const T mL = L[0] * aL, mR = R[0] * aR;
-    f[0] = mL + mR + k * (L[0] - R[0]);
-    f[1] = wL * ptL + wR * ptR + (mL * L[1] + mR * R[1] + k * (L[0] * L[1] - R[0] * R[1]) - bn2);
-    f[2] = mL * L[2] + mR * R[2] - bn * (wL * L[6] + wR * R[6]) + k * (L[0] * L[2] - R[0] * R[2]);
-    f[3] = mL * L[3] + mR * R[3] - bn * (wL * L[7] + wR * R[7]) + k * (L[0] * L[3] - R[0] * R[3]);
     const T EL = L[4] * igm1 + T(0.5) * (L[0] * (L[1] * L[1] + L[2] * L[2] + L[3] * L[3]) + b2L);
     const T ER = R[4] * igm1 + T(0.5) * (R[0] * (R[1] * R[1] + R[2] * R[2] + R[3] * R[3]) + b2R);
     const T vbL = L[1] * bn + L[2] * L[6] + L[3] * L[7], vbR = R[1] * bn + R[2] * R[6] + R[3] * R[7];
     f[4] = aL * (EL + ptL) + aR * (ER + ptR) - bn * (wL * vbL + wR * vbR) + k * (EL - ER);
-    f[5] = T(0);
-    f[6] = aL * L[6] + aR * R[6] - bn * (wL * L[2] + wR * R[2]) + k * (L[6] - R[6]);
     f[7] = aL * L[7] + aR * R[7] - bn * (wL * L[3] + wR * R[3]) + k * (L[7] - R[7]);
+    f[3] = mL * L[3] + mR * R[3] - bn * (wL * L[7] + wR * R[7]) + k * (L[0] * L[3] - R[0] * R[3]);
+    f[6] = aL * L[6] + aR * R[6] - bn * (wL * L[2] + wR * R[2]) + k * (L[6] - R[6]);
+    f[2] = mL * L[2] + mR * R[2] - bn * (wL * L[6] + wR * R[6]) + k * (L[0] * L[2] - R[0] * R[2]);
+    f[1] = wL * ptL + wR * ptR + (mL * L[1] + mR * R[1] + k * (L[0] * L[1] - R[0] * R[1]) - bn2);
+    f[0] = mL + mR + k * (L[0] - R[0]);
+    f[5] = T(0);
     f[8] = T(0);
 }
 
