@@ -107,7 +107,7 @@ GLM_DEV unsigned short hy_enc_log2s(float l2)
 GLM_DEV float hy_f16_to_f32(unsigned short h) { return (float)__builtin_bit_cast(_Float16, h); }
 GLM_DEV unsigned short hy_f32_to_f16(float x) { return __builtin_bit_cast(unsigned short, (_Float16)x); }
 template <typename T>
-GLM_DEV T hy_exp2(T x) { return (T)exp2f((float)x); }
+GLM_HD T hy_exp2(T x) { return (T)exp2f((float)x); }
 
 // spike_25d.cu:196-202 prim_from_cons (:183-194 with scalars: s = (rho s) / rho; with LG the scalar
 // planes already hold log2 X, :188-190)
@@ -129,8 +129,8 @@ GLM_DEV void hy_c2p(const T c[NV], T q[NV], const HydroArgs<T>& a)
 
 // a*b + c as one operation.  The flux functions below are compiled without contraction and write their
 // fused operations out, so that every copy of them (two rows, three faces, three directions) rounds alike.
-GLM_DEV double tfma(double a, double b, double c) { return __builtin_fma(a, b, c); }
-GLM_DEV float tfma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+GLM_HD double tfma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+GLM_HD float tfma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
 // spike_25d.cu:245-255 toCons (with LG the scalars are log2 X, decoded for the conserved rho X, :248-250)
 template <typename T, int NV, bool LG = false>
@@ -192,42 +192,45 @@ GLM_DEV void hy_states(const T l[NV], const T c[NV], const T r[NV], T lo[NV], T 
 // (riemann_fb, :335-376).  With CMA the scalar fluxes of the HLL fan are the mass flux times the upwind
 // face value (:321, :367).
 //
-// F = [sR FL - sL FR + sL sR (UR - UL)] / (sR - sL) = wL (FL - sL UL) + wR (FR - sR UR) with
-// wL = sR / (sR - sL) and wR = -sL / (sR - sL).  FL - sL UL needs no momenta and no flux of its own (its mass
-// part rho (u - sL) times each velocity is its momentum part); speeds clamped at 0 make it the upwind flux
-// on supersonic faces, and speeds -+max(|u| + a) make it LLF: two selects instead of one per component.
+// F = wL FL + wR FR + k (UL - UR) with wL = sR / (sR - sL), wR = -sL / (sR - sL) and k = -sL wL; weights
+// of 1/2 and k = max(|u| + a)/2 make it LLF: three selects instead of one per component.  The jumps are formed
+// before they are multiplied: as wL (FL - sL UL) + wR (FR - sR UR), 12 operations less, the terms -+k U are
+// rounded before they cancel, and at Mach 0.01 with 2% jumps the mass flux loses a factor of 70 of its accuracy.
 template <typename T, int D, bool FB, int NV, bool CMA, bool LG = false>
-GLM_DEV void hy_riemann(const T L[NV], const T R[NV], T F[NV], const HydroArgs<T>& a)
+GLM_HD void hy_riemann(const T L[NV], const T R[NV], T F[NV], const HydroArgs<T>& a)
 {
 #pragma clang fp contract(off)
-    const T uL = L[1 + D], uR = R[1 + D];
     const T aL = tsqrt_pos(a.gamma * L[4] * trcp(L[0])), aR = tsqrt_pos(a.gamma * R[4] * trcp(R[0]));
-    T sL = tmin(tmin(uL - aL, uR - aR), T(0)), sR = tmax(tmax(uL + aL, uR + aR), T(0));
-    bool llf = false;
+    const T sL = tmin(tmin(L[1 + D] - aL, R[1 + D] - aR), T(0)), sR = tmax(tmax(L[1 + D] + aL, R[1 + D] + aR), T(0));
+    const bool llf = FB && (L[0] < a.fb_dmin || L[4] < a.fb_pmin || R[0] < a.fb_dmin || R[4] < a.fb_pmin);
+    const T inv = trcp(sR - sL);
+    T wL = sR * inv, wR = -sL * inv, k = -sL * wL;
     if (FB) {
-        llf = L[0] < a.fb_dmin || L[4] < a.fb_pmin || R[0] < a.fb_dmin || R[4] < a.fb_pmin;
-        const T sm = tmax(tabs(uL) + aL, tabs(uR) + aR);
-        sL = llf ? -sm : sL;
-        sR = llf ? sm : sR;
+        const T sm = tmax(tabs(L[1 + D]) + aL, tabs(R[1 + D]) + aR);
+        wL = llf ? T(0.5) : wL;
+        wR = llf ? T(0.5) : wR;
+        k = llf ? T(0.5) * sm : k;
     }
-    const T inv = trcp(sR - sL), wL = sR * inv, wR = -sL * inv;
-    const T dL = uL - sL, dR = uR - sR;
-    const T mL = wL * (L[0] * dL), mR = wR * (R[0] * dR);
-    F[0] = mL + mR;
+    const T bL = wL * L[1 + D], bR = wR * R[1 + D];
+    const T mL = L[0] * bL, mR = R[0] * bR;
+    F[0] = tfma(k, L[0] - R[0], tfma(L[0], bL, mR));
 #pragma unroll
-    for (int c = 1; c < 4; ++c) F[c] = tfma(mL, L[c], mR * R[c]);
+    for (int c = 1; c < 4; ++c) {
+        const T uy = R[0] * R[c];
+        F[c] = tfma(k, tfma(L[0], L[c], -uy), tfma(mL, L[c], bR * uy));
+    }
     F[1 + D] = F[1 + D] + tfma(wL, L[4], wR * R[4]);
     const T EL = tfma(L[4], a.igm1, T(0.5) * L[0] * tfma(L[1], L[1], tfma(L[2], L[2], L[3] * L[3])));
     const T ER = tfma(R[4], a.igm1, T(0.5) * R[0] * tfma(R[1], R[1], tfma(R[2], R[2], R[3] * R[3])));
-    F[4] = tfma(wL, tfma(EL, dL, L[4] * uL), wR * tfma(ER, dR, R[4] * uR));
+    F[4] = tfma(k, EL - ER, tfma(bL, EL + L[4], bR * (ER + R[4])));
 #pragma unroll
     for (int v = 5; v < NV; ++v) {
-        if (CMA) {
+        if (CMA && !llf) {
             const T x = F[0] >= T(0) ? L[v] : R[v];
             F[v] = F[0] * (LG ? hy_exp2(x) : x);
-            if (FB && llf) F[v] = tfma(mL, LG ? hy_exp2(L[v]) : L[v], mR * (LG ? hy_exp2(R[v]) : R[v]));
         } else {
-            F[v] = tfma(mL, L[v], mR * R[v]);
+            const T xL = LG ? hy_exp2(L[v]) : L[v], ux = R[0] * (LG ? hy_exp2(R[v]) : R[v]);
+            F[v] = tfma(k, tfma(L[0], xL, -ux), tfma(mL, xL, bR * ux));
         }
     }
 }

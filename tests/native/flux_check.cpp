@@ -1,6 +1,6 @@
 // flux_check.cpp -- the kernels' two-wave fluxes (HLL, LLF) as host functions, for their rounding error and their
 // one-sided limits.  Built by tests/native/Makefile (a host-only pass of hipcc); used by the CPU tests.
-#include "../../glmmhdturb_amd/csrc/physics.hpp"
+#include "../../glmmhdturb_amd/csrc/hydro_march.hpp"
 
 using namespace glm;
 
@@ -19,9 +19,21 @@ void mhd(int llf, const T* L, const T* R, T* f, long n, double gamma)
     }
 }
 
+// n faces normal to x: states of seven values each (rho, vx, vy, vz, p and two scalars), solved by HLL or LLF
+template <typename T>
+void hydro(int llf, const T* L, const T* R, T* f, long n, double gamma)
+{
+    HydroArgs<T> a;
+    a.gamma = (T)gamma; a.igm1 = (T)(1.0 / (gamma - 1.0));
+    a.fb_dmin = llf ? T(1e30) : T(0); a.fb_pmin = T(0);
+    for (long i = 0; i < n; ++i) hy_riemann<T, 0, true, 7, false>(L + 7 * i, R + 7 * i, f + 7 * i, a);
+}
+
 }  // namespace
 
 extern "C" {
 void fc_mhd_f32(int llf, const float* L, const float* R, float* f, long n, double g) { mhd(llf, L, R, f, n, g); }
 void fc_mhd_f64(int llf, const double* L, const double* R, double* f, long n, double g) { mhd(llf, L, R, f, n, g); }
+void fc_hydro_f32(int llf, const float* L, const float* R, float* f, long n, double g) { hydro(llf, L, R, f, n, g); }
+void fc_hydro_f64(int llf, const double* L, const double* R, double* f, long n, double g) { hydro(llf, L, R, f, n, g); }
 }

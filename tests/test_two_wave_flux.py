@@ -1,5 +1,5 @@
-"""The two-wave fluxes (csrc/physics.hpp two_wave_x: HLL and LLF) against 80-bit arithmetic on states down to Mach
-0.01, where U_L - U_R has to be formed before it is multiplied by the wave speeds."""
+"""The two-wave fluxes (HLL and LLF: csrc/physics.hpp two_wave_x, csrc/hydro_march.hpp hy_riemann) against 80-bit
+arithmetic on states down to Mach 0.01, where U_L - U_R has to be formed before it is multiplied by the wave speeds."""
 import ctypes as C
 import os
 
@@ -71,3 +71,17 @@ def test_mhd_flux_error_follows_the_jump(mach, jump, dtype, llf):
     for c, (fl, fr, d) in terms.items():
         err = abs(f[c] - (wl * fl + wr * fr + d))
         assert np.all(err <= 8 * np.finfo(dtype).eps * (size[c] + abs(d))), (c, float((err / (size[c] + abs(d))).max()))
+
+
+@pytest.mark.parametrize("llf", [0, 1], ids=["hll", "llf"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("mach,jump", [(0.01, 0.02), (0.1, 0.02), (1.0, 0.02), (1.0, 0.5)])
+def test_hydro_flux_error_follows_the_jump(mach, jump, dtype, llf):
+    """The mass flux, with the same bound."""
+    L, R = pair(7, mach, jump, dtype)
+    f = solve("fc_hydro_f32" if dtype == np.float32 else "fc_hydro_f64", llf, L, R).T
+    l, r = L.astype(X).T, R.astype(X).T
+    wl, wr, k = two_wave(l, r, llf, lambda q: np.sqrt(X(G) * q[4] / q[0]))
+    fl, fr, d = l[0] * l[1], r[0] * r[1], k * (l[0] - r[0])
+    err = abs(f[0] - (wl * fl + wr * fr + d))
+    assert np.all(err <= 8 * np.finfo(dtype).eps * (abs(fl) + abs(fr) + abs(d)))
