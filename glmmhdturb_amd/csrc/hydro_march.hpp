@@ -196,13 +196,37 @@ GLM_DEV void hy_states(const T l[NV], const T c[NV], const T r[NV], T lo[NV], T 
 // of 1/2 and k = max(|u| + a)/2 make it LLF: three selects instead of one per component.  The jumps are formed
 // before they are multiplied: as wL (FL - sL UL) + wR (FR - sR UR), 12 operations less, the terms -+k U are
 // rounded before they cancel, and at Mach 0.01 with 2% jumps the mass flux loses a factor of 70 of its accuracy.
-template <typename T, int D, bool FB, int NV, bool CMA, bool LG = false>
-GLM_HD void hy_riemann(const T L[NV], const T R[NV], T F[NV], const HydroArgs<T>& a)
+//
+// Where both waves go one way the flux is that side's, and nothing of the other side enters it, be it infinite or
+// NaN.  By a branch, or with SEL by selects: the branch is the faster one (480^3 FP32 1.99 ms, with
+// selects 2.05) except in the FP64 builds whose registers it makes spill (256^3 705 us with 36 B spilled,
+// with selects 670; PPM1D at 192^3 488 and 376).
+template <typename T, int D, bool FB, int NV, bool CMA, bool LG = false, bool SEL = false>
+GLM_HD void hy_riemann(const T L_[NV], const T R_[NV], T F[NV], const HydroArgs<T>& a)
 {
 #pragma clang fp contract(off)
+    T L[NV], R[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) { L[v] = L_[v]; R[v] = R_[v]; }
     const T aL = tsqrt_pos(a.gamma * L[4] * trcp(L[0])), aR = tsqrt_pos(a.gamma * R[4] * trcp(R[0]));
-    const T sL = tmin(tmin(L[1 + D] - aL, R[1 + D] - aR), T(0)), sR = tmax(tmax(L[1 + D] + aL, R[1 + D] + aR), T(0));
+    const T sL = tmin(L[1 + D] - aL, R[1 + D] - aR), sR = tmax(L[1 + D] + aL, R[1 + D] + aR);
     const bool llf = FB && (L[0] < a.fb_dmin || L[4] < a.fb_pmin || R[0] < a.fb_dmin || R[4] < a.fb_pmin);
+    const bool up = sL >= T(0) && !llf, down = sR <= T(0) && !llf;
+    if (!SEL && (up || down)) {
+        T X[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) X[v] = up ? L[v] : R[v];
+        const T m = X[0] * X[1 + D];
+        const T E = tfma(X[4], a.igm1, T(0.5) * X[0] * tfma(X[1], X[1], tfma(X[2], X[2], X[3] * X[3])));
+        F[0] = m;
+#pragma unroll
+        for (int c = 1; c < 4; ++c) F[c] = m * X[c];
+        F[1 + D] = F[1 + D] + X[4];
+        F[4] = (E + X[4]) * X[1 + D];
+#pragma unroll
+        for (int v = 5; v < NV; ++v) F[v] = m * (LG ? hy_exp2(X[v]) : X[v]);
+        return;
+    }
     const T inv = trcp(sR - sL);
     T wL = sR * inv, wR = -sL * inv, k = -sL * wL;
     if (FB) {
@@ -210,6 +234,13 @@ GLM_HD void hy_riemann(const T L[NV], const T R[NV], T F[NV], const HydroArgs<T>
         wL = llf ? T(0.5) : wL;
         wR = llf ? T(0.5) : wR;
         k = llf ? T(0.5) * sm : k;
+    }
+    if (SEL) {   // both sides the one
+#pragma unroll
+        for (int v = 0; v < NV; ++v) { L[v] = down ? R_[v] : L_[v]; R[v] = up ? L_[v] : R_[v]; }
+        wL = up || down ? T(1) : wL;
+        wR = up || down ? T(0) : wR;
+        k = up || down ? T(0) : k;
     }
     const T bL = wL * L[1 + D], bR = wR * R[1 + D];
     const T mL = L[0] * bL, mR = R[0] * bR;
@@ -285,6 +316,7 @@ hydro_march_kernel(HydroArgs<T> a)
     constexpr bool LG = FMT == HY_U16SP;      // species held as log2 X
     constexpr bool PRIM = FMT == HY_F16P || FMT == HY_U16P;   // primitive storage: no conversion on load
     constexpr bool fb = FB && SV == HY_PLM;
+    constexpr bool sel = sizeof(T) == 8 && GLM_HY_WAVES(T, NSP, SV) > 1 && !fb;   // hy_riemann
     static_assert(FMT == HY_CONS || (sizeof(T) == 4 && (FMT != HY_U16SP || (NSP == 2 && CMA)) &&
                                      (FMT == HY_U16SP || NSP == 0)), "compact formats: FP32; U16SP with 2 CMA species");
     __shared__ T P[2][NV][HM_NPL];   // primitives of plane j in P[j & 1]
@@ -430,7 +462,7 @@ hydro_march_kernel(HydroArgs<T> a)
 #pragma unroll
                     for (int v = 0; v < NV; ++v) { hi[v] = l[v]; lo[v] = c[v]; }
                 }
-                hy_riemann<T, 0, fb, NV, CMA, LG>(hi, lo, F, a);
+                hy_riemann<T, 0, fb, NV, CMA, LG, sel>(hi, lo, F, a);
 #pragma unroll
                 for (int v = 0; v < NV; ++v) div[r][v] = lane_next(F[v]) - F[v];
             }
@@ -451,7 +483,7 @@ hydro_march_kernel(HydroArgs<T> a)
 #pragma unroll
                     for (int v = 0; v < NV; ++v) { up[v] = c[v]; lo[v] = n[v]; }
                 }
-                hy_riemann<T, 1, fb, NV, CMA, LG>(up, lo, F1, a);
+                hy_riemann<T, 1, fb, NV, CMA, LG, sel>(up, lo, F1, a);
                 if (f > 0) {
 #pragma unroll
                     for (int v = 0; v < NV; ++v) div[f - 1][v] += F1[v] - F0[v];
@@ -467,7 +499,7 @@ hydro_march_kernel(HydroArgs<T> a)
             lds(k, li + r * HM_LX, p0);
             prim(pre[r], pn);
             hy_states<T, 2, NV, SV>(p0, pp[r], pn, lo, hi, a);
-            hy_riemann<T, 2, fb, NV, CMA, LG>(zprev[r], lo, F, a);
+            hy_riemann<T, 2, fb, NV, CMA, LG, sel>(zprev[r], lo, F, a);
             if (k >= k0 && own[r]) {
 #pragma unroll
                 for (int v = 0; v < NV; ++v) div[r][v] += F[v] - Fz[r][v];

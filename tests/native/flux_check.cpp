@@ -19,14 +19,15 @@ void mhd(int llf, const T* L, const T* R, T* f, long n, double gamma)
     }
 }
 
-// n faces normal to x: states of seven values each (rho, vx, vy, vz, p and two scalars), solved by HLL or LLF
-template <typename T>
+// n faces normal to x: states of seven values each (rho, vx, vy, vz, p and two scalars), solved by HLL or LLF;
+// SEL: the one-sided fluxes by selects
+template <typename T, bool SEL = false>
 void hydro(int llf, const T* L, const T* R, T* f, long n, double gamma)
 {
     HydroArgs<T> a;
     a.gamma = (T)gamma; a.igm1 = (T)(1.0 / (gamma - 1.0));
     a.fb_dmin = llf ? T(1e30) : T(0); a.fb_pmin = T(0);
-    for (long i = 0; i < n; ++i) hy_riemann<T, 0, true, 7, false>(L + 7 * i, R + 7 * i, f + 7 * i, a);
+    for (long i = 0; i < n; ++i) hy_riemann<T, 0, true, 7, false, false, SEL>(L + 7 * i, R + 7 * i, f + 7 * i, a);
 }
 
 }  // namespace
@@ -36,4 +37,6 @@ void fc_mhd_f32(int llf, const float* L, const float* R, float* f, long n, doubl
 void fc_mhd_f64(int llf, const double* L, const double* R, double* f, long n, double g) { mhd(llf, L, R, f, n, g); }
 void fc_hydro_f32(int llf, const float* L, const float* R, float* f, long n, double g) { hydro(llf, L, R, f, n, g); }
 void fc_hydro_f64(int llf, const double* L, const double* R, double* f, long n, double g) { hydro(llf, L, R, f, n, g); }
+void fc_hydro_sel_f32(int llf, const float* L, const float* R, float* f, long n, double g) { hydro<float, true>(llf, L, R, f, n, g); }
+void fc_hydro_sel_f64(int llf, const double* L, const double* R, double* f, long n, double g) { hydro<double, true>(llf, L, R, f, n, g); }
 }

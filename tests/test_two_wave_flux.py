@@ -85,3 +85,32 @@ def test_hydro_flux_error_follows_the_jump(mach, jump, dtype, llf):
     fl, fr, d = l[0] * l[1], r[0] * r[1], k * (l[0] - r[0])
     err = abs(f[0] - (wl * fl + wr * fr + d))
     assert np.all(err <= 8 * np.finfo(dtype).eps * (abs(fl) + abs(fr) + abs(d)))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("name", ["fc_hydro", "fc_hydro_sel"])
+def test_supersonic_hydro_flux_is_the_upwind_sides(name, dtype):
+    """Both waves to one side: that side's flux, with its own roundings only, whatever the other side holds."""
+    name += "_f32" if dtype == np.float32 else "_f64"
+    L, R = pair(7, 0.5, 0.1, dtype, 500)
+    for q in (L, R):
+        q[:, 1] = 3 + abs(q[:, 1])   # above every sound speed of the pair
+        q[:, 5:] = 0.3
+    m = L[:, 0] * L[:, 1]
+    E = L[:, 4].astype(X) / (X(G) - 1) + L[:, 0] * (L[:, 1:4].astype(X) ** 2).sum(1) / 2
+    up = solve(name, 0, L, R)
+    assert np.array_equal(up[:, 0], m)
+    for c in (2, 3, 5, 6):
+        assert np.array_equal(up[:, c], m * L[:, c])
+    # the product and the sum with p, whether fused or not; E's terms, p and the product with u
+    eps = np.finfo(dtype).eps
+    assert np.all(abs(up[:, 1] - (L[:, 0].astype(X) * L[:, 1] * L[:, 1] + L[:, 4])) <= 2 * eps * abs(up[:, 1]))
+    assert np.all(abs(up[:, 4] - (E + L[:, 4]) * L[:, 1]) <= 6 * eps * abs(up[:, 4]))
+    flip = np.array([1, -1, 1, 1, 1, 1, 1], dtype)   # the mirrored face
+    down = solve(name, 0, R * flip, L * flip)
+    assert np.array_equal(down * flip, -up)
+    for v, x in [(0, np.nan), (1, np.nan), (2, np.nan), (3, np.inf), (4, np.nan), (5, np.nan), (6, np.inf), (1, np.inf), (0, np.inf)]:
+        bad = R.copy()
+        bad[:, v] = x
+        assert np.array_equal(solve(name, 0, L, bad), up), (v, x)
+        assert np.array_equal(solve(name, 0, bad * flip, L * flip), down), (v, x)
