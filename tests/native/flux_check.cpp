@@ -30,6 +30,14 @@ void hydro(int llf, const T* L, const T* R, T* f, long n, double gamma)
     for (long i = 0; i < n; ++i) hy_riemann<T, 0, true, 7, false, false, SEL>(L + 7 * i, R + 7 * i, f + 7 * i, a);
 }
 
+template <typename T>
+void update(const T* q, const T* div, T* u, long n, double dtdx)
+{
+    HydroArgs<T> a;
+    a.igm1 = T(2.5); a.dtdx = (T)dtdx;
+    for (long i = 0; i < n; ++i) hy_update<T, 7>(q + 7 * i, div + 7 * i, u + 7 * i, a);
+}
+
 }  // namespace
 
 extern "C" {
@@ -39,4 +47,6 @@ void fc_hydro_f32(int llf, const float* L, const float* R, float* f, long n, dou
 void fc_hydro_f64(int llf, const double* L, const double* R, double* f, long n, double g) { hydro(llf, L, R, f, n, g); }
 void fc_hydro_sel_f32(int llf, const float* L, const float* R, float* f, long n, double g) { hydro<float, true>(llf, L, R, f, n, g); }
 void fc_hydro_sel_f64(int llf, const double* L, const double* R, double* f, long n, double g) { hydro<double, true>(llf, L, R, f, n, g); }
+void fc_update_f32(const float* q, const float* div, float* u, long n, double dtdx) { update(q, div, u, n, dtdx); }
+void fc_update_f64(const double* q, const double* div, double* u, long n, double dtdx) { update(q, div, u, n, dtdx); }
 }

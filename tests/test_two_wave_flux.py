@@ -114,3 +114,20 @@ def test_supersonic_hydro_flux_is_the_upwind_sides(name, dtype):
         bad[:, v] = x
         assert np.array_equal(solve(name, 0, L, bad), up), (v, x)
         assert np.array_equal(solve(name, 0, bad * flip, L * flip), down), (v, x)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_hydro_update_rounds_a_value_once(dtype):
+    """Density, momenta and scalars: one rounding at the value's size and one at the change's."""
+    q, div = pair(7, 1.0, 0.5, dtype)
+    q[:, 5:] = 0.3
+    u = np.empty_like(q)
+    ptr = [a.ctypes.data_as(C.c_void_p) for a in (q, div, u)]
+    if not os.path.exists(LIB):
+        pytest.skip("host flux build is missing (tests/native)")
+    k = dtype(0.05)
+    getattr(C.CDLL(LIB), "fc_update_f32" if dtype == np.float32 else "fc_update_f64")(*ptr, C.c_long(len(q)), C.c_double(k))
+    for c in (0, 1, 2, 3, 5, 6):
+        d = X(k) * div[:, c]
+        x = (q[:, 0].astype(X) * q[:, c] if c else q[:, 0].astype(X)) - d
+        assert np.all(abs(u[:, c] - x) <= 0.5 * np.finfo(dtype).eps * (1.001 * abs(x) + abs(d))), c
