@@ -134,5 +134,5 @@ def check(code: int) -> None:
 
 def plane_array(ptrs):
     """Host array of device plane addresses (the float** / void* const* of the ABI)."""
-    arr = (C.c_void_p * len(ptrs))(*ptrs)
+    arr = (C.c_void_p * len(ptrs))(*map(int, ptrs))
     return arr, arr
