@@ -199,8 +199,9 @@ glm_ctx* glm_create(int nx, int ny, int nz, int precision)
         ctx_free(c);
         return nullptr;
     }
-    if (hipMemset(c->d_cmax, 0, 4 * sizeof(unsigned long long)) != hipSuccess) {
-        set_err(GLM_ERR_HIP, "glm_create: hipMemset failed");
+    // waited for: the null stream's work is not ordered before that of a non-blocking stream the context may get
+    if (hipMemset(c->d_cmax, 0, 4 * sizeof(unsigned long long)) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
+        set_err(GLM_ERR_HIP, "glm_create: clearing the result slots failed");
         ctx_free(c);
         return nullptr;
     }
