@@ -126,7 +126,7 @@ struct glm_ens {
     double clock_khz;
     // device tables
     EnsBox* d_eb;
-    void* d_ma;            // MarchArgs<T>[nbox]
+    void* d_ma;            // MarchArgs<T>[nbox] (replaced with the tile list)
     OUBox* d_ou;
     EnsTile* d_tiles;         // flat tile list: box and its local tile (replaced when the layout changes)
     unsigned int* d_queue;
@@ -281,38 +281,53 @@ int grid_of(const glm_ens* e, int total, int persistent)
     return g < total ? g : total;
 }
 
-// The tile list of a layout in device memory (the caller's to free).
-int upload_tiles(const Layout& L, EnsTile** out)
+// A host table in new device memory (the caller's to free).  A failure is taken off the runtime, or the next launch
+// would report it.
+int upload(const void* src, size_t bytes, void** out)
 {
-    if (hipMalloc(out, L.tiles.size() * sizeof(EnsTile)) != hipSuccess)
-        return set_err(GLM_ERR_ALLOC, "glm_ens: tile list allocation failed");
-    if (hipMemcpy(*out, L.tiles.data(), L.tiles.size() * sizeof(EnsTile), hipMemcpyHostToDevice) != hipSuccess) {
+    if (hipMalloc(out, bytes) != hipSuccess) {
+        *out = nullptr;
+        (void)hipGetLastError();
+        return set_err(GLM_ERR_ALLOC, "glm_ens: table allocation failed");
+    }
+    if (hipMemcpy(*out, src, bytes, hipMemcpyHostToDevice) != hipSuccess) {
         (void)hipFree(*out);
         *out = nullptr;
-        return set_err(GLM_ERR_HIP, "glm_ens: tile list upload failed");
+        (void)hipGetLastError();
+        return set_err(GLM_ERR_HIP, "glm_ens: table upload failed");
     }
     return GLM_OK;
 }
+int upload_tiles(const Layout& L, EnsTile** out) { return upload(L.tiles.data(), L.tiles.size() * sizeof(EnsTile), (void**)out); }
 
+// The boxes' march arguments for a layout, in device memory.  The step control rewrites the per-step
+// fields every sweep; the rest comes from here.
+template <typename T>
+int upload_args(const glm_ens* e, const Layout& L, void** out)
+{
+    auto v = make_args<T>(e, L, nullptr);
+    for (int b = 0; b < e->nbox; ++b) v[b].cmax = &e->d_eb[b].cmax;
+    return upload(v.data(), v.size() * sizeof v[0], out);
+}
+
+// Both tables of the new layout are in place before the old ones go: a call that fails leaves the ensemble,
+// and the graph that points to its tables, as they were.
 int apply_config(glm_ens* e, int zreq, int persistent, int ord)
 {
     Layout L = make_layout(e, zreq, ord);
     if (L.total <= 0) return set_err(GLM_ERR_ARG, "glm_ens: empty tile list");
     HIPCHK(hipStreamSynchronize(e->stream));
     EnsTile* tiles = nullptr;
+    void* ma = nullptr;
     if (int err = upload_tiles(L, &tiles)) return err;
-    if (e->d_tiles) (void)hipFree(e->d_tiles);
-    e->d_tiles = tiles;
-    // the step control rewrites the per-step fields every sweep; the rest comes from here
-    if (e->prec == 8) {
-        auto v = make_args<double>(e, L, nullptr);
-        for (int b = 0; b < e->nbox; ++b) v[b].cmax = &e->d_eb[b].cmax;
-        HIPCHK(hipMemcpy(e->d_ma, v.data(), v.size() * sizeof v[0], hipMemcpyHostToDevice));
-    } else {
-        auto v = make_args<float>(e, L, nullptr);
-        for (int b = 0; b < e->nbox; ++b) v[b].cmax = &e->d_eb[b].cmax;
-        HIPCHK(hipMemcpy(e->d_ma, v.data(), v.size() * sizeof v[0], hipMemcpyHostToDevice));
+    if (int err = e->prec == 8 ? upload_args<double>(e, L, &ma) : upload_args<float>(e, L, &ma)) {
+        (void)hipFree(tiles);
+        return err;
     }
+    if (e->d_tiles) (void)hipFree(e->d_tiles);
+    if (e->d_ma) (void)hipFree(e->d_ma);
+    e->d_tiles = tiles;
+    e->d_ma = ma;
     e->zchunk = zreq; e->persistent = persistent; e->order = ord;
     e->total = L.total;
     e->grid = grid_of(e, L.total, persistent);
@@ -419,7 +434,6 @@ glm_ens* glm_ens_create(int nbox, const glm_ens_box* boxes, const glm_params* sc
     e->clock_khz = khz > 0 ? (double)khz : 100000.0;
     const size_t logn = (size_t)ENS_LOG * nbox;
     if (hipMalloc(&e->d_eb, nbox * sizeof(EnsBox)) != hipSuccess ||
-        hipMalloc(&e->d_ma, nbox * ma_bytes(precision)) != hipSuccess ||
         hipMalloc(&e->d_ou, nbox * sizeof(OUBox)) != hipSuccess ||
         hipMalloc(&e->d_queue, NXCD * sizeof(unsigned int)) != hipSuccess ||
         hipMalloc(&e->d_sweep, sizeof(long long)) != hipSuccess ||

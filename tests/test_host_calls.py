@@ -43,3 +43,49 @@ def test_a_new_contexts_slots_are_zero_on_every_stream():
     at = [i for i, x in enumerate(log) if x.startswith("memset")]
     assert at and any(x in ("sync (nil)", "sync device") for x in log[at[-1] + 1:])
     h.lib.glm_destroy(ctx)
+
+
+def boxes(n=3, edge=32):
+    out = (_lib.GLMEnsBox * n)()
+    for b, x in enumerate(out):
+        x.nx = x.ny = x.nz = edge
+        for v in range(9):
+            x.u0[v], x.u1[v] = 0x20000000 + 0x1000000 * b + 0x10000 * v, 0x40000000 + 0x1000000 * b + 0x10000 * v
+        x.boxlen, x.courant, x.ch_scale, x.turb_T = 1.0, 0.3, 0.25, 1.0
+    return out
+
+
+def ensemble(h, bx):
+    e = h.lib.glm_ens_create(len(bx), bx, C.byref(step_args(Params(N=32, nz=32), 1.0, 0.0)), 8)
+    assert e
+    return e
+
+
+def march(line):
+    m = re.search(r"boxes (\S+) tiles (\S+) total (\d+)", line)
+    return int(m[1], 16), int(m[2], 16), int(m[3])
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("call", [("hipMalloc", 1), ("hipMalloc", 2), ("hipMemcpy", 1), ("hipMemcpy", 2)])
+def test_a_failed_configure_leaves_the_ensemble_as_it_was(call, graph):
+    """The next sweep runs the old layout, whose tables are still allocated and of its size."""
+    h = Host()
+    bx = boxes()
+    e = ensemble(h, bx)
+    if graph:
+        assert h.lib.glm_ens_graph(e, 1) == 0
+    assert h.lib.glm_ens_step(e, 1) == 0
+    before = march([x for x in h.log() if "ens_march" in x][-1])
+    h.fail(*call)
+    assert h.lib.glm_ens_configure(e, 1, 0, 1) != 0
+    assert h.lib.glm_ens_step(e, 1) == 0
+    after = march([x for x in h.log() if "ens_march" in x][-1])
+    assert after == before
+    assert h.lib.fh_live(after[0]) > 0 and h.lib.fh_live(after[1]) == 8 * after[2]
+    # and a configure that succeeds replaces them
+    assert h.lib.glm_ens_configure(e, 1, 0, 1) == 0
+    assert h.lib.glm_ens_step(e, 1) == 0
+    new = march([x for x in h.log() if "ens_march" in x][-1])
+    assert new[2] > before[2] and h.lib.fh_live(new[1]) == 8 * new[2] and h.lib.fh_live(new[0]) > 0
+    h.lib.glm_ens_destroy(e)
