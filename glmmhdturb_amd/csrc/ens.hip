@@ -38,7 +38,8 @@ constexpr int ENS_MAX_BOXES = 1024;
 template <typename T>
 __global__ void __launch_bounds__(ENS_MAX_BOXES) ens_ctl_kernel(EnsBox* eb, MarchArgs<T>* ma, OUBox* ou, int nbox,
                                                                 long long* sweep, unsigned int* queue, double* log,
-                                                                unsigned long long* t0, unsigned long long* t1)
+                                                                unsigned long long* t0, unsigned long long* t1,
+                                                                int* host_parity)
 {
     __shared__ long long s_sw;
     if (threadIdx.x == 0) {
@@ -85,7 +86,8 @@ __global__ void __launch_bounds__(ENS_MAX_BOXES) ens_ctl_kernel(EnsBox* eb, Marc
     m.glm_fac = (T)fac;
     m.ramp = (T)ramp;
     m.dt = (T)dt;
-    e.parity = 1 - par;
+    e.parity = 1 - par;   // every box starts at 0 and flips in each sweep
+    if (b == 0) __hip_atomic_store(host_parity, 1 - par, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     e.t = t + dt;
     e.nstep += 1;
     double* lg = log + ((size_t)slot * nbox + b) * 8;
@@ -138,7 +140,7 @@ struct glm_ens {
     int total, grid;
     // graph
     int use_graph;
-    long long enqueued;    // sweeps enqueued since the last reset: each flips every box's buffers
+    int* h_parity;         // pinned and device-mapped: the buffers' parity, by the step control
     hipGraph_t graph;
     hipGraphExec_t exec;
 };
@@ -158,6 +160,7 @@ void ens_free(glm_ens* e)
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (OUBox& o : e->ou) ou_box_free(o);
+    if (e->h_parity) (void)hipHostFree(e->h_parity);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
 }
@@ -341,11 +344,11 @@ int enqueue_sweep(glm_ens* e)
     if (e->prec == 8) {
         hipLaunchKernelGGL((ens_ctl_kernel<double>), dim3(1), dim3(nt), 0, e->stream, e->d_eb,
                            (MarchArgs<double>*)e->d_ma, e->d_ou, e->nbox, e->d_sweep, e->d_queue, e->d_log, e->d_t0,
-                           e->d_t1);
+                           e->d_t1, e->h_parity);
     } else {
         hipLaunchKernelGGL((ens_ctl_kernel<float>), dim3(1), dim3(nt), 0, e->stream, e->d_eb,
                            (MarchArgs<float>*)e->d_ma, e->d_ou, e->nbox, e->d_sweep, e->d_queue, e->d_log, e->d_t0,
-                           e->d_t1);
+                           e->d_t1, e->h_parity);
     }
     HIPCHK(hipGetLastError());
     if (e->any_turb) HIPCHK(launch_ou_advance(e->prec, e->d_ou, e->nbox, e->gmax, e->nbmax, -1, e->stream));
@@ -439,7 +442,8 @@ glm_ens* glm_ens_create(int nbox, const glm_ens_box* boxes, const glm_params* sc
         hipMalloc(&e->d_sweep, sizeof(long long)) != hipSuccess ||
         hipMalloc(&e->d_log, logn * 8 * sizeof(double)) != hipSuccess ||
         hipMalloc(&e->d_t0, logn * sizeof(unsigned long long)) != hipSuccess ||
-        hipMalloc(&e->d_t1, logn * sizeof(unsigned long long)) != hipSuccess)
+        hipMalloc(&e->d_t1, logn * sizeof(unsigned long long)) != hipSuccess ||
+        hipHostMalloc((void**)&e->h_parity, sizeof(int), hipHostMallocMapped) != hipSuccess)
         return fail(GLM_ERR_ALLOC, "glm_ens_create: device allocation failed");
     e->gmax = 2; e->nbmax = 1;
     for (int b = 0; b < nbox; ++b) {
@@ -490,6 +494,7 @@ int glm_ens_reset(glm_ens* e)
         }
     }
     HIPCHK(hipMemcpy(e->d_eb, eb.data(), eb.size() * sizeof(EnsBox), hipMemcpyHostToDevice));
+    *e->h_parity = 0;
     HIPCHK(hipMemcpyAsync(e->d_ou, e->ou.data(), e->nbox * sizeof(OUBox), hipMemcpyHostToDevice, e->stream));
     const long long minus1 = -1;
     HIPCHK(hipMemcpyAsync(e->d_sweep, &minus1, sizeof minus1, hipMemcpyHostToDevice, e->stream));
@@ -502,7 +507,6 @@ int glm_ens_reset(glm_ens* e)
     if (e->prec == 8) hipLaunchKernelGGL((ens_ctot_kernel<double>), grid, dim3(256), 0, e->stream, e->d_eb, (const MarchArgs<double>*)e->d_ma);
     else hipLaunchKernelGGL((ens_ctot_kernel<float>), grid, dim3(256), 0, e->stream, e->d_eb, (const MarchArgs<float>*)e->d_ma);
     HIPCHK(hipGetLastError());
-    e->enqueued = 0;
     HIPCHK(hipStreamSynchronize(e->stream));
     return GLM_OK;
 }
@@ -516,7 +520,6 @@ int glm_ens_step(glm_ens* e, int nsweeps)
             int err = enqueue_sweep(e);
             if (err) return err;
         }
-        e->enqueued += 1;
     }
     return GLM_OK;
 }
@@ -557,7 +560,7 @@ int glm_ens_current(glm_ens* e, int box, void** planes)
 {
     if (!e || !planes || box < 0 || box >= e->nbox) return set_err(GLM_ERR_ARG, "glm_ens_current: bad argument");
     HIPCHK(hipStreamSynchronize(e->stream));
-    const int par = (int)(e->enqueued & 1);   // the step control starts at u0 and flips every box in each sweep
+    const int par = *(volatile int*)e->h_parity;
     for (int v = 0; v < 9; ++v) planes[v] = par ? e->box[box].u1[v] : e->box[box].u0[v];
     return GLM_OK;
 }

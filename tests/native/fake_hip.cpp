@@ -202,7 +202,7 @@ hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void** args, size_t, hip
     } else if (clear) {
         memset(*(void**)args[0], 0, 8 * (size_t) * (int*)args[1]);
     } else if (control) {
-        *(*(long long**)args[4]) += 1;   // the sweep number
+        **(int**)args[9] = (int)(++**(long long**)args[4] + 1) & 1;   // the sweep number, and the buffers' parity
     }
     return hipSuccess;
 }

@@ -89,3 +89,21 @@ def test_a_failed_configure_leaves_the_ensemble_as_it_was(call, graph):
     new = march([x for x in h.log() if "ens_march" in x][-1])
     assert new[2] > before[2] and h.lib.fh_live(new[1]) == 8 * new[2] and h.lib.fh_live(new[0]) > 0
     h.lib.glm_ens_destroy(e)
+
+
+def test_current_buffers_are_the_devices_after_a_failed_sweep():
+    """The step control has flipped the buffers when the march behind it cannot be launched."""
+    h = Host()
+    bx = boxes(2)
+    e = ensemble(h, bx)
+    out, _ = _lib.plane_array([0] * 9)
+    for sweep in range(3):
+        h.fail("hipLaunchKernel", 1 + sweep % 2)   # the control, the march, the control
+        assert h.lib.glm_ens_step(e, 1) != 0
+        n = h.lib.glm_ens_sweeps(e)
+        assert n == (0, 1, 1)[sweep]
+        for b in range(2):
+            assert h.lib.glm_ens_current(e, b, out) == 0
+            assert list(out) == list(bx[b].u1 if n % 2 else bx[b].u0)
+    assert h.lib.glm_ens_reset(e) == 0 and h.lib.glm_ens_current(e, 0, out) == 0 and list(out) == list(bx[0].u0)
+    h.lib.glm_ens_destroy(e)
