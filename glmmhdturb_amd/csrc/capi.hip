@@ -90,13 +90,16 @@ static int resident_of(const void* fn, int threads, int key, ResidentOf& out)
     return GLM_OK;
 }
 
+// Where in h_out a call's result arrives: words of its own, as its caller's memory was.
+enum HostWord { OUT_DIAG = 0, OUT_CFL = GLM_NDIAG, OUT_REDUCTION, OUT_FDOT, OUT_WORDS };
+
 struct glm_ctx {
     int nx, ny, nz, prec;
     size_t n;
     hipStream_t stream;
     unsigned long long* d_cmax;  // [0],[1] march CFL ping-pong, [2] CT step CFL, [3] standalone reductions
     bool red_dirty;              // slot 3 may hold a value: a reduction was started and not read back
-    unsigned long long* h_out;   // pinned and device-mapped: results of the calls that wait for them
+    unsigned long long* h_out;   // pinned and device-mapped: results of the calls that wait for them (HostWord)
     int cfl_parity;              // slot the next march step accumulates into
     int cfl_slot;                // slot holding the CFL max of the last step with want_cfl (-1: none)
     void* d_parts;
@@ -128,11 +131,11 @@ static void ctx_free(glm_ctx* c)
 
 // Wait for the context's stream and return the 8 bytes of a device slot; clear: zero the slot behind them.
 // (An 8-byte hipMemcpyAsync to the caller's memory took about 6 us more than the one-lane kernel.)
-static int read_slot(glm_ctx* c, unsigned long long* slot, bool clear, double* out)
+static int read_slot(glm_ctx* c, unsigned long long* slot, bool clear, HostWord word, double* out)
 {
-    HIPCHK(launch_publish_u64(slot, c->h_out, clear, c->stream));
+    HIPCHK(launch_publish_u64(slot, c->h_out + word, clear, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    memcpy(out, c->h_out, sizeof *out);
+    memcpy(out, c->h_out + word, sizeof *out);
     return GLM_OK;
 }
 
@@ -145,7 +148,7 @@ static int begin_reduction(glm_ctx* c)
 }
 static int end_reduction(glm_ctx* c, double* out)
 {
-    if (int e = read_slot(c, c->d_cmax + 3, true, out)) return e;
+    if (int e = read_slot(c, c->d_cmax + 3, true, OUT_REDUCTION, out)) return e;
     c->red_dirty = false;
     return GLM_OK;
 }
@@ -194,7 +197,7 @@ glm_ctx* glm_create(int nx, int ny, int nz, int precision)
     c->cfl_slot = -1;
     if (hipMalloc(&c->d_cmax, 4 * sizeof(unsigned long long)) != hipSuccess ||
         hipMalloc(&c->d_parts, np * diag_part_bytes()) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_out, GLM_NDIAG * sizeof(double), hipHostMallocMapped) != hipSuccess) {
+        hipHostMalloc((void**)&c->h_out, OUT_WORDS * sizeof(double), hipHostMallocMapped) != hipSuccess) {
         set_err(GLM_ERR_ALLOC, "glm_create: allocation failed");
         ctx_free(c);
         return nullptr;
@@ -308,7 +311,7 @@ int glm_cfl_max(glm_ctx* ctx, double* cmax)
 {
     if (!ctx || !cmax) return set_err(GLM_ERR_ARG, "glm_cfl_max: null argument");
     if (ctx->cfl_slot < 0) return set_err(GLM_ERR_STATE, "glm_cfl_max: no step with want_cfl has run");
-    return read_slot(ctx, ctx->d_cmax + ctx->cfl_slot, false, cmax);
+    return read_slot(ctx, ctx->d_cmax + ctx->cfl_slot, false, OUT_CFL, cmax);
 }
 
 }  // extern "C"
@@ -370,11 +373,11 @@ int glm_diagnostics(glm_ctx* ctx, void* const* q, const glm_params* p, double* o
     if (!e) e = check_params(p);
     if (e) return e;
     if (ctx->prec == 8)
-        HIPCHK(launch_diag<double>(cptr9<double>(q), ctx->nx, ctx->ny, ctx->nz, p->dx, p->smallr, ctx->d_parts, (double*)ctx->h_out, ctx->stream));
+        HIPCHK(launch_diag<double>(cptr9<double>(q), ctx->nx, ctx->ny, ctx->nz, p->dx, p->smallr, ctx->d_parts, (double*)(ctx->h_out + OUT_DIAG), ctx->stream));
     else
-        HIPCHK(launch_diag<float>(cptr9<float>(q), ctx->nx, ctx->ny, ctx->nz, p->dx, p->smallr, ctx->d_parts, (double*)ctx->h_out, ctx->stream));
+        HIPCHK(launch_diag<float>(cptr9<float>(q), ctx->nx, ctx->ny, ctx->nz, p->dx, p->smallr, ctx->d_parts, (double*)(ctx->h_out + OUT_DIAG), ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    memcpy(out, ctx->h_out, GLM_NDIAG * sizeof(double));
+    memcpy(out, ctx->h_out + OUT_DIAG, GLM_NDIAG * sizeof(double));
     return GLM_OK;
 }
 
@@ -565,7 +568,7 @@ int glm_adjoint_force_dot(glm_ctx* ctx, int reset, double* out)
     if (!ctx || !out) return set_err(GLM_ERR_ARG, "glm_adjoint_force_dot: null argument");
     *out = 0.0;
     if (!ctx->d_fdot) return GLM_OK;
-    return read_slot(ctx, (unsigned long long*)ctx->d_fdot, reset != 0, out);
+    return read_slot(ctx, (unsigned long long*)ctx->d_fdot, reset != 0, OUT_FDOT, out);
 }
 
 // CT step paths: the multi-pass kernel sequence, the fused z-march, the staged 3-D tiles.

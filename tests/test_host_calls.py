@@ -107,3 +107,23 @@ def test_current_buffers_are_the_devices_after_a_failed_sweep():
             assert list(out) == list(bx[b].u1 if n % 2 else bx[b].u0)
     assert h.lib.glm_ens_reset(e) == 0 and h.lib.glm_ens_current(e, 0, out) == 0 and list(out) == list(bx[0].u0)
     h.lib.glm_ens_destroy(e)
+
+
+def test_waiting_calls_return_through_words_of_their_own():
+    """Two threads that wait for different results of one context do not get each other's."""
+    h = Host()
+    start = len(h.log())
+    ctx = h.lib.glm_create(16, 16, 16, 8)
+    mapped = [x.split() for x in h.log(start) if x.startswith("malloc")][-1]
+    base, size = int(mapped[1], 16), int(mapped[2])
+    a = step_args(Params(N=16, nz=16, gamma=1.4), 1e-3, 0.0, want_cfl=True)
+    out = C.c_double()
+    assert h.lib.glm_step(ctx, planes(), planes(base=0x30000000), C.byref(a)) == 0
+    assert h.lib.glm_cfl_max(ctx, C.byref(out)) == 0
+    assert h.lib.glm_ctot_max(ctx, planes(), C.byref(a), C.byref(out)) == 0
+    assert h.lib.glm_step_adjoint(ctx, planes(), planes(base=0x30000000), planes(base=0x50000000), C.byref(a), None) == 0
+    assert h.lib.glm_adjoint_force_dot(ctx, 1, C.byref(out)) == 0
+    words = [int(x.split("host ")[1], 16) for x in h.log() if "publish_u64" in x]
+    assert len(set(words)) == len(words) == 3
+    assert all(base + 8 * _lib.NDIAG <= w <= base + size - 8 for w in words)   # behind the diagnostics
+    h.lib.glm_destroy(ctx)
