@@ -13,12 +13,17 @@ namespace glm {
 
 // Gas pressure (gamma-1)(E - rho v^2/2 - B^2/2), floored (ct_mhd.jl:26-34).  With FP32 state the
 // subtraction is carried out in FP64, as in the GLM path: E can be dominated by the kinetic or
-// magnetic part.
+// magnetic part.  The fused operations are written out and no others are made: the pressure has the same bits
+// at every place the march takes it (its window's first planes and its loop, near and wide planes), which
+// chunk lengths must not show.
 template <typename T>
 GLM_DEV T ct_pressure(T E, T rho, T vx, T vy, T vz, T bx, T by, T bz, T gamma, T smallp)
 {
+#pragma clang fp contract(off)
     const double r = rho, u = vx, v = vy, w = vz, b1 = bx, b2 = by, b3 = bz;
-    const double e = (double)E - 0.5 * r * (u * u + v * v + w * w) - 0.5 * (b1 * b1 + b2 * b2 + b3 * b3);
+    const double vv = __builtin_fma(w, w, __builtin_fma(v, v, u * u));
+    const double bb = __builtin_fma(b3, b3, __builtin_fma(b2, b2, b1 * b1));
+    const double e = __builtin_fma(-0.5, bb, __builtin_fma(-0.5 * r, vv, (double)E));
     return tmax((T)(((double)gamma - 1.0) * e), smallp);
 }
 
