@@ -25,4 +25,15 @@ hipError_t launch_adj_front_pr<GLM_PRED, GLM_RIEM>(const MarchArgs<double>& m, c
     return hipErrorInvalidValue;
 }
 
+template <>
+const void* adj_front_ptr_pr<GLM_PRED, GLM_RIEM>(int recon, int slope)
+{
+#define GLM_CASE(RC, SL) \
+    if (recon == RC && slope == SL) return (const void*)&adj_front_kernel<GLM_PRED, GLM_RIEM, RC, SL>;
+    GLM_CASE(RECON_PLM, SLOPE_MONCEN) GLM_CASE(RECON_PPM, SLOPE_MONCEN)
+    GLM_CASE(RECON_PLM, SLOPE_MINMOD) GLM_CASE(RECON_PPM, SLOPE_MINMOD)
+#undef GLM_CASE
+    return nullptr;
+}
+
 }  // namespace glm

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include "physics.hpp"
+#include "tiling.hpp"
 
 namespace glm {
 
@@ -36,12 +37,23 @@ struct MarchArgs;
 // One (predictor, Riemann) family of front kernels (adj_front.hpp), built from adj_front_inst.hip.
 template <int PRED, int RIEM>
 hipError_t launch_adj_front_pr(const MarchArgs<double>& m, const AdjArgs& a, int recon, int slope, hipStream_t st);
+template <int PRED, int RIEM>
+const void* adj_front_ptr_pr(int recon, int slope);   // the kernel (occupancy queries)
+
+// Concurrent workgroups of a scheme's reverse kernels on the present device (the front half, the back half,
+// the HLLD adjoint) and the modelled chunk lengths of the two marches on a grid.
+struct AdjResident {
+    Resident front, back, hlld;
+    int zfront, zback;
+};
+hipError_t adj_resident(int nx, int ny, int nz, int pred, int riem, int recon, int slope, AdjResident& out);
+
 // Launch the reverse step and add the step's sum of (kick acceleration adjoint . acceleration)
 // to *fdot (device).  With fused, the face-state and predictor adjoints and the gather run as one
 // z-march kernel (adj_march.hpp, z planes per tile: zchunk, 0 = the occupancy model) where a z plane
 // of the scratch is below 4 GiB; otherwise as the separate passes 5 and 6.  a.scr and a.part must come
 // from a scratch of adj_scratch_bytes(n).  Returns hipErrorInvalidValue for an unsupported scheme.
-hipError_t launch_step_adjoint(AdjArgs a, void* scratch, int pred, int riem, int recon, int slope, double* fdot,
-                               bool fused, int zchunk, hipStream_t st);
+hipError_t launch_step_adjoint(AdjArgs a, const AdjResident& r, void* scratch, int pred, int riem, int recon,
+                               int slope, double* fdot, bool fused, int zchunk, hipStream_t st);
 
 }  // namespace glm

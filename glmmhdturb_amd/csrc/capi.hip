@@ -116,6 +116,8 @@ struct glm_ctx {
     double* d_fdot;
     // concurrent march workgroups of the last march variant of each kind
     ResidentOf march_res, ct_res, hydro_res;
+    int adj_key;                 // the reverse step's scheme adj_res was asked for (0: none yet)
+    AdjResident adj_res;
 };
 
 static void ctx_free(glm_ctx* c)
@@ -544,7 +546,14 @@ static int step_adjoint_impl(glm_ctx* ctx, void* const* u0, void* const* lam1, v
     a.mh_revert = p->mh_revert; a.face_guard = p->face_guard; a.update_floor = p->update_floor;
     a.do_turb = p->do_turb;
     a.afield = (const double*)afield;
-    hipError_t he = launch_step_adjoint(a, ctx->adj_scratch, p->predictor, p->riemann, p->recon, p->slope, ctx->d_fdot,
+    const int key = 1 + ((p->predictor * 4 + p->riemann) * 4 + p->recon) * 4 + p->slope;
+    if (ctx->adj_key != key) {
+        const hipError_t re = adj_resident(a.nx, a.ny, a.nz, p->predictor, p->riemann, p->recon, p->slope, ctx->adj_res);
+        if (re == hipErrorInvalidValue) return set_err(GLM_ERR_ARG, "glm_step_adjoint: unsupported scheme");
+        HIPCHK(re);
+        ctx->adj_key = key;
+    }
+    hipError_t he = launch_step_adjoint(a, ctx->adj_res, ctx->adj_scratch, p->predictor, p->riemann, p->recon, p->slope, ctx->d_fdot,
                                         fused, p->zchunk, ctx->stream);
     if (he == hipErrorInvalidValue) return set_err(GLM_ERR_ARG, "glm_step_adjoint: unsupported scheme");
     HIPCHK(he);

@@ -127,3 +127,18 @@ def test_waiting_calls_return_through_words_of_their_own():
     assert len(set(words)) == len(words) == 3
     assert all(base + 8 * _lib.NDIAG <= w <= base + size - 8 for w in words)   # behind the diagnostics
     h.lib.glm_destroy(ctx)
+
+
+def test_the_reverse_step_fits_the_device_it_finds():
+    """Fewer CUs: the HLLD adjoint's grid is what is resident, the marches take longer chunks."""
+    grids = {}
+    for cus in (256, 64):
+        h = Host(cus, 1)
+        ctx = h.lib.glm_create(64, 64, 64, 8)
+        a = step_args(Params(N=64, nz=64, gamma=1.4), 1e-3, 0.0, riemann="hlld", recon="ppm")
+        assert h.lib.glm_step_adjoint(ctx, planes(), planes(base=0x30000000), planes(base=0x50000000), C.byref(a), None) == 0
+        for k in ("adj_riemann", "adj_front", "adj_back"):
+            grids[k, cus] = int(re.search(r"grid (\d+)", [x for x in h.log() if k in x][-1])[1])
+        h.lib.glm_destroy(ctx)
+    assert grids["adj_riemann", 256] == 256 and grids["adj_riemann", 64] == 64
+    assert grids["adj_front", 64] < grids["adj_front", 256] and grids["adj_back", 64] < grids["adj_back", 256]
