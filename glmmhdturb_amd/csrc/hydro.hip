@@ -93,7 +93,7 @@ hipError_t launch_hydro_march(void* const* q, void* const* o, const HydroArgsHos
     a.nx = h.nx; a.ny = h.ny; a.nz = h.nz;
     hydro_tiling<T>(h.nx, h.ny, h.nz, h.zchunk, res, a.tiles_x, a.tiles_y, a.nzc, a.zchunk);
     a.gamma = (T)h.gamma; a.gm1 = (T)(h.gamma - 1.0); a.igm1 = (T)(1.0 / (h.gamma - 1.0));
-    a.dtdx = (T)h.dtdx; a.half_dtdx = (T)(0.5 * h.dtdx);
+    a.dtdx = (T)h.dtdx;
     a.smallr = (T)h.smallr; a.smallp = (T)h.smallp;
     a.fb_dmin = (T)h.fb_dmin; a.fb_pmin = (T)h.fb_pmin;
     const long nblk = (long)a.tiles_x * a.tiles_y * a.nzc;

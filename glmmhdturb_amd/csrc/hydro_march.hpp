@@ -63,7 +63,7 @@ struct HydroArgs {
     unsigned short* oh[HM_NVMAX];
     int nx, ny, nz;
     int tiles_x, tiles_y, nzc, zchunk;
-    T gm1, igm1, gamma, dtdx, half_dtdx, smallr, smallp, fb_dmin, fb_pmin;
+    T gm1, igm1, gamma, dtdx, smallr, smallp, fb_dmin, fb_pmin;
 };
 
 // uint16 codecs (spike_25d.cu:157-168): log2 over [-110, 0] (species), velocity linear over
