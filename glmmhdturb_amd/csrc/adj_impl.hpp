@@ -32,7 +32,8 @@ struct Cell {
 };
 // Scratch index: the ADJ_NPLANES values of a cell row lie together, row by row.  As planes of n cells the
 // 60 to 120 streams of a pass were as many pages, and every access of a wavefront a translation of its
-// own: the Riemann adjoint took 618 us at 128^3 (505 now), the reverse step as a whole 6% more.
+// own: at 128^3 the Riemann adjoint took 618 us instead of 505 (before its loads were requested ahead), the reverse step
+// as a whole 6% more.
 GLM_DEV size_t adj_index(const AdjArgs& a, int i, int j, int k)
 {
     return (size_t)i + (size_t)a.nx * ADJ_NPLANES * ((size_t)j + (size_t)a.ny * k);

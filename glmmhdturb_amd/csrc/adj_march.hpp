@@ -31,7 +31,7 @@ namespace glm {
 
 // Workgroups a CU (wavefronts a SIMD).  The normal-only predictor couples the variables of each
 // direction's face states, does not fit 256 registers and is faster with 512 (its reverse step with PPM
-// + MonCen at 128^3: 2.05 against 3.03 ms; with the full predictor 2.30 against 2.09).
+// and HLLD at 128^3: 1.62 against 2.64 ms).  The full predictor's fits and needs no second half (1.59).
 constexpr int adj_waves(int pred) { return pred == PRED_FULL ? 2 : 1; }
 constexpr int ADJ_GRP = 2;     // variables in work at a time
 // LDS rows: odd pitches, so that the ring's columns (one lane a row) fall on different banks.

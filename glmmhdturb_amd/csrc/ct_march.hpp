@@ -112,12 +112,14 @@ struct CTMarchLDS {
 
 // A column (x, y) of the grid and the byte offsets, within a z plane, of its cells and of their upper x
 // and y neighbours, for planes below 4 GiB: the plane's base is one for the wavefront and an access adds
-// its offset itself.  (64-bit lane addresses, a multiplication or two and an addition each, were 4% of a
-// plane's instructions: the HLLD + PLM step at 256^3 FP64 2.43 -> 2.24 ms.)  Where the offsets are used
-// (192^3, us with 64-bit addresses and with offsets): FP64 PLM HLLD 886 -> 829 (HLL 632 -> 633); FP32 PLM
-// HLLD 416 -> 415, PPM HLL 374 -> 347, PPM HLLD 486 -> 448.  Not in the FP64 builds at one wavefront a SIMD,
-// which have the registers and wait longer for the pointers (PPM HLL 924 -> 985, HLLD 1097 -> 1125; species
-// HLL 1018 -> 1078, HLLD 1148 -> 1218), nor for FP32 PLM HLL (324 -> 327) and species (HLLD 521 -> 526).
+// its offset itself, where 64-bit lane addresses take a multiplication or two and an addition each.  256^3 in
+// us with 64-bit addresses and with offsets, for LLF, HLL and HLLD:
+//   used:      FP64 PLM 1558, 1589, 2146 -> 1529, 1543, 1977
+//              FP32 PPM 1094, 1102, 1242 -> 948, 958, 1091; FP32 PLM HLLD 1069 -> 1025
+//   not used:  FP32 PLM LLF and HLL 870, 856 -> 907, 906; with species 1254, 1262, 1348 -> 1272, 1284, 1405
+//              FP64 PPM 2362, 2410, 2718 -> 2509, 2577, 2907; PLM with species 2498, 2523, 2823 -> 2646, 2661, 3003
+// (the FP64 builds not using them run one wavefront a SIMD, have the registers and wait longer for the
+// pointers).  64^3 to 192^3 are on the same side, or within 1% of the line.
 template <typename T, int RIEM, int NS, int RC>
 constexpr bool CM_OFFSETS = NS == 0 && (sizeof(T) == 8 ? RC == RECON_PLM : RIEM == RIEM_HLLD || RC != RECON_PLM);
 struct CmColumn {
@@ -240,8 +242,8 @@ ct_march_kernel(CTMArgs<T> a_)
     const CmColumn col = cm_column<T>(gx, gy, nx, ny);
     const int lo = (ty + 1) * CM_PX + (tx + 1);
     const int li = ty * CM_LX + tx;
-    const bool helper = tid >= CM_NO;   // the halo wavefront, which has no update, brings in the two-cell ring (when
-                                        // the first owned one did: 2.70 ms at 256^3 FP64, now 2.46)
+    const bool helper = tid >= CM_NO;   // the halo wavefront, which has no update, brings in the two-cell ring (by
+                                        // the first owned one the HLLD + PLM step at 256^3 FP64 took 10% longer)
     int hx = 0, hy = 0;
     cm_helper_cell(helper ? tid - CM_NO : 0, hx, hy);
     const CmColumn hcol =

@@ -247,7 +247,8 @@ GLM_HD double fast_speed(double rho, double p, double b2, double bn, const Phys<
 }
 // The larger of two states' fast speeds with a common normal field (HLLD's): one outer root, of the larger
 // square; in FP64 no reciprocal either: with N/D the larger square over the common denominator,
-// sqrt(N/D) = N / sqrt(N D), from the reciprocal square root estimate and one Goldschmidt step.
+// sqrt(N/D) = N / sqrt(N D), from the reciprocal square root estimate and one Goldschmidt step.  N D is of the size of
+// p rho^3, so densities and pressures may reach 1e75 together (hlld_x has floors of its own at 1e-12).
 template <typename T>
 GLM_HD T fast_speed_sq(T rho, T p, T b2, T bn, const Phys<T>& s)
 {
