@@ -22,7 +22,7 @@
 //   y: four cells' states and three faces for a lane's two rows, from the LDS plane;
 //   z: one cell's states and one face per plane and row; the upper state is carried to the next plane.
 // Per owned cell that is 4 slopes and half steps and 3.5 solves (times 32/30), where a lane per column
-// with both its faces in each direction took 8 and 5: 480^3 FP32 2.52 -> 1.90 ms.
+// with both its faces in each direction took 8 and 5: 480^3 FP32 2.52 -> 1.90 ms (1.99 with the flux sums below).
 //   LDS holds the primitives of planes k and k+1 over the tile grown by two cells (34 x 20): a lane's own
 // cells reach plane k+2 in registers, the halo's plane k+1 is fetched during plane k, so one barrier
 // per plane suffices.  The loop starts two planes early so that the chunk's first z states and face
@@ -302,11 +302,11 @@ inline void hydro_tiling(int nx, int ny, int nz, int zchunk_req, const Resident&
     march_tiles(nx, ny, nz, HM_OX, HM_OY, zchunk_req, r, 0.7, sizeof(T) == 8 ? 0.9 : 0.6, tiles_x, tiles_y, nzc, zchunk);
 }
 
-// Resident wavefronts per SIMD that the register allocation is held to.  FP32: 3 (168 registers, no
-// spills; at 4, 128 registers with 20 B of spills, 480^3 took 2.01 ms instead of 1.90, the fallback build
-// 2.63 instead of 1.97), with scalars 2 (2.58 ms; 3 with 36 B of spills 2.89).  FP64: 2 (3.58 ms; the
-// fallback build with 60 B of spills 4.21, at one wavefront 4.11), with scalars or donor seams, which
-// would spill 136-550 B at 256 registers, 1 (scalars 5.11 ms, at two 9.86; donor 3.72, at two 6.05).
+// Resident wavefronts per SIMD that the register allocation is held to (480^3).  FP32: 3 (144 to 168 registers,
+// no spills, 2.09 ms; at 4, 128 registers with 76 B of spills, 2.55), with scalars 2 (2.83 ms; 3 with 108 B of
+// spills 3.60).  FP64: 2 (4.23 ms, at one 4.57; with the fallback 4.38 and 4.74, PPM1D 5.57 and 5.79), with
+// scalars or donor seams, which would spill 140-552 B at 256 registers, 1 (scalars 5.9 ms, at two 9.7; donor
+// 4.8, at two 6.5).
 #ifndef GLM_HY_WAVES
 #define GLM_HY_WAVES(T, NSP, SV) (sizeof(T) == 8 ? ((NSP) || (SV) == HY_DONOR ? 1 : 2) : ((NSP) ? 2 : 3))
 #endif
