@@ -82,10 +82,17 @@ hipError_t launch_ou_advance(int prec, const OUBox* d_boxes, int nbox, int gmax,
     dim3 bl(256);
     hipLaunchKernelGGL(ou_band_step_kernel, dim3(blocks_for(nb * nb * nb, nbox), nbox), bl, 0, st, d_boxes, step_all);
     hipLaunchKernelGGL(ou_pass_x_kernel, dim3(blocks_for(3 * nb * nb * g, nbox), nbox), bl, 0, st, d_boxes, step_all);
-    // one plane of the y and z passes in LDS where its nb x g complex values fit (kmax 3 on a 64^3 forcing
-    // grid: 7 KB); the separate passes for wide bands on large grids
+    // The y and z passes as one kernel, a workgroup a plane, where a plane's nb x g complex values fit LDS and either
+    // the planes fill the device or a plane has so few terms that the launch saved is the larger part.  One kernel
+    // against two, whole advances in us: 8 boxes on 64^3 with kmax 3: 70 against 117; two of them (384 planes, where
+    // the lines cross): 38 against 41, with kmax 16 218 against 197; one: 33.6 against 28.5, with kmax 16 186
+    // against 111.  One on 32^3 with kmax 3: 17.7 against 19.0, kmax 5 (15136 terms a plane): 26.5 against 24.1.
+    // An ensemble (step_all < 0) launches the passes in each sweep, due or not, so there the launch counts for more:
+    // one box of 32^3 with kmax 3 on 64^3 takes 33 us a sweep with one kernel and 35.6 with two, with kmax 16
+    // on a box of 64^3 117 and 104.
     const size_t lds = 2 * nb * g * sizeof(double);
-    if (lds <= 64 * 1024) {
+    const bool filled = 3 * g * nbox >= 384, few_terms = nb * g * (nb + g) <= (step_all < 0 ? 40000u : 10000u);
+    if (lds <= 64 * 1024 && (filled || few_terms)) {
         dim3 gp((unsigned)(3 * g), nbox);
         if (prec == 8) hipLaunchKernelGGL((ou_pass_yz_kernel<double>), gp, bl, lds, st, d_boxes, step_all);
         else hipLaunchKernelGGL((ou_pass_yz_kernel<float>), gp, bl, lds, st, d_boxes, step_all);

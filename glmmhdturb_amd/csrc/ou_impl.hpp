@@ -100,6 +100,11 @@ __global__ void ou_band_step_kernel(const OUBox* boxes, long long step_all)
     }
 }
 
+// (sr, si) += (xr, xi) * (cs, sn), with the fused operations written out: the passes below and the kernel that
+// joins two of them give the same bits, whichever a number of boxes takes.
+GLM_DEV double band_re(double sr, double xr, double xi, double cs, double sn) { return sr + fma(xr, cs, -(xi * sn)); }
+GLM_DEV double band_im(double si, double xr, double xi, double cs, double sn) { return si + fma(xi, cs, xr * sn); }
+
 // x pass: w1[c][ed][eb][i] = sum_ea F[c][ed][eb][ea] * exp(+2 pi i a i / g)
 __global__ void ou_pass_x_kernel(const OUBox* boxes, long long step_all)
 {
@@ -116,8 +121,8 @@ __global__ void ou_pass_x_kernel(const OUBox* boxes, long long step_all)
         double sr = 0.0, si = 0.0;
         for (int ea = 0; ea < nb; ++ea) {
             const int tw = (band_mode(ea, nb, K, g) * i) % g;
-            sr += xr[ea] * b.cs[tw] - xi[ea] * b.sn[tw];
-            si += xr[ea] * b.sn[tw] + xi[ea] * b.cs[tw];
+            sr = band_re(sr, xr[ea], xi[ea], b.cs[tw], b.sn[tw]);
+            si = band_im(si, xr[ea], xi[ea], b.cs[tw], b.sn[tw]);
         }
         b.w1r[t] = sr;
         b.w1i[t] = si;
@@ -140,8 +145,8 @@ __global__ void ou_pass_y_kernel(const OUBox* boxes, long long step_all)
         for (int eb = 0; eb < nb; ++eb) {
             const int tw = (band_mode(eb, nb, K, g) * j) % g;
             const double xr = b.w1r[base + (size_t)eb * g], xi = b.w1i[base + (size_t)eb * g];
-            sr += xr * b.cs[tw] - xi * b.sn[tw];
-            si += xr * b.sn[tw] + xi * b.cs[tw];
+            sr = band_re(sr, xr, xi, b.cs[tw], b.sn[tw]);
+            si = band_im(si, xr, xi, b.cs[tw], b.sn[tw]);
         }
         b.w2r[t] = sr;
         b.w2i[t] = si;
@@ -166,7 +171,7 @@ __global__ void ou_pass_z_kernel(const OUBox* boxes, long long step_all)
         for (int ed = 0; ed < nb; ++ed) {
             const int tw = (band_mode(ed, nb, K, g) * k) % g;
             const size_t at = (c * nb + ed) * gg + ij;
-            sr += b.w2r[at] * b.cs[tw] - b.w2i[at] * b.sn[tw];
+            sr = band_re(sr, b.w2r[at], b.w2i[at], b.cs[tw], b.sn[tw]);
         }
         af[t] = (T)(sr * b.scale);
     }
@@ -175,7 +180,8 @@ __global__ void ou_pass_z_kernel(const OUBox* boxes, long long step_all)
 // The y and z passes as one: a workgroup takes one (component, j) plane, sums w2[ed][i] for it into LDS and
 // the g x g outputs (k, i) from there, so w2 does not go through memory.  The twiddle index (mode * j) mod g
 // of successive modes is carried by addition (with a division per term the y and z passes of 16 boxes on 32^3..64^3
-// forcing grids took 125 us, now 75).  The sums run over the modes in the passes' order.
+// forcing grids took 125 us, now 75).  The sums run over the modes in the passes' order.  What bounds it with few
+// boxes is the number of planes: launch_ou_advance then takes the passes.
 template <typename T>
 __global__ void __launch_bounds__(256) ou_pass_yz_kernel(const OUBox* boxes, long long step_all)
 {
@@ -198,8 +204,8 @@ __global__ void __launch_bounds__(256) ou_pass_yz_kernel(const OUBox* boxes, lon
             for (int eb = 0; eb < nb; ++eb) {
                 if (eb == K + 1) tw = jump_j;
                 const double xr = b.w1r[base + (size_t)eb * g], xi = b.w1i[base + (size_t)eb * g];
-                sr += xr * b.cs[tw] - xi * b.sn[tw];
-                si += xr * b.sn[tw] + xi * b.cs[tw];
+                sr = band_re(sr, xr, xi, b.cs[tw], b.sn[tw]);
+                si = band_im(si, xr, xi, b.cs[tw], b.sn[tw]);
                 tw += j;
                 if (tw >= g) tw -= g;
             }
@@ -213,7 +219,7 @@ __global__ void __launch_bounds__(256) ou_pass_yz_kernel(const OUBox* boxes, lon
             int tw = 0;   // (band_mode(ed) * k) mod g
             for (int ed = 0; ed < nb; ++ed) {
                 if (ed == K + 1) tw = (int)(((size_t)band_mode(ed, nb, K, g) * k) % g);
-                sr += w2r[ed * g + i] * b.cs[tw] - w2i[ed * g + i] * b.sn[tw];
+                sr = band_re(sr, w2r[ed * g + i], w2i[ed * g + i], b.cs[tw], b.sn[tw]);
                 tw += k;
                 if (tw >= g) tw -= g;
             }

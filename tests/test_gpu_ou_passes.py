@@ -24,3 +24,19 @@ def test_ou_advance_matches_dense_transform(orc, g, kmax):
     got = s.afield().cpu().numpy().reshape(-1)
     # nb terms an axis, each within a few ulps of the largest partial sum
     assert np.max(np.abs(got - fo.afield)) <= 1e-13 * g * max(np.max(np.abs(fo.afield)), 1e-300)
+
+
+# separate passes for the box alone (96 or 192 planes of many terms), one kernel for the boxes together
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n,g,kmax", [(4, 32, 5.0), (4, 33, 16.0), (3, 64, 3.0), (2, 64, 31.0)])
+def test_a_box_alone_and_among_others_has_the_same_bits(n, g, kmax, prec):
+    from glmmhdturb_amd.ensemble import BoxSpec, Ensemble, single_box_run
+    boxes = [BoxSpec(N=8, seed=7 + b, amp=3e3, turb_gs=g, turb_kmax=kmax, turb_Ndt=20) for b in range(n)]
+    ens = Ensemble(boxes, precision=prec)
+    ens.step(5)
+    ens.sync()
+    log = ens.log(n - 1, 5)
+    assert log[0]["ou_due"] and log[4]["ramp"] > 0
+    _, u, _ = single_box_run(boxes[-1], ens.scheme, 5, prec, log=log)
+    assert torch.equal(ens.current(n - 1), u) and float(u[1].abs().max()) > 0
+    ens.close()

@@ -142,3 +142,26 @@ def test_the_reverse_step_fits_the_device_it_finds():
         h.lib.glm_destroy(ctx)
     assert grids["adj_riemann", 256] == 256 and grids["adj_riemann", 64] == 64
     assert grids["adj_front", 64] < grids["adj_front", 256] and grids["adj_back", 64] < grids["adj_back", 256]
+
+
+# (boxes, forcing grid, kmax, one kernel): few planes of many terms each: separate passes; enough planes, either side
+# of the line; planes of few terms, more of them in an ensemble; a plane past LDS
+@pytest.mark.parametrize("n,g,kmax,one", [(1, 64, 3.0, False), (1, 64, 16.0, False), (1, 32, 5.0, False), (2, 64, 3.0, True),
+                                          (3, 32, 8.0, True), (3, 32, 16.0, False), (4, 32, 16.0, True), (1, 128, 3.0, True),
+                                          (1, 32, 3.0, True), (1, 16, 8.0, True), (8, 128, 16.0, False)])
+def test_the_forcing_passes_are_joined_where_that_is_faster(n, g, kmax, one):
+    h = Host()
+    if n == 1:
+        ctx = h.lib.glm_create(16, 16, 16, 8)
+        assert h.lib.glm_ou_setup(ctx, g, 1.0, kmax, 0.5, 100, 0.0, 1.0, 7) == 0
+        assert h.lib.glm_ou_advance(ctx) == 0
+        h.lib.glm_destroy(ctx)
+    else:
+        bx = boxes(n)
+        for x in bx:
+            x.do_turb, x.g, x.ndt, x.kmin, x.kmax, x.amp = 1, g, 100, 1.0, kmax, 1.0
+        e = ensemble(h, bx)
+        assert h.lib.glm_ens_step(e, 1) == 0
+        h.lib.glm_ens_destroy(e)
+    passes = [re.search(r"ou_pass_[xyz]+", x)[0] for x in h.log() if "ou_pass_" in x]
+    assert passes == (["ou_pass_x", "ou_pass_yz"] if one else ["ou_pass_x", "ou_pass_y", "ou_pass_z"])
